@@ -8,8 +8,10 @@
 //     on key order, so this is the reference's "every block of the own segment, element mask original key
 //     position > query position" with half the tiles and one masked tile instead of all.
 // Work decomposition
-//   A work item is TWO adjacent 128-query blocks of one head, served by one workgroup (8 waves, two per
-//   SIMD): waves 0-3 take the first block, waves 4-7 the second, 32 queries per wave.  A small kernel
+//   A work item is TWO adjacent 128-query blocks of one head, served by one workgroup (4 waves, one per
+//   SIMD): wave w takes queries 32 w .. 32 w + 31 of either block, so that the waves finish a tile together also where
+//   only one block visits it -- above all the item's last tile, the second block's diagonal one, which then takes half a
+//   tile's time.  A small kernel
 //   first merges the two visit lists of every item (ascending key-block indices, own-segment blocks
 //   appended) into one list in HBM; every merged tile is copied ONCE into LDS for both query blocks, which
 //   halves the L2 -> LDS traffic and doubles the time a tile stays in flight.  K and V tiles are
@@ -36,15 +38,14 @@
 //   sums from one more matrix product, ones x P, i.e. of the rounded values; the output is normalised once at
 //   the end.
 // Tile kinds
-//   * fast tiles: a software pipeline over the four 32-key sub-tiles -- S of sub-tile k+1, exponentials
-//     of sub-tile k and P.V of sub-tile k-1 are issued interleaved, LDS fragments are read two slots
-//     ahead.  Exponentials are taken against a LAZY reference maximum: it is not updated per tile; a row
+//   * fast tiles: a software pipeline over the four 32-key sub-tiles in a static schedule (pbs_attn_tile.h): one
+//     matrix instruction, one unit of exponential work, and so on; the next tile's copies go out in between.
+//     Exponentials are taken against a LAZY reference maximum: it is not updated per tile; a row
 //     sum of one tile above 2^14 triggers a uniform rescale (exact, all terms share the reference); an
 //     overflow marks the row and the whole workgroup redoes it without speculation.  The first tile of a
-//     row takes its reference from the exact maximum over its first 32 keys.  The diagonal tile runs the
+//     row takes its reference from the exact maximum over sixteen of its first keys.  The diagonal tile runs the
 //     same pipeline and zeroes the exponentials of keys after the query (key-in-tile > query-in-block).
-//   * careful tiles (a row whose first tile is the diagonal one, and the redo pass): one 32-key sub-tile at a
-//     time, exact running maximum, classic online softmax.
+//   * careful tiles (the redo pass): one 32-key sub-tile at a time, exact running maximum, classic online softmax.
 //   An item's tiles come in the order permuted tiles, own-segment tiles before the diagonal, diagonal tile, and
 //   each kind has a loop of its own (see the loops): one tile body per loop keeps the accumulators in place.
 #include "pbs_attn_tile.h"
@@ -60,7 +61,7 @@ struct AttnArgs {
   const uint16_t* pvt;   // (B*Hq, nb, 128, 128) permuted V blocks, transposed
   const uint16_t* k;     // original K at the KV heads, caller's strides
   const uint16_t* v;     // original V at the KV heads, caller's strides
-  const uint16_t* plist; // (B*Hq * npair, cap) merged visit lists
+  const uint16_t* plist; // (B*Hq * npair, cap) merged visit lists, in item order
   int* queue;            // 8 work counters, one per XCD
   int cap;               // entries per list row (multiple of 8)
   uint16_t* o;
@@ -74,15 +75,18 @@ struct AttnArgs {
 
 typedef const __attribute__((address_space(4))) struct AttnArgs* ArgsPtr;
 
-// ---- merged visit list of a pair of query blocks, built once per pass by its own kernel:
-// row (bh * npair + pair) of `plist`: [0] = number of tiles, [1 ..] = entries kb | ENT_ORIG? | use_first << 14 |
+// ---- merged visit list of a pair of query blocks, built once per pass by its own kernel.  Row `item` of `plist` (items
+// are numbered head by head, the long pairs of a head first) starts with a header that saves the attention kernel its
+// divisions -- [0] number of tiles, [1] batch, [2] query head, [3] KV head, [4] first query block -- and holds from
+// LIST_HEADER on entries kb | ENT_ORIG? | use_first << 14 |
 // use_second << 15: the union of the two visit lists (ascending), then the own segments in ORIGINAL key order
 // (blocks first-of-segment .. query block, shared where the two blocks share a segment).  Block 0 also clears
 // the work counters of the attention kernel that follows on the stream.
+constexpr int LIST_HEADER = 8;
 constexpr int MERGE_THREADS = 256;
 __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const int32_t* __restrict__ cols, const int32_t* __restrict__ cnt,
                                                                uint16_t* __restrict__ plist, int* __restrict__ queue, int nb,
-                                                               int bps, int cap, const uint8_t* __restrict__ own_needed) {
+                                                               int bps, int cap, int Hq, int group, const uint8_t* __restrict__ own_needed) {
   __shared__ uint8_t flags0[4096], flags1[4096];
   __shared__ int wsum[MERGE_THREADS / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -134,10 +138,19 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
     if (x < wave) w += ws;
     total += ws;
   }
-  uint16_t* out = plist + (int64_t)blockIdx.x * cap;
+  uint16_t* out = plist + ((int64_t)bh * npair + (npair - 1 - pair)) * cap;
+  if (tid == 0) {
+    const int h = bh % Hq;
+    out[1] = (uint16_t)(bh / Hq);
+    out[2] = (uint16_t)h;
+    out[3] = (uint16_t)(h / group);
+    out[4] = (uint16_t)(2 * pair);
+  }
+  uint16_t* const header = out;
+  out += LIST_HEADER;
   for (int kb = k0; kb < k1; ++kb) {
     const int f = flags0[kb] | flags1[kb];
-    if (f) out[1 + w++] = (uint16_t)(kb | (f << 14));
+    if (f) out[w++] = (uint16_t)(kb | (f << 14));
   }
   const int qb0 = 2 * pair, qb1 = second ? qb0 + 1 : qb0;
   const int sf0 = (qb0 / bps) * bps, sf1 = (qb1 / bps) * bps;
@@ -146,23 +159,23 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
     // one-block segments with an optional diagonal: a query block's own block is listed only where its flag is set
     if (tid == 0) {
       int n = total;
-      if (own_needed[(int64_t)bh * nb + qb0]) out[1 + n++] = (uint16_t)(qb0 | ENT_ORIG | (1u << 14));
-      if (second && own_needed[(int64_t)bh * nb + qb1]) out[1 + n++] = (uint16_t)(qb1 | ENT_ORIG | (2u << 14));
+      if (own_needed[(int64_t)bh * nb + qb0]) out[n++] = (uint16_t)(qb0 | ENT_ORIG | (1u << 14));
+      if (second && own_needed[(int64_t)bh * nb + qb1]) out[n++] = (uint16_t)(qb1 | ENT_ORIG | (2u << 14));
       // every list ends with an own-segment entry: a pair with neither own block listed gets the first one's, used by
       // neither query block.  The attention kernel's item protocol -- first tile in flight, claim and hand-over of the
       // next item at the last tiles -- then needs no empty case and none where a permuted tile ends the item; a query
       // block that used no tile writes zeros
-      if (n == total) out[1 + n++] = (uint16_t)(qb0 | ENT_ORIG);
-      out[0] = (uint16_t)n;
+      if (n == total) out[n++] = (uint16_t)(qb0 | ENT_ORIG);
+      header[0] = (uint16_t)n;
     }
     return;
   }
   for (int t = tid; t < n_own; t += MERGE_THREADS) {
     const int kb = sf0 + t;
     const int f = (kb <= qb0 ? 1 : 0) | ((second && kb >= sf1) ? 2 : 0);
-    out[1 + total + t] = (uint16_t)(kb | ENT_ORIG | (f << 14));
+    out[total + t] = (uint16_t)(kb | ENT_ORIG | (f << 14));
   }
-  if (tid == 0) out[0] = (uint16_t)(total + n_own);
+  if (tid == 0) header[0] = (uint16_t)(total + n_own);
 }
 
 // Ticket t of the counter of a range of `count` items starting at `begin` -> work item.  Items are numbered head by
@@ -186,21 +199,21 @@ __device__ __forceinline__ void stage_list_async(const uint16_t* src, int chunks
   const uint32_t src_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)src0);
   const uint32_t src_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(src0 >> 32));
   const uint64_t srcu = ((uint64_t)src_hi << 32) | (uint64_t)src_lo;
-  for (int p = 0; p * 512 < chunks; ++p) {
-    const int chunk = p * 512 + tid;
+  for (int p = 0; p * THREADS < chunks; ++p) {
+    const int chunk = p * THREADS + tid;
     const uint32_t voff = (uint32_t)chunk * 16u;
     if (chunk < chunks) {
-      register uint32_t m0v asm("m0") = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_byte + p * 8192 + wave * 1024));
-      asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(voff), "s"(srcu) : "memory");
+      register uint32_t m0v asm("m0") = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_byte + p * (THREADS * 16) + wave * 1024));
+      asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(voff), "s"(srcu) : "memory");   // (wait states: see copy_tile_now)
     }
   }
 }
 
-__global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
+__global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // starts at LDS offset 0
+  RESERVE_ACC_REGS();
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int grp = wave >> 2, wq = wave & 3;
-
+  
   // Work items = (head, pair of query blocks), ordered head by head with the long rows of a head first and cut
   // into eight contiguous ranges of about equal work, one per XCD (blockIdx % 8): an XCD works through one
   // head at a time, so its resident workgroups walk the same permuted K/V stream at about the same pace and
@@ -237,52 +250,80 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
   int nxt = q_end;   // the next item is claimed late in the current one: an item claimed early waits for this
                      // workgroup while others may be idle
   bool has_nxt = false;
-  const uint32_t use_bit = 1u << (14 + grp);
 
-  // base pointers of one head's tiles: permuted K, permuted V^T, original K rows, original-order V^T
-  struct HeadBase {
+  // an item's coordinates, from the header of its list in LDS, and the base pointers of its head's tiles: permuted K,
+  // permuted V^T, original K and V rows
+  struct Item {
+    int n_tiles, b, h, qb0;
     const uint16_t *pk, *pvt, *korig, *vorig;
     uint32_t k_ss, v_ss;
     int S;
   };
-  auto head_base = [&](ArgsPtr ap, int bh_e) __attribute__((always_inline)) {
-    HeadBase hb;
-    const int Hq_e = ap->Hq, Hkv_e = ap->Hkv, nb_e = ap->nb;
-    const int b_e = bh_e / Hq_e, kvh = (bh_e % Hq_e) / (Hq_e / Hkv_e);
-    hb.pk = ap->pk + (int64_t)bh_e * nb_e * BS * D;
-    hb.pvt = ap->pvt + (int64_t)bh_e * nb_e * BS * D;
-    hb.korig = ap->k + b_e * ap->k_sb + kvh * ap->k_sh;
-    hb.vorig = ap->v + b_e * ap->v_sb + kvh * ap->v_sh;
-    hb.k_ss = ap->k_ss;
-    hb.v_ss = ap->v_ss;
-    hb.S = ap->S;
-    return hb;
+  auto read_item = [&](ArgsPtr ap, const uint16_t* list) __attribute__((always_inline)) {
+    Item t;
+    const u32x4 hd = *reinterpret_cast<const u32x4*>(list);
+    const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)hd[0]), w1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)hd[1]);
+    t.n_tiles = (int)(w0 & 0xffffu);
+    t.b = (int)(w0 >> 16);
+    t.h = (int)(w1 & 0xffffu);
+    t.qb0 = (int)__builtin_amdgcn_readfirstlane((int)hd[2]) & 0xffff;
+    const int64_t tiles = (int64_t)(t.b * ap->Hq + t.h) * ap->nb * (BS * D), kvh = (int)(w1 >> 16);
+    t.pk = ap->pk + tiles;
+    t.pvt = ap->pvt + tiles;
+    t.korig = ap->k + t.b * ap->k_sb + kvh * ap->k_sh;
+    t.vorig = ap->v + t.b * ap->v_sb + kvh * ap->v_sh;
+    t.k_ss = ap->k_ss;
+    t.v_ss = ap->v_ss;
+    t.S = ap->S;
+    return t;
   };
-  // copy of one visit-list entry's K and V^T tiles into the buffers at LDS byte offset `buf`
-  auto stage_entry = [&](const HeadBase& hb, uint32_t e, uint32_t buf, int lane, uint32_t lane_off) __attribute__((always_inline)) {
-    const int kb_e = (int)(e & ENT_KB);
-    if (PBS_UNLIKELY(e & ENT_ORIG)) {
-      // the lane id is formed afresh: offsets derived from the item's one are loop invariants that get hoisted out of
-      // the tile loop and, when registers run out there, spilled and reloaded per tile
-      stage_krows_async(hb.korig + (int64_t)kb_e * BS * hb.k_ss, hb.k_ss, hb.S - kb_e * BS, buf, wave, lane_id_here());
-      stage_vrows_async(hb.vorig + (int64_t)kb_e * BS * hb.v_ss, hb.v_ss, hb.S - kb_e * BS, LDS_V0 + buf, wave, lane_id_here());
+  auto first_entry = [&](const uint16_t* list) __attribute__((always_inline)) {
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)list[LIST_HEADER]);
+  };
+  // Aims the tile copy at the tile of list entry `e`, into the buffers at LDS byte offset `buf`: the addresses here, and
+  // where the kind of tile changes the per-lane offsets (16 registers).  The copy in hand at a tile's head is always the
+  // one that fetched that tile, so the tile loops, which run over tiles of one kind, leave the offsets alone: written
+  // under a branch of such a loop they would be copied twice per tile.
+  TileCopy copy;
+  auto aim_perm = [&](const Item& t, uint32_t e, uint32_t buf) __attribute__((always_inline)) {
+    const int64_t tile = (int64_t)(e & ENT_KB) * (BS * D);
+    copy.lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(buf + (uint32_t)wave * 8192u));
+    copy.k = uniform64((uint64_t)(uintptr_t)(t.pk + tile) - COPY_BIAS);
+    copy.v = uniform64((uint64_t)(uintptr_t)(t.pvt + tile) - COPY_BIAS);
+  };
+  auto aim_rows = [&](const Item& t, uint32_t e, uint32_t buf) __attribute__((always_inline)) {
+    const int64_t row = (int64_t)(e & ENT_KB) * BS;
+    copy.lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(buf + (uint32_t)wave * 8192u));
+    copy.k = uniform64((uint64_t)(uintptr_t)(t.korig + row * t.k_ss) - COPY_BIAS);
+    copy.v = uniform64((uint64_t)(uintptr_t)(t.vorig + row * t.v_ss) - COPY_BIAS);
+  };
+  auto rows_of = [&](const Item& t, uint32_t e) __attribute__((always_inline)) { return t.S - (int)(e & ENT_KB) * BS; };   // >= 128 but for the last block
+  auto aim_anew = [&](const Item& t, uint32_t e, uint32_t buf) __attribute__((always_inline)) {
+    // the lane ids are formed afresh: what is derived from the item's one gets hoisted out of the tile loops
+    if (e & ENT_ORIG) {
+      aim_rows(t, e, buf);
+      copy_offsets_rows(copy, t.k_ss, t.v_ss, rows_of(t, e), wave, lane_id_here());
     } else {
-      // the first wave of every SIMD issues its own share and that of the SIMD's second wave (rows 16 further: the
-      // same chunk, 4096 bytes on), which goes straight on to the matrix instructions of the current tile: the copy
-      // instructions of a tile then queue behind the barrier in four waves instead of eight
-      if (wave < 4) {
-        const uint16_t* ks = hb.pk + (int64_t)kb_e * BS * D;
-        const uint16_t* vs = hb.pvt + (int64_t)kb_e * BS * D;
-        stage_tile_async(ks, buf, wave, lane_off ^ k_copy_xor(wave));
-        stage_tile_async(ks, buf, wave + 4, (lane_off + 4096u) ^ k_copy_xor(wave + 4));
-        stage_tile_async(vs, LDS_V0 + buf, wave, lane_off);
-        stage_tile_async(vs, LDS_V0 + buf, wave + 4, lane_off + 4096u);
-      }
+      aim_perm(t, e, buf);
+      copy_offsets_perm(copy, wave, lane_id_here());
     }
   };
-  auto list_row = [&](ArgsPtr ap, int item) __attribute__((always_inline)) {
-    const int bh_i = item / npair, pair_i = npair - 1 - item % npair;
-    return ap->plist + ((int64_t)bh_i * npair + pair_i) * ap->cap;
+  auto list_row = [&](ArgsPtr ap, int item) __attribute__((always_inline)) { return ap->plist + (int64_t)item * ap->cap; };
+  // an item's Q^T fragments (B operand): column i16 of group qg is query 32 wave + 16 (qg % 2) + i16 of block qg / 2,
+  // d = 32 kd + 8 g4 + 0..7.  Rows past the end of the sequence compute on the last row's values and are never stored.
+  auto load_q = [&](ArgsPtr aq, const Item& t, auto set) __attribute__((always_inline)) {
+    const int ln = lane_id_here();
+    const int64_t q_ss = aq->q_ss;
+    const uint16_t* qhead = aq->q + t.b * aq->q_sb + t.h * aq->q_sh + 8 * (ln >> 4);
+    const int last = t.S - 1, pos0 = t.qb0 * BS + 32 * wave + (ln & 15);
+    static_for<QG>([&](auto qc) __attribute__((always_inline)) {
+      constexpr int qg = decltype(qc)::value, st = decltype(set)::value;
+      const uint16_t* qrow = qhead + (int64_t)min(pos0 + (qg >> 1) * BS + (qg & 1) * 16, last) * q_ss;
+      q_load<qg, 0, st>(qrow);
+      q_load<qg, 1, st>(qrow + 32);
+      q_load<qg, 2, st>(qrow + 64);
+      q_load<qg, 3, st>(qrow + 96);
+    });
   };
 
   // the first item's list, then its first tile
@@ -292,18 +333,20 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
   uint32_t li = 0;        // which list buffer holds the current item's list
   uint32_t par = 0;       // which tile buffers hold the current item's first tile (0 or 0x8000)
   {
-    stage_entry(head_base(a0, cur / npair), (uint32_t)__builtin_amdgcn_readfirstlane((int)reinterpret_cast<const uint16_t*>(smem + LDS_LIST)[1]), 0u,
-                (int)threadIdx.x & 63, async_lane_offset(wave, (int)threadIdx.x & 63));
+    const uint16_t* list0 = reinterpret_cast<const uint16_t*>(smem + LDS_LIST);
+    aim_anew(read_item(a0, list0), first_entry(list0), 0u);
   }
+  copy_tile_now(copy);
 
   bool careful_only = false;   // the current pass repeats an item without speculation
+  bool q_ready = false;        // the item's queries have been loaded ahead
+  bool stores_out = false;     // the previous item's last sixteen vector memory operations are its output stores
   for (;;) {
     const uint16_t* mlist = reinterpret_cast<const uint16_t*>(smem + LDS_LIST + li * LIST_BYTES);
     const uint16_t* nlist = reinterpret_cast<const uint16_t*>(smem + LDS_LIST + (li ^ 1u) * LIST_BYTES);
     ArgsPtr ap = PBS_ARGS();
     // everything per lane is derived afresh from the lane id in every item: nothing but scalars lives across items
     const int lane = lane_id_here();
-    const int tid = wave * 64 + lane;
     const int i16 = lane & 15, g4 = lane >> 4;
     // per-lane LDS byte offsets of the fragments inside buffer 0; XOR 0x8000 switches buffer.
     //   K fragment (sub-tile ks, row tile T, d-step kd) : (koff0 ^ kd << 6) + T * 1024 + ks * 8192
@@ -320,30 +363,20 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
       ka[n] = koff0 ^ (uint32_t)(n << 6) ^ par;
       va[n] = voff0 ^ (uint32_t)(n << 6) ^ par;
     }
-    const uint32_t lane_off = async_lane_offset(wave, lane);
     int claim = 0;   // ticket of the next item: in flight during one tile
 
-    const int bh = cur / npair;
-    const int pair = npair - 1 - cur % npair;
-    const HeadBase hb = head_base(ap, bh);
-    const int b = bh / ap->Hq, h = bh % ap->Hq;
-    const int qb = 2 * pair + grp;
-    const bool qb_valid = qb < ap->nb;
+    const Item hb = read_item(ap, mlist);
+    const int qb0 = hb.qb0, n_tiles = hb.n_tiles;
     const float c_log2 = ap->scale_log2;
-    const int qpos = qb * BS + 32 * wq + i16;
 
-    // Q^T fragments (B operand): query column 16 qg + i16, d = 32 kd + 8 g4 + 0..7.  Rows past the end of the
-    // sequence compute on the last row's values and are never stored.
-    bf16x8 qf[2][4];
-#pragma unroll
-    for (int qg = 0; qg < 2; ++qg) {
-      const uint16_t* qrow = ap->q + b * ap->q_sb + h * ap->q_sh + (int64_t)min(qpos + 16 * qg, ap->S - 1) * ap->q_ss;
-#pragma unroll
-      for (int kd = 0; kd < 4; ++kd) qf[qg][kd] = *reinterpret_cast<const bf16x8*>(qrow + 32 * kd + 8 * g4);
+    // the item's queries: loaded ahead at the previous item's last tile, or from here (they are complete at the wait for
+    // the first tile's copies)
+    if (!careful_only) {
+      if (q_ready) q_advance();
+      else load_q(ap, hb, std::integral_constant<int, 0>{});
     }
-    const int n_tiles = __builtin_amdgcn_readfirstlane((int)mlist[0]);
     // the next item: claimed three tiles before the end of this one (the counter's latency passes under a
-    // tile), published and its list and queries requested one tile later, its first tile requested at the last
+    // tile), published and its list requested one tile later, its queries and its first tile requested at the last
     // tile.  Items of fewer than three tiles finish these steps after their loop.
     const int claim_it = careful_only ? -8 : max(n_tiles - 3, 0);
     auto publish_and_fetch = [&]() __attribute__((always_inline)) {   // between the wait for this thread's loads and the barrier ...
@@ -352,54 +385,35 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
     auto adopt_next = [&]() __attribute__((always_inline)) {          // ... and after the barrier
       nxt = ticket_item(q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]), PBS_ARGS()->interleave, npair);
       has_nxt = nxt < q_end;
-      if (has_nxt) {
-        ArgsPtr an = PBS_ARGS();
-        const int ln = lane_id_here();
-        stage_list_async(list_row(an, nxt), an->cap >> 3, LDS_LIST + (li ^ 1u) * LIST_BYTES, wave, wave * 64 + ln);
-        // the next item's queries are read once, from HBM: bring this wave's 32 rows into L2 now (copies into a
-        // landing area nobody reads), so that the loads at the top of the item find them there
-        const int bh_n = nxt / npair, qb_n = 2 * (npair - 1 - nxt % npair) + grp;
-        const int pos0 = qb_n * BS + 32 * wq;
-        if (pos0 + 32 <= an->S) {
-          const int64_t q_ss = an->q_ss;
-          const uint16_t* qn = an->q + (bh_n / an->Hq) * an->q_sb + (bh_n % an->Hq) * an->q_sh + (int64_t)pos0 * q_ss;
-          const uint32_t voff = (uint32_t)((ln >> 4) * (uint32_t)q_ss * 2u + (ln & 15) * 16u);
-#pragma unroll
-          for (int n = 0; n < 8; ++n) {
-            const uint64_t base = (uint64_t)(uintptr_t)(qn + 4 * n * q_ss);
-            const uint32_t b_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base);
-            const uint32_t b_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32));
-            const uint64_t bu = ((uint64_t)b_hi << 32) | b_lo;
-            register uint32_t m0v asm("m0") = (uint32_t)__builtin_amdgcn_readfirstlane((int)(LDS_DUMP + wave * 1024));
-            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(voff), "s"(bu) : "memory");
-          }
-        }
-      }
+      if (has_nxt)
+        stage_list_async(list_row(PBS_ARGS(), nxt), PBS_ARGS()->cap >> 3, LDS_LIST + (li ^ 1u) * LIST_BYTES, wave, wave * 64 + lane_id_here());
+    };
+    // the next item's queries and first tile, once its list has landed
+    auto aim_at_next = [&](uint32_t buf) __attribute__((always_inline)) {
+      ArgsPtr an = PBS_ARGS();
+      const Item t = read_item(an, nlist);
+      load_q(an, t, std::integral_constant<int, Q_NEXT>{});
+      aim_anew(t, first_entry(nlist), buf);
     };
 
     {
-      f32x4 o[8][2];   // [d tile][query column group]
-      {
-        float zero = 0.f;   // opaque: a constant zero vector would be kept (and spilled) as registers of its own
-        asm volatile("" : "+v"(zero));
+      o_clear();
+      float m_ref[QG], l_row[QG];   // reference maxima and row sums of queries 16 qg + i16, identical in the four lanes i16 + 16 g
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-          for (int qg = 0; qg < 2; ++qg)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[dt][qg][r] = zero;
+      for (int qg = 0; qg < QG; ++qg) {
+        m_ref[qg] = -INFINITY;
+        l_row[qg] = 0.f;
       }
-      float m_ref[2] = {-INFINITY, -INFINITY};   // reference maxima of queries i16 and 16 + i16, identical in the four lanes i16 + 16 g
-      float l_row[2] = {0.f, 0.f};               // row sums of queries i16 and 16 + i16, identical in the four lanes too
-      bool first = true, poisoned = false;
-      bool all_seen = false;     // every query of this wave has a finite reference maximum (wave-uniform)
+      bool poisoned = false;
+      uint32_t unseen = 3u << 14;   // use bits of the query blocks that have seen no tile yet (their reference is still -inf)
 
       if (careful_only) {
         // the redo pass starts the item over: its first tile goes back into the buffers it had (the next
         // item's first tile, if it was on its way there, is fetched again at the end of this pass)
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
-        stage_entry(hb, (uint32_t)__builtin_amdgcn_readfirstlane((int)mlist[1]), par, lane, lane_off);
+        aim_anew(hb, first_entry(mlist), par);
+        copy_tile_now(copy);
       }
       uint32_t bufx = par;
       auto next_buffers = [&]() __attribute__((always_inline)) {
@@ -410,87 +424,86 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
           va[n] ^= 0x8000u;
         }
       };
-      // what every tile starts with: wait for its copies, hand over the buffers of the tile before, and request the
-      // copies of the tile after it (or, at the last tile, of the next item's first tile)
-      uint32_t e_cur = (uint32_t)__builtin_amdgcn_readfirstlane((int)mlist[1]);   // the entry of the current tile
-      uint32_t e_nxt = 0;                                                        // of the next one, set by tile_head
-      uint16_t e_ahead = mlist[2];                                               // per lane, not yet made uniform
-      // `may_be_last`: the item's last tile is an own-segment tile (merge_pair_lists_kernel ends every list with one),
-      // so the loop over the permuted tiles always has a next entry to request and carries no code for the next item's
-      // first tile
-      auto tile_head = [&](int it, auto may_be_last) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this thread's share of tile `it` (and of the next list) has landed
+      // a tile's copies are awaited at the end of the tile before it.  Vector memory operations complete in order, so
+      // behind an item's first tile (and its queries) the previous item's stores may still be on their way
+      auto wait_copies = [&]() __attribute__((always_inline)) { __builtin_amdgcn_s_waitcnt(0x0f70); };   // vmcnt(0)
+      if (stores_out) __builtin_amdgcn_s_waitcnt(0x4f70);   // vmcnt(16)
+      else wait_copies();
+      uint32_t e_cur = first_entry(mlist);         // the entry of the current tile
+      uint32_t e_nxt = 0;                          // of the next one, set by tile_head
+      uint16_t e_ahead = mlist[LIST_HEADER + 1];   // per lane, not yet made uniform
+      // what every tile starts with: hand over the buffers of the tile before
+      auto tile_head = [&](int it) __attribute__((always_inline)) {
         if (PBS_UNLIKELY(it == claim_it + 1)) publish_and_fetch();
-        __syncthreads();                      // every share has; every wave is done with tile it - 1
-        if (PBS_UNLIKELY(it == claim_it + 1)) adopt_next();
-        if (PBS_UNLIKELY(it == claim_it) && wave == 0 && lane_id_here() == 0) claim = atomicAdd(PBS_ARGS()->queue + vic, 1);
+        __syncthreads();                      // every wave's share of tile `it` has landed; every wave is done with tile it - 1
+        if (PBS_UNLIKELY((unsigned)(it - claim_it) < 2u)) {
+          if (it != claim_it) adopt_next();
+          else if (wave == 0 && lane_id_here() == 0) claim = atomicAdd(PBS_ARGS()->queue + vic, 1);
+        }
         // the list entries are read from LDS one tile ahead of their use (the read's latency would otherwise sit in
         // front of the copy requests of every tile): `e_ahead` holds entry it + 1, requested at the tile before
         e_nxt = (uint32_t)__builtin_amdgcn_readfirstlane((int)e_ahead);
-        e_ahead = mlist[3 + it];
-        if (!decltype(may_be_last)::value || PBS_LIKELY(it + 1 < n_tiles))
-          stage_entry(hb, e_nxt, bufx ^ 0x8000u, lane, lane_off);
-        else if (has_nxt && (careful_only || n_tiles >= 3))   // shorter items: after the loop, once the list has landed
-          stage_entry(head_base(PBS_ARGS(), nxt / npair), (uint32_t)__builtin_amdgcn_readfirstlane((int)nlist[1]), bufx ^ 0x8000u, lane, lane_off);
+        e_ahead = mlist[LIST_HEADER + 2 + it];
       };
-      constexpr std::integral_constant<bool, true> any_tile{};
-      constexpr std::integral_constant<bool, false> not_the_last{};
-      // first tile of a row, every key visible: the exact maximum over its first 32 keys is a good enough reference
-      // to start the pipelined path (later keys move it up lazily)
-      auto first_reference = [&]() __attribute__((always_inline)) {
-        first = false;
-        float mx[2] = {-INFINITY, -INFINITY};
+      // at the item's last tile: the next item's first tile
+      auto aim_past_item = [&]() __attribute__((always_inline)) {
+        if (has_nxt && (careful_only || n_tiles >= 3)) aim_at_next(bufx ^ 0x8000u);   // shorter items: after the loop, once the list has landed
+        else copy.lds ^= 0x8000u;   // nothing to fetch: the same tile again, into buffers nobody reads (a pipelined tile always copies)
+      };
+      // logits of the 16-key row tile at byte offset `at` of the K buffer against the wave's queries
+      auto logits_of = [&](f32x4 (&s)[QG], int at) __attribute__((always_inline)) {
+        bf16x8 fk[4];
 #pragma unroll
-        for (int T = 0; T < 2; ++T) {
-          f32x4 s0[2] = {(f32x4){0}, (f32x4){0}};
+        for (int kd = 0; kd < 4; ++kd) fk[kd] = ldsf(ka[kd] + at);
+        static_for<4>([&](auto kc) __attribute__((always_inline)) {
+          constexpr int kd = decltype(kc)::value;
+          static_for<QG>([&](auto qc) __attribute__((always_inline)) { mfma_s<decltype(qc)::value, kd, kd == 0>(s[decltype(qc)::value], fk[kd]); });
+        });
+        MFMA_FENCE();
+      };
+      // first tile of a row: the exact maximum over the visible ones of its keys 0-3, 8-11, 16-19 and 24-27 is a good
+      // enough reference to start the pipelined path (later keys move it up lazily); in a diagonal tile every query sees
+      // key 0 at least, so the reference is finite there too
+      auto first_reference = [&](auto masked, uint32_t ent) __attribute__((always_inline)) {
+        f32x4 s0[QG];
+        logits_of(s0, 0);
+        const int ln = lane_id_here();
+        const int qrel8 = 32 * wave + (ln & 15) - 8 * (ln >> 4);
 #pragma unroll
-          for (int kd = 0; kd < 4; ++kd) {
-            const bf16x8 fk = ldsf(ka[kd] + T * 1024);
+        for (int qg = 0; qg < QG; ++qg) {
+          float mx = -INFINITY;
 #pragma unroll
-            for (int qg = 0; qg < 2; ++qg) s0[qg] = PBS_MFMA(fk, qf[qg][kd], s0[qg]);
-          }
-#pragma unroll
-          for (int qg = 0; qg < 2; ++qg)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mx[qg] = fmaxf(mx[qg], s0[qg][r]);
+          for (int r = 0; r < 4; ++r)
+            if (!(decltype(masked)::value >> qg & 1) || r - 16 * (qg & 1) <= qrel8) mx = fmaxf(mx, s0[qg][r]);
+          const float m_new = max_over_lane_groups(mx) * c_log2;
+          if (ent & unseen & (1u << (14 + (qg >> 1)))) m_ref[qg] = m_new;
         }
-#pragma unroll
-        for (int qg = 0; qg < 2; ++qg) m_ref[qg] = max_over_lane_groups(mx[qg]) * c_log2;
-        all_seen = true;
+        unseen &= ~ent;
       };
-      // careful tile: classic online softmax, one 32-key sub-tile at a time.  The redo pass, and a diagonal tile
-      // while some query has not seen a single key yet (its reference maximum is still -inf)
-      auto careful_tile = [&](uint32_t ent, bool masked) __attribute__((always_inline)) {
-        first = false;
+      // careful tile (the redo pass): classic online softmax, one 32-key sub-tile at a time
+      auto careful_tile = [&](uint32_t ent) __attribute__((always_inline)) {
+        MFMA_FENCE();
 #pragma nounroll
         for (int ks = 0; ks < 4; ++ks) {   // a real loop: the rare path stays small, in code and in registers
-          f32x4 s[2][2];   // [T][qg]
+          f32x4 s[2][QG];   // [T][qg]
+          logits_of(s[0], ks * 8192);
+          logits_of(s[1], ks * 8192 + 1024);
+          const int ln = lane_id_here();   // keep the compares inside the tile (see fast_tile)
+          const int qrel8 = 32 * wave + (ln & 15) - 8 * (ln >> 4);
 #pragma unroll
-          for (int T = 0; T < 2; ++T) {
-            s[T][0] = (f32x4){0};
-            s[T][1] = (f32x4){0};
-#pragma unroll
-            for (int kd = 0; kd < 4; ++kd) {
-              const bf16x8 fk = ldsf(ka[kd] + T * 1024 + ks * 8192);
-#pragma unroll
-              for (int qg = 0; qg < 2; ++qg) s[T][qg] = PBS_MFMA(fk, qf[qg][kd], s[T][qg]);
-            }
-          }
-          if (masked) {
-            const int ln = lane_id_here();   // keep the compares inside the tile (see fast_tile)
-            const int qrel8 = 32 * wq + (ln & 15) - 8 * (ln >> 4);
+          for (int qg = 0; qg < QG; ++qg) {
+            const bool used = (ent >> (14 + (qg >> 1))) & 1u;
+            const bool masked = (ent & ENT_ORIG) && (int)(ent & ENT_KB) == qb0 + (qg >> 1);
 #pragma unroll
             for (int T = 0; T < 2; ++T)
 #pragma unroll
-              for (int qg = 0; qg < 2; ++qg)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                  if (32 * ks + 4 * T + r - 16 * qg > qrel8) s[T][qg][r] = -INFINITY;
+              for (int r = 0; r < 4; ++r)
+                if (!used || (masked && 32 * ks + 4 * T + r - 16 * (qg & 1) > qrel8)) s[T][qg][r] = -INFINITY;
           }
-          float alpha[2];
-          bf16x8 pf[2];
+          float alpha[QG];
+          bf16x8 pf[QG];
 #pragma unroll
-          for (int qg = 0; qg < 2; ++qg) {
+          for (int qg = 0; qg < QG; ++qg) {
             float mx = fmaxf(fmaxf(s[0][qg][0], s[0][qg][1]), fmaxf(s[0][qg][2], s[0][qg][3]));
             mx = fmaxf(mx, fmaxf(fmaxf(s[1][qg][0], s[1][qg][1]), fmaxf(s[1][qg][2], s[1][qg][3])));
             mx = max_over_lane_groups(mx);
@@ -507,24 +520,19 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
             }
             l_row[qg] = l_row[qg] * alpha[qg] + sum_over_lane_groups(rs);
           }
-          if (__any(alpha[0] != 1.0f || alpha[1] != 1.0f)) {
-#pragma unroll
-            for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-              for (int qg = 0; qg < 2; ++qg)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o[dt][qg][r] *= alpha[qg];
+          if (__any(alpha[0] != 1.0f || alpha[1] != 1.0f || alpha[2] != 1.0f || alpha[3] != 1.0f)) {
+            static_for<QG>([&](auto qc) __attribute__((always_inline)) { o_scale<decltype(qc)::value>(alpha[decltype(qc)::value]); });
           }
-#pragma unroll
-          for (int dt = 0; dt < 8; ++dt) {
+          MFMA_FENCE();
+          static_for<8>([&](auto dc) __attribute__((always_inline)) {
+            constexpr int dt = decltype(dc)::value;
             const bf16x8 fv = (ent & ENT_ORIG)
                                   ? ldsf_transposed(vrow_lane_addr(LDS_V0 + (va[0] & 0x8000u), lane_id_here()) + dt * 128 + ks * 8192)
                                   : ldsf((va[0] ^ (uint32_t)(ks << 6)) + dt * 4096);
-#pragma unroll
-            for (int qg = 0; qg < 2; ++qg) o[dt][qg] = PBS_MFMA(fv, pf[qg], o[dt][qg]);
-          }
+            static_for<QG>([&](auto qc) __attribute__((always_inline)) { mfma_o<dt, decltype(qc)::value>(fv, pf[decltype(qc)::value]); });
+          });
+          MFMA_FENCE();
         }
-        all_seen = !__any(m_ref[0] == -INFINITY || m_ref[1] == -INFINITY);
       };
       // The merged list holds the permuted tiles of earlier segments first, then the tiles of the own segments in
       // ascending order: for a query block those before its own block, its own (diagonal) block, and -- for the first
@@ -532,38 +540,76 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
       // pass: a loop whose body updates the 64 accumulator registers on one path only keeps them in place, where
       // alternative tile bodies inside one loop cost a copy of all of them per tile (and the registers for it).
       int it = 0;
+      constexpr uint32_t USE0 = 1u << 14, USE1 = 1u << 15;
       if (PBS_UNLIKELY(careful_only)) {
         for (; it < n_tiles; ++it, next_buffers(), e_cur = e_nxt) {
-          tile_head(it, any_tile);
-          if (!(e_cur & use_bit) || !qb_valid) continue;
-          careful_tile(e_cur, (e_cur & ENT_ORIG) && (int)(e_cur & ENT_KB) == qb);
+          tile_head(it);
+          if (it + 1 < n_tiles) aim_anew(hb, e_nxt, bufx ^ 0x8000u);
+          else aim_past_item();
+          copy_tile_now(copy);
+          if (e_cur & (USE0 | USE1)) careful_tile(e_cur);
+          wait_copies();
         }
       } else {
-        for (; it < n_tiles; ++it, next_buffers(), e_cur = e_nxt) {          // permuted tiles
-          if (PBS_UNLIKELY(e_cur & ENT_ORIG)) break;
-          tile_head(it, not_the_last);
-          if (PBS_UNLIKELY(!(e_cur & use_bit) || !qb_valid)) continue;
-          if (PBS_UNLIKELY(first)) first_reference();
-          fast_tile<false, PREFETCH_SLOTS, false>(o, qf, ka, va, c_log2, m_ref, l_row, poisoned, wq);
-        }
-        for (; it < n_tiles; ++it, next_buffers(), e_cur = e_nxt) {          // own-segment tiles before the diagonal: every key visible
-          if ((int)(e_cur & ENT_KB) >= qb) break;
-          tile_head(it, any_tile);
-          if (!(e_cur & use_bit) || !qb_valid) continue;
-          if (first) first_reference();
-          fast_tile<false, PREFETCH_SLOTS, true>(o, qf, ka, va, c_log2, m_ref, l_row, poisoned, wq);
-        }
-        if (it < n_tiles && (int)(e_cur & ENT_KB) == qb) {   // the diagonal tile
-          tile_head(it, any_tile);
-          if ((e_cur & use_bit) && qb_valid) {
-            if (first || !all_seen) careful_tile(e_cur, true);
-            else fast_tile<true, PREFETCH_SLOTS, true>(o, qf, ka, va, c_log2, m_ref, l_row, poisoned, wq);
-          }
+        auto next_tile = [&]() __attribute__((always_inline)) {
           ++it;
           next_buffers();
           e_cur = e_nxt;
+        };
+        auto visit = [&](auto masked, auto v_rows) __attribute__((always_inline)) {
+          if (PBS_UNLIKELY(e_cur & unseen)) first_reference(masked, e_cur);
+          fast_tile<0, decltype(masked)::value, decltype(v_rows)::value>(ka, va, c_log2, e_cur & USE0, e_cur & USE1, m_ref, l_row,
+                                                                         poisoned, wave, copy);
+        };
+        constexpr std::integral_constant<int, 0> all_visible{};
+        constexpr std::integral_constant<int, 3> diagonal0{};
+        // permuted tiles (an item's last tile never is one), the last one apart
+        if (!(e_cur & ENT_ORIG)) {
+          for (;;) {
+            tile_head(it);
+            if (PBS_UNLIKELY(e_nxt & ENT_ORIG)) break;
+            aim_perm(hb, e_nxt, bufx ^ 0x8000u);
+            visit(all_visible, std::false_type{});
+            wait_copies();
+            next_tile();
+          }
+          aim_anew(hb, e_nxt, bufx ^ 0x8000u);
+          visit(all_visible, std::false_type{});
+          wait_copies();
+          next_tile();
         }
-        for (; it < n_tiles; ++it, next_buffers(), e_cur = e_nxt) tile_head(it, any_tile);   // tiles of the pair's other block only
+        // own-segment tiles before the first diagonal: every key visible, a diagonal tile follows; the last one apart
+        if ((int)(e_cur & ENT_KB) < qb0) {
+          for (;;) {
+            tile_head(it);
+            if ((int)(e_nxt & ENT_KB) >= qb0) break;
+            aim_rows(hb, e_nxt, bufx ^ 0x8000u);
+            visit(all_visible, std::true_type{});
+            wait_copies();
+            next_tile();
+          }
+          aim_anew(hb, e_nxt, bufx ^ 0x8000u);
+          visit(all_visible, std::true_type{});
+          wait_copies();
+          next_tile();
+        }
+        if ((int)(e_cur & ENT_KB) == qb0) {   // the first block's diagonal tile, or the place-holder of a pair that uses none
+          tile_head(it);
+          const bool more = it + 1 < n_tiles;
+          if (more) aim_anew(hb, e_nxt, bufx ^ 0x8000u);
+          else aim_past_item();
+          if (e_cur & (USE0 | USE1)) visit(diagonal0, std::true_type{});
+          else copy_tile_now(copy);
+          if (more) wait_copies();
+          next_tile();
+        }
+        if (it < n_tiles) {   // the second block's diagonal tile, which nobody else sees
+          tile_head(it);
+          aim_past_item();
+          if (e_cur & unseen) first_reference(std::integral_constant<int, 12>{}, e_cur);
+          fast_tile<2, 12, true>(ka, va, c_log2, false, true, m_ref, l_row, poisoned, wave, copy);
+          next_tile();
+        }
       }
       if (!careful_only && n_tiles < 3) {
         if (n_tiles < 2) {
@@ -574,68 +620,66 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
         }
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
-        if (has_nxt)
-          stage_entry(head_base(PBS_ARGS(), nxt / npair), (uint32_t)__builtin_amdgcn_readfirstlane((int)nlist[1]), bufx, lane, lane_off);
+        if (has_nxt) {
+          aim_at_next(bufx);
+          copy_tile_now(copy);
+        }
       }
       if (poisoned) misc[1] = 1;
       __syncthreads();   // every wave is done with the last tile
       if (!careful_only && misc[1] != 0) {   // the whole workgroup redoes both rows without speculation
         careful_only = true;
+        stores_out = false;
         continue;
       }
 
-      // ---- epilogue: normalise, transpose through LDS (same swizzle), coalesced 16-byte stores.  The staging
-      // area is the pair of buffers the last tile sat in (the other pair is receiving the next item's first
-      // tile): its K buffer for the first query block, its V buffer for the second.
+      // ---- epilogue: normalise, transpose through LDS (rows of 16 chunks of 16 bytes, chunk XOR row % 16), coalesced
+      // stores of four whole rows each.  The staging area is the pair of buffers the last tile sat in (the other pair is
+      // receiving the next item's first tile), 16 KB per wave: no barrier, the next one hands the buffers on.
       // a query block that used no tile (no selected block and no own block: possible only with an optional diagonal)
       // has a zero sum and writes zeros, as the reference does for a row without selected blocks
-      float inv[2];
+      MFMA_FENCE();
+      float inv[QG];
 #pragma unroll
-      for (int qg = 0; qg < 2; ++qg) {
+      for (int qg = 0; qg < QG; ++qg) {
         const float l_all = l_row[qg];
         inv[qg] = l_all == 0.f ? 0.f : 1.0f / l_all;
       }
       // lane-dependent addresses of the epilogue come from a fresh opaque lane id: derived from the item's one
       // they would be computed at the top of the item and held across the tile loop
       const int lane_e = lane_id_here();
-      const int i_e = lane_e & 15, g_e = lane_e >> 4;
-      const uint32_t last_buf = par ^ (((n_tiles - 1) & 1) ? 0x8000u : 0u);
-      uint16_t* os = reinterpret_cast<uint16_t*>(smem + last_buf + (grp ? LDS_V0 : 0u));
+      const uint32_t stage = (par ^ (((n_tiles - 1) & 1) ? 0x8000u : 0u)) + (wave >> 1 ? LDS_V0 : 0u) + (wave & 1) * 16384u;
+      uint8_t* wr = smem + stage + (lane_e & 15) * 256 + ((lane_e >> 4) & 1) * 8;
+      const int wr_c = (lane_e >> 5) ^ (lane_e & 15);      // chunk of d tile 0, swizzled; d tile dt: ^ 2 dt
+      static_for<8 * QG>([&](auto ic) __attribute__((always_inline)) {
+        constexpr int dt = decltype(ic)::value % 8, qg = decltype(ic)::value / 8;
+        const f32x4 o4 = o_get<dt, qg>();
+        bf16x4 v4;
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt)
+        for (int cc = 0; cc < 4; ++cc) v4[cc] = (__bf16)(o4[cc] * inv[qg]);
+        *reinterpret_cast<bf16x4*>(wr + qg * 4096 + ((wr_c ^ (2 * dt)) * 16)) = v4;
+      });
+      ArgsPtr ae = PBS_ARGS();
+      const int64_t o_ss = ae->o_ss;
+      const int pos0 = qb0 * BS + 32 * wave + (lane_e >> 4);      // this lane's first row
+      uint16_t* obase = ae->o + hb.b * ae->o_sb + hb.h * ae->o_sh + pos0 * o_ss + (lane_e & 15) * 8;
+      const uint8_t* rd = smem + stage + (lane_e >> 4) * 256;
+      const bool full = (qb0 + 2) * BS <= hb.S;
+      auto out_rows = [&](auto all) __attribute__((always_inline)) {
 #pragma unroll
-        for (int qg = 0; qg < 2; ++qg) {
-          const int row = 32 * wq + 16 * qg + i_e;
-          const int c = 2 * dt + (g_e >> 1);   // 16-byte chunk of d = 16 dt + 4 g + 0..3
-          bf16x4 v4;
-#pragma unroll
-          for (int cc = 0; cc < 4; ++cc) v4[cc] = (__bf16)(o[dt][qg][cc] * inv[qg]);
-          *reinterpret_cast<bf16x4*>(os + row * D + ((c ^ (row & 15)) * 8) + 4 * (g_e & 1)) = v4;
+        for (int n = 0; n < 16; ++n) {              // rows 4 n .. 4 n + 3 of the wave's 64: n < 8 of the first block
+          const int row = 4 * n + (lane_e >> 4), rel = (n >> 3) * BS + 4 * (n & 7);
+          if (decltype(all)::value || pos0 + rel < hb.S)
+            *reinterpret_cast<u32x4*>(obase + rel * o_ss) = *reinterpret_cast<const u32x4*>(rd + n * 1024 + (((lane_e & 15) ^ (row & 15)) * 16));
         }
-      __syncthreads();
-      if (qb_valid) {
-        ArgsPtr ae = PBS_ARGS();
-        const int bh_e = cur / npair;
-        uint16_t* obase = ae->o + (bh_e / ae->Hq) * ae->o_sb + (bh_e % ae->Hq) * ae->o_sh;
-        const int S_e = ae->S;
-        const int64_t o_ss = ae->o_ss;
-        // the query block index is rebuilt from the thread id here: keeping it alive across the tile loop
-        // costs a register the loop does not have
-        const int tid_e = wave * 64 + lane_e;
-        const int qb_e = 2 * (npair - 1 - cur % npair) + (tid_e >> 8);
-        const int t256 = tid_e & 255;
-        const uint16_t* os_e = reinterpret_cast<const uint16_t*>(smem + last_buf + ((tid_e >> 8) ? LDS_V0 : 0u));
-#pragma unroll
-        for (int n = 0; n < 8; ++n) {
-          const int ci = t256 + 256 * n;
-          const int row = ci >> 4, c = ci & 15;
-          const int pos = qb_e * BS + row;
-          if (pos < S_e)
-            *reinterpret_cast<u32x4*>(obase + (int64_t)pos * o_ss + c * 8) =
-                *reinterpret_cast<const u32x4*>(os_e + row * D + ((c ^ (row & 15)) * 8));
-        }
-      }
+      };
+      // both blocks whole: every lane stores sixteen times 16 bytes, i.e. at least sixteen vector memory operations follow
+      // the copies of the next item's first tile, which `stores_out` relies on
+      if (PBS_LIKELY(full)) out_rows(std::true_type{});
+      else out_rows(std::false_type{});
+      stores_out = full;
     }
+    bool stolen = false;
     if (!has_nxt) {
       // the range is used up: serve the other XCDs' ranges, one after the other.  No look-ahead on this path:
       // claim, fetch the list, request the first tile, each after the other
@@ -655,14 +699,17 @@ __global__ __launch_bounds__(512, 2) void sparse_attn_kernel(AttnArgs a) {
         }
       }
       if (has_nxt) {
+        stolen = true;
         stage_list_async(list_row(as, nxt), as->cap >> 3, LDS_LIST + (li ^ 1u) * LIST_BYTES, wave, wave * 64 + lane_id_here());
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
-        stage_entry(head_base(as, nxt / npair), (uint32_t)__builtin_amdgcn_readfirstlane((int)nlist[1]),
-                    par ^ ((n_tiles & 1) ? 0x8000u : 0u), lane, lane_off);
+        aim_anew(read_item(as, nlist), first_entry(nlist), par ^ ((n_tiles & 1) ? 0x8000u : 0u));
+        copy_tile_now(copy);
       }
     }
     if (!has_nxt) break;
+    q_ready = !stolen;
+    if (stolen) stores_out = false;
     careful_only = false;
     par ^= (n_tiles & 1) ? 0x8000u : 0u;
     li ^= 1u;
@@ -678,9 +725,9 @@ std::atomic<int> g_cu_count[64];           // CUs of device d (0: not looked up 
 
 }  // namespace
 
-// entries per merged list row (a multiple of 8: rows stay 16-byte aligned): the count, at most nb blocks of
+// uint16 per merged list row (a multiple of 8: rows stay 16-byte aligned): the header, at most nb blocks of
 // earlier segments, at most bps + 1 own-segment blocks
-static int list_cap(int nb, int bps) { return (1 + nb + std::min(bps, nb) + 1 + 7) / 8 * 8; }
+static int list_cap(int nb, int bps) { return (LIST_HEADER + nb + std::min(bps, nb) + 1 + 7) / 8 * 8; }
 
 // workspace: 256 bytes of work counters, then one merged visit list per pair of query blocks
 
@@ -749,7 +796,7 @@ static int sparse_attn_launch(const void* q, const void* perm_k, const void* per
   PBS_REQUIRE(a.nb <= 4096, "pbs_sparse_attn_fwd: more than 4096 blocks per sequence (%d)", a.nb);
   // eight ranges of equal estimated work: the row pair p of a head costs about p + 1 (causal length)
   const int64_t npair = (a.nb + 1) / 2;
-  PBS_REQUIRE((int64_t)a.BH * npair < (1ll << 28), "pbs_sparse_attn_fwd: launch too large");
+  PBS_REQUIRE((int64_t)a.BH * npair < (1ll << 28) && B < 65536 && Hq < 65536, "pbs_sparse_attn_fwd: launch too large");
   const double head_work = 0.5 * (double)npair * (double)(npair + 1);
   int max_items = 0;
   for (int x = 0; x <= 8; ++x) {
@@ -803,7 +850,7 @@ static int sparse_attn_launch(const void* q, const void* perm_k, const void* per
     return (int)attr;
   }
   hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * npair)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
-                     (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.bps, a.cap, own_block_needed);
-  hipLaunchKernelGGL(sparse_attn_kernel, dim3((unsigned)n_wg), dim3(512), LDS_TOTAL, (hipStream_t)stream, a);
+                     (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.bps, a.cap, Hq, Hq / Hkv, own_block_needed);
+  hipLaunchKernelGGL(sparse_attn_kernel, dim3((unsigned)n_wg), dim3(THREADS), LDS_TOTAL, (hipStream_t)stream, a);
   return pbs_check_launch("pbs_sparse_attn_fwd");
 }

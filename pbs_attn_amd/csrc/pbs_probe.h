@@ -15,7 +15,7 @@ int pbs_mfma_probe(const void* operands, int iters, int shape_32x32x16, float* s
 double pbs_mfma_probe_flop(int iters);
 
 /* the attention kernel's tile pipeline alone.  256
- * workgroups of 8 waves each run `iters` unmasked 128-key tiles for their 256 queries (2 x 128 x 128 block pairs
+ * workgroups of 4 waves each run `iters` unmasked 128-key tiles for their 256 queries (2 x 128 x 128 block pairs
  * per workgroup and tile, 8.389 MFLOP each) out of LDS, with the kernel's barrier per tile and, if `with_copies`,
  * its asynchronous copies of the next tile (64 KB from a ring of `n_src_tiles` >= 2 K / V^T tile pairs of 65536
  * bytes each at `tiles`, whose first 32 KB also serve as the queries; the workgroups of an XCD copy the same tile at

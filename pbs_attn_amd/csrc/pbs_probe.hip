@@ -75,12 +75,13 @@ namespace {
 // fast_tile sustains by itself.  V_ROWS: the tiles are handled as the kernel handles a tile of the query block's own
 // segment (K and V copied row by row, V fragments by transposing reads).  Workgroup 0 reports its shader-clock and
 // 100 MHz ticks.
-template <bool V_ROWS>
-__global__ __launch_bounds__(512, 2) void tile_probe_kernel(const uint16_t* __restrict__ tiles, int n_src, int iters, int with_copies,
-                                                            float* __restrict__ sink, unsigned long long* __restrict__ clocks) {
+template <bool V_ROWS, bool COPIES>
+__global__ __launch_bounds__(THREADS, 1) void tile_probe_kernel(const uint16_t* __restrict__ tiles, int n_src, int iters,
+                                                                float* __restrict__ sink, unsigned long long* __restrict__ clocks) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  RESERVE_ACC_REGS();
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  for (int i = threadIdx.x; i < (int)(4 * TILE_BYTES / 16); i += 512)   // both buffer pairs start as copies of the first tiles
+  for (int i = threadIdx.x; i < (int)(4 * TILE_BYTES / 16); i += THREADS)   // both buffer pairs start as copies of the first tiles
     reinterpret_cast<u32x4*>(smem)[i] = reinterpret_cast<const u32x4*>(tiles)[i % (2 * TILE_BYTES / 16)];
   __syncthreads();
   const int lane = lane_id_here();
@@ -88,64 +89,59 @@ __global__ __launch_bounds__(512, 2) void tile_probe_kernel(const uint16_t* __re
   const int krow = 8 * (i16 >> 2) + (i16 & 3);
   const uint32_t koff0 = (uint32_t)(krow * 256 + ((g4 ^ i16) * 16));
   const uint32_t voff0 = LDS_V0 + (uint32_t)(i16 * 256 + ((g4 ^ i16) * 16));
-  const uint32_t lane_off = async_lane_offset(wave, lane);
-  bf16x8 qf[2][4];
-#pragma unroll
-  for (int qg = 0; qg < 2; ++qg)
-#pragma unroll
-    for (int kd = 0; kd < 4; ++kd)
-      qf[qg][kd] = *reinterpret_cast<const bf16x8*>(tiles + (wave * 32 + 16 * qg + i16) * D + 32 * kd + 8 * g4);
-  f32x4 o[8][2];
-  float zero = 0.f;
-  asm volatile("" : "+v"(zero));
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-    for (int qg = 0; qg < 2; ++qg)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[dt][qg][r] = zero;
-  float m_ref[2] = {8.f, 8.f}, l_part[2] = {0.f, 0.f}, c_log2 = 0.12751743f;   // exp2(s / sqrt(128) * log2 e - 8): no rescale on N(0, 1) data
+  static_for<QG>([&](auto qc) __attribute__((always_inline)) {
+    constexpr int qg = decltype(qc)::value;
+    const uint16_t* qrow = tiles + (wave * 64 + 16 * qg + i16) * D + 8 * g4;
+    q_load<qg, 0>(qrow);
+    q_load<qg, 1>(qrow + 32);
+    q_load<qg, 2>(qrow + 64);
+    q_load<qg, 3>(qrow + 96);
+  });
+  o_clear();
+  float m_ref[QG] = {8.f, 8.f, 8.f, 8.f}, l_part[QG] = {0.f, 0.f, 0.f, 0.f};
+  float c_log2 = 0.12751743f;   // exp2(s / sqrt(128) * log2 e - 8): no rescale on N(0, 1) data
   asm volatile("" : "+s"(c_log2));
   bool poisoned = false;
   uint32_t bufx = 0;
+  TileCopy copy;
+  if (V_ROWS) copy_offsets_rows(copy, D, D, BS, wave, lane);
+  else copy_offsets_perm(copy, wave, lane);
+  uint32_t ka[4], va[4];
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    ka[n] = koff0 ^ (uint32_t)(n << 6);
+    va[n] = voff0 ^ (uint32_t)(n << 6);
+  }
   const unsigned long long c0 = __builtin_amdgcn_s_memtime(), r0 = __builtin_amdgcn_s_memrealtime();
-  for (int it = 0; it < iters; ++it, bufx ^= 0x8000u) {
+  for (int it = 0; it < iters; ++it) {
     __builtin_amdgcn_s_waitcnt(0x0f70);
     __syncthreads();
-    if (with_copies) {
-      // the 32 workgroups of an XCD (blockIdx % 8) copy the same tile at the same step, as the kernel's workgroups
-      // of an XCD walk one head's K / V stream together and share it in that XCD's L2
-      const uint16_t* src = tiles + (size_t)((it * 7 + (int)(blockIdx.x & 7) * 29) % n_src) * (2 * BS * D);
-      if (V_ROWS) {
-        stage_krows_async(src, D, BS, bufx ^ 0x8000u, wave, lane_id_here());
-        stage_vrows_async(src + BS * D, D, BS, LDS_V0 + (bufx ^ 0x8000u), wave, lane_id_here());
-      } else {
-        if (wave < 4) {   // as the kernel does: the first wave of every SIMD issues the second wave's share too
-          stage_tile_async(src, bufx ^ 0x8000u, wave, lane_off ^ k_copy_xor(wave));
-          stage_tile_async(src, bufx ^ 0x8000u, wave + 4, (lane_off + 4096u) ^ k_copy_xor(wave + 4));
-          stage_tile_async(src + BS * D, LDS_V0 + (bufx ^ 0x8000u), wave, lane_off);
-          stage_tile_async(src + BS * D, LDS_V0 + (bufx ^ 0x8000u), wave + 4, lane_off + 4096u);
-        }
-      }
-    }
-    uint32_t ka[4], va[4];
+    // the 32 workgroups of an XCD (blockIdx % 8) copy the same tile at the same step, as the kernel's workgroups
+    // of an XCD walk one head's K / V stream together and share it in that XCD's L2
+    const uint16_t* src = tiles + (size_t)((it * 7 + (int)(blockIdx.x & 7) * 29) % n_src) * (2 * BS * D);
+    copy.k = uniform64((uint64_t)(uintptr_t)src - COPY_BIAS);
+    copy.v = uniform64((uint64_t)(uintptr_t)(src + BS * D) - COPY_BIAS);
+    copy.lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)((bufx ^ 0x8000u) + (uint32_t)wave * 8192u));
+    fast_tile<0, 0, V_ROWS, COPIES>(ka, va, c_log2, true, true, m_ref, l_part, poisoned, wave, copy);
+    bufx ^= 0x8000u;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      ka[n] = koff0 ^ (uint32_t)(n << 6) ^ bufx;
-      va[n] = voff0 ^ (uint32_t)(n << 6) ^ bufx;
+      ka[n] ^= 0x8000u;
+      va[n] ^= 0x8000u;
     }
-    fast_tile<false, PREFETCH_SLOTS, V_ROWS>(o, qf, ka, va, c_log2, m_ref, l_part, poisoned, wave & 3);
   }
   __builtin_amdgcn_s_waitcnt(0x0f70);
   const unsigned long long c1 = __builtin_amdgcn_s_memtime(), r1 = __builtin_amdgcn_s_memrealtime();
-  float s = l_part[0] + l_part[1] + m_ref[0] + m_ref[1] + (poisoned ? 1.f : 0.f);
+  MFMA_FENCE();
+  float s = poisoned ? 1.f : 0.f;
 #pragma unroll
-  for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-    for (int qg = 0; qg < 2; ++qg)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s += o[dt][qg][r];
-  sink[blockIdx.x * 512 + threadIdx.x] = s;
+  for (int q = 0; q < QG; ++q) s += l_part[q] + m_ref[q];
+  static_for<8 * QG>([&](auto ic) __attribute__((always_inline)) {
+    const f32x4 o4 = o_get<decltype(ic)::value / QG, decltype(ic)::value % QG>();
+    s += (o4[0] + o4[1]) + (o4[2] + o4[3]);
+  });
+  sink[blockIdx.x * 2 * THREADS + threadIdx.x] = s;
+  sink[(blockIdx.x * 2 + 1) * THREADS + threadIdx.x] = l_part[0] + l_part[1] + l_part[2] + l_part[3];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     clocks[0] = c1 - c0;
     clocks[1] = r1 - r0;
@@ -158,18 +154,15 @@ extern "C" int pbs_attn_tile_probe(const void* tiles, int n_src_tiles, int iters
                                    unsigned long long* clocks, void* stream) {
   PBS_REQUIRE(tiles && sink && clocks && iters > 0 && n_src_tiles >= 2, "pbs_attn_tile_probe: bad arguments");
   PBS_REQUIRE(((uintptr_t)tiles % 16) == 0, "pbs_attn_tile_probe: tiles must be 16-byte aligned");
-  const bool v_rows = (with_copies & 2) != 0;
-  const void* kernel = v_rows ? (const void*)tile_probe_kernel<true> : (const void*)tile_probe_kernel<false>;
-  hipError_t attr = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_TOTAL);
+  const bool v_rows = (with_copies & 2) != 0, copies = (with_copies & 1) != 0;
+  auto* kernel = v_rows ? (copies ? tile_probe_kernel<true, true> : tile_probe_kernel<true, false>)
+                        : (copies ? tile_probe_kernel<false, true> : tile_probe_kernel<false, false>);
+  hipError_t attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_TOTAL);
   if (attr != hipSuccess) {
     pbs_set_error("pbs_attn_tile_probe: cannot reserve %u bytes of LDS: %s", LDS_TOTAL, hipGetErrorString(attr));
     return (int)attr;
   }
-  if (v_rows)
-    hipLaunchKernelGGL(tile_probe_kernel<true>, dim3(256), dim3(512), LDS_TOTAL, (hipStream_t)stream, (const uint16_t*)tiles,
-                       n_src_tiles, iters, with_copies & 1, sink, clocks);
-  else
-    hipLaunchKernelGGL(tile_probe_kernel<false>, dim3(256), dim3(512), LDS_TOTAL, (hipStream_t)stream, (const uint16_t*)tiles,
-                       n_src_tiles, iters, with_copies & 1, sink, clocks);
+  hipLaunchKernelGGL(kernel, dim3(256), dim3(THREADS), LDS_TOTAL, (hipStream_t)stream, (const uint16_t*)tiles, n_src_tiles,
+                     iters, sink, clocks);
   return pbs_check_launch("pbs_attn_tile_probe");
 }
