@@ -80,8 +80,8 @@ typedef const __attribute__((address_space(4))) struct AttnArgs* ArgsPtr;
 // divisions -- [0] number of tiles, [1] batch, [2] query head, [3] KV head, [4] first query block -- and holds from
 // LIST_HEADER on entries kb | ENT_ORIG? | use_first << 14 |
 // use_second << 15: the union of the two visit lists (ascending), then the own segments in ORIGINAL key order
-// (blocks first-of-segment .. query block, shared where the two blocks share a segment).  Block 0 also clears
-// the work counters of the attention kernel that follows on the stream.
+// (blocks first-of-segment .. query block, shared where the two blocks share a segment).  Without `cols` every block of
+// every earlier segment is visited.  Block 0 also clears the work counters of the attention kernel that follows on the stream.
 constexpr int LIST_HEADER = 8;
 constexpr int MERGE_THREADS = 256;
 __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const int32_t* __restrict__ cols, const int32_t* __restrict__ cnt,
@@ -94,10 +94,12 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
   const int bh = blockIdx.x / npair, pair = blockIdx.x % npair;
   if (blockIdx.x == 0 && tid < 8) queue[tid] = 0;
   const bool second = 2 * pair + 1 < nb;
+  const int qb0 = 2 * pair, qb1 = second ? qb0 + 1 : qb0;
+  const int sf0 = (qb0 / bps) * bps, sf1 = (qb1 / bps) * bps;
   const int32_t* l0 = cols + ((int64_t)bh * nb + 2 * pair) * nb;
   const int32_t* l1 = l0 + (second ? nb : 0);
-  const int n0 = cnt[(int64_t)bh * nb + 2 * pair];
-  const int n1 = second ? cnt[(int64_t)bh * nb + 2 * pair + 1] : 0;
+  const int n0 = cols ? cnt[(int64_t)bh * nb + 2 * pair] : 0;
+  const int n1 = cols && second ? cnt[(int64_t)bh * nb + 2 * pair + 1] : 0;
   constexpr int MAX_PER = 4096 / MERGE_THREADS;
   int c0[MAX_PER], c1[MAX_PER];
 #pragma unroll
@@ -107,8 +109,8 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
     c1[u] = i < n1 ? l1[i] : 0;
   }
   for (int i = tid; i < nb; i += MERGE_THREADS) {
-    flags0[i] = 0;
-    flags1[i] = 0;
+    flags0[i] = !cols && i < sf0 ? 1 : 0;
+    flags1[i] = !cols && second && i < sf1 ? 2 : 0;
   }
   __syncthreads();
 #pragma unroll
@@ -152,8 +154,6 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
     const int f = flags0[kb] | flags1[kb];
     if (f) out[w++] = (uint16_t)(kb | (f << 14));
   }
-  const int qb0 = 2 * pair, qb1 = second ? qb0 + 1 : qb0;
-  const int sf0 = (qb0 / bps) * bps, sf1 = (qb1 / bps) * bps;
   const int n_own = qb1 - sf0 + 1;
   if (own_needed) {
     // one-block segments with an optional diagonal: a query block's own block is listed only where its flag is set
@@ -736,19 +736,13 @@ extern "C" size_t pbs_sparse_attn_workspace_bytes(int B, int Hq, int S, int segm
   return 256 + (size_t)B * Hq * npair * cap * 2;
 }
 
-static int sparse_attn_launch(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
-                              const int32_t* csr_cols, const int32_t* csr_cnt, void* out, int B, int Hq, int Hkv, int S,
-                              int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
-                              int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
-                              int64_t o_sh, int64_t o_ss, float softmax_scale, const uint8_t* own_block_needed, void* workspace,
-                              void* stream);
-
 extern "C" int pbs_sparse_attn_fwd(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
                                    const int32_t* csr_cols, const int32_t* csr_cnt, void* out, int B, int Hq, int Hkv, int S,
                                    int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
                                    int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
                                    int64_t o_sb, int64_t o_sh, int64_t o_ss, float softmax_scale, void* workspace, void* stream) {
-  return sparse_attn_launch(q, perm_k, perm_vt, k, v, csr_cols, csr_cnt, out, B, Hq, Hkv, S, head_dim, block_size, segment_size,
+  PBS_REQUIRE(csr_cols && csr_cnt, "pbs_sparse_attn_fwd: null tensor pointer");
+  return pbs_sparse_attn_launch(q, perm_k, perm_vt, k, v, csr_cols, csr_cnt, out, B, Hq, Hkv, S, head_dim, block_size, segment_size,
                             q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale, nullptr,
                             workspace, stream);
 }
@@ -761,18 +755,19 @@ extern "C" int pbs_sparse_attn_fwd_optional_diagonal(const void* q, const void* 
                                                      int64_t v_ss, int64_t o_sb, int64_t o_sh, int64_t o_ss, float softmax_scale,
                                                      void* workspace, void* stream) {
   PBS_REQUIRE(own_block_needed, "pbs_sparse_attn_fwd_optional_diagonal: null own_block_needed");
-  return sparse_attn_launch(q, perm_k, perm_vt, k, v, csr_cols, csr_cnt, out, B, Hq, Hkv, S, head_dim, block_size, block_size,
+  PBS_REQUIRE(csr_cols && csr_cnt, "pbs_sparse_attn_fwd: null tensor pointer");
+  return pbs_sparse_attn_launch(q, perm_k, perm_vt, k, v, csr_cols, csr_cnt, out, B, Hq, Hkv, S, head_dim, block_size, block_size,
                             q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale,
                             own_block_needed, workspace, stream);
 }
 
-static int sparse_attn_launch(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
+int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
                               const int32_t* csr_cols, const int32_t* csr_cnt, void* out, int B, int Hq, int Hkv, int S,
                               int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
                               int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
                               int64_t o_sh, int64_t o_ss, float softmax_scale, const uint8_t* own_block_needed, void* workspace,
                               void* stream) {
-  PBS_REQUIRE(q && perm_k && perm_vt && k && v && csr_cols && csr_cnt && out, "pbs_sparse_attn_fwd: null tensor pointer");
+  PBS_REQUIRE(q && perm_k && perm_vt && k && v && out, "pbs_sparse_attn_fwd: null tensor pointer");
   PBS_REQUIRE(workspace && ((uintptr_t)workspace % 256) == 0, "pbs_sparse_attn_fwd: workspace must be a 256-byte aligned device buffer of pbs_sparse_attn_workspace_bytes()");
   PBS_REQUIRE(head_dim == D && block_size == BS, "pbs_sparse_attn_fwd: head_dim and block_size must be 128 (got %d, %d)", head_dim, block_size);
   PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0, "pbs_sparse_attn_fwd: bad shape");
