@@ -81,18 +81,20 @@ typedef const __attribute__((address_space(4))) struct AttnArgs* ArgsPtr;
 // LIST_HEADER on entries kb | ENT_ORIG? | use_first << 14 |
 // use_second << 15: the union of the two visit lists (ascending), then the own segments in ORIGINAL key order
 // (blocks first-of-segment .. query block, shared where the two blocks share a segment).  Without `cols` every block of
-// every earlier segment is visited.  Block 0 also clears the work counters of the attention kernel that follows on the stream.
+// every earlier segment is visited.  Block 0 also sets the work counters of the attention kernel that follows on the
+// stream: its workgroups start on the first `first_tickets` tickets of their ranges without asking.
 constexpr int LIST_HEADER = 8;
 constexpr int MERGE_THREADS = 256;
 __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const int32_t* __restrict__ cols, const int32_t* __restrict__ cnt,
                                                                uint16_t* __restrict__ plist, int* __restrict__ queue, int nb,
-                                                               int bps, int cap, int Hq, int group, const uint8_t* __restrict__ own_needed) {
+                                                               int bps, int cap, int Hq, int group, int first_tickets,
+                                                               const uint8_t* __restrict__ own_needed) {
   __shared__ uint8_t flags0[4096], flags1[4096];
   __shared__ int wsum[MERGE_THREADS / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int npair = (nb + 1) >> 1;
   const int bh = blockIdx.x / npair, pair = blockIdx.x % npair;
-  if (blockIdx.x == 0 && tid < 8) queue[tid] = 0;
+  if (blockIdx.x == 0 && tid < 8) queue[tid] = first_tickets;
   const bool second = 2 * pair + 1 < nb;
   const int qb0 = 2 * pair, qb1 = second ? qb0 + 1 : qb0;
   const int sf0 = (qb0 / bps) * bps, sf1 = (qb1 / bps) * bps;
@@ -229,23 +231,46 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   const int xcd = blockIdx.x & 7;
   int q_begin = a0->xcd_start[xcd], q_end = a0->xcd_start[xcd + 1];   // the range being served: this XCD's, later others'
   int vic = xcd, vic_tried = 0;
-  int* misc = reinterpret_cast<int*>(smem + LDS_MISC);   // [1] redo flag, [2] first item, [4] next item
-  // the first item: from this XCD's range, or, when that one is empty or already handed out, from the next XCD's
-  // range that still has items
-  int cur;
-  for (;;) {
-    if (threadIdx.x == 0) {
-      misc[2] = q_begin + atomicAdd(a0->queue + vic, 1);
-      misc[1] = 0;
+  int* misc = reinterpret_cast<int*>(smem + LDS_MISC);   // [1] redo flag, [4] next item, [5] ranges with items left
+  // Another range that still has items, once this one is used up: true with the item in `found` and the range in
+  // vic / q_begin / q_end.  All eight counters are read at once, and a range whose counter has passed its end is skipped
+  // without asking for a ticket (counters only grow): at the end of a launch, when every range is used up, that is one round
+  // trip to memory instead of seven.
+  int found = 0;
+  auto claim_elsewhere = [&]() __attribute__((always_inline)) {
+    if (vic_tried >= 7) return false;
+    ArgsPtr as = PBS_ARGS();
+    __syncthreads();   // everyone has read the previous ticket
+    if (wave == 0) {
+      const int ln = lane_id_here();
+      bool left = false;
+      if (ln < 8) left = as->xcd_start[ln] + __hip_atomic_load(as->queue + ln, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < as->xcd_start[ln + 1];
+      const uint64_t ranges = __ballot(left);
+      if (ln == 0) misc[5] = (int)ranges;
     }
     __syncthreads();
-    cur = ticket_item(q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[2]), a0->interleave, npair);
-    if (cur < q_end) break;
-    if (++vic_tried > 7) return;
-    vic = (xcd + vic_tried) & 7;
-    q_begin = a0->xcd_start[vic];
-    q_end = a0->xcd_start[vic + 1];
-    __syncthreads();   // everyone has read the ticket before the next one is written
+    const int ranges = __builtin_amdgcn_readfirstlane(misc[5]);
+    while (vic_tried < 7) {
+      ++vic_tried;
+      vic = (xcd + vic_tried) & 7;
+      if (!(ranges >> vic & 1)) continue;
+      q_begin = as->xcd_start[vic];
+      q_end = as->xcd_start[vic + 1];
+      __syncthreads();   // everyone has read the previous ticket
+      if (wave == 0 && lane_id_here() == 0) misc[4] = q_begin + atomicAdd(as->queue + vic, 1);
+      __syncthreads();
+      found = ticket_item(q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]), as->interleave, npair);
+      if (found < q_end) return true;
+    }
+    return false;
+  };
+  // The first item: workgroup n of an XCD takes ticket n, without asking (the counters start behind these tickets); where the
+  // range is shorter than that, an item of another one.
+  if (threadIdx.x == 0) misc[1] = 0;
+  int cur = ticket_item(q_begin, q_end, q_begin + ((int)blockIdx.x >> 3), a0->interleave, npair);
+  if (PBS_UNLIKELY(cur >= q_end)) {
+    if (!claim_elsewhere()) return;
+    cur = found;
   }
   int nxt = q_end;   // the next item is claimed late in the current one: an item claimed early waits for this
                      // workgroup while others may be idle
@@ -684,20 +709,8 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       // the range is used up: serve the other XCDs' ranges, one after the other.  No look-ahead on this path:
       // claim, fetch the list, request the first tile, each after the other
       ArgsPtr as = PBS_ARGS();
-      while (vic_tried < 7) {
-        ++vic_tried;
-        vic = (xcd + vic_tried) & 7;
-        q_begin = as->xcd_start[vic];
-        q_end = as->xcd_start[vic + 1];
-        __syncthreads();   // everyone has read the previous ticket
-        if (wave == 0 && lane_id_here() == 0) misc[4] = q_begin + atomicAdd(as->queue + vic, 1);
-        __syncthreads();
-        nxt = ticket_item(q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]), as->interleave, npair);
-        if (nxt < q_end) {
-          has_nxt = true;
-          break;
-        }
-      }
+      has_nxt = claim_elsewhere();
+      if (has_nxt) nxt = found;
       if (has_nxt) {
         stolen = true;
         stage_list_async(list_row(as, nxt), as->cap >> 3, LDS_LIST + (li ^ 1u) * LIST_BYTES, wave, wave * 64 + lane_id_here());
@@ -845,7 +858,7 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
     return (int)attr;
   }
   hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * npair)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
-                     (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.bps, a.cap, Hq, Hq / Hkv, own_block_needed);
+                     (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.bps, a.cap, Hq, Hq / Hkv, (int)(n_wg / 8), own_block_needed);
   hipLaunchKernelGGL(sparse_attn_kernel, dim3((unsigned)n_wg), dim3(THREADS), LDS_TOTAL, (hipStream_t)stream, a);
   return pbs_check_launch("pbs_sparse_attn_fwd");
 }

@@ -21,7 +21,7 @@ constexpr int TILE_BYTES = BS * D * 2;            // 32 KB
 constexpr uint32_t LDS_V0 = 2 * TILE_BYTES;       // K buffers at 0 / 32 KB, V buffers at 64 / 96 KB
 constexpr uint32_t LDS_LIST = 4 * TILE_BYTES;     // two merged visit lists (current item, next item), uint16 entries
 constexpr uint32_t LIST_BYTES = 9728;             // header + at most 4096 + 511 + 1 entries, rounded up
-constexpr uint32_t LDS_MISC = LDS_LIST + 2 * LIST_BYTES;   // ints: [1] redo flag, [2] first work item, [4] next work item
+constexpr uint32_t LDS_MISC = LDS_LIST + 2 * LIST_BYTES;   // ints: [1] redo flag, [4] next work item, [5] ranges with items left
 constexpr uint32_t LDS_TOTAL = LDS_MISC + 1024;   // 151 552 bytes of the CU's 160 KB
 constexpr int THREADS = 256;                      // four waves, one per SIMD
 constexpr int QG = 4;                             // query column groups of 16 per wave: 64 queries
