@@ -83,7 +83,6 @@ typedef const __attribute__((address_space(4))) struct AttnArgs* ArgsPtr;
 // (blocks first-of-segment .. query block, shared where the two blocks share a segment).  Without `cols` every block of
 // every earlier segment is visited.  Block 0 also sets the work counters of the attention kernel that follows on the
 // stream: its workgroups start on the first `first_tickets` tickets of their ranges without asking.
-constexpr int LIST_HEADER = 8;
 constexpr int MERGE_THREADS = 256;
 __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const int32_t* __restrict__ cols, const int32_t* __restrict__ cnt,
                                                                uint16_t* __restrict__ plist, int* __restrict__ queue, int nb,
@@ -755,7 +754,7 @@ extern "C" int pbs_sparse_attn_fwd(const void* q, const void* perm_k, const void
                                    int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
                                    int64_t o_sb, int64_t o_sh, int64_t o_ss, float softmax_scale, void* workspace, void* stream) {
   PBS_REQUIRE(csr_cols && csr_cnt, "pbs_sparse_attn_fwd: null tensor pointer");
-  return pbs_sparse_attn_launch(q, perm_k, perm_vt, k, v, csr_cols, csr_cnt, out, B, Hq, Hkv, S, head_dim, block_size, segment_size,
+  return pbs_sparse_attn_launch(q, perm_k, perm_vt, k, v, csr_cols, csr_cnt, false, out, B, Hq, Hkv, S, head_dim, block_size, segment_size,
                             q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale, nullptr,
                             workspace, stream);
 }
@@ -769,42 +768,15 @@ extern "C" int pbs_sparse_attn_fwd_optional_diagonal(const void* q, const void* 
                                                      void* workspace, void* stream) {
   PBS_REQUIRE(own_block_needed, "pbs_sparse_attn_fwd_optional_diagonal: null own_block_needed");
   PBS_REQUIRE(csr_cols && csr_cnt, "pbs_sparse_attn_fwd: null tensor pointer");
-  return pbs_sparse_attn_launch(q, perm_k, perm_vt, k, v, csr_cols, csr_cnt, out, B, Hq, Hkv, S, head_dim, block_size, block_size,
+  return pbs_sparse_attn_launch(q, perm_k, perm_vt, k, v, csr_cols, csr_cnt, false, out, B, Hq, Hkv, S, head_dim, block_size, block_size,
                             q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale,
                             own_block_needed, workspace, stream);
 }
 
-int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
-                              const int32_t* csr_cols, const int32_t* csr_cnt, void* out, int B, int Hq, int Hkv, int S,
-                              int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
-                              int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
-                              int64_t o_sh, int64_t o_ss, float softmax_scale, const uint8_t* own_block_needed, void* workspace,
-                              void* stream) {
-  PBS_REQUIRE(q && perm_k && perm_vt && k && v && out, "pbs_sparse_attn_fwd: null tensor pointer");
-  PBS_REQUIRE(workspace && ((uintptr_t)workspace % 256) == 0, "pbs_sparse_attn_fwd: workspace must be a 256-byte aligned device buffer of pbs_sparse_attn_workspace_bytes()");
-  PBS_REQUIRE(head_dim == D && block_size == BS, "pbs_sparse_attn_fwd: head_dim and block_size must be 128 (got %d, %d)", head_dim, block_size);
-  PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0, "pbs_sparse_attn_fwd: bad shape");
-  PBS_REQUIRE(segment_size > 0 && segment_size % block_size == 0, "pbs_sparse_attn_fwd: segment_size must be a multiple of block_size");
-  PBS_REQUIRE(segment_size / block_size <= 511, "pbs_sparse_attn_fwd: more than 511 blocks per segment");
-  PBS_REQUIRE(q_sb % 8 == 0 && q_sh % 8 == 0 && q_ss % 8 == 0 && o_sb % 8 == 0 && o_sh % 8 == 0 && o_ss % 8 == 0 &&
-                  k_sb % 8 == 0 && k_sh % 8 == 0 && k_ss % 8 == 0 && v_sb % 8 == 0 && v_sh % 8 == 0 && v_ss % 8 == 0,
-              "pbs_sparse_attn_fwd: strides must keep rows 16-byte aligned");
-  PBS_REQUIRE(k_ss >= D && k_ss < (1 << 22), "pbs_sparse_attn_fwd: key row stride %lld outside [128, 2^22)", (long long)k_ss);
-  PBS_REQUIRE(v_ss >= D && v_ss < (1 << 22), "pbs_sparse_attn_fwd: value row stride %lld outside [128, 2^22)", (long long)v_ss);
-  PBS_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)out % 16) == 0 && ((uintptr_t)perm_k % 16) == 0 &&
-                  ((uintptr_t)perm_vt % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0,
-              "pbs_sparse_attn_fwd: pointers must be 16-byte aligned");
-  AttnArgs a;
-  a.q = (const uint16_t*)q; a.pk = (const uint16_t*)perm_k; a.pvt = (const uint16_t*)perm_vt;
-  a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
-  a.o = (uint16_t*)out;
-  a.BH = B * Hq; a.Hq = Hq; a.Hkv = Hkv; a.S = S; a.nb = (S + BS - 1) / BS; a.bps = segment_size / block_size;
-  a.q_sb = q_sb; a.q_sh = q_sh; a.q_ss = q_ss; a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = (uint32_t)k_ss; a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = (uint32_t)v_ss; a.o_sb = o_sb; a.o_sh = o_sh; a.o_ss = o_ss;
-  a.scale_log2 = softmax_scale * 1.4426950408889634f;
-  PBS_REQUIRE(a.nb <= 4096, "pbs_sparse_attn_fwd: more than 4096 blocks per sequence (%d)", a.nb);
+// the eight ranges of work items (AttnArgs::xcd_start) and the ticket order; returns the items of the longest range
+static int plan_ranges(AttnArgs& a) {
   // eight ranges of equal estimated work: the row pair p of a head costs about p + 1 (causal length)
   const int64_t npair = (a.nb + 1) / 2;
-  PBS_REQUIRE((int64_t)a.BH * npair < (1ll << 28) && B < 65536 && Hq < 65536, "pbs_sparse_attn_fwd: launch too large");
   const double head_work = 0.5 * (double)npair * (double)(npair + 1);
   int max_items = 0;
   for (int x = 0; x <= 8; ++x) {
@@ -832,22 +804,76 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
     for (a.interleave = 1; (1 << (a.interleave - 1)) < nh; ++a.interleave) {}
     for (int x = 0; x <= 8; ++x) a.xcd_start[x] = (int)(x * (int64_t)nh * npair);
   }
-  a.cap = list_cap(a.nb, a.bps);
-  PBS_REQUIRE((uint32_t)a.cap * 2 <= LIST_BYTES, "pbs_sparse_attn_fwd: visit list too long");
-  a.queue = (int*)workspace;
-  a.plist = (const uint16_t*)((char*)workspace + 256);
-  // the kernel's dynamic LDS size is raised once per device, not per call; the CU count is looked up once too
+  return max_items;
+}
+
+// one workgroup per CU (the kernel's LDS leaves room for one), a multiple of 8 so that every XCD gets its share; fewer when
+// there are fewer items.  The CU count is looked up once per device.
+static int64_t workgroups(int max_items) {
   int dev = 0;
-  hipError_t attr = hipGetDevice(&dev);
-  const bool tracked = attr == hipSuccess && dev >= 0 && dev < 64;
+  const bool tracked = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64;
   int n_cu = tracked ? g_cu_count[dev].load(std::memory_order_relaxed) : 0;
   if (n_cu <= 0) {
     if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cu <= 0) n_cu = 256;
     if (tracked) g_cu_count[dev].store(n_cu, std::memory_order_relaxed);
   }
-  // one workgroup per CU (the kernel's LDS leaves room for one), a multiple of 8 so that every XCD gets its share;
-  // fewer when there are fewer items
-  const int64_t n_wg = std::min<int64_t>((int64_t)8 * max_items, (int64_t)(n_cu + 7) / 8 * 8);
+  return std::min<int64_t>((int64_t)8 * max_items, (int64_t)(n_cu + 7) / 8 * 8);
+}
+
+PairLists pbs_pair_lists(int B, int Hq, int Hkv, int S, int block_size, int segment_size, void* workspace) {
+  AttnArgs a;
+  a.BH = B * Hq;
+  a.nb = (S + block_size - 1) / block_size;
+  PairLists l;
+  l.plist = (uint16_t*)((char*)workspace + 256);
+  l.queue = (int*)workspace;
+  l.cap = list_cap(a.nb, segment_size / block_size);
+  l.Hq = Hq;
+  l.group = Hq / Hkv;
+  l.first_tickets = (int)(workgroups(plan_ranges(a)) / 8);
+  return l;
+}
+
+int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
+                              const int32_t* csr_cols, const int32_t* csr_cnt, bool lists_built, void* out, int B, int Hq, int Hkv, int S,
+                              int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                              int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
+                              int64_t o_sh, int64_t o_ss, float softmax_scale, const uint8_t* own_block_needed, void* workspace,
+                              void* stream) {
+  PBS_REQUIRE(q && perm_k && perm_vt && k && v && out, "pbs_sparse_attn_fwd: null tensor pointer");
+  PBS_REQUIRE(workspace && ((uintptr_t)workspace % 256) == 0, "pbs_sparse_attn_fwd: workspace must be a 256-byte aligned device buffer of pbs_sparse_attn_workspace_bytes()");
+  PBS_REQUIRE(head_dim == D && block_size == BS, "pbs_sparse_attn_fwd: head_dim and block_size must be 128 (got %d, %d)", head_dim, block_size);
+  PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0, "pbs_sparse_attn_fwd: bad shape");
+  PBS_REQUIRE(segment_size > 0 && segment_size % block_size == 0, "pbs_sparse_attn_fwd: segment_size must be a multiple of block_size");
+  PBS_REQUIRE(segment_size / block_size <= 511, "pbs_sparse_attn_fwd: more than 511 blocks per segment");
+  PBS_REQUIRE(q_sb % 8 == 0 && q_sh % 8 == 0 && q_ss % 8 == 0 && o_sb % 8 == 0 && o_sh % 8 == 0 && o_ss % 8 == 0 &&
+                  k_sb % 8 == 0 && k_sh % 8 == 0 && k_ss % 8 == 0 && v_sb % 8 == 0 && v_sh % 8 == 0 && v_ss % 8 == 0,
+              "pbs_sparse_attn_fwd: strides must keep rows 16-byte aligned");
+  PBS_REQUIRE(k_ss >= D && k_ss < (1 << 22), "pbs_sparse_attn_fwd: key row stride %lld outside [128, 2^22)", (long long)k_ss);
+  PBS_REQUIRE(v_ss >= D && v_ss < (1 << 22), "pbs_sparse_attn_fwd: value row stride %lld outside [128, 2^22)", (long long)v_ss);
+  PBS_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)out % 16) == 0 && ((uintptr_t)perm_k % 16) == 0 &&
+                  ((uintptr_t)perm_vt % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0,
+              "pbs_sparse_attn_fwd: pointers must be 16-byte aligned");
+  AttnArgs a;
+  a.q = (const uint16_t*)q; a.pk = (const uint16_t*)perm_k; a.pvt = (const uint16_t*)perm_vt;
+  a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
+  a.o = (uint16_t*)out;
+  a.BH = B * Hq; a.Hq = Hq; a.Hkv = Hkv; a.S = S; a.nb = (S + BS - 1) / BS; a.bps = segment_size / block_size;
+  a.q_sb = q_sb; a.q_sh = q_sh; a.q_ss = q_ss; a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = (uint32_t)k_ss; a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = (uint32_t)v_ss; a.o_sb = o_sb; a.o_sh = o_sh; a.o_ss = o_ss;
+  a.scale_log2 = softmax_scale * 1.4426950408889634f;
+  PBS_REQUIRE(a.nb <= 4096, "pbs_sparse_attn_fwd: more than 4096 blocks per sequence (%d)", a.nb);
+  const int64_t npair = (a.nb + 1) / 2;
+  PBS_REQUIRE((int64_t)a.BH * npair < (1ll << 28) && B < 65536 && Hq < 65536, "pbs_sparse_attn_fwd: launch too large");
+  const int max_items = plan_ranges(a);
+  a.cap = list_cap(a.nb, a.bps);
+  PBS_REQUIRE((uint32_t)a.cap * 2 <= LIST_BYTES, "pbs_sparse_attn_fwd: visit list too long");
+  a.queue = (int*)workspace;
+  a.plist = (const uint16_t*)((char*)workspace + 256);
+  const int64_t n_wg = workgroups(max_items);
+  int dev = 0;
+  hipError_t attr = hipGetDevice(&dev);
+  const bool tracked = attr == hipSuccess && dev >= 0 && dev < 64;
+  // the kernel's dynamic LDS size is raised once per device, not per call
   if (attr == hipSuccess && !(tracked && (g_lds_reserved.load(std::memory_order_acquire) >> dev & 1))) {
     if (const int rc = pbs_require_no_static_lds((const void*)sparse_attn_kernel, "pbs_sparse_attn_fwd")) return rc;
     attr = hipFuncSetAttribute((const void*)sparse_attn_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_TOTAL);
@@ -857,7 +883,8 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
     pbs_set_error("pbs_sparse_attn_fwd: cannot reserve %u bytes of LDS: %s", LDS_TOTAL, hipGetErrorString(attr));
     return (int)attr;
   }
-  hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * npair)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
+  if (!lists_built)
+    hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * npair)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
                      (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.bps, a.cap, Hq, Hq / Hkv, (int)(n_wg / 8), own_block_needed);
   hipLaunchKernelGGL(sparse_attn_kernel, dim3((unsigned)n_wg), dim3(THREADS), LDS_TOTAL, (hipStream_t)stream, a);
   return pbs_check_launch("pbs_sparse_attn_fwd");

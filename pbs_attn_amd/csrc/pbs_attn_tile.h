@@ -2,7 +2,7 @@
 // tile copies, MFMA fragment reads and the software pipeline over one 128 x 128 tile (fast_tile).  Shared by the
 // attention kernel and by the bench-only probe that times this pipeline by itself.
 #pragma once
-#include "pbs_common.h"
+#include "pbs_lists.h"
 #include <type_traits>
 #include <utility>
 
@@ -25,8 +25,6 @@ constexpr uint32_t LDS_MISC = LDS_LIST + 2 * LIST_BYTES;   // ints: [1] redo fla
 constexpr uint32_t LDS_TOTAL = LDS_MISC + 1024;   // 151 552 bytes of the CU's 160 KB
 constexpr int THREADS = 256;                      // four waves, one per SIMD
 constexpr int QG = 4;                             // query column groups of 16 per wave: 64 queries
-constexpr uint32_t ENT_KB = 0x1fffu;              // visit-list entry: key block ...
-constexpr uint32_t ENT_ORIG = 0x2000u;            // ... | tile of the un-permuted K / V (own segment) | use bits 14, 15
 
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 

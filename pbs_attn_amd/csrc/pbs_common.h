@@ -24,15 +24,6 @@ int pbs_check_launch(const char* what);         // hipGetLastError -> positive c
 // with the message set.
 int pbs_require_no_static_lds(const void* kernel, const char* what);
 
-// pbs_sparse_attn_fwd (and its optional-diagonal form, with own_block_needed) after their null checks.  csr_cols null:
-// every block of every earlier segment is visited and csr_cnt is not read.
-int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
-                           const int32_t* csr_cols, const int32_t* csr_cnt, void* out, int B, int Hq, int Hkv, int S,
-                           int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
-                           int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
-                           int64_t o_sh, int64_t o_ss, float softmax_scale, const uint8_t* own_block_needed, void* workspace,
-                           void* stream);
-
 #define PBS_REQUIRE(cond, ...)                      \
   do {                                              \
     if (!(cond)) return pbs_arg_error(__VA_ARGS__); \

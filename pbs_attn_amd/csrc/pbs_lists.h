@@ -1,0 +1,41 @@
+// Merged visit lists of the pairs of query blocks: their layout, shared by the kernels that write them (the block
+// selection, or the merge of two CSR rows) and the attention kernel that reads them.
+#pragma once
+#include "pbs_common.h"
+
+constexpr int LIST_HEADER = 8;              // uint16 entries in front of a row's tiles: [0] number of tiles, [1] batch, [2] query head,
+                                            // [3] KV head, [4] first query block of the pair
+constexpr uint32_t ENT_KB = 0x1fffu;        // visit-list entry: key block ...
+constexpr uint32_t ENT_ORIG = 0x2000u;      // ... | tile of the un-permuted K / V (own segment) | use bits 14, 15
+
+// Where the lists go: row `bh * npair + (npair - 1 - pair)` of `plist`, `cap` entries each, and the attention kernel's eight
+// work counters, which start at `first_tickets`.
+struct PairLists {
+  uint16_t* plist;
+  int* queue;
+  int cap, Hq, group, first_tickets;   // group: query heads per KV head
+};
+// of the lists that pbs_sparse_attn_launch expects in `workspace` with lists_built set
+PairLists pbs_pair_lists(int B, int Hq, int Hkv, int S, int block_size, int segment_size, void* workspace);
+
+// pbs_sparse_attn_fwd (and its optional-diagonal form, with own_block_needed) after their null checks.  lists_built: the
+// visit lists and counters are in the workspace already.  Otherwise they are merged from the CSR rows or, with csr_cols
+// null (csr_cnt is not read), hold every block of every earlier segment.
+int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
+                           const int32_t* csr_cols, const int32_t* csr_cnt, bool lists_built, void* out, int B, int Hq, int Hkv, int S,
+                           int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                           int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
+                           int64_t o_sh, int64_t o_ss, float softmax_scale, const uint8_t* own_block_needed, void* workspace,
+                           void* stream);
+
+// The selection of pbs_select_blocks for rows of block probabilities that are non-zero in the blocks of earlier segments
+// only, up to PBS_PAIR_SELECT_MAX_BLOCKS blocks, straight into the merged lists.  first_blk: the block that holds original
+// key 0, per row, or null.
+constexpr int PBS_PAIR_SELECT_MAX_BLOCKS = 2048;
+int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold_per_row, float threshold, const int32_t* first_blk,
+                          int rows, int S, int block_size, int segment_size, uint8_t* block_needed, const PairLists& lists,
+                          void* stream);
+// pbs_segment_argsort; first_blk, if not null, receives per row the block of `block_size` that holds original key 0 (there has
+// to be a complete segment)
+int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,
+                               int S_pad, int segment_size, void* stream);

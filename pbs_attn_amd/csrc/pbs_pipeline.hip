@@ -1,6 +1,6 @@
 // Whole PBS prefill attention in one call: every stage enqueued on one stream out of one caller-provided
 // workspace (no allocation, no synchronisation, one host round trip instead of ten).
-#include "pbs_common.h"
+#include "pbs_lists.h"
 
 #include "../../include/pbs_hip.h"   // the stage entry points, type-checked against the public ABI
 
@@ -34,8 +34,9 @@ Layout make_layout(int B, int Hq, int Hkv, int S, int D, int block_size, int seg
   L.pooled_k = take(rows * nb * D * 2);
   L.pooled_q = take(rows * nb * D * 2);
   L.probs = take(rows * nb * nb * 4);
-  L.cols = take(rows * nb * nb * 4);
-  L.cnt = take(rows * nb * 4);
+  const bool csr = nb > PBS_PAIR_SELECT_MAX_BLOCKS;   // shorter rows: the selection writes the attention kernel's lists itself
+  L.cols = take(csr ? rows * nb * nb * 4 : 0);
+  L.cnt = take(csr ? rows * nb * 4 : 0);
   L.needed = take(rows * nb);
   L.select_ws = take(pbs_select_blocks_workspace_bytes((int)rows));
   L.attn_ws = off;
@@ -107,7 +108,7 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
   // 32.2 -> 20.7 us).  (Permuted tiles: none is listed, any aligned address will do.)
   const bool own_tiles_only = segment_size >= s_pad;
   if (own_tiles_only)
-    return pbs_sparse_attn_launch(q, w, w, k, v, nullptr, nullptr, out, B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb,
+    return pbs_sparse_attn_launch(q, w, w, k, v, nullptr, nullptr, false, out, B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb,
                                   q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale, nullptr,
                                   w + L.attn_ws, stream);
   if (one_segment || nseg == 0 || (nseg == 1 && rem == 0)) {
@@ -115,12 +116,14 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
   } else {
     if ((rc = pbs_score_keys(q, k, (float*)(w + L.scores), B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh,
                              q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;
-    if ((rc = pbs_segment_argsort((const float*)(w + L.scores), (int32_t*)(w + L.idx), rows, S, s_pad, segment_size, stream))) return rc;
+    if ((rc = pbs_segment_argsort_launch((const float*)(w + L.scores), (int32_t*)(w + L.idx), (int32_t*)(w + L.select_ws), block_size,
+                                         rows, S, s_pad, segment_size, stream))) return rc;
   }
   // With a real threshold the permuted K / V are gathered AFTER the selection, and only the blocks some query
   // block visits: the estimate needs no more than the pooled permuted key blocks, which come straight from K.
   // (Every candidate selected: everything is visited, one full gather.)
   uint8_t* needed = threshold_is_int_one ? nullptr : w + L.needed;
+  const bool pair_lists = !threshold_is_int_one && nb <= PBS_PAIR_SELECT_MAX_BLOCKS;
   if (threshold_is_int_one) {
     if ((rc = pbs_gather_kv(k, v, (const int32_t*)(w + L.idx), w + L.perm_k, w + L.perm_vt, nullptr, B, Hq, Hkv,
                             S, head_dim, block_size, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, key_pool_max, nullptr, stream))) return rc;
@@ -128,26 +131,28 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
     if ((rc = pbs_pool_blocks(q, k, (const int32_t*)(w + L.idx), w + L.pooled_q, w + L.pooled_k, needed, B, Hq, Hkv, S,
                               head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, query_pool_max, key_pool_max,
                               stream))) return rc;
-    // (up to 1024 blocks the selection reads a row's candidate entries only: the others are not written)
-    if (nb <= 1024) {
+    // (the selection into pair lists reads a row's candidate entries only: the others are not written)
+    if (pair_lists) {
       if ((rc = pbs_block_logits_softmax_candidates_only(w + L.pooled_q, w + L.pooled_k, (float*)(w + L.probs), rows, nb,
                                                          head_dim, segment_size / block_size, stream))) return rc;
+      if ((rc = pbs_select_pair_lists((const float*)(w + L.probs), threshold_per_row, threshold,
+                                      force_select_first_block ? (const int32_t*)(w + L.select_ws) : nullptr, rows, S, block_size,
+                                      segment_size, needed,
+                                      pbs_pair_lists(B, Hq, Hkv, S, block_size, segment_size, w + L.attn_ws), stream))) return rc;
     } else {
       if ((rc = pbs_block_logits_softmax(w + L.pooled_q, w + L.pooled_k, (float*)(w + L.probs), rows, nb, head_dim,
                                          segment_size / block_size, stream))) return rc;
+      if ((rc = pbs_select_blocks((const float*)(w + L.probs), threshold_per_row, threshold, /*threshold_is_int_one=*/0,
+                                  force_select_first_block, /*candidate_rule=*/1, (const int32_t*)(w + L.idx), rows, S, block_size,
+                                  segment_size, nullptr, nullptr, (int32_t*)(w + L.cols), (int32_t*)(w + L.cnt), needed,
+                                  w + L.select_ws, L.attn_ws - L.select_ws, stream))) return rc;
     }
-  }
-  if (!threshold_is_int_one) {
-    if ((rc = pbs_select_blocks((const float*)(w + L.probs), threshold_per_row, threshold, /*threshold_is_int_one=*/0,
-                                force_select_first_block, /*candidate_rule=*/1, (const int32_t*)(w + L.idx), rows, S, block_size,
-                                segment_size, nullptr, nullptr, (int32_t*)(w + L.cols), (int32_t*)(w + L.cnt), needed,
-                                w + L.select_ws, L.attn_ws - L.select_ws, stream))) return rc;
     if ((rc = pbs_gather_kv(k, v, (const int32_t*)(w + L.idx), w + L.perm_k, w + L.perm_vt, nullptr, B, Hq, Hkv,
                             S, head_dim, block_size, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, key_pool_max, needed, stream))) return rc;
   }
   // (every candidate selected: the lists follow from the block numbers)
-  const int32_t* cols = threshold_is_int_one ? nullptr : (const int32_t*)(w + L.cols);
-  return pbs_sparse_attn_launch(q, w + L.perm_k, w + L.perm_vt, k, v, cols, (const int32_t*)(w + L.cnt), out, B, Hq, Hkv, S,
+  const int32_t* cols = threshold_is_int_one || pair_lists ? nullptr : (const int32_t*)(w + L.cols);
+  return pbs_sparse_attn_launch(q, w + L.perm_k, w + L.perm_vt, k, v, cols, (const int32_t*)(w + L.cnt), pair_lists, out, B, Hq, Hkv, S,
                                 head_dim, block_size, segment_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb,
                                 o_sh, o_ss, softmax_scale, nullptr, w + L.attn_ws, stream);
 }

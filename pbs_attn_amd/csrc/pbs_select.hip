@@ -11,7 +11,7 @@
 //     own segment itself, in original key order).
 // Rows of up to 1024 blocks take the wave-level variant further down (one wave per row,
 // the row in registers).
-#include "pbs_common.h"
+#include "pbs_lists.h"
 #include <utility>
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 #include <float.h>
@@ -211,10 +211,10 @@ __global__ __launch_bounds__(256) void select_blocks_kernel(SelectArgs a) {
 
 
 // ---------------------------------------------------------------------------------------------
-// Wave-level variant (rows of up to 1024 blocks): ONE wave per row, the row lives in registers.
-//   * bitonic network on the 32-bit value keys, NPL keys per lane: strides below NPL are register
-//     compare-exchanges, larger strides exchange with lane ^ (stride / NPL); no barriers; the stable order's
-//     tie-break by index is applied only where it matters, at the value where the threshold is reached;
+// Wave-level variant (rows of up to 2048 blocks): ONE wave per row, the row lives in registers.
+//   * bitonic network on the 32-bit value keys, NPL keys per lane, no barriers and no LDS: strides below NPL are register
+//     compare-exchanges, larger strides exchange with lane ^ (stride / NPL) by row moves of the vector unit; the stable
+//     order's tie-break by index is applied only where it matters, at the value where the threshold is reached;
 //   * the running sum is first taken as a parallel float64 prefix (local prefixes + wave scan).  It
 //     differs from the sequential sum by < 1e-12, so "float32(prefix) >= threshold" is decided from it
 //     unless some prefix up to the first hit lies within 1e-11 of the float32 rounding boundary of the
@@ -222,28 +222,90 @@ __global__ __launch_bounds__(256) void select_blocks_kernel(SelectArgs a) {
 //     decision is the one the sequential float64 sum gives;
 //   * flags, own-segment minima, masks and the compacted visit list as in the block-level kernel.
 // ---------------------------------------------------------------------------------------------
-// The bitonic network on 32-bit keys, NPL per lane: a compare-exchange is a minimum and a maximum.
+// the value of lane ^ X.  Strides 1 .. 8 are moves inside a row of sixteen lanes, 16 and 32 exchange rows.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_move(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, false);
+}
+// {own, partner's} in either order: what a minimum, maximum or median does not mind
+struct TwoOf {
+  uint32_t a, b;
+};
+template <int X>
+__device__ __forceinline__ TwoOf with_lane_xor(uint32_t v) {
+  if constexpr (X == 1) return {v, dpp_move<0xB1>(v)};                        // quad_perm 1 0 3 2
+  else if constexpr (X == 2) return {v, dpp_move<0x4E>(v)};                   // quad_perm 2 3 0 1
+  else if constexpr (X == 4) return {v, dpp_move<0x1B>(dpp_move<0x141>(v))};  // mirrored in eight lanes, then in four
+  else if constexpr (X == 8) return {v, dpp_move<0x128>(v)};                  // rotated by eight in sixteen
+  else if constexpr (X == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return {r[0], r[1]};
+  } else {
+    static_assert(X == 32, "lane distance");
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return {r[0], r[1]};
+  }
+}
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+  TwoOf t = with_lane_xor<1>(v);
+  v = min(t.a, t.b);
+  t = with_lane_xor<2>(v);
+  v = min(t.a, t.b);
+  t = with_lane_xor<4>(v);
+  v = min(t.a, t.b);
+  t = with_lane_xor<8>(v);
+  v = min(t.a, t.b);
+  t = with_lane_xor<16>(v);
+  v = min(t.a, t.b);
+  t = with_lane_xor<32>(v);
+  return min(t.a, t.b);
+}
+// the median of three: the minimum of a and b where c is 0, their maximum where it is ~0
+__device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c) { return max(min(a, b), min(max(a, b), c)); }
+
+// one stage of the network: LS is the lane distance
+template <int NPL, int LS>
+__device__ __forceinline__ void cross_lane_stage(uint32_t (&k)[NPL], int lane) {
+  uint32_t side = lane & LS ? ~0u : 0u;   // the upper lane keeps the maximum
+  asm("" : "+v"(side));                   // (a value, not a condition: one median per key instead of two compares and a select)
+#pragma unroll
+  for (int r = 0; r < NPL; ++r) {
+    const TwoOf t = with_lane_xor<LS>(k[r]);
+    k[r] = med3_u32(t.a, t.b, side);
+  }
+}
+// The bitonic network on 32-bit keys, NPL per lane.  Where the direction of a stage depends on the lane, the keys of the
+// descending lanes are complemented for the phase, so that every exchange is a plain minimum and maximum.
 template <int NPL>
 __device__ __forceinline__ void wave_bitonic_sort_u32(uint32_t (&k)[NPL], int lane) {
   constexpr int N = 64 * NPL;
+  uint32_t flipped = 0;
 #pragma unroll
   for (int size = 2; size <= N; size <<= 1) {
+    if (size >= NPL) {
+      const uint32_t flip = (lane & (size / NPL)) ? ~0u : 0u;
+      const uint32_t change = flip ^ flipped;
+#pragma unroll
+      for (int r = 0; r < NPL; ++r) k[r] ^= change;
+      flipped = flip;
+    }
 #pragma unroll
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
       if (stride >= NPL) {
-        const int lstride = stride / NPL;
-        const bool keep_min = ((lane & lstride) == 0) == ((lane & (size / NPL)) == 0);
-#pragma unroll
-        for (int r = 0; r < NPL; ++r) {
-          const uint32_t o = (uint32_t)__shfl_xor((int)k[r], lstride, 64);
-          k[r] = keep_min ? min(k[r], o) : max(k[r], o);
+        switch (stride / NPL) {
+          case 1: cross_lane_stage<NPL, 1>(k, lane); break;
+          case 2: cross_lane_stage<NPL, 2>(k, lane); break;
+          case 4: cross_lane_stage<NPL, 4>(k, lane); break;
+          case 8: cross_lane_stage<NPL, 8>(k, lane); break;
+          case 16: cross_lane_stage<NPL, 16>(k, lane); break;
+          default: cross_lane_stage<NPL, 32>(k, lane); break;
         }
       } else {
 #pragma unroll
         for (int r = 0; r < NPL; ++r) {
           if ((r & stride) == 0) {
             const int p = r | stride;
-            const bool up = (size >= NPL) ? ((lane & (size / NPL)) == 0) : ((r & size) == 0);
+            const bool up = size >= NPL || (r & size) == 0;
             const uint32_t lo = min(k[r], k[p]), hi = max(k[r], k[p]);
             k[r] = up ? lo : hi;
             k[p] = up ? hi : lo;
@@ -254,18 +316,12 @@ __device__ __forceinline__ void wave_bitonic_sort_u32(uint32_t (&k)[NPL], int la
   }
 }
 
-// one wave decides row `rq` ((row, qb - qb_lo) flattened) of the group of rows [qb_lo, qb_hi) x all heads
+// One wave decides row (head `row`, query block qb): flag[0 .. nb) (this wave's, in LDS) becomes the selection.
 template <int NPL>
-__device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t rq, int total_rows, uint8_t* smem_w) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+__device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb, uint8_t* flag) {
+  const int lane = threadIdx.x & 63;
   const int nb = a.nb;
-  const int nb_pad = (nb + 15) & ~15;
-  uint8_t* flag = smem_w + wave * nb_pad;
-  if (rq >= total_rows) return;
-  const int nqb = a.qb_hi - a.qb_lo;
-  const int row = (int)(rq / nqb), qb = a.qb_lo + (int)(rq % nqb);
   const int seg_first = (qb / a.bps) * a.bps;
-  const int seg_end = min(seg_first + a.bps, nb);
   const int64_t row_off = ((int64_t)row * nb + qb) * nb;
 
   for (int kb = lane; kb < nb; kb += 64) flag[kb] = 0;
@@ -277,66 +333,80 @@ __device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t 
     // entries that are zero by construction sort behind every candidate (ties keep index order) and add nothing
     // to the running sum: the row is sorted up to its last candidate only (the launch is sized for that)
     const int count = a.cand_rule == 1 ? seg_first : a.cand_rule == 2 ? min(qb + 1, nb) : nb;
-    uint64_t k[NPL];
+    // value keys, ascending key = descending value; lane l holds entries l * NPL .. l * NPL + NPL - 1, so that the order of
+    // (lane, register) is the order of the indices.  No entry has the key ~0, which stands for "none".
+    uint32_t k0v[NPL];
+    float raw[NPL];
+    if (NPL >= 4 && (nb & 3) == 0 && ((uintptr_t)a.P & 15) == 0) {
+      // whole 16-byte pieces: the one that holds the last candidate ends inside the row (nb is a multiple of four)
+#pragma unroll
+      for (int r = 0; r < NPL; r += 4) {
+        const int i = lane * NPL + r;
+        f32x4 x = {0.f, 0.f, 0.f, 0.f};
+        if (i < count) x = *reinterpret_cast<const f32x4*>(p + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (r + e < NPL) raw[r + e] = x[e];
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < NPL; ++r) {
+        const int i = lane * NPL + r;
+        raw[r] = i < count ? p[i] : 0.f;
+      }
+    }
 #pragma unroll
     for (int r = 0; r < NPL; ++r) {
-      const int i = lane * NPL + r;
-      uint64_t key = ~0ull;
-      if (i < count) {
-        float v = p[i];
-        if (v != v) v = 0.f;
-        else if (v == INFINITY) v = FLT_MAX;
-        else if (v == -INFINITY) v = -FLT_MAX;
-        key = desc_stable_key(v, (uint32_t)i);
-      }
-      k[r] = key;
+      float v = raw[r];
+      if (v != v) v = 0.f;
+      else if (v == INFINITY) v = FLT_MAX;
+      else if (v == -INFINITY) v = -FLT_MAX;
+      k0v[r] = lane * NPL + r < count ? ~f32_orderable(v) : ~0u;
     }
     const float thr = a.thr_rows ? a.thr_rows[row] : a.thr;
 
     // Rows whose mass sits in a few blocks need no sort: the largest remaining entry is taken out of the row
-    // (smallest composite key: value descending, ties by index -- the order of the sort) and added to the
+    // (value descending, ties by index -- the order of the sort) and added to the
     // sequential float64 sum until float32(sum) reaches the threshold: the reference's decision, term by term.
     // Tried only when EXTRACT_MAX times the row's largest value can reach the threshold; a row that does not
     // get there in EXTRACT_MAX steps is sorted whole like any other.
     bool decided = false;
     if (NPL > 1) {
       constexpr int EXTRACT_MAX = 16;
-      uint64_t best = k[0];
+      uint32_t mine = k0v[0];   // the smallest key of this lane
 #pragma unroll
-      for (int r = 1; r < NPL; ++r) best = k[r] < best ? k[r] : best;
+      for (int r = 1; r < NPL; ++r) mine = min(mine, k0v[r]);
+      uint32_t best = wave_min_u32(mine);
+      if (best != ~0u && (float)((double)f32_from_orderable(~best) * EXTRACT_MAX) >= thr) {
+        uint32_t w[NPL];
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        const uint64_t o = shfl_xor_u64(best, off);
-        best = o < best ? o : best;
-      }
-      if (best != ~0ull && (float)((double)desc_key_value(best) * EXTRACT_MAX) >= thr) {
-        uint64_t w[NPL];
-#pragma unroll
-        for (int r = 0; r < NPL; ++r) w[r] = k[r];
+        for (int r = 0; r < NPL; ++r) w[r] = k0v[r];
         double cum = 0.0;
-        uint32_t my_idx = 0;
+        int my_idx = 0;
         int taken = 0;
         for (int it = 0; it < EXTRACT_MAX; ++it) {
-          if (it > 0) {
-            best = w[0];
+          if (best == ~0u) break;   // the row has no further entry: not reached, let the sort path say so
+          // the lowest lane that holds the key, and its lowest register that does
+          const int owner = __builtin_ctzll(__ballot(mine == best));
+          int at = 0;
 #pragma unroll
-            for (int r = 1; r < NPL; ++r) best = w[r] < best ? w[r] : best;
+          for (int r = NPL - 1; r >= 0; --r) at = w[r] == best ? r : at;
+          const int gone = lane == owner ? at : NPL;
+          mine = ~0u;
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-              const uint64_t o = shfl_xor_u64(best, off);
-              best = o < best ? o : best;
-            }
-            if (best == ~0ull) break;   // the row has no further entry: not reached, let the sort path say so
+          for (int r = 0; r < NPL; ++r) {
+            w[r] = r == gone ? ~0u : w[r];
+            mine = min(mine, w[r]);
           }
-          if (lane == it) my_idx = (uint32_t)best;
-#pragma unroll
-          for (int r = 0; r < NPL; ++r) w[r] = (w[r] == best) ? ~0ull : w[r];
-          cum += (double)desc_key_value(best);
+          const int idx = owner * NPL + __builtin_amdgcn_readlane(at, owner);
+          if (lane == it) my_idx = idx;
+          cum += (double)f32_from_orderable(~best);
           taken = it + 1;
           if ((float)cum >= thr) {
             decided = true;
             break;
           }
+          best = wave_min_u32(mine);
         }
         if (decided && lane < taken) flag[my_idx] = 1;
       }
@@ -345,22 +415,16 @@ __device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t 
     // The sort runs on the 32-bit value keys alone (ascending key = descending value).  Entries of equal value are
     // interchangeable in the running sum; which of them the stable order takes first matters only for the value at
     // which the threshold is reached, and is settled there by index (below).
-    uint32_t kv[NPL], k0v[NPL];
+    uint32_t kv[NPL];
 #pragma unroll
-    for (int r = 0; r < NPL; ++r) kv[r] = k0v[r] = (uint32_t)(k[r] >> 32);
+    for (int r = 0; r < NPL; ++r) kv[r] = k0v[r];
     wave_bitonic_sort_u32<NPL>(kv, lane);
 
-    float v[NPL];
-#pragma unroll
-    for (int r = 0; r < NPL; ++r) v[r] = (lane * NPL + r < count) ? f32_from_orderable(~kv[r]) : 0.f;
+    auto value = [&](int r) __attribute__((always_inline)) { return lane * NPL + r < count ? f32_from_orderable(~kv[r]) : 0.f; };
     // parallel float64 prefix
-    double loc[NPL];
     double c = 0.0;
 #pragma unroll
-    for (int r = 0; r < NPL; ++r) {
-      c += (double)v[r];
-      loc[r] = c;
-    }
+    for (int r = 0; r < NPL; ++r) c += (double)value(r);
     double incl = c;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -371,12 +435,15 @@ __device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t 
     if (lane == 0) excl = 0.0;
     // float32 rounding boundary of the threshold (midpoint to its predecessor), as a double
     const double mid = 0.5 * ((double)thr + (double)nextafterf(thr, -INFINITY));
+    const double tol = 1e-11 * fmax(1.0, fabs(mid));
     uint32_t reach = 0, amb = 0;
+    c = 0.0;
 #pragma unroll
     for (int r = 0; r < NPL; ++r) {
-      const double cp = excl + loc[r];
+      c += (double)value(r);
+      const double cp = excl + c;
       reach |= ((float)cp >= thr ? 1u : 0u) << r;
-      amb |= (fabs(cp - mid) <= 1e-11 * fmax(1.0, fabs(mid)) ? 1u : 0u) << r;
+      amb |= (fabs(cp - mid) <= tol ? 1u : 0u) << r;
     }
     int first = reach ? lane * NPL + __builtin_ctz(reach) : INT_MAX;
 #pragma unroll
@@ -394,7 +461,7 @@ __device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t 
         uint32_t rch = 0;
 #pragma unroll
         for (int r = 0; r < NPL; ++r) {
-          cs += (double)v[r];
+          cs += (double)value(r);
           rch |= ((float)cs >= thr ? 1u : 0u) << r;
         }
         const uint32_t rl = (uint32_t)__builtin_amdgcn_readlane((int)rch, L);
@@ -409,10 +476,10 @@ __device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t 
     if (first >= 0) {
       // the selection is ranks 0 .. first of the stable order: every entry above the value at rank `first`, and of
       // the entries equal to it the m lowest indices, m = first + 1 - (number of entries above it)
-      uint32_t mine = 0;
+      uint32_t at_first = 0;
 #pragma unroll
-      for (int r = 0; r < NPL; ++r) mine = (r == first % NPL) ? kv[r] : mine;
-      const uint32_t kstar = (uint32_t)__builtin_amdgcn_readlane((int)mine, first / NPL);
+      for (int r = 0; r < NPL; ++r) at_first = (r == first % NPL) ? kv[r] : at_first;
+      const uint32_t kstar = (uint32_t)__builtin_amdgcn_readlane((int)at_first, first / NPL);
       int above = 0, ties = 0;
 #pragma unroll
       for (int r = 0; r < NPL; ++r) {
@@ -445,6 +512,22 @@ __device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t 
     const int fb = a.first_blk[row];
     if (fb >= 0 && fb < nb) flag[fb] = 1;
   }
+}
+
+// one wave decides row `rq` ((row, qb - qb_lo) flattened) of the group of rows [qb_lo, qb_hi) x all heads
+template <int NPL>
+__device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t rq, int total_rows, uint8_t* smem_w) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nb = a.nb;
+  const int nb_pad = (nb + 15) & ~15;
+  uint8_t* flag = smem_w + wave * nb_pad;
+  if (rq >= total_rows) return;
+  const int nqb = a.qb_hi - a.qb_lo;
+  const int row = (int)(rq / nqb), qb = a.qb_lo + (int)(rq % nqb);
+  const int seg_first = (qb / a.bps) * a.bps;
+  const int seg_end = min(seg_first + a.bps, nb);
+  const int64_t row_off = ((int64_t)row * nb + qb) * nb;
+  decide_row<NPL>(a, row, qb, flag);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -499,6 +582,100 @@ __global__ __launch_bounds__(256) void select_blocks_groups_kernel(SelectArgs a,
     case 4: select_row_by_wave<4>(a, rq, total, smem_w); break;
     case 8: select_row_by_wave<8>(a, rq, total, smem_w); break;
     default: select_row_by_wave<16>(a, rq, total, smem_w); break;
+  }
+}
+
+// ---- the single-call path: selection straight into the merged lists that the attention kernel reads (pbs_lists.h).
+// A workgroup decides the rows of two pairs of query blocks, one wave each, into flags in LDS; then the first wave of a
+// pair writes the pair's list and the second one the gather's flags.  No CSR rows (4 bytes per visited block and row, written
+// here and read back) and no launch that merges them.  Groups are in pairs here: qb_lo / qb_hi are pair numbers.
+// LONG: rows of 1025 .. 2048 candidates, in a kernel of their own: the register need of 32 entries per lane would cost the shorter
+// rows two thirds of their waves.
+template <bool LONG>
+__global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, PairLists l, SelectGroups gr, int rows) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem_w[];
+  int g = 0;
+  while (g + 1 < gr.n && (int)blockIdx.x >= gr.wg_end[g]) ++g;
+  const int wg0 = g == 0 ? 0 : gr.wg_end[g - 1];
+  const int n_pairs = gr.qb_hi[g] - gr.qb_lo[g], total = rows * n_pairs;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int unit = ((int)blockIdx.x - wg0) * 2 + (wave >> 1);
+  const bool live = unit < total;
+  const int row = live ? unit / n_pairs : 0, pair = gr.qb_lo[g] + (live ? unit - row * n_pairs : 0);
+  const int nb = a.nb, nb_pad = (nb + 15) & ~15, npair = (nb + 1) >> 1;
+  const int qb0 = 2 * pair, qb = qb0 + (wave & 1);
+  uint8_t* flag = smem_w + wave * nb_pad;
+  if (blockIdx.x == 0 && threadIdx.x < 8) l.queue[threadIdx.x] = l.first_tickets;
+  if (live && qb < nb) {
+    if constexpr (LONG) {
+      decide_row<32>(a, row, qb, flag);
+    } else {
+      switch (gr.npl[g]) {
+        case 1: decide_row<1>(a, row, qb, flag); break;
+        case 2: decide_row<2>(a, row, qb, flag); break;
+        case 4: decide_row<4>(a, row, qb, flag); break;
+        case 8: decide_row<8>(a, row, qb, flag); break;
+        default: decide_row<16>(a, row, qb, flag); break;
+      }
+    }
+  }
+  __syncthreads();
+  if (!live) return;
+  const bool second = qb0 + 1 < nb;
+  const int qb1 = second ? qb0 + 1 : qb0;
+  const int sf0 = (qb0 / a.bps) * a.bps, sf1 = (qb1 / a.bps) * a.bps;
+  const int end1 = second ? sf1 : 0, end = max(sf0, end1);   // a row's flags count up to its own segment
+  const uint32_t* f0 = reinterpret_cast<const uint32_t*>(smem_w + (wave & 2) * nb_pad);
+  const uint32_t* f1 = reinterpret_cast<const uint32_t*>(smem_w + ((wave & 2) + 1) * nb_pad);
+  // the flags of blocks 4 x .. 4 x + 3, a byte each: bit 0 visited by the first query block, bit 1 by the second
+  auto visited = [&](int x) __attribute__((always_inline)) {
+    auto below = [&](int n) __attribute__((always_inline)) {   // bytes of blocks below n
+      const int valid = n - 4 * x;
+      return valid >= 4 ? ~0u : valid <= 0 ? 0u : (1u << (8 * valid)) - 1u;
+    };
+    const uint32_t m0 = below(sf0), m1 = below(end1);
+    return (m0 ? f0[x] & m0 : 0u) | (m1 ? f1[x] & m1 : 0u) << 1;
+  };
+  if (wave & 1) {
+    if (a.needed)
+      for (int x = lane; 4 * x < end; x += 64) {
+        const uint32_t v = visited(x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (v >> (8 * e) & 3u) a.needed[(int64_t)row * nb + 4 * x + e] = 1;   // every writer stores the same value
+      }
+    return;
+  }
+  uint16_t* header = l.plist + ((int64_t)row * npair + (npair - 1 - pair)) * l.cap;
+  uint16_t* out = header + LIST_HEADER;
+  int base = 0;
+  for (int x0 = 0; 4 * x0 < end; x0 += 64) {
+    const int x = x0 + lane;
+    const uint32_t v = 4 * x < end ? visited(x) : 0u;
+    const int n = __popc((v | v >> 1) & 0x01010101u);
+    // prefix of n (0 .. 4) over the lanes, a bit of it at a time
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint64_t b0 = __ballot(n & 1), b1 = __ballot(n & 2), b2 = __ballot(n & 4);
+    int w = base + __popcll(b0 & below) + 2 * __popcll(b1 & below) + 4 * __popcll(b2 & below);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t use = v >> (8 * e) & 3u;
+      if (use) out[w++] = (uint16_t)((uint32_t)(4 * x + e) | use << 14);
+    }
+    base += __popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2);
+  }
+  const int n_own = qb1 - sf0 + 1;
+  for (int t = lane; t < n_own; t += 64) {
+    const int kb = sf0 + t;
+    const uint32_t use = (kb <= qb0 ? 1u : 0u) | (second && kb >= sf1 ? 2u : 0u);
+    out[base + t] = (uint16_t)((uint32_t)kb | ENT_ORIG | use << 14);
+  }
+  if (lane == 0) {
+    header[0] = (uint16_t)(base + n_own);
+    header[1] = (uint16_t)(row / l.Hq);
+    header[2] = (uint16_t)(row % l.Hq);
+    header[3] = (uint16_t)(row % l.Hq / l.group);
+    header[4] = (uint16_t)qb0;
   }
 }
 
@@ -628,4 +805,49 @@ extern "C" int pbs_select_blocks(const float* block_attn_scores, const float* th
   const size_t lds = (size_t)a.n_pow2 * sizeof(uint64_t) + (size_t)((nb + 15) / 16) * 16;
   hipLaunchKernelGGL(select_blocks_kernel, dim3(nb, rows), dim3(256), lds, st, a);
   return pbs_check_launch("pbs_select_blocks");
+}
+
+int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold_per_row, float threshold, const int32_t* first_blk,
+                          int rows, int S, int block_size, int segment_size, uint8_t* block_needed, const PairLists& lists,
+                          void* stream) {
+  const int nb = (S + block_size - 1) / block_size, npair = (nb + 1) / 2;
+  PBS_REQUIRE(rows > 0 && rows <= 65535 && nb <= PBS_PAIR_SELECT_MAX_BLOCKS, "pbs_select_pair_lists: bad shape");
+  SelectArgs a = {};
+  a.P = block_attn_scores; a.thr_rows = threshold_per_row; a.thr = threshold;
+  a.force_first = first_blk != nullptr;
+  a.first_blk = const_cast<int32_t*>(first_blk);
+  a.nb = nb; a.bs = block_size; a.bps = segment_size / block_size; a.S = S;
+  a.needed = block_needed;
+  a.cand_rule = 1;
+  // groups of pairs whose second row's candidates fit 64 * npl sorted entries, longest first
+  int npl[6], lo[6], hi[6], n = 0, from = 0;
+  for (int x = 1; x <= 32 && from < npair; x *= 2) {
+    const int64_t blocks = (64 * x / a.bps + 1) * (int64_t)a.bps;   // query blocks with at most 64 x candidates
+    const int to = blocks >= nb ? npair : (int)(blocks / 2);
+    if (to > from) {
+      npl[n] = x; lo[n] = from; hi[n] = to;
+      ++n;
+      from = to;
+    }
+  }
+  const size_t lds = (size_t)4 * ((nb + 15) & ~15);
+  SelectGroups gr;
+  gr.n = 0;
+  int wgs = 0;
+  for (int x = n - 1; x >= 0; --x) {
+    if (npl[x] == 32) {
+      SelectGroups one;
+      one.n = 1;
+      one.npl[0] = 32; one.qb_lo[0] = lo[x]; one.qb_hi[0] = hi[x];
+      one.wg_end[0] = (rows * (hi[x] - lo[x]) + 1) / 2;
+      hipLaunchKernelGGL(select_pair_lists_kernel<true>, dim3((unsigned)one.wg_end[0]), dim3(256), lds, (hipStream_t)stream, a, lists, one, rows);
+      continue;
+    }
+    gr.npl[gr.n] = npl[x]; gr.qb_lo[gr.n] = lo[x]; gr.qb_hi[gr.n] = hi[x];
+    wgs += (rows * (hi[x] - lo[x]) + 1) / 2;
+    gr.wg_end[gr.n++] = wgs;
+  }
+  if (wgs)
+    hipLaunchKernelGGL(select_pair_lists_kernel<false>, dim3((unsigned)wgs), dim3(256), lds, (hipStream_t)stream, a, lists, gr, rows);
+  return pbs_check_launch("pbs_select_pair_lists");
 }

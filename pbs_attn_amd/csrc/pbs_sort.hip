@@ -4,13 +4,13 @@
 // composite keys (inverted order-preserving score bits << 32 | local index), so
 // equal scores keep ascending index order whatever the network does.  The
 // trailing partial segment and the padding up to a whole block keep identity order.
-#include "pbs_common.h"
+#include "pbs_lists.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 
 namespace {
 
 __global__ __launch_bounds__(256) void segment_argsort_kernel(const float* scores, int32_t* idx, int S, int Sc,
-                                                              int S_pad, int seg, int n_pow2) {
+                                                              int S_pad, int seg, int n_pow2, int32_t* first_blk, int block_size) {
   extern __shared__ uint64_t keys[];
   const int row = blockIdx.y;
   const int nseg = Sc / seg;
@@ -27,12 +27,15 @@ __global__ __launch_bounds__(256) void segment_argsort_kernel(const float* score
     keys[i] = i < seg ? desc_stable_key(src[i], (uint32_t)i) : ~0ull;
   bitonic_sort_lds(keys, n_pow2);
   for (int i = threadIdx.x; i < seg; i += blockDim.x) out[base + i] = base + (int32_t)(uint32_t)keys[i];
+  if (first_blk && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < seg; i += blockDim.x)
+      if ((uint32_t)keys[i] == 0) first_blk[row] = i / block_size;
 }
 
 }  // namespace
 
-extern "C" int pbs_segment_argsort(const float* scores, int32_t* key_indices, int rows, int S, int S_pad,
-                                   int segment_size, void* stream) {
+int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,
+                               int S_pad, int segment_size, void* stream) {
   PBS_REQUIRE(key_indices, "pbs_segment_argsort: null index pointer");
   PBS_REQUIRE(rows > 0 && S > 0 && S_pad >= S, "pbs_segment_argsort: bad shape rows=%d S=%d S_pad=%d", rows, S, S_pad);
   PBS_REQUIRE(segment_size > 0 && segment_size <= 8192, "pbs_segment_argsort: segment_size %d outside (0, 8192]", segment_size);
@@ -43,6 +46,12 @@ extern "C" int pbs_segment_argsort(const float* scores, int32_t* key_indices, in
   const int n_pow2 = next_pow2_int(segment_size);
   PBS_REQUIRE(rows <= 65535, "pbs_segment_argsort: too many rows (%d)", rows);
   hipLaunchKernelGGL(segment_argsort_kernel, dim3(nseg + tail_blocks, rows), dim3(256), (size_t)n_pow2 * sizeof(uint64_t),
-                     (hipStream_t)stream, scores, key_indices, S, Sc, S_pad, segment_size, n_pow2);
+                     (hipStream_t)stream, scores, key_indices, S, Sc, S_pad, segment_size, n_pow2,
+                     first_blk, block_size);
   return pbs_check_launch("pbs_segment_argsort");
+}
+
+extern "C" int pbs_segment_argsort(const float* scores, int32_t* key_indices, int rows, int S, int S_pad,
+                                   int segment_size, void* stream) {
+  return pbs_segment_argsort_launch(scores, key_indices, nullptr, 1, rows, S, S_pad, segment_size, stream);
 }

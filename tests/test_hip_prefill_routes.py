@@ -35,3 +35,18 @@ def _single_and_staged(dev, B, Hq, Hkv, S, seg, thr, kind="uniform_heavy", **kw)
 ])
 def test_routes_without_a_selection(dev, B, Hq, Hkv, S, seg, thr):
     assert torch.equal(*_single_and_staged(dev, B, Hq, Hkv, S, seg, thr))
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,seg,thr,kind,kw", [
+    (2, 3, 1, 1111, 384, 0.8, "uniform_heavy", dict(query_pool_mode="max", key_pool_mode="max")),   # odd blocks per segment, pairs across segments
+    (1, 4, 2, 257, 256, 0.9, "uniform_heavy", {}),                  # one complete segment, the last pair a single row
+    (1, 5, 5, 130 * 128 + 1, 128, "rows", "strong_uniform", {}),    # groups of 64 / 128 / 256 candidates that end inside a pair
+    (1, 2, 1, 66 * 128, 128, 1.0, "strong_heavy", dict(force_select_first_block=False)),   # sums that may never reach the threshold
+    (1, 2, 2, 9000, 512, 0.0, "uniform_heavy", {}),                 # rows without candidates are flagged too
+    (1, 2, 1, 1024 * 128, 1024, 0.9, "strong_heavy", {}),           # 1024 blocks: the longest rows of the short kernel
+    (1, 1, 1, 1025 * 128 + 7, 384, 0.9, "strong_uniform", {}),      # beyond: lists against the block-level sort
+    (1, 1, 1, 2048 * 128, 128, 0.95, "uniform_heavy", {}),          # the longest rows of the list-writing selection
+    (1, 1, 1, 2048 * 128 + 1, 2048, 0.3, "uniform_heavy", {}),      # one block more: CSR rows and a merge
+])
+def test_selection_into_pair_lists(dev, B, Hq, Hkv, S, seg, thr, kind, kw):
+    assert torch.equal(*_single_and_staged(dev, B, Hq, Hkv, S, seg, thr, kind, **kw))
