@@ -136,56 +136,79 @@ __global__ __launch_bounds__(256, 2) void score_kernel(ScoreArgs a) {
       if (st + 1 < n_stages)
         stage_keys_async(kbase + (int64_t)(key_lo + (st + 1) * STAGE_KEYS) * a.k_ss, a.k_ss, buf ^ STAGE_BYTES, wave, nwaves, lane);
       if (!active) continue;
-#pragma unroll
-      for (int sub = 0; sub < STAGE_KEYS / KEYS_PER_WAVE_STEP; ++sub) {
-        const int key = key_lo + st * STAGE_KEYS + sub * KEYS_PER_WAVE_STEP + j;   // always < Sc
-        bf16x8 kf[8];
+      // Eight logit tiles (32 keys x 32 queries) per stage, one ahead: the matrix instructions of tile i + 1 go out among the
+      // vector work of tile i (left to itself the compiler issues a tile's eight in a row, each waiting for the one
+      // before).  What bounds the pass is the vector unit: per pair of logits 4 conversions, 2 multiplications, 2 multiply-adds,
+      // 2 exponentials (two slots each), 2 additions and, here, a maximum.  Both passes together: 256k head shard
+      // 210 -> 193 us, 128k 418 -> 397 us, 32k 111 -> 107 us (with the one-instruction rounding of pbs_common.h).
+      constexpr int TILES = 4 * STAGE_KEYS / KEYS_PER_WAVE_STEP;
+      bf16x8 kf[8];
+      f32x16 acc_next = {0};
+      auto load_keys = [&](int sub) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) kf[t] = lds_frag(buf + (uint32_t)sub * 8192u + (frag0 ^ (uint32_t)(t << 5)));
-
+      };
+      auto multiply = [&](int qt) __attribute__((always_inline)) {
+        acc_next = (f32x16){0};
+#pragma unroll
+        for (int t = 0; t < 8; ++t)   // rows = keys and columns = queries, or (FINAL) the other way round
+          acc_next = FINAL ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[qt][t], kf[t], acc_next, 0, 0, 0)
+                           : __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t], qf[qt][t], acc_next, 0, 0, 0);
+      };
+      load_keys(0);
+      multiply(0);
+      __builtin_amdgcn_sched_barrier(0);
+      float accp = 0.f;
+#pragma unroll
+      for (int i = 0; i < TILES; ++i) {
+        const int sub = i >> 2, qt = i & 3;
+        const f32x16 acc = acc_next;
+        if (qt == 3 && i + 1 < TILES) load_keys(sub + 1);
+        if (i + 1 < TILES) multiply((i + 1) & 3);
         if (!FINAL) {
-          // S^T tile: rows = keys, column = query j of sub-tile qt
+          float v[16], mx = -INFINITY;   // logits before the log2(e) factor
 #pragma unroll
-          for (int qt = 0; qt < 4; ++qt) {
-            f32x16 acc = {0};
-#pragma unroll
-            for (int t = 0; t < 8; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t], qf[qt][t], acc, 0, 0, 0);
-            float v[16], mx = -INFINITY;   // logits before the log2(e) factor
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-              const f32x2 l2 = logit2(acc[r], acc[r + 1], a.inv_sqrt_d);
-              v[r] = l2.x;
-              v[r + 1] = l2.y;
-              mx = fmaxf(fmaxf(mx, l2.x), l2.y);
-            }
-            const float m_new = fmaxf(m_run[qt], mx * LOG2E);
-            float sum = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sum += __builtin_amdgcn_exp2f(__builtin_fmaf(v[r], LOG2E, -m_new));
-            l_run[qt] = l_run[qt] * __builtin_amdgcn_exp2f(m_run[qt] - m_new) + sum;
-            m_run[qt] = m_new;
+          for (int r = 0; r < 16; r += 2) {
+            const f32x2 l2 = logit2(acc[r], acc[r + 1], a.inv_sqrt_d);
+            v[r] = l2.x;
+            v[r + 1] = l2.y;
+            mx = fmaxf(fmaxf(mx, l2.x), l2.y);
           }
+          const float m_new = fmaxf(m_run[qt], mx * LOG2E);
+          float sum = 0.f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sum += __builtin_amdgcn_exp2f(__builtin_fmaf(v[r], LOG2E, -m_new));
+          l_run[qt] = l_run[qt] * __builtin_amdgcn_exp2f(m_run[qt] - m_new) + sum;
+          m_run[qt] = m_new;
         } else {
-          // S tile: rows = queries of sub-tile qt, column = key j
-          float accp = 0.f;
 #pragma unroll
-          for (int qt = 0; qt < 4; ++qt) {
-            f32x16 acc = {0};
-#pragma unroll
-            for (int t = 0; t < 8; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[qt][t], kf[t], acc, 0, 0, 0);
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-              const float4 st4 = *reinterpret_cast<const float4*>(&s_stats[32 * qt + 8 * r4 + 4 * half]);
-              const f32x2 la = logit2(acc[4 * r4 + 0], acc[4 * r4 + 1], a.inv_sqrt_d);
-              const f32x2 lb = logit2(acc[4 * r4 + 2], acc[4 * r4 + 3], a.inv_sqrt_d);
-              accp += __builtin_amdgcn_exp2f(__builtin_fmaf(la.x, LOG2E, -st4.x));
-              accp += __builtin_amdgcn_exp2f(__builtin_fmaf(la.y, LOG2E, -st4.y));
-              accp += __builtin_amdgcn_exp2f(__builtin_fmaf(lb.x, LOG2E, -st4.z));
-              accp += __builtin_amdgcn_exp2f(__builtin_fmaf(lb.y, LOG2E, -st4.w));
-            }
+          for (int r4 = 0; r4 < 4; ++r4) {
+            const float4 st4 = *reinterpret_cast<const float4*>(&s_stats[32 * qt + 8 * r4 + 4 * half]);
+            const f32x2 la = logit2(acc[4 * r4 + 0], acc[4 * r4 + 1], a.inv_sqrt_d);
+            const f32x2 lb = logit2(acc[4 * r4 + 2], acc[4 * r4 + 3], a.inv_sqrt_d);
+            accp += __builtin_amdgcn_exp2f(__builtin_fmaf(la.x, LOG2E, -st4.x));
+            accp += __builtin_amdgcn_exp2f(__builtin_fmaf(la.y, LOG2E, -st4.y));
+            accp += __builtin_amdgcn_exp2f(__builtin_fmaf(lb.x, LOG2E, -st4.z));
+            accp += __builtin_amdgcn_exp2f(__builtin_fmaf(lb.y, LOG2E, -st4.w));
           }
-          accp += xhalf_f32(accp);
-          if (half == 0) a.scores[(int64_t)bh * a.Sc + key] = accp * (1.0f / NQ);
+        }
+        if (i + 1 < TILES) {
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+            if (qt == 3 && t == 0) {   // the next keys, and time for them to arrive
+              __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+              __builtin_amdgcn_sched_group_barrier(0x2, 30, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x2, 11, 0);                           // vector instructions
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                            // a matrix instruction
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (FINAL && qt == 3) {
+          const float total = accp + xhalf_f32(accp);
+          accp = 0.f;
+          const int key = key_lo + st * STAGE_KEYS + sub * KEYS_PER_WAVE_STEP + j;   // always < Sc
+          if (half == 0) a.scores[(int64_t)bh * a.Sc + key] = total * (1.0f / NQ);
         }
       }
     }
