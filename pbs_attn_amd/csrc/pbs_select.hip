@@ -274,43 +274,73 @@ __device__ __forceinline__ void cross_lane_stage(uint32_t (&k)[NPL], int lane) {
     k[r] = med3_u32(t.a, t.b, side);
   }
 }
-// The bitonic network on 32-bit keys, NPL per lane.  Where the direction of a stage depends on the lane, the keys of the
-// descending lanes are complemented for the phase, so that every exchange is a plain minimum and maximum.
+// the stages of strides 2^n - 1 .. 1 inside a lane's keys, ascending or, for `size` < NPL, by the register's place
+template <int NPL>
+__device__ __forceinline__ void local_stages(uint32_t (&k)[NPL], int size) {
+#pragma unroll
+  for (int stride = min(size, NPL) >> 1; stride > 0; stride >>= 1) {
+#pragma unroll
+    for (int r = 0; r < NPL; ++r) {
+      if ((r & stride) == 0) {
+        const int p = r | stride;
+        const bool up = size >= NPL || (r & size) == 0;
+        const uint32_t lo = min(k[r], k[p]), hi = max(k[r], k[p]);
+        k[r] = up ? lo : hi;
+        k[p] = up ? hi : lo;
+      }
+    }
+  }
+}
+// a phase: runs of NPL * LANES / 2 keys become runs of NPL * LANES (LANES 1: a lane's own keys).  Where the direction depends
+// on the lane, the keys of the descending lanes are complemented for the phase, so that every exchange is a plain minimum
+// and maximum; `flipped` is the complement the keys carry from the phase before.
+template <int NPL>
+__device__ __forceinline__ void begin_phase(uint32_t (&k)[NPL], int lanes, int lane, uint32_t& flipped) {
+  const uint32_t flip = (lane & lanes) ? ~0u : 0u, change = flip ^ flipped;
+#pragma unroll
+  for (int r = 0; r < NPL; ++r) k[r] ^= change;
+  flipped = flip;
+}
+template <int NPL, int LANES>
+__device__ __forceinline__ void phase(uint32_t (&k)[NPL], int lane, uint32_t& flipped) {
+  begin_phase<NPL>(k, LANES, lane, flipped);
+  if constexpr (LANES >= 64) cross_lane_stage<NPL, 32>(k, lane);
+  if constexpr (LANES >= 32) cross_lane_stage<NPL, 16>(k, lane);
+  if constexpr (LANES >= 16) cross_lane_stage<NPL, 8>(k, lane);
+  if constexpr (LANES >= 8) cross_lane_stage<NPL, 4>(k, lane);
+  if constexpr (LANES >= 4) cross_lane_stage<NPL, 2>(k, lane);
+  if constexpr (LANES >= 2) cross_lane_stage<NPL, 1>(k, lane);
+  local_stages<NPL>(k, NPL);
+}
+// The bitonic network on 32-bit keys, NPL per lane.  Short rows have it unrolled.  With 32 keys per lane the phases that
+// reach across lanes are a loop over one copy of each stage: unrolled, the compiler gave the long rows twice the time
+// (rows of 1025 .. 2048 blocks of a 256k head shard: 361 us unrolled, 169 us as a loop; the short rows of a 4k prompt: 6.2
+// unrolled against 7.5 us).
 template <int NPL>
 __device__ __forceinline__ void wave_bitonic_sort_u32(uint32_t (&k)[NPL], int lane) {
-  constexpr int N = 64 * NPL;
+#pragma unroll
+  for (int size = 2; size < NPL; size <<= 1) local_stages<NPL>(k, size);
   uint32_t flipped = 0;
-#pragma unroll
-  for (int size = 2; size <= N; size <<= 1) {
-    if (size >= NPL) {
-      const uint32_t flip = (lane & (size / NPL)) ? ~0u : 0u;
-      const uint32_t change = flip ^ flipped;
-#pragma unroll
-      for (int r = 0; r < NPL; ++r) k[r] ^= change;
-      flipped = flip;
-    }
-#pragma unroll
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      if (stride >= NPL) {
-        switch (stride / NPL) {
-          case 1: cross_lane_stage<NPL, 1>(k, lane); break;
-          case 2: cross_lane_stage<NPL, 2>(k, lane); break;
-          case 4: cross_lane_stage<NPL, 4>(k, lane); break;
-          case 8: cross_lane_stage<NPL, 8>(k, lane); break;
-          case 16: cross_lane_stage<NPL, 16>(k, lane); break;
-          default: cross_lane_stage<NPL, 32>(k, lane); break;
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < NPL; ++r) {
-          if ((r & stride) == 0) {
-            const int p = r | stride;
-            const bool up = size >= NPL || (r & size) == 0;
-            const uint32_t lo = min(k[r], k[p]), hi = max(k[r], k[p]);
-            k[r] = up ? lo : hi;
-            k[p] = up ? hi : lo;
-          }
-        }
+  if constexpr (NPL < 32) {
+    phase<NPL, 1>(k, lane, flipped);
+    phase<NPL, 2>(k, lane, flipped);
+    phase<NPL, 4>(k, lane, flipped);
+    phase<NPL, 8>(k, lane, flipped);
+    phase<NPL, 16>(k, lane, flipped);
+    phase<NPL, 32>(k, lane, flipped);
+    phase<NPL, 64>(k, lane, flipped);
+  } else {
+#pragma nounroll
+    for (int lanes = 1; lanes <= 64; lanes <<= 1) {
+      begin_phase<NPL>(k, lanes, lane, flipped);
+      switch (lanes) {   // strides from lanes / 2 lanes down to one
+        case 64: cross_lane_stage<NPL, 32>(k, lane); [[fallthrough]];
+        case 32: cross_lane_stage<NPL, 16>(k, lane); [[fallthrough]];
+        case 16: cross_lane_stage<NPL, 8>(k, lane); [[fallthrough]];
+        case 8: cross_lane_stage<NPL, 4>(k, lane); [[fallthrough]];
+        case 4: cross_lane_stage<NPL, 2>(k, lane); [[fallthrough]];
+        case 2: cross_lane_stage<NPL, 1>(k, lane); [[fallthrough]];
+        default: local_stages<NPL>(k, NPL); break;
       }
     }
   }
