@@ -1,5 +1,6 @@
 """GPU: the routes of the single-call path (pbs_prefill_attn_fwd) against the stage-by-stage calls, bit for bit: the same
 tiles in the same order, whatever kernel wrote the visit lists.  Shapes at the edges of the routes."""
+import numpy as np
 import pytest
 import torch
 
@@ -50,3 +51,27 @@ def test_routes_without_a_selection(dev, B, Hq, Hkv, S, seg, thr):
 ])
 def test_selection_into_pair_lists(dev, B, Hq, Hkv, S, seg, thr, kind, kw):
     assert torch.equal(*_single_and_staged(dev, B, Hq, Hkv, S, seg, thr, kind, **kw))
+
+
+@pytest.mark.parametrize("seg", [1, 2, 7, 100, 128, 130, 256, 384, 512, 1000, 1024, 1025, 2048, 2049])
+def test_segment_sort_is_stable_for_every_score(dev, seg):
+    """One wave per segment up to 2048 keys, a workgroup beyond: against a stable sort of the same scores, with ties, both
+    zeros, infinities, subnormals and NaN (which counts as the largest), a partial last segment and block padding."""
+    from pbs_attn_amd import ops
+    nseg, rows = 3, 5
+    S = nseg * seg + seg // 2
+    g = torch.Generator().manual_seed(seg)
+    x = torch.randn((1, rows, nseg * seg), generator=g)
+    x[:, 1] = x[:, 1].round()                                   # many ties
+    x[:, 2] = torch.rand((nseg * seg,), generator=g) * 1e-38    # subnormal and tiny
+    special = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan"), 1e-45, -1e-45, 3.4e38])
+    x[:, 3] = special[torch.randint(0, 8, (nseg * seg,), generator=g)]
+    x[:, 4] = 0.0
+    idx = ops.segment_argsort(x.to(dev), S, seg, 128).cpu().long()
+    s_pad = (S + 127) // 128 * 128
+    v = x.view(rows, nseg, seg).double().numpy()
+    nan = np.isnan(v)
+    order = np.lexsort((np.broadcast_to(np.arange(seg), v.shape), -np.where(nan, 0.0, v), ~nan), axis=-1)
+    want = torch.from_numpy(order + np.arange(nseg)[:, None] * seg).view(1, rows, nseg * seg)
+    tail = torch.arange(nseg * seg, s_pad).expand(1, rows, -1)
+    assert torch.equal(idx, torch.cat((want, tail), -1))
