@@ -1,10 +1,10 @@
 // Key scoring: mean over the last 128 queries of softmax(Q_last K^T / sqrt(D))
 // over all keys of the complete segments (no causal mask).
 //
-// Three launches, K is read twice (each time once per workgroup, through LDS) and never re-materialised:
+// Two or three launches, K is read twice (each time once per workgroup, through LDS) and never re-materialised:
 //   (all exponentials are base 2 on logits pre-multiplied by log2(e))
 //   1. score_partial : per (head, key chunk) online (max, sum-exp) of every query row
-//   2. score_reduce  : fold the chunk partials into row max + log2(row sum)
+//   2. score_reduce  : fold the chunk partials into row max + log2(row sum) (short sequences: part of 3)
 //   3. score_final   : recompute the logits and emit the per-key mean probability
 // Logits reproduce the rounding points of a bf16 matmul followed by a bf16
 // divide: fp32 accumulate -> bf16 -> / sqrt(D) -> bf16.
@@ -57,7 +57,9 @@ constexpr float LOG2E = 1.4426950408889634f;
 constexpr int STAGE_KEYS = 64;
 constexpr uint32_t STAGE_BYTES = STAGE_KEYS * D * 2;      // 16 KB
 constexpr uint32_t LDS_STATS = 2 * STAGE_BYTES;           // per wave: NQ floats (row max + log2 row sum)
-constexpr uint32_t LDS_SCORE_TOTAL = LDS_STATS + 4 * NQ * 4;
+constexpr uint32_t LDS_SCORE_TOTAL = LDS_STATS + 4 * NQ * 4;   // (SPLIT: NQ statistics and 4 x STAGE_KEYS sums)
+constexpr int SPLIT_MAX_CHUNKS = 32;                      // the final pass of the split form folds a query's chunks itself
+static_assert(STAGE_KEYS == PBS_WAVE && NQ + 4 * STAGE_KEYS <= 4 * NQ, "sums and statistics of the split form");
 
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
@@ -83,27 +85,33 @@ __device__ __forceinline__ void stage_keys_async(const uint16_t* rows, int64_t k
   }
 }
 
-// One wave per query head of the KV group; the waves of a workgroup share the staged key rows.
-template <bool FINAL>
-__global__ __launch_bounds__(256, 2) void score_kernel(ScoreArgs a) {
+// One wave per query head of the KV group; the waves of a workgroup share the staged key rows.  SPLIT (short sequences, see
+// score_plan): the four waves take 32 queries each of ONE head.
+// Waves per SIMD: the final pass of the split form needs 147 registers and would spill 18 of them at four.
+template <bool FINAL, bool SPLIT>
+__global__ __launch_bounds__(256, SPLIT ? (FINAL ? 3 : 4) : 2) void score_kernel(ScoreArgs a) {
+  constexpr int QT = SPLIT ? 1 : NQ / 32;   // query tiles of a wave
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // starts at LDS offset 0: this kernel has no static LDS
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int j = lane & 31, half = lane >> 5;
   const int G = a.Hq / a.Hkv;
-  const int b = blockIdx.y / a.Hkv, kvh = blockIdx.y % a.Hkv;
+  const int b = blockIdx.y / (SPLIT ? a.Hq : a.Hkv), in_batch = blockIdx.y % (SPLIT ? a.Hq : a.Hkv);
+  const int kvh = SPLIT ? in_batch / G : in_batch;
+  const int q_first = SPLIT ? 32 * wave : 0;
   const int chunk = blockIdx.x;
   const int key_lo = chunk * a.chunk_keys;
   const int key_hi = min(key_lo + a.chunk_keys, a.Sc);   // chunk_keys and Sc are multiples of STAGE_KEYS
   const int nwaves = (int)blockDim.x >> 6;
   const uint16_t* kbase = a.k + b * a.k_sb + kvh * a.k_sh;
-  float* s_stats = reinterpret_cast<float*>(smem + LDS_STATS) + wave * NQ;   // p = exp2(logit - stat)
+  float* s_stats = reinterpret_cast<float*>(smem + LDS_STATS) + wave * (32 * QT);   // p = exp2(logit - stat)
+  float* s_sums = reinterpret_cast<float*>(smem + LDS_STATS) + NQ;   // SPLIT: a wave's sums of the stage's keys
   // LDS byte offset of fragment 0 of key row j inside a stage buffer; fragment t lies at frag0 ^ (t << 5),
   // rows 32 .. 63 of the stage 8 KB further on
   const uint32_t frag0 = (uint32_t)(j * 256 + ((half ^ (j & 15)) * 16));
   const int n_stages = (key_hi - key_lo) / STAGE_KEYS;
 
-  for (int g0 = 0; g0 < G; g0 += nwaves) {
-    const int g = g0 + wave;
+  for (int g0 = 0; g0 < (SPLIT ? 1 : G); g0 += nwaves) {
+    const int g = SPLIT ? in_batch - kvh * G : g0 + wave;
     const bool active = g < G;
     const int h = kvh * G + (active ? g : 0);
     const int bh = b * a.Hq + h;
@@ -112,19 +120,36 @@ __global__ __launch_bounds__(256, 2) void score_kernel(ScoreArgs a) {
     __syncthreads();   // every wave is done with the stage buffers (and the statistics) of the previous group of heads
     stage_keys_async(kbase + (int64_t)key_lo * a.k_ss, a.k_ss, 0u, wave, nwaves, lane);
 
-    // the head's 128 scoring queries, resident for the whole chunk
-    bf16x8 qf[4][8];
+    // the wave's scoring queries, resident for the whole chunk
+    bf16x8 qf[QT][8];
 #pragma unroll
-    for (int qt = 0; qt < 4; ++qt)
+    for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-      for (int t = 0; t < 8; ++t) qf[qt][t] = load_frag(qbase + (int64_t)(32 * qt + j) * a.q_ss, t, half);
+      for (int t = 0; t < 8; ++t) qf[qt][t] = load_frag(qbase + (int64_t)(q_first + 32 * qt + j) * a.q_ss, t, half);
 
-    if (FINAL && active)
+    if (FINAL && SPLIT) {
+      // a query's chunks are few enough to be folded here: two lanes a query, all loads in flight
+      const float* p = a.part + ((int64_t)bh * a.nchunk * NQ + q_first + j) * 2;
+      float2 ml[SPLIT_MAX_CHUNKS / 2];
+#pragma unroll
+      for (int c = 0; c < SPLIT_MAX_CHUNKS / 2; ++c)
+        ml[c] = *reinterpret_cast<const float2*>(p + (int64_t)min(2 * c + half, a.nchunk - 1) * NQ * 2);
+      float m = ml[0].x, l = 0.f;   // (a chunk read twice does not move the maximum)
+#pragma unroll
+      for (int c = 1; c < SPLIT_MAX_CHUNKS / 2; ++c) m = fmaxf(m, ml[c].x);
+      m = fmaxf(m, xhalf_f32(m));
+#pragma unroll
+      for (int c = 0; c < SPLIT_MAX_CHUNKS / 2; ++c)
+        l += 2 * c + half < a.nchunk ? ml[c].y * __builtin_amdgcn_exp2f(ml[c].x - m) : 0.f;
+      l += xhalf_f32(l);
+      if (half == 0) s_stats[j] = m + __builtin_amdgcn_logf(l);   // log base 2
+    } else if (FINAL && active) {
       for (int i = lane; i < NQ; i += 64) s_stats[i] = a.stats[(int64_t)bh * NQ + i];
+    }
 
-    float m_run[4], l_run[4];
+    float m_run[QT], l_run[QT];
 #pragma unroll
-    for (int qt = 0; qt < 4; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
       m_run[qt] = -INFINITY;
       l_run[qt] = 0.f;
     }
@@ -136,12 +161,12 @@ __global__ __launch_bounds__(256, 2) void score_kernel(ScoreArgs a) {
       if (st + 1 < n_stages)
         stage_keys_async(kbase + (int64_t)(key_lo + (st + 1) * STAGE_KEYS) * a.k_ss, a.k_ss, buf ^ STAGE_BYTES, wave, nwaves, lane);
       if (!active) continue;
-      // Eight logit tiles (32 keys x 32 queries) per stage, one ahead: the matrix instructions of tile i + 1 go out among the
+      // Eight logit tiles (32 keys x 32 queries) per stage (SPLIT: two), one ahead: the matrix instructions of tile i + 1 go out among the
       // vector work of tile i (left to itself the compiler issues a tile's eight in a row, each waiting for the one
       // before).  What bounds the pass is the vector unit: per pair of logits 4 conversions, 2 multiplications, 2 multiply-adds,
       // 2 exponentials (two slots each), 2 additions and, here, a maximum.  Both passes together: 256k head shard
       // 210 -> 193 us, 128k 418 -> 397 us, 32k 111 -> 107 us (with the one-instruction rounding of pbs_common.h).
-      constexpr int TILES = 4 * STAGE_KEYS / KEYS_PER_WAVE_STEP;
+      constexpr int TILES = QT * STAGE_KEYS / KEYS_PER_WAVE_STEP;
       bf16x8 kf[8];
       f32x16 acc_next = {0};
       auto load_keys = [&](int sub) __attribute__((always_inline)) {
@@ -161,10 +186,10 @@ __global__ __launch_bounds__(256, 2) void score_kernel(ScoreArgs a) {
       float accp = 0.f;
 #pragma unroll
       for (int i = 0; i < TILES; ++i) {
-        const int sub = i >> 2, qt = i & 3;
+        const int sub = i / QT, qt = i % QT;
         const f32x16 acc = acc_next;
-        if (qt == 3 && i + 1 < TILES) load_keys(sub + 1);
-        if (i + 1 < TILES) multiply((i + 1) & 3);
+        if (qt == QT - 1 && i + 1 < TILES) load_keys(sub + 1);
+        if (i + 1 < TILES) multiply((i + 1) % QT);
         if (!FINAL) {
           float v[16], mx = -INFINITY;   // logits before the log2(e) factor
 #pragma unroll
@@ -195,7 +220,7 @@ __global__ __launch_bounds__(256, 2) void score_kernel(ScoreArgs a) {
         if (i + 1 < TILES) {
 #pragma unroll
           for (int t = 0; t < 8; ++t) {
-            if (qt == 3 && t == 0) {   // the next keys, and time for them to arrive
+            if (qt == QT - 1 && t == 0) {   // the next keys, and time for them to arrive
               __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
               __builtin_amdgcn_sched_group_barrier(0x2, 30, 0);
             }
@@ -204,22 +229,34 @@ __global__ __launch_bounds__(256, 2) void score_kernel(ScoreArgs a) {
           }
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (FINAL && qt == 3) {
+        if (FINAL && qt == QT - 1) {
           const float total = accp + xhalf_f32(accp);
           accp = 0.f;
-          const int key = key_lo + st * STAGE_KEYS + sub * KEYS_PER_WAVE_STEP + j;   // always < Sc
-          if (half == 0) a.scores[(int64_t)bh * a.Sc + key] = total * (1.0f / NQ);
+          const int in_stage = sub * KEYS_PER_WAVE_STEP + j;
+          const int key = key_lo + st * STAGE_KEYS + in_stage;   // always < Sc
+          if (half == 0) {
+            if (SPLIT) s_sums[wave * STAGE_KEYS + in_stage] = total;
+            else a.scores[(int64_t)bh * a.Sc + key] = total * (1.0f / NQ);
+          }
+        }
+      }
+      if (FINAL && SPLIT) {
+        __syncthreads();   // (the next stage's sums are written behind its first barrier)
+        if (wave == 0) {
+          const float* s = s_sums + lane;
+          a.scores[(int64_t)bh * a.Sc + key_lo + st * STAGE_KEYS + lane] =
+              ((s[0] + s[STAGE_KEYS]) + (s[2 * STAGE_KEYS] + s[3 * STAGE_KEYS])) * (1.0f / NQ);
         }
       }
     }
     if (!FINAL && active) {
 #pragma unroll
-      for (int qt = 0; qt < 4; ++qt) {
+      for (int qt = 0; qt < QT; ++qt) {
         const float m_o = xhalf_f32(m_run[qt]), l_o = xhalf_f32(l_run[qt]);
         const float m_new = fmaxf(m_run[qt], m_o);
         const float l_new = l_run[qt] * __builtin_amdgcn_exp2f(m_run[qt] - m_new) + l_o * __builtin_amdgcn_exp2f(m_o - m_new);
         if (half == 0) {
-          float* p = a.part + (((int64_t)bh * a.nchunk + chunk) * NQ + 32 * qt + j) * 2;
+          float* p = a.part + (((int64_t)bh * a.nchunk + chunk) * NQ + q_first + 32 * qt + j) * 2;
           p[0] = m_new;
           p[1] = l_new;
         }
@@ -268,12 +305,34 @@ int chunks_for(int Sc, int chunk_keys) { return (Sc + chunk_keys - 1) / chunk_ke
 // Keys per workgroup.  With one query head per KV head a workgroup is a single wave and starts from a
 // quarter of the keys; short sequences get shorter chunks until the launch has enough workgroups to
 // fill the chip (each workgroup re-reads its heads' 128 queries, so chunks stay >= 64 keys).
-int chunk_keys_for(int B, int Hq, int Hkv, int Sc) {
+//
+// The split form (a workgroup's waves share one head's queries) has 4 G workgroups for every 4 query heads of a KV head, a
+// quarter of the serial work and registers per wave, and folds the chunk partials without a launch of its own, but it stages each
+// key row once per query head.  It takes:
+//   * short sequences, where the grouped form leaves the chip idle or waiting.  Whole pass, grouped -> split, us: 28 / 4 heads x
+//     1000 keys 93.9 -> 72.9 (the three launches 37.4 -> 14.2, two launches), 32 / 8 x 600 66.7 -> 57.4, x 4096 191.9 -> 184.0, x 6000
+//     338 -> 328, 16 / 4 x 12000 526 -> 516; equal at 32 / 8 x 8192 (501, 504) and 4 / 1 x 30000, slower at 4 / 1 x 40000 (654 -> 681:
+//     SPLIT_MAX_CHUNKS workgroups a head no longer fill the chip), hence the two limits;
+//   * groups that leave waves of the grouped form idle: 28 / 4 x 9000 601 -> 567, 16 / 16 x 20000 783 -> 763 and x 131072 1485 ->
+//     1409, 8 / 8 x 131072 790 -> 760, 16 / 8 x 32768 460 -> 430, 14 / 2 x 65536 632 -> 624; at 28 / 4 x 65536, where an eighth is
+//     idle, the two are equal (1193, 1196), hence the limit for groups with less than a quarter idle.
+struct ScorePlan {
+  bool split;
+  int chunk_keys, nchunk;
+};
+ScorePlan score_plan(int B, int Hq, int Hkv, int Sc) {
   const bool grouped = Hq / Hkv > 1;
   int chunk = grouped ? KEYS_PER_WG : KEYS_PER_WG / 4;
   const int64_t want = grouped ? 512 : 2048;
   while (chunk > 64 && (int64_t)chunks_for(Sc, chunk) * B * Hkv < want) chunk /= 2;
-  return chunk;
+  const int64_t heads = (int64_t)B * Hq, keys = heads * Sc;
+  const int G = Hq / Hkv, slots = (G + 3) / 4 * 4, idle = slots - G;
+  const bool small = keys <= 3 << 16 && Sc <= 16384;
+  const bool uneven = idle > 0 && heads >= 8 && (4 * idle >= slots || keys <= 1 << 20);
+  const bool split = (small || uneven) && heads <= 65535;
+  if (split)
+    while (chunks_for(Sc, chunk) > SPLIT_MAX_CHUNKS) chunk *= 2;
+  return {split, chunk, chunks_for(Sc, chunk)};
 }
 
 }  // namespace
@@ -282,7 +341,7 @@ extern "C" size_t pbs_score_keys_workspace_bytes(int B, int Hq, int Hkv, int S, 
   if (segment_size <= 0 || B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv) return 0;
   const int Sc = (S / segment_size) * segment_size;
   if (Sc == 0) return 0;
-  return (size_t)B * Hq * ((size_t)chunks_for(Sc, chunk_keys_for(B, Hq, Hkv, Sc)) + 1) * NQ * 2 * sizeof(float);
+  return (size_t)B * Hq * ((size_t)score_plan(B, Hq, Hkv, Sc).nchunk + 1) * NQ * 2 * sizeof(float);
 }
 
 namespace {
@@ -315,23 +374,32 @@ int score_keys_launch(const char* who, const void* q, const void* k, float* scor
   a.q_sb = q_sb; a.q_sh = q_sh; a.q_ss = q_ss;
   a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = k_ss;
   a.inv_sqrt_d = (float)(1.0 / sqrt((double)head_dim));
-  a.chunk_keys = chunk_keys_for(B, Hq, Hkv, Sc);
-  a.nchunk = chunks_for(Sc, a.chunk_keys);
+  const ScorePlan plan = score_plan(B, Hq, Hkv, Sc);
+  a.chunk_keys = plan.chunk_keys;
+  a.nchunk = plan.nchunk;
   a.part = (float*)workspace;
   a.stats = a.part + (size_t)B * Hq * a.nchunk * NQ * 2;
   a.scores = scores;
   static std::atomic<bool> lds_checked{false};   // once per process: a property of the code object
   if (!lds_checked.load(std::memory_order_acquire)) {
-    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<false>, who)) return rc;
-    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true>, who)) return rc;
+    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<false, false>, who)) return rc;
+    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, false>, who)) return rc;
+    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<false, true>, who)) return rc;
+    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, true>, who)) return rc;
     lds_checked.store(true, std::memory_order_release);
   }
   hipStream_t st = (hipStream_t)stream;
+  if (plan.split) {
+    const dim3 grid(a.nchunk, B * Hq);
+    hipLaunchKernelGGL((score_kernel<false, true>), grid, dim3(256), LDS_SCORE_TOTAL, st, a);
+    hipLaunchKernelGGL((score_kernel<true, true>), grid, dim3(256), LDS_SCORE_TOTAL, st, a);
+    return pbs_check_launch(who);
+  }
   dim3 grid(a.nchunk, B * Hkv);
   const dim3 block(Hq / Hkv > 1 ? 256 : 64);
-  hipLaunchKernelGGL(score_kernel<false>, grid, block, LDS_SCORE_TOTAL, st, a);
+  hipLaunchKernelGGL((score_kernel<false, false>), grid, block, LDS_SCORE_TOTAL, st, a);
   hipLaunchKernelGGL(score_reduce_kernel, dim3(B * Hq), dim3(NQ * REDUCE_LANES), 0, st, a);
-  hipLaunchKernelGGL(score_kernel<true>, grid, block, LDS_SCORE_TOTAL, st, a);
+  hipLaunchKernelGGL((score_kernel<true, false>), grid, block, LDS_SCORE_TOTAL, st, a);
   return pbs_check_launch(who);
 }
 

@@ -75,3 +75,22 @@ def test_segment_sort_is_stable_for_every_score(dev, seg):
     want = torch.from_numpy(order + np.arange(nseg)[:, None] * seg).view(1, rows, nseg * seg)
     tail = torch.arange(nseg * seg, s_pad).expand(1, rows, -1)
     assert torch.equal(idx, torch.cat((want, tail), -1))
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,seg", [
+    (1, 1, 1, 130, 128), (2, 7, 1, 1000, 128), (1, 4, 1, 2048, 128), (1, 4, 1, 2190, 128),   # 2 .. 32 chunks of 64, 17 of 128 keys
+    (1, 12, 3, 16384, 128), (1, 12, 3, 16512, 128),   # the longest sequence of the split scoring, and one block more
+    (1, 8, 4, 26880, 256), (3, 5, 5, 1111, 256),      # groups that would leave waves idle: 27 chunks of 1024, and a ragged batch
+])
+def test_key_scores_at_the_edges_of_the_split_form(dev, B, Hq, Hkv, S, seg):
+    """Tolerance: logits are bf16 values, and one that falls the other way on a near tie of the rounding moves its
+    probability by 2^-8 of the logit (|logit| < 6 here: under 3 %); sums of 128 of them move far less on average."""
+    from oracle import pbs_oracle as O
+    from pbs_attn_amd import ops
+    q, k, _ = small_case(B, Hq, Hkv, S, seed=S + Hq)
+    ref = O.key_scores(q, k, 128, seg)
+    got = ops.score_keys(q.to(dev), k.to(dev), 128, seg).cpu()
+    assert got.shape == ref.shape
+    rel = (got - ref).abs() / ref.abs().clamp_min(1e-12)
+    assert rel.max().item() < 3e-2 and rel.mean().item() < 2e-3
+    assert torch.allclose(got.sum(-1), torch.ones(B, Hq), atol=2e-3)
