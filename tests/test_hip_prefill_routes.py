@@ -38,6 +38,24 @@ def test_routes_without_a_selection(dev, B, Hq, Hkv, S, seg, thr):
     assert torch.equal(*_single_and_staged(dev, B, Hq, Hkv, S, seg, thr))
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,S,scale", [
+    (1, 32, 8, 77, 1), (3, 5, 5, 700, 1), (1, 28, 4, 1000, 1), (1, 32, 8, 2048, 1),   # an item or less per workgroup
+    (1, 33, 3, 2048, 1), (1, 64, 8, 1100, 1),                                         # more items: the list kernel
+    (1, 4, 2, 900, 20), (1, 2, 1, 2048, 20),   # exponents that overflow: the item is repeated from the same list
+])
+def test_one_segment_with_lists_formed_by_the_attention_kernel(dev, B, Hq, Hkv, S, scale):
+    q, k, v = (x.to(dev) for x in small_case(B, Hq, Hkv, S, seed=S))
+    q, k = q * scale, k * scale
+    single = P.permuted_block_sparse_attn_fwd(q, k, v, 128, 2048, 0.9, True)
+    P.stage_timer = _NullTimer()
+    try:
+        staged = P.permuted_block_sparse_attn_fwd(q, k, v, 128, 2048, 0.9, True)
+    finally:
+        P.stage_timer = None
+    assert torch.isfinite(single.float()).all()
+    assert torch.equal(single, staged)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,S,seg,thr,kind,kw", [
     (2, 3, 1, 1111, 384, 0.8, "uniform_heavy", dict(query_pool_mode="max", key_pool_mode="max")),   # odd blocks per segment, pairs across segments
     (1, 4, 2, 257, 256, 0.9, "uniform_heavy", {}),                  # one complete segment, the last pair a single row
