@@ -14,7 +14,9 @@ HEAD_DIM = 128
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device, without a Stream object around it (a pass of a few dozen tokens is bound by
+    the host)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t):
@@ -23,8 +25,12 @@ def _ptr(t):
 
 def _rows16(t: torch.Tensor) -> torch.Tensor:
     """Kernels need unit stride on head_dim and 16-byte aligned rows."""
-    if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:-1]) or t.data_ptr() % 16:
-        t = t.contiguous()
+    *lead, last = t.stride()
+    if last != 1 or t.data_ptr() % 16:
+        return t.contiguous()
+    for s in lead:
+        if s % 8:
+            return t.contiguous()
     return t
 
 
@@ -295,24 +301,23 @@ def prefill_attn_fwd(q, k, v, block_size, segment_size, threshold, force_select_
     lib = _lib.load()
     q, k, v = _rows16(q), _rows16(k), _rows16(v)
     B, Hq, S, D = q.shape
-    Hkv = k.shape[1]
+    Hkv, device = k.shape[1], q.device
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
-    is_int_one, thr_rows, thr = _threshold_args(threshold, B, Hq, q.device)
+    is_int_one, thr_rows, thr = _threshold_args(threshold, B, Hq, device)
     if S > segment_size and segment_size // block_size > 511:
         raise _lib.PbsHipError(
             f"a segment of {segment_size // block_size} blocks exceeds the attention kernel's limit of 511: "
             f"use a smaller segment_size")
-    out = torch.empty((B, Hq, S, D), dtype=q.dtype, device=q.device)
+    out = torch.empty((B, Hq, S, D), dtype=torch.bfloat16, device=device)
     ws_bytes = lib.pbs_prefill_attn_workspace_bytes(B, Hq, Hkv, S, D, block_size, segment_size)
-    ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=q.device)
+    ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=device)
     _lib.check(lib.pbs_prefill_attn_fwd(
-        _ptr(q), _ptr(k), _ptr(v), _ptr(out), B, Hq, Hkv, S, D, block_size, segment_size,
-        q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-        v.stride(0), v.stride(1), v.stride(2), out.stride(0), out.stride(1), out.stride(2),
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Hq, Hkv, S, D, block_size, segment_size,
+        *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], Hq * S * D, S * D, D,
         thr, _ptr(thr_rows), int(is_int_one), int(bool(force_select_first_block)),
         int(query_pool_mode == "max"), int(key_pool_mode == "max"), softmax_scale,
-        _ptr(ws), ws.numel(), _stream()), "pbs_prefill_attn_fwd")
+        ws.data_ptr(), max(ws_bytes, 256), _stream()), "pbs_prefill_attn_fwd")
     return out
 
 
