@@ -151,7 +151,7 @@ def tile_pipeline(torch, iters=6000):
     rings = {"zeros": torch.zeros(n_src * 32768, dtype=torch.bfloat16, device=dev),
              "normal": torch.randn(n_src * 32768, generator=gen).to(torch.bfloat16).to(dev)}
     st = torch.cuda.current_stream().cuda_stream
-    out = {"kernel": "fast tiles of 128 keys x 256 queries per workgroup, 256 workgroups x 8 waves, barrier per tile",
+    out = {"kernel": "fast tiles of 128 keys x 256 queries per workgroup, 256 workgroups x 4 waves, barrier per tile",
            "flop_per_tile_step": 2 * FLOP_PER_BLOCK_PAIR}
     for name, ring in rings.items():
         for copies in (1, 0):

@@ -11,14 +11,15 @@
 //   A work item is TWO adjacent 128-query blocks of one head, served by one workgroup (4 waves, one per
 //   SIMD): wave w takes queries 32 w .. 32 w + 31 of either block, so that the waves finish a tile together also where
 //   only one block visits it -- above all the item's last tile, the second block's diagonal one, which then takes half a
-//   tile's time.  A small kernel
-//   first merges the two visit lists of every item (ascending key-block indices, own-segment blocks
-//   appended) into one list in HBM; every merged tile is copied ONCE into LDS for both query blocks, which
+//   tile's time.  The two
+//   visit lists of every item come merged into one list in HBM (ascending key-block indices, own-segment blocks appended),
+//   written by the block selection, by the list kernel below from CSR rows, or, for a sequence inside one segment, formed in
+//   LDS by the workgroup itself; every merged tile is copied ONCE into LDS for both query blocks, which
 //   halves the L2 -> LDS traffic and doubles the time a tile stays in flight.  K and V tiles are
 //   double-buffered (2 x 64 KB) and fetched one tile ahead with asynchronous global -> LDS copies (no
 //   registers), one workgroup barrier per tile.
 //   The attention kernel is PERSISTENT: one workgroup per CU takes item after item from a counter (one per
-//   XCD, over that XCD's share of the items; when it runs dry, the other XCDs' counters).  The tile pipeline
+//   XCD, over that XCD's share of the items; when it runs dry, the other XCDs' counters), the first one without asking.  The tile pipeline
 //   runs across items: the next item is claimed three tiles before the end of the current one, its list and
 //   its queries (into L2) are requested one tile later, its first K / V tiles at the last tile, so that an
 //   item's fixed costs (list, first tile, write-out of the previous item) overlap attention work.  With short

@@ -7,7 +7,7 @@
 #include <utility>
 
 // branch hints: they decide which side of a branch is laid out as the fall-through.  A taken branch refills the
-// wave's instruction buffer, and in the tile loop all eight waves of a workgroup take it at about the same time with
+// wave's instruction buffer, and in the tile loop all four waves of a workgroup take it at about the same time with
 // the matrix pipes idle, so the common path of that loop has to be the straight one.
 #define PBS_LIKELY(x) __builtin_expect(!!(x), 1)
 #define PBS_UNLIKELY(x) __builtin_expect(!!(x), 0)

@@ -9,8 +9,8 @@
 //   * emit the dense byte masks and the visit list: the ascending selected key blocks of
 //     strictly earlier segments (the attention kernel adds the causal part of the row's
 //     own segment itself, in original key order).
-// Rows of up to 1024 blocks take the wave-level variant further down (one wave per row,
-// the row in registers).
+// Rows of up to 1024 blocks (2048 on the single-call path, which writes the attention kernel's merged lists instead of
+// CSR rows) take the wave-level variant further down (one wave per row, the row in registers).
 #include "pbs_lists.h"
 #include "pbs_wave.h"
 #include <utility>
