@@ -20,8 +20,8 @@
 //   registers), one workgroup barrier per tile.
 //   The attention kernel is PERSISTENT: one workgroup per CU takes item after item from a counter (one per
 //   XCD, over that XCD's share of the items; when it runs dry, the other XCDs' counters), the first one without asking.  The tile pipeline
-//   runs across items: the next item is claimed three tiles before the end of the current one, its list and
-//   its queries (into L2) are requested one tile later, its first K / V tiles at the last tile, so that an
+//   runs across items: the next item is claimed three tiles before the end of the current one, its list is
+//   requested one tile later, its queries and its first K / V tiles at the last tile, so that an
 //   item's fixed costs (list, first tile, write-out of the previous item) overlap attention work.  With short
 //   visit lists (a few tiles per item) that is the difference between waiting for HBM three times per item
 //   and once.
@@ -416,12 +416,6 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     const int qb0 = hb.qb0, n_tiles = hb.n_tiles;
     const float c_log2 = ap->scale_log2;
 
-    // the item's queries: loaded ahead at the previous item's last tile, or from here (they are complete at the wait for
-    // the first tile's copies)
-    if (!careful_only) {
-      if (q_ready) q_advance();
-      else load_q(ap, hb, std::integral_constant<int, 0>{});
-    }
     // the next item: claimed three tiles before the end of this one (the counter's latency passes under a
     // tile), published and its list requested one tile later, its queries and its first tile requested at the last
     // tile.  Items of fewer than three tiles finish these steps after their loop.
@@ -444,7 +438,6 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     };
 
     {
-      o_clear();
       float m_ref[QG], l_row[QG];   // reference maxima and row sums of queries 16 qg + i16, identical in the four lanes i16 + 16 g
 #pragma unroll
       for (int qg = 0; qg < QG; ++qg) {
@@ -454,14 +447,6 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       bool poisoned = false;
       uint32_t unseen = 3u << 14;   // use bits of the query blocks that have seen no tile yet (their reference is still -inf)
 
-      if (careful_only) {
-        // the redo pass starts the item over: its first tile goes back into the buffers it had (the next
-        // item's first tile, if it was on its way there, is fetched again at the end of this pass)
-        __builtin_amdgcn_s_waitcnt(0x0f70);
-        __syncthreads();
-        aim_anew(hb, first_entry(mlist), par);
-        copy_tile_now(copy);
-      }
       uint32_t bufx = par;
       auto next_buffers = [&]() __attribute__((always_inline)) {
         bufx ^= 0x8000u;
@@ -471,11 +456,33 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
           va[n] ^= 0x8000u;
         }
       };
-      // a tile's copies are awaited at the end of the tile before it.  Vector memory operations complete in order, so
-      // behind an item's first tile (and its queries) the previous item's stores may still be on their way
+      // a tile's copies are awaited at the end of the tile before it, those of an item's first tile here, and with them the
+      // item's queries.  Loads from inline assembly are unknown to the compiler and not interlocked by the hardware, so nothing
+      // may touch their registers before this wait (tests/test_attention_registers.py follows every path through the compiled
+      // code); the accumulators are cleared in its shadow.
       auto wait_copies = [&]() __attribute__((always_inline)) { __builtin_amdgcn_s_waitcnt(0x0f70); };   // vmcnt(0)
-      if (stores_out) __builtin_amdgcn_s_waitcnt(0x4f70);   // vmcnt(16)
-      else wait_copies();
+      if (PBS_UNLIKELY(careful_only)) {
+        // the redo pass starts the item over: its first tile goes back into the buffers it had (the next
+        // item's first tile, if it was on its way there, is fetched again at the end of this pass)
+        wait_copies();
+        __syncthreads();
+        aim_anew(hb, first_entry(mlist), par);
+        copy_tile_now(copy);
+        o_clear();
+        wait_copies();
+      } else if (q_ready) {
+        // requested at the previous item's last tile, and after them the sixteen copies of this item's first tile.  Vector
+        // memory operations complete in order: vmcnt(16) leaves the sixteen youngest on their way, which are the previous
+        // item's stores or, where it had fewer, copies
+        o_clear();
+        __builtin_amdgcn_s_waitcnt(0x4f70);   // vmcnt(16)
+        if (!stores_out) wait_copies();
+        q_advance();
+      } else {
+        load_q(ap, hb, std::integral_constant<int, 0>{});
+        o_clear();
+        wait_copies();
+      }
       uint32_t e_cur = first_entry(mlist);         // the entry of the current tile
       uint32_t e_nxt = 0;                          // of the next one, set by tile_head
       uint16_t e_ahead = mlist[LIST_HEADER + 1];   // per lane, not yet made uniform

@@ -230,7 +230,8 @@ __device__ __forceinline__ void o_scale(float alpha) {
     asm volatile("v_accvgpr_write_b32 a[%1], %0" ::"v"(x), "n"(r));
   });
 }
-// this lane's 16 bytes of a Q^T fragment, straight into the accumulation registers; complete after the next vmcnt(0)
+// this lane's 16 bytes of a Q^T fragment, straight into the accumulation registers.  They are there only once a vmcnt wait
+// has covered the load, and nobody waits by himself: neither the compiler nor the hardware.
 template <int Q, int KD, int SET = 0>
 __device__ __forceinline__ void q_load(const uint16_t* src) {
   constexpr int r = q_reg(Q, KD) + SET;
