@@ -437,11 +437,11 @@ __device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_
   for (int q = Q0; q < QG; ++q) negm[q] = (q < 2 ? use0 : use1) ? -m_ref[q] : -INFINITY;
   // The diagonal tile, by sub-tile k of 32 keys against the wave's 32 queries of the block: k < wave visible, k > wave
   // hidden, k == wave the triangle key 8 g + 4 T + r > query 16 (q % 2) + i.  The probabilities of masked column groups,
-  // as bf16 pairs, are ANDed with the triangle's bits (one register per pair, the same for both blocks), all ones where
-  // k < wave, and a hidden sub-tile has reference +inf: 2 vector instructions per pair of logits (comparing and selecting
-  // per logit takes 4, and held up the diagonal tile by 1300 cycles).
-  uint32_t tri[2][2][2];        // [T][q % 2][pair]
-  float negm_k[MASKED ? 4 : 1][QG];
+  // as bf16 pairs, are ANDed with all ones, zero or the triangle's bits (one register per pair, the same for both blocks),
+  // whatever they are: a later key's logit may be NaN or infinite without a trace.  2 vector instructions per pair of logits
+  // (comparing and selecting per logit takes 4, and held up the diagonal tile by 1300 cycles).
+  uint32_t tri[2][2][2];          // [T][q % 2][pair]
+  uint32_t some[MASKED ? 4 : 1], all[MASKED ? 4 : 1];   // all ones where k <= wave, where k < wave
   if (MASKED) {
     const int ln = lane_id_here();          // nothing below may be formed outside the tile
     const int qrel8 = (ln & 15) - 8 * (ln >> 4);
@@ -453,12 +453,14 @@ __device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_
         for (int pr = 0; pr < 2; ++pr) {
           const int key = 4 * T + 2 * pr - 16 * q;
           tri[T][q][pr] = (key <= qrel8 ? 0xffffu : 0u) | (key + 1 <= qrel8 ? 0xffff0000u : 0u);
+          asm volatile("" : "+v"(tri[T][q][pr]));   // (formed here, not in the gaps)
         }
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int q = Q0; q < QG; ++q)
-        if (MASKED >> q & 1) negm_k[k][q] = k > wave ? -INFINITY : negm[q];
+    for (int k = 0; k < 4; ++k) {
+      some[k] = k <= wave ? ~0u : 0u;
+      all[k] = k < wave ? ~0u : 0u;
+      asm volatile("" : "+v"(some[k]), "+v"(all[k]));
+    }
   }
   uint32_t vr = 0;
   if (V_ROWS) vr = vrow_lane_addr(LDS_V0 + (va[0] & 0x8000u), lane_id_here());   // va[] carries the buffer switch in bit 15
@@ -515,7 +517,7 @@ __device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_
       constexpr int combo = u / UNITS_PER_COMBO, unit = u % UNITS_PER_COMBO, k = combo / (2 * NQ), T = combo / NQ & 1, q = combo % NQ;
       auto scaled = [&](auto rc) __attribute__((always_inline)) {
         constexpr int r = decltype(rc)::value;
-        x[r] = __builtin_fmaf(sacc[k & 1][T][q][r], c_log2, (MASKED >> (Q0 + q) & 1) ? negm_k[MASKED ? k : 0][Q0 + q] : negm[Q0 + q]);
+        x[r] = __builtin_fmaf(sacc[k & 1][T][q][r], c_log2, negm[Q0 + q]);
       };
       if constexpr (unit == 0) { scaled(std::integral_constant<int, 0>{}); scaled(std::integral_constant<int, 1>{}); }
       if constexpr (unit == 1) e[0] = __builtin_amdgcn_exp2f(x[0]);
@@ -525,7 +527,7 @@ __device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_
 #pragma unroll
         for (int pr = 0; pr < 2; ++pr) {
           uint32_t two = __builtin_bit_cast(uint32_t, (bf16x2){(__bf16)e[2 * pr], (__bf16)e[2 * pr + 1]});
-          if constexpr (MASKED >> (Q0 + q) & 1) two &= tri[T][q & 1][pr] | (k < wave ? 0xffffffffu : 0u);
+          if constexpr (MASKED >> (Q0 + q) & 1) two &= (tri[T][q & 1][pr] & some[k]) | all[k];
           pbuf[k & 1][q][2 * T + pr] = two;
         }
       }
