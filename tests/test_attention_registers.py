@@ -117,10 +117,12 @@ def _unfinished_reads(body):
                 m = re.search(r"vmcnt\((\d+)\)", " ".join(t))
                 if m:
                     state = {r: n for r, n in state.items() if n < int(m[1])}
-            if op.startswith(("s_branch", "s_cbranch")):
+            # where its block leaves the lane mask alone, some lane is always there
+            some_lane = op.startswith("s_cbranch_exec") and not any("exec" in tok for u in code[head:i] for tok in u[1:])
+            if op.startswith(("s_branch", "s_cbranch")) and not (some_lane and op == "s_cbranch_execz"):
                 flow(at[t[1]], state)
-            if op == "s_cbranch_execnz" and not any("exec" in tok for u in code[head:i] for tok in u[1:]):
-                break   # where its block leaves the lane mask alone, some lane is always there and the branch is taken
+            if some_lane and op == "s_cbranch_execnz":
+                break
             if op == "s_setpc_b64":   # a branch out of a conditional one's reach: getpc, add (label - .Lpost_getpc), addc, setpc
                 flow(at[re.search(r"\((\.LBB\w+)-\.Lpost_getpc", " ".join(code[i - 2]))[1]], state)
             if op in ("s_branch", "s_endpgm", "s_setpc_b64"):
