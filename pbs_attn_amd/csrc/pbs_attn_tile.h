@@ -281,7 +281,7 @@ struct MfmaOp { int kind, k, T, x, q, frag; };   // kind 0: S (sub-tile k, row t
 constexpr int N_FRAG = 64, UNITS_PER_COMBO = 7;
 constexpr int FRAG_BUFS = 6, FRAG_AHEAD = 11;   // fragment registers; how many matrix instructions ahead of its use a fragment is read
 constexpr int COPY_FIRST_GAP = 2, COPY_GAP_STEP = 8;
-// NQ: the column groups the tile is worked on for, four or (a tile that only the pair's second block sees) two
+// NQ: the column groups the tile is worked on for, four or (a tile that only one of the pair's blocks sees) two
 template <int NQ>
 struct TileSchedule {
   static constexpr int N_MFMA = 68 * NQ, N_UNITS = 8 * NQ * UNITS_PER_COMBO;
@@ -418,23 +418,23 @@ constexpr int lds_reads_younger(int f, int i, bool v_rows) {
 // ka[kd] / va[ks]: this lane's byte addresses of the K fragments of d-step kd (row tile 0, sub-tile 0) and of the V^T
 // fragments of sub-tile ks (d tile 0) in the tile's buffers: held in registers and switched between the two buffers
 // once per tile, so that a fragment read needs no address arithmetic.
-// Q0: the first column group that sees the tile (0, or 2: only the pair's second block does).  MASKED: the column groups
+// Q0, NQ: the column groups that see the tile: all four, or the two of one of the pair's blocks.  (A block that does not visit
+// a tile takes no part in it at all: with probabilities of zero instead, an infinity or a NaN of the tile's V would get
+// into its rows.)  MASKED: the column groups
 // (bits) whose diagonal block the tile is, read in original key order: logits of keys that lie after the query
 // (key-in-tile > query-in-block) get no probability.  V_ROWS: the tile's V is a tile of the caller's tensor, and its fragments
 // come from transposing reads; otherwise it is a transposed (V^T) tile and they are plain 16-byte reads.
-// Exponentials are taken against a LAZY reference maximum (see pbs_attn.hip); `use0` / `use1` say whether the pair's first
-// / second block visits the tile at all (if not, its reference is +inf here and its probabilities are zero).  Row sums
+// Exponentials are taken against a LAZY reference maximum (see pbs_attn.hip).  Row sums
 // come from one more matrix instruction per sub-tile and column group, ones x P, whose every output row is the sum over
 // the sub-tile's 32 keys of the probabilities as the P.V product sees them (rounded to bf16).
 // `copy`: the next tile's copies, a piece every COPY_GAP_STEP matrix instructions.
-template <int Q0, int MASKED, bool V_ROWS, bool COPIES = true>
-__device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_t (&va)[4], float c_log2, bool use0, bool use1,
-                                          float (&m_ref)[QG], float (&l_row)[QG], bool& poisoned, int wave, const TileCopy& copy) {
-  constexpr int NQ = QG - Q0;
+template <int Q0, int NQ, int MASKED, bool V_ROWS, bool COPIES = true>
+__device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_t (&va)[4], float c_log2, float (&m_ref)[QG],
+                                          float (&l_row)[QG], bool& poisoned, int wave, const TileCopy& copy) {
   typedef TileSchedule<NQ> Sched;
   float negm[QG];
 #pragma unroll
-  for (int q = Q0; q < QG; ++q) negm[q] = (q < 2 ? use0 : use1) ? -m_ref[q] : -INFINITY;
+  for (int q = Q0; q < Q0 + NQ; ++q) negm[q] = -m_ref[q];
   // The diagonal tile, by sub-tile k of 32 keys against the wave's 32 queries of the block: k < wave visible, k > wave
   // hidden, k == wave the triangle key 8 g + 4 T + r > query 16 (q % 2) + i.  The probabilities of masked column groups,
   // as bf16 pairs, are ANDed with all ones, zero or the triangle's bits (one register per pair, the same for both blocks),

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(THREADS, 1) void tile_probe_kernel(const uint16_t* 
     copy.k = uniform64((uint64_t)(uintptr_t)src - COPY_BIAS);
     copy.v = uniform64((uint64_t)(uintptr_t)(src + BS * D) - COPY_BIAS);
     copy.lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)((bufx ^ 0x8000u) + (uint32_t)wave * 8192u));
-    fast_tile<0, 0, V_ROWS, COPIES>(ka, va, c_log2, true, true, m_ref, l_part, poisoned, wave, copy);
+    fast_tile<0, QG, 0, V_ROWS, COPIES>(ka, va, c_log2, m_ref, l_part, poisoned, wave, copy);
     bufx ^= 0x8000u;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {

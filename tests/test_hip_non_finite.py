@@ -61,3 +61,18 @@ def _check(dev, Hq, S, seg, token, bad_k, bad_v, seed, scale=1):
 ])
 def test_later_keys_of_the_diagonal_block(dev, S, seg, token, bad):
     _check(dev, 3, S, seg, token, bad, None, S + token)
+
+
+@pytest.mark.parametrize("scale", [1, 20])   # 20: exponents that overflow, the item is repeated
+@pytest.mark.parametrize("bad_k,bad_v", [(float("nan"), None), (float("inf"), None), (None, float("nan")), (None, float("inf"))])
+@pytest.mark.parametrize("S,seg,token", [
+    (2048, 256, 300), (1900, 128, 5),   # a permuted tile that one block of a pair selected
+    (1100, 384, 300),                   # the first block's own segment ends inside the pair; a last pair of one block
+    (2048, 384, 130),                   # ... a tile before its diagonal
+])
+def test_blocks_that_did_not_select_the_token(dev, S, seg, token, bad_k, bad_v, scale):
+    seed = S + seg
+    mask = _random_lists(3, (S + 127) // 128, seg // 128, seed)[0][..., token // 128]
+    first, second = mask[..., :-1:2], mask[..., 1::2]
+    assert (first & ~second).any() and (second & ~first).any()
+    _check(dev, 3, S, seg, token, bad_k, bad_v, seed, scale)
