@@ -44,9 +44,10 @@
 //     Exponentials are taken against a LAZY reference maximum: it is not updated per tile; a row
 //     sum of one tile above 2^14 triggers a uniform rescale (exact, all terms share the reference); an
 //     overflow marks the row and the whole workgroup redoes it without speculation.  The first tile of a
-//     row takes its reference from the exact maximum over sixteen of its first keys.  The diagonal tile runs the
-//     same pipeline and zeroes the exponentials of keys after the query (key-in-tile > query-in-block).
-//   * careful tiles (the redo pass): one 32-key sub-tile at a time, exact running maximum, classic online softmax.
+//     row takes its reference from the exact maximum over its first 32 keys.  The diagonal tile runs the
+//     same pipeline and zeroes the probabilities of keys after the query (key-in-tile > query-in-block).
+//   * careful tiles (the redo pass, and a diagonal tile that is its block's first tile): one 32-key sub-tile at a time, exact
+//     running maximum, classic online softmax.
 //   An item's tiles come in the order permuted tiles, own-segment tiles before the diagonal, diagonal tile, and
 //   each kind has a loop of its own (see the loops): one tile body per loop keeps the accumulators in place.
 #include "pbs_attn_tile.h"
@@ -504,96 +505,104 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
         if (has_nxt && (careful_only || n_tiles >= 3)) aim_at_next(bufx ^ 0x8000u);   // shorter items: after the loop, once the list has landed
         else copy.lds ^= 0x8000u;   // nothing to fetch: the same tile again, into buffers nobody reads (a pipelined tile always copies)
       };
-      // logits of the 16-key row tile at byte offset `at` of the K buffer against the wave's queries
-      auto logits_of = [&](f32x4 (&s)[QG], int at) __attribute__((always_inline)) {
-        bf16x8 fk[4];
+      // logits of the 32 keys at byte offset `at` of the K buffer against the queries of column groups Q0 .. Q0 + NQ - 1
+      auto logits_of = [&](auto q0c, auto& s, int at) __attribute__((always_inline)) {
+        constexpr int Q0 = decltype(q0c)::value, NQ = sizeof(s[0]) / sizeof(s[0][0]);
+        static_for<2>([&](auto tc) __attribute__((always_inline)) {
+          constexpr int T = decltype(tc)::value;
+          bf16x8 fk[4];
 #pragma unroll
-        for (int kd = 0; kd < 4; ++kd) fk[kd] = ldsf(ka[kd] + at);
-        static_for<4>([&](auto kc) __attribute__((always_inline)) {
-          constexpr int kd = decltype(kc)::value;
-          static_for<QG>([&](auto qc) __attribute__((always_inline)) { mfma_s<decltype(qc)::value, kd, kd == 0>(s[decltype(qc)::value], fk[kd]); });
+          for (int kd = 0; kd < 4; ++kd) fk[kd] = ldsf(ka[kd] + at + T * 1024);
+          static_for<4>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int kd = decltype(kc)::value;
+            static_for<NQ>([&](auto qc) __attribute__((always_inline)) {
+              constexpr int q = decltype(qc)::value;
+              mfma_s<Q0 + q, kd, kd == 0>(s[T][q], fk[kd]);
+            });
+          });
         });
         MFMA_FENCE();
       };
-      // first tile of a row: the exact maximum over the visible ones of its keys 0-3, 8-11, 16-19 and 24-27 is a good
-      // enough reference to start the pipelined path (later keys move it up lazily); in a diagonal tile every query sees
-      // key 0 at least, so the reference is finite there too
-      auto first_reference = [&](auto masked, uint32_t ent) __attribute__((always_inline)) {
-        f32x4 s0[QG];
-        logits_of(s0, 0);
-        const int ln = lane_id_here();
-        const int qrel8 = 32 * wave + (ln & 15) - 8 * (ln >> 4);
+      // first tile of a row, every key visible: the exact maximum over its first 32 keys is a good enough reference
+      // to start the pipelined path (later keys move it up lazily).  (Over 16 keys the results' error against 64-bit arithmetic was 0.5 to 1 %
+      // larger: a reference that is the maximum has the probability 1, which bf16 holds exactly.)
+      auto first_reference = [&](uint32_t ent) __attribute__((always_inline)) {
+        f32x4 s0[2][QG];
+        logits_of(std::integral_constant<int, 0>{}, s0, 0);
 #pragma unroll
         for (int qg = 0; qg < QG; ++qg) {
           float mx = -INFINITY;
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (!(decltype(masked)::value >> qg & 1) || r - 16 * (qg & 1) <= qrel8) mx = fmaxf(mx, s0[qg][r]);
+          for (int T = 0; T < 2; ++T)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s0[T][qg][r]);
           const float m_new = max_over_lane_groups(mx) * c_log2;
           if (ent & unseen & (1u << (14 + (qg >> 1)))) m_ref[qg] = m_new;
         }
         unseen &= ~ent;
       };
-      // careful tile (the redo pass): classic online softmax, one 32-key sub-tile at a time
-      auto careful_tile = [&](uint32_t ent) __attribute__((always_inline)) {
+      // careful tile, for one of the pair's blocks: classic online softmax, one 32-key sub-tile at a time.  The redo pass, and a
+      // diagonal tile that is its block's first tile (the 128 keys of a sequence's first block, or a block that
+      // selected nothing: with a reference from some of so few keys the error against 64-bit arithmetic was 3 % larger)
+      auto careful_tile = [&](auto bc, uint32_t ent) __attribute__((always_inline)) {
+        constexpr int block = decltype(bc)::value, Q0 = 2 * block;
+        const bool masked = (ent & ENT_ORIG) && (int)(ent & ENT_KB) == qb0 + block;
+        // of a diagonal tile the sub-tiles up to the wave's own (the rest is hidden), none where its queries lie past the sequence
+        const int n_sub = !masked ? 4 : (qb0 + block) * BS + 32 * wave < hb.S ? wave + 1 : 0;
         MFMA_FENCE();
 #pragma nounroll
-        for (int ks = 0; ks < 4; ++ks) {   // a real loop: the rare path stays small, in code and in registers
-          f32x4 s[2][QG];   // [T][qg]
-          logits_of(s[0], ks * 8192);
-          logits_of(s[1], ks * 8192 + 1024);
-          const int ln = lane_id_here();   // keep the compares inside the tile (see fast_tile)
-          const int qrel8 = 32 * wave + (ln & 15) - 8 * (ln >> 4);
-#pragma unroll
-          for (int qg = 0; qg < QG; ++qg) {
-            const bool used = (ent >> (14 + (qg >> 1))) & 1u;
-            const bool masked = (ent & ENT_ORIG) && (int)(ent & ENT_KB) == qb0 + (qg >> 1);
+        for (int ks = 0; ks < n_sub; ++ks) {   // a real loop: the rare path stays small, in code and in registers
+          f32x4 s[2][2];   // [T][column group - Q0]
+          logits_of(std::integral_constant<int, Q0>{}, s, ks * 8192);
+          if (masked) {
+            const int ln = lane_id_here();   // keep the compares inside the tile (see fast_tile)
+            const int qrel8 = 32 * wave + (ln & 15) - 8 * (ln >> 4);
 #pragma unroll
             for (int T = 0; T < 2; ++T)
 #pragma unroll
-              for (int r = 0; r < 4; ++r)
-                if (!used || (masked && 32 * ks + 4 * T + r - 16 * (qg & 1) > qrel8)) s[T][qg][r] = -INFINITY;
-          }
-          float alpha[QG];
-          bf16x8 pf[QG];
+              for (int q = 0; q < 2; ++q)
 #pragma unroll
-          for (int qg = 0; qg < QG; ++qg) {
-            float mx = fmaxf(fmaxf(s[0][qg][0], s[0][qg][1]), fmaxf(s[0][qg][2], s[0][qg][3]));
-            mx = fmaxf(mx, fmaxf(fmaxf(s[1][qg][0], s[1][qg][1]), fmaxf(s[1][qg][2], s[1][qg][3])));
+                for (int r = 0; r < 4; ++r)
+                  if (32 * ks + 4 * T + r - 16 * q > qrel8) s[T][q][r] = -INFINITY;
+          }
+          float alpha[2];
+          bf16x8 pf[2];
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            float mx = fmaxf(fmaxf(s[0][q][0], s[0][q][1]), fmaxf(s[0][q][2], s[0][q][3]));
+            mx = fmaxf(mx, fmaxf(fmaxf(s[1][q][0], s[1][q][1]), fmaxf(s[1][q][2], s[1][q][3])));
             mx = max_over_lane_groups(mx);
-            const float m_new = fmaxf(m_ref[qg], mx * c_log2);
+            const float m_new = fmaxf(m_ref[Q0 + q], mx * c_log2);
             const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-            alpha[qg] = __builtin_amdgcn_exp2f(m_ref[qg] - m_use);
-            m_ref[qg] = m_new;
+            alpha[q] = __builtin_amdgcn_exp2f(m_ref[Q0 + q] - m_use);
+            m_ref[Q0 + q] = m_new;
             float rs = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-              const float pe = __builtin_amdgcn_exp2f(s[e >> 2][qg][e & 3] * c_log2 - m_use);
+              const float pe = __builtin_amdgcn_exp2f(s[e >> 2][q][e & 3] * c_log2 - m_use);
               rs += pe;
-              pf[qg][e] = (__bf16)pe;
+              pf[q][e] = (__bf16)pe;
             }
-            l_row[qg] = l_row[qg] * alpha[qg] + sum_over_lane_groups(rs);
+            l_row[Q0 + q] = l_row[Q0 + q] * alpha[q] + sum_over_lane_groups(rs);
           }
-          if (__any(alpha[0] != 1.0f || alpha[1] != 1.0f || alpha[2] != 1.0f || alpha[3] != 1.0f)) {
-            static_for<QG>([&](auto qc) __attribute__((always_inline)) { o_scale<decltype(qc)::value>(alpha[decltype(qc)::value]); });
+          if (__any(alpha[0] != 1.0f || alpha[1] != 1.0f)) {
+            o_scale<Q0>(alpha[0]);
+            o_scale<Q0 + 1>(alpha[1]);
           }
           MFMA_FENCE();
-          static_for<2>([&](auto bc) __attribute__((always_inline)) {   // (a block that does not visit the tile: see fast_tile)
-            constexpr int block = decltype(bc)::value;
-            if ((ent >> (14 + block)) & 1u) {
-              static_for<8>([&](auto dc) __attribute__((always_inline)) {
-                constexpr int dt = decltype(dc)::value;
-                const bf16x8 fv = (ent & ENT_ORIG)
-                                      ? ldsf_transposed(vrow_lane_addr(LDS_V0 + (va[0] & 0x8000u), lane_id_here()) + dt * 128 + ks * 8192)
-                                      : ldsf((va[0] ^ (uint32_t)(ks << 6)) + dt * 4096);
-                mfma_o<dt, 2 * block>(fv, pf[2 * block]);
-                mfma_o<dt, 2 * block + 1>(fv, pf[2 * block + 1]);
-              });
-            }
+          static_for<8>([&](auto dc) __attribute__((always_inline)) {
+            constexpr int dt = decltype(dc)::value;
+            const bf16x8 fv = (ent & ENT_ORIG)
+                                  ? ldsf_transposed(vrow_lane_addr(LDS_V0 + (va[0] & 0x8000u), lane_id_here()) + dt * 128 + ks * 8192)
+                                  : ldsf((va[0] ^ (uint32_t)(ks << 6)) + dt * 4096);
+            mfma_o<dt, Q0>(fv, pf[0]);
+            mfma_o<dt, Q0 + 1>(fv, pf[1]);
           });
           MFMA_FENCE();
         }
       };
+      constexpr std::integral_constant<int, 0> block0{};
+      constexpr std::integral_constant<int, 1> block1{};
       // The merged list holds the permuted tiles of earlier segments first, then the tiles of the own segments in
       // ascending order: for a query block those before its own block, its own (diagonal) block, and -- for the first
       // block of a pair -- the second block's, which it skips.  Each kind has a loop of its own, and so has the redo
@@ -607,7 +616,8 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
           if (it + 1 < n_tiles) aim_anew(hb, e_nxt, bufx ^ 0x8000u);
           else aim_past_item();
           copy_tile_now(copy);
-          if (e_cur & (USE0 | USE1)) careful_tile(e_cur);
+          if (e_cur & USE0) careful_tile(block0, e_cur);
+          if (e_cur & USE1) careful_tile(block1, e_cur);
           wait_copies();
         }
       } else {
@@ -623,7 +633,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
         auto visit = [&](auto masked, auto v_rows) __attribute__((always_inline)) {
           constexpr int MASKED = decltype(masked)::value;
           constexpr bool V_ROWS = decltype(v_rows)::value;
-          if (PBS_UNLIKELY(e_cur & unseen)) first_reference(masked, e_cur);
+          if (PBS_UNLIKELY(e_cur & unseen)) first_reference(e_cur);
           if (PBS_LIKELY((e_cur & (USE0 | USE1)) == (USE0 | USE1)))
             fast_tile<0, 4, MASKED, V_ROWS>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
           else if (V_ROWS || (e_cur & USE0))   // (of own-segment tiles the second block alone visits its diagonal one only)
@@ -668,16 +678,30 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
           const bool more = it + 1 < n_tiles;
           if (more) aim_anew(hb, e_nxt, bufx ^ 0x8000u);
           else aim_past_item();
-          if (e_cur & (USE0 | USE1)) visit(diagonal0, std::true_type{});
-          else copy_tile_now(copy);
+          if (PBS_UNLIKELY(e_cur & unseen & USE0)) {
+            copy_tile_now(copy);
+            careful_tile(block0, e_cur);
+            if (e_cur & USE1) {
+              if (unseen & USE1) first_reference(USE1);
+              fast_tile<2, 2, 0, true, false>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
+            }
+          } else if (e_cur & (USE0 | USE1)) {
+            visit(diagonal0, std::true_type{});
+          } else {
+            copy_tile_now(copy);
+          }
           if (more) wait_copies();
           next_tile();
         }
         if (it < n_tiles) {   // the second block's diagonal tile, which nobody else sees
           tile_head(it);
           aim_past_item();
-          if (e_cur & unseen) first_reference(std::integral_constant<int, 12>{}, e_cur);
-          fast_tile<2, 2, 12, true>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
+          if (PBS_UNLIKELY(e_cur & unseen)) {
+            copy_tile_now(copy);
+            careful_tile(block1, e_cur);
+          } else {
+            fast_tile<2, 2, 12, true>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
+          }
           next_tile();
         }
       }
