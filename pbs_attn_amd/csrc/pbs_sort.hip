@@ -7,6 +7,7 @@
 #include "pbs_lists.h"
 #include "pbs_wave.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
+#include <algorithm>
 
 namespace {
 
@@ -104,7 +105,8 @@ template <int NPL>
 __global__ __launch_bounds__(256) void segment_argsort_wave_kernel(const float* scores, int32_t* idx, int Sc, int S_pad, int seg, int n_units,
                                                                    int rows, int32_t* first_blk, int block_size) {
   const int lane = threadIdx.x & 63;
-  const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // a segment of a row, or a piece of its identity tail
+  // a segment of a row, or a piece of its identity tail
+  const int64_t unit = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int row = (int)(unit / n_units), s = (int)(unit - (int64_t)row * n_units);
   if (row >= rows) return;
   const int base = s * seg;
@@ -159,7 +161,11 @@ int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_
   PBS_REQUIRE(rows <= 65535, "pbs_segment_argsort: too many rows (%d)", rows);
   if (segment_size <= 2048) {
     const int n_units = nseg + tail_blocks;
-    const dim3 grid((unsigned)(((int64_t)rows * n_units + 3) / 4));
+    // a launch holds fewer than 2^32 work-items along a dimension: rows of very many segments go on along y
+    const int64_t wgs = ((int64_t)rows * n_units + 3) / 4, gx = std::min<int64_t>(wgs, 1 << 23);
+    const int64_t gy = (wgs + gx - 1) / gx;
+    PBS_REQUIRE(gy <= 65535, "pbs_segment_argsort: launch too large");
+    const dim3 grid((unsigned)gx, (unsigned)gy);
     auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, scores, key_indices, Sc, S_pad, segment_size, n_units, rows,
                          first_blk, block_size);

@@ -95,6 +95,20 @@ def test_segment_sort_is_stable_for_every_score(dev, seg):
     assert torch.equal(idx, torch.cat((want, tail), -1))
 
 
+def test_segment_sort_of_more_work_items_than_one_grid_dimension_holds(dev):
+    """65535 rows x 1088 units (1025 segments of two keys, 63 pieces of the identity tail) are 2^26 waves of 64 and more."""
+    from pbs_attn_amd import ops
+    rows, S, seg = 65535, 2050, 2
+    x = torch.rand((1, rows, S), device=dev)
+    idx = ops.segment_argsort(x, S, seg, 128)[0]
+    pairs = x.view(rows, S // 2, 2)
+    second_first = (pairs[..., 1] > pairs[..., 0]).int()
+    base = torch.arange(0, S, 2, device=dev, dtype=torch.int32)
+    assert torch.equal(idx[:, :S:2], base + second_first)
+    assert torch.equal(idx[:, 1:S:2], base + 1 - second_first)
+    assert torch.equal(idx[:, S:], torch.arange(S, idx.shape[1], device=dev, dtype=torch.int32).expand(rows, -1))
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,S,seg", [
     (1, 1, 1, 130, 128), (2, 7, 1, 1000, 128), (1, 4, 1, 2048, 128), (1, 4, 1, 2190, 128),   # 2 .. 32 chunks of 64, 17 of 128 keys
     (1, 12, 3, 16384, 128), (1, 12, 3, 16512, 128),   # the longest sequence of the split scoring, and one block more
