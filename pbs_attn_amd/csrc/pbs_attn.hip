@@ -10,9 +10,8 @@
 // Work decomposition
 //   A work item is TWO adjacent 128-query blocks of one head, served by one workgroup (4 waves, one per
 //   SIMD): wave w takes queries 32 w .. 32 w + 31 of either block, so that the waves finish a tile together also where
-//   only one block visits it -- above all the item's last tile, the second block's diagonal one, which then takes half a
-//   tile's time.  The two
-//   visit lists of every item come merged into one list in HBM (ascending key-block indices, own-segment blocks appended),
+//   only one block visits it, as always the item's last tile, the second block's diagonal one; such a tile takes half a
+//   tile's time.  The two visit lists of every item come merged into one list in HBM (ascending key-block indices, own-segment blocks appended),
 //   written by the block selection, by the list kernel below from CSR rows, or, for a sequence inside one segment, formed in
 //   LDS by the workgroup itself; every merged tile is copied ONCE into LDS for both query blocks, which
 //   halves the L2 -> LDS traffic and doubles the time a tile stays in flight.  K and V tiles are
@@ -49,7 +48,7 @@
 //   * careful tiles (the redo pass, and a diagonal tile that is its block's first tile): one 32-key sub-tile at a time, exact
 //     running maximum, classic online softmax.
 //   An item's tiles come in the order permuted tiles, own-segment tiles before the diagonal, diagonal tile, and
-//   each kind has a loop of its own (see the loops): one tile body per loop keeps the accumulators in place.
+//   each kind has a loop of its own (see the loops).
 #include "pbs_attn_tile.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 #include <atomic>
@@ -218,7 +217,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // starts at LDS offset 0
   RESERVE_ACC_REGS();
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  
+
   // Work items = (head, pair of query blocks), ordered head by head with the long rows of a head first and cut
   // into eight contiguous ranges of about equal work, one per XCD (blockIdx % 8): an XCD works through one
   // head at a time, so its resident workgroups walk the same permuted K/V stream at about the same pace and
@@ -606,8 +605,9 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       // The merged list holds the permuted tiles of earlier segments first, then the tiles of the own segments in
       // ascending order: for a query block those before its own block, its own (diagonal) block, and -- for the first
       // block of a pair -- the second block's, which it skips.  Each kind has a loop of its own, and so has the redo
-      // pass: a loop whose body updates the 64 accumulator registers on one path only keeps them in place, where
-      // alternative tile bodies inside one loop cost a copy of all of them per tile (and the registers for it).
+      // pass: what differs between kinds -- the sixteen per-lane offsets of the tile copy, the fragment reads of V, the masks
+      // -- is then fixed inside a loop, and its common path is straight code.  (O's 128 accumulation registers are named, see
+      // pbs_attn_tile.h, and stay in place whatever the loops look like.)
       int it = 0;
       constexpr uint32_t USE0 = 1u << 14, USE1 = 1u << 15;
       if (PBS_UNLIKELY(careful_only)) {
@@ -793,7 +793,9 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     cur = nxt;
     nxt = q_end;
     has_nxt = false;
-    if (wave == 0 && lane_id_here() == 0) misc[1] = 0;   // read by everyone before the epilogue's barrier, set again only after the next item's barriers
+    // (nobody is still to read it: it was zero when this item's last barrier had been passed, or the item was a repetition, which
+    // does not read it; the next item's barriers lie before it can be set again)
+    if (wave == 0 && lane_id_here() == 0) misc[1] = 0;
   }
 }
 

@@ -12,7 +12,6 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 
 // ---- error reporting across the C ABI (thread-local message) --------------
 extern "C" const char* pbs_last_error(void);
@@ -39,14 +38,12 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return u >> 16;
 }
-__device__ __forceinline__ float round_bf16(float f) { return bf16_bits_to_f32(f32_to_bf16_bits(f)); }
 
 // two values rounded to bf16 (nearest even), returned as floats.  A conversion instruction packs two values; with a zero
 // as the lower one its result IS the float of the rounded upper one, so two conversions replace one and the two
-// instructions that take the pair apart (scoring
-// passes at 128k: 211 -> 198 us each, 1020 -> 892 vector instructions per 128 logits of a lane)
+// instructions that take the pair apart (scoring passes at 128k: 211 -> 198 us each, 1020 -> 892 vector instructions per
+// 128 logits of a lane)
 typedef __attribute__((ext_vector_type(2))) float f32x2;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 __device__ __forceinline__ f32x2 hw_round_bf16x2(f32x2 x) {
   const bf16x2 a = __builtin_convertvector((f32x2){0.f, x.x}, bf16x2), b = __builtin_convertvector((f32x2){0.f, x.y}, bf16x2);
   return (f32x2){__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)};

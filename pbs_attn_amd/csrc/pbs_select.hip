@@ -56,10 +56,6 @@ __global__ __launch_bounds__(1024) void first_token_block_kernel(const int32_t* 
   if (threadIdx.x == 0) first_blk[blockIdx.x] = found;
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int lane_mask) {
-  const uint32_t lo = __shfl_xor((uint32_t)v, lane_mask, 64), hi = __shfl_xor((uint32_t)(v >> 32), lane_mask, 64);
-  return ((uint64_t)hi << 32) | lo;
-}
 __device__ __forceinline__ double shfl_up_f64(double v, int delta) {
   const uint64_t u = __builtin_bit_cast(uint64_t, v);
   const uint32_t lo = __shfl_up((uint32_t)u, delta, 64), hi = __shfl_up((uint32_t)(u >> 32), delta, 64);
