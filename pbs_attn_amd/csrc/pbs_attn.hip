@@ -45,8 +45,8 @@
 //     overflow marks the row and the whole workgroup redoes it without speculation.  The first tile of a
 //     row takes its reference from the exact maximum over its first 32 keys.  The diagonal tile runs the
 //     same pipeline and zeroes the probabilities of keys after the query (key-in-tile > query-in-block).
-//   * careful tiles (the redo pass, and a diagonal tile that is its block's first tile): one 32-key sub-tile at a time, exact
-//     running maximum, classic online softmax.
+//   * careful tiles (the redo pass): one 32-key sub-tile at a time, exact running maximum, classic online softmax; so, in vector
+//     registers, a diagonal tile that is its block's first tile.
 //   An item's tiles come in the order permuted tiles, own-segment tiles before the diagonal, diagonal tile, and
 //   each kind has a loop of its own (see the loops).
 #include "pbs_attn_tile.h"
@@ -504,8 +504,9 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
         if (has_nxt && (careful_only || n_tiles >= 3)) aim_at_next(bufx ^ 0x8000u);   // shorter items: after the loop, once the list has landed
         else copy.lds ^= 0x8000u;   // nothing to fetch: the same tile again, into buffers nobody reads (a pipelined tile always copies)
       };
-      // logits of the 32 keys at byte offset `at` of the K buffer against the queries of column groups Q0 .. Q0 + NQ - 1
-      auto logits_of = [&](auto q0c, auto& s, int at) __attribute__((always_inline)) {
+      // logits of the 32 keys at byte offset `at` of the K buffer against the queries of column groups Q0 .. Q0 + NQ - 1 (the
+      // fence behind them is the caller's); `between` goes out after every d-step
+      auto logits_of = [&](auto q0c, auto& s, int at, auto between) __attribute__((always_inline)) {
         constexpr int Q0 = decltype(q0c)::value, NQ = sizeof(s[0]) / sizeof(s[0][0]);
         static_for<2>([&](auto tc) __attribute__((always_inline)) {
           constexpr int T = decltype(tc)::value;
@@ -518,71 +519,80 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
               constexpr int q = decltype(qc)::value;
               mfma_s<Q0 + q, kd, kd == 0>(s[T][q], fk[kd]);
             });
+            between(std::integral_constant<int, 4 * T + kd>{});
           });
         });
-        MFMA_FENCE();
       };
       // first tile of a row, every key visible: the exact maximum over its first 32 keys is a good enough reference
       // to start the pipelined path (later keys move it up lazily).  (Over 16 keys the results' error against 64-bit arithmetic was 0.5 to 1 %
       // larger: a reference that is the maximum has the probability 1, which bf16 holds exactly.)
-      auto first_reference = [&](uint32_t ent) __attribute__((always_inline)) {
-        f32x4 s0[2][QG];
-        logits_of(std::integral_constant<int, 0>{}, s0, 0);
+      auto first_reference = [&](auto q0c, uint32_t ent) __attribute__((always_inline)) {   // for column groups q0c .. QG - 1
+        constexpr int Q0 = decltype(q0c)::value;
+        f32x4 s0[2][QG - Q0];
+        logits_of(q0c, s0, 0, [](auto) {});
+        MFMA_FENCE();
 #pragma unroll
-        for (int qg = 0; qg < QG; ++qg) {
-          float mx = -INFINITY;
-#pragma unroll
-          for (int T = 0; T < 2; ++T)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s0[T][qg][r]);
+        for (int qg = Q0; qg < QG; ++qg) {
+          const f32x4 a = s0[0][qg - Q0], b = s0[1][qg - Q0];
+          const float mx = max3(max3(a[0], a[1], a[2]), max3(a[3], b[0], b[1]), max3(b[2], b[3], b[3]));
           const float m_new = max_over_lane_groups(mx) * c_log2;
           if (ent & unseen & (1u << (14 + (qg >> 1)))) m_ref[qg] = m_new;
         }
         unseen &= ~ent;
       };
-      // careful tile, for one of the pair's blocks: classic online softmax, one 32-key sub-tile at a time.  The redo pass, and a
-      // diagonal tile that is its block's first tile (the 128 keys of a sequence's first block, or a block that
-      // selected nothing: with a reference from some of so few keys the error against 64-bit arithmetic was 3 % larger)
+      // online softmax over the 32 keys with logits s ([row tile][column group]): the running maxima m move up, the sums l follow;
+      // alpha is what earlier sums are to be scaled by, pf the probabilities
+      auto online_step = [&](const f32x4 (&s)[2][2], float (&m)[2], float (&l)[2], float (&alpha)[2], bf16x8 (&pf)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          float mx = max3(s[0][q][0], s[0][q][1], s[0][q][2]);
+          mx = max3(mx, s[0][q][3], s[1][q][0]);
+          mx = max3(mx, s[1][q][1], s[1][q][2]);
+          mx = max_over_lane_groups(max3(mx, mx, s[1][q][3]));
+          const float m_new = fmaxf(m[q], mx * c_log2);
+          const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+          alpha[q] = __builtin_amdgcn_exp2f(m[q] - m_use);
+          m[q] = m_new;
+          float rs = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float pe = __builtin_amdgcn_exp2f(s[e >> 2][q][e & 3] * c_log2 - m_use);
+            rs += pe;
+            pf[q][e] = (__bf16)pe;
+          }
+          l[q] = l[q] * alpha[q] + sum_over_lane_groups(rs);
+        }
+      };
+      // the logits of sub-tile ks of a block's diagonal tile: keys after the query out
+      auto hide_later_keys = [&](f32x4 (&s)[2][2], int ks) __attribute__((always_inline)) {
+        const int ln = lane_id_here();   // keep the compares inside the tile (see fast_tile)
+        const int qrel8 = 32 * (wave - ks) + (ln & 15) - 8 * (ln >> 4);
+#pragma unroll
+        for (int T = 0; T < 2; ++T)
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (4 * T + r - 16 * q > qrel8) s[T][q][r] = -INFINITY;
+      };
+      // careful tile (the redo pass), for one of the pair's blocks: classic online softmax, one 32-key sub-tile at a time
       auto careful_tile = [&](auto bc, uint32_t ent) __attribute__((always_inline)) {
         constexpr int block = decltype(bc)::value, Q0 = 2 * block;
         const bool masked = (ent & ENT_ORIG) && (int)(ent & ENT_KB) == qb0 + block;
-        // of a diagonal tile the sub-tiles up to the wave's own (the rest is hidden), none where its queries lie past the sequence
-        const int n_sub = !masked ? 4 : (qb0 + block) * BS + 32 * wave < hb.S ? wave + 1 : 0;
         MFMA_FENCE();
 #pragma nounroll
-        for (int ks = 0; ks < n_sub; ++ks) {   // a real loop: the rare path stays small, in code and in registers
+        for (int ks = 0; ks < 4; ++ks) {   // a real loop: the rare path stays small, in code and in registers
           f32x4 s[2][2];   // [T][column group - Q0]
-          logits_of(std::integral_constant<int, Q0>{}, s, ks * 8192);
-          if (masked) {
-            const int ln = lane_id_here();   // keep the compares inside the tile (see fast_tile)
-            const int qrel8 = 32 * wave + (ln & 15) - 8 * (ln >> 4);
-#pragma unroll
-            for (int T = 0; T < 2; ++T)
-#pragma unroll
-              for (int q = 0; q < 2; ++q)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                  if (32 * ks + 4 * T + r - 16 * q > qrel8) s[T][q][r] = -INFINITY;
-          }
-          float alpha[2];
+          logits_of(std::integral_constant<int, Q0>{}, s, ks * 8192, [](auto) {});
+          MFMA_FENCE();
+          if (masked) hide_later_keys(s, ks);
+          float m[2] = {m_ref[Q0], m_ref[Q0 + 1]}, l[2] = {l_row[Q0], l_row[Q0 + 1]}, alpha[2];
           bf16x8 pf[2];
+          online_step(s, m, l, alpha, pf);
 #pragma unroll
           for (int q = 0; q < 2; ++q) {
-            float mx = fmaxf(fmaxf(s[0][q][0], s[0][q][1]), fmaxf(s[0][q][2], s[0][q][3]));
-            mx = fmaxf(mx, fmaxf(fmaxf(s[1][q][0], s[1][q][1]), fmaxf(s[1][q][2], s[1][q][3])));
-            mx = max_over_lane_groups(mx);
-            const float m_new = fmaxf(m_ref[Q0 + q], mx * c_log2);
-            const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-            alpha[q] = __builtin_amdgcn_exp2f(m_ref[Q0 + q] - m_use);
-            m_ref[Q0 + q] = m_new;
-            float rs = 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const float pe = __builtin_amdgcn_exp2f(s[e >> 2][q][e & 3] * c_log2 - m_use);
-              rs += pe;
-              pf[q][e] = (__bf16)pe;
-            }
-            l_row[Q0 + q] = l_row[Q0 + q] * alpha[q] + sum_over_lane_groups(rs);
+            m_ref[Q0 + q] = m[q];
+            l_row[Q0 + q] = l[q];
           }
           if (__any(alpha[0] != 1.0f || alpha[1] != 1.0f)) {
             o_scale<Q0>(alpha[0]);
@@ -598,6 +608,66 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
             mfma_o<dt, Q0 + 1>(fv, pf[1]);
           });
           MFMA_FENCE();
+        }
+      };
+      // A diagonal tile that is its block's first tile (the first 128 keys of a sequence, or a block that selected nothing): online
+      // softmax as well, since with a reference from some of so few keys the error against 64-bit arithmetic was 3 %
+      // larger.  The logits come first, the next tile's copies between them, and the sums stay in vector registers, O being
+      // zero so far; sub-tiles up to the wave's own (the rest is hidden), none where its queries lie past the sequence.
+      auto first_diagonal_tile = [&](auto bc) __attribute__((always_inline)) {
+        constexpr int block = decltype(bc)::value, Q0 = 2 * block;
+        if ((qb0 + block) * BS + 32 * wave >= hb.S) {
+          copy_tile_now(copy);
+          return;
+        }
+        f32x4 s[4][2][2], o[8][2];
+        asm volatile("s_nop 4");   // (as in copy_tile_now)
+        static_for<4>([&](auto kc) __attribute__((always_inline)) {
+          constexpr int ks = decltype(kc)::value;
+          logits_of(std::integral_constant<int, Q0>{}, s[ks], ks * 8192, [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = 8 * ks + decltype(ic)::value;
+            if constexpr (i % 2 == 0) copy_piece<i / 2>(copy);
+          });
+        });
+        const uint32_t vr = vrow_lane_addr(LDS_V0 + (va[0] & 0x8000u), lane_id_here());
+        float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+        MFMA_FENCE();
+        static_for<4>([&](auto kc) __attribute__((always_inline)) {
+          constexpr int ks = decltype(kc)::value;
+          if (ks == 0 || ks <= wave) {
+            if (ks == wave) hide_later_keys(s[ks], ks);
+            float alpha[2];
+            bf16x8 pf[2];
+            online_step(s[ks], m, l, alpha, pf);
+            if constexpr (ks > 0) {
+#pragma unroll
+              for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                  for (int r = 0; r < 4; ++r) o[dt][q][r] *= alpha[q];
+            }
+            bf16x8 fv[8];
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) fv[dt] = ldsf_transposed(vr + dt * 128 + ks * 8192);
+            MFMA_FENCE();
+            static_for<8>([&](auto dc) __attribute__((always_inline)) {
+              constexpr int dt = decltype(dc)::value;
+              mfma_v<ks == 0>(o[dt][0], fv[dt], pf[0]);
+              mfma_v<ks == 0>(o[dt][1], fv[dt], pf[1]);
+            });
+            MFMA_FENCE();
+          }
+        });
+        static_for<8>([&](auto dc) __attribute__((always_inline)) {
+          constexpr int dt = decltype(dc)::value;
+          o_set<dt, Q0>(o[dt][0]);
+          o_set<dt, Q0 + 1>(o[dt][1]);
+        });
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          m_ref[Q0 + q] = m[q];
+          l_row[Q0 + q] = l[q];
         }
       };
       constexpr std::integral_constant<int, 0> block0{};
@@ -633,7 +703,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
         auto visit = [&](auto masked, auto v_rows) __attribute__((always_inline)) {
           constexpr int MASKED = decltype(masked)::value;
           constexpr bool V_ROWS = decltype(v_rows)::value;
-          if (PBS_UNLIKELY(e_cur & unseen)) first_reference(e_cur);
+          if (PBS_UNLIKELY(e_cur & unseen)) first_reference(std::integral_constant<int, 0>{}, e_cur);
           if (PBS_LIKELY((e_cur & (USE0 | USE1)) == (USE0 | USE1)))
             fast_tile<0, 4, MASKED, V_ROWS>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
           else if (V_ROWS || (e_cur & USE0))   // (of own-segment tiles the second block alone visits its diagonal one only)
@@ -679,10 +749,9 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
           if (more) aim_anew(hb, e_nxt, bufx ^ 0x8000u);
           else aim_past_item();
           if (PBS_UNLIKELY(e_cur & unseen & USE0)) {
-            copy_tile_now(copy);
-            careful_tile(block0, e_cur);
+            first_diagonal_tile(block0);
             if (e_cur & USE1) {
-              if (unseen & USE1) first_reference(USE1);
+              if (unseen & USE1) first_reference(std::integral_constant<int, 2>{}, USE1);
               fast_tile<2, 2, 0, true, false>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
             }
           } else if (e_cur & (USE0 | USE1)) {
@@ -697,8 +766,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
           tile_head(it);
           aim_past_item();
           if (PBS_UNLIKELY(e_cur & unseen)) {
-            copy_tile_now(copy);
-            careful_tile(block1, e_cur);
+            first_diagonal_tile(block1);
           } else {
             fast_tile<2, 2, 12, true>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
           }

@@ -167,6 +167,14 @@ __device__ __forceinline__ uint32_t vrow_lane_addr(uint32_t v_buf, int lane) {
 
 #define PBS_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0)
 
+// the largest of three logits (a NaN only if all are), one instruction: the compiler puts one more per operand in front, to quieten
+// signalling NaNs, of which matrix instructions have none
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
 // over the four lanes l, l ^ 16, l ^ 32, l ^ 48 that share a query column, by row exchanges of the vector unit (a shuffle
 // goes through LDS)
 template <class F>
@@ -250,6 +258,20 @@ __device__ __forceinline__ void mfma_s(f32x4& d, const bf16x8& k) {
   constexpr int r = q_reg(Q, KD);
   if constexpr (FROM_ZERO) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, a[%2:%3], 0" : "=v"(d) : "v"(k), "n"(r), "n"(r + 3));
   else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, a[%2:%3], %0" : "+v"(d) : "v"(k), "n"(r), "n"(r + 3));
+}
+// the same with the sums in vector registers
+template <bool FROM_ZERO>
+__device__ __forceinline__ void mfma_v(f32x4& d, const bf16x8& v, const bf16x8& p) {
+  if constexpr (FROM_ZERO) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=v"(d) : "v"(v), "v"(p));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(v), "v"(p));
+}
+template <int DT, int Q>
+__device__ __forceinline__ void o_set(const f32x4& x) {
+  constexpr int r = o_reg(DT, Q);
+  asm volatile("v_accvgpr_write_b32 a[%1], %0" ::"v"(x[0]), "n"(r));
+  asm volatile("v_accvgpr_write_b32 a[%1], %0" ::"v"(x[1]), "n"(r + 1));
+  asm volatile("v_accvgpr_write_b32 a[%1], %0" ::"v"(x[2]), "n"(r + 2));
+  asm volatile("v_accvgpr_write_b32 a[%1], %0" ::"v"(x[3]), "n"(r + 3));
 }
 template <int DT, int Q>
 __device__ __forceinline__ void mfma_o(const bf16x8& v, const bf16x8& p) {

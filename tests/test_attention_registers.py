@@ -1,7 +1,7 @@
 """The attention kernel keeps O and Q^T in accumulation registers that it names itself, and issues its matrix
 instructions, tile copies and query loads from inline assembly, which the compiler does not look into.  What that relies
 on is checked in the compiled code: the compiler uses no accumulation register of its own, nothing is spilled to memory,
-and an address that a vector instruction has put into scalar registers is not read by a memory instruction within the
+results of matrix instructions are given their time, an address that a vector instruction has put into scalar registers is not read by a memory instruction within the
 five wait states the hardware asks for; and a load into an accumulation register is awaited before the register is read."""
 import os
 import re
@@ -155,3 +155,31 @@ def test_loads_into_accumulation_registers_are_awaited_on_every_path(kernels):
     for name, body in kernels[1].items():
         assert re.search(r"global_load_dwordx4 a\[", body), name
         assert not _unfinished_reads(body), name
+
+
+def _vector_regs(token):
+    m = re.fullmatch(r"v\[(\d+):(\d+)\]", token) or re.fullmatch(r"[-|]*v(\d+)()\|?", token)
+    return range(int(m[1]), int(m[2] or m[1]) + 1) if m else ()
+
+
+def test_results_of_matrix_instructions_have_settled(kernels):
+    """The result of a matrix instruction may be touched by other instructions 11 wait states after it, what a vector instruction
+    wrote may be read by a matrix instruction 3 states after it.  The compiler sees to that for its own matrix
+    instructions only.  In order of the code; a matrix instruction counts as the four states for which it holds the pipe."""
+    for name, body in kernels[1].items():
+        issued, written, now = {}, {}, 0
+        for line in body.splitlines():
+            t = line.split(";")[0].replace(",", " ").split()
+            if not t or t[0].startswith(".") or t[0].endswith(":"):
+                continue
+            if t[0].startswith("v_mfma"):
+                assert all(now - written.get(r, -9) >= 3 for tok in t[2:4] for r in _vector_regs(tok)), (name, line)
+                issued.update(dict.fromkeys(_vector_regs(t[1]), now))
+                now += 4
+                continue
+            assert all(now - issued.get(r, -99) > 11 for tok in t[1:] for r in _vector_regs(tok)), (name, line)
+            if t[0].startswith("v_"):
+                for r in _vector_regs(t[1]):
+                    written[r] = now
+                    issued.pop(r, None)
+            now += 1 + (int(t[1]) if t[0] == "s_nop" else 0)
