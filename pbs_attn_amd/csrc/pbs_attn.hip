@@ -613,7 +613,9 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       // A diagonal tile that is its block's first tile (the first 128 keys of a sequence, or a block that selected nothing): online
       // softmax as well, since with a reference from some of so few keys the error against 64-bit arithmetic was 3 %
       // larger.  The logits come first, the next tile's copies between them, and the sums stay in vector registers, O being
-      // zero so far; sub-tiles up to the wave's own (the rest is hidden), none where its queries lie past the sequence.
+      // zero so far; sub-tiles up to the wave's own (the rest is hidden), none where its queries lie past the sequence.  (Attention
+      // launch, pipelined form -> this: 77 tokens 10.3 -> 10.4 us, 128 tokens 10.4 -> 11.0, 256 tokens on 16 heads 12.9 -> 15.0; with
+      // the careful tile above 77 tokens took 13.0 and 256 about 18.)
       auto first_diagonal_tile = [&](auto bc) __attribute__((always_inline)) {
         constexpr int block = decltype(bc)::value, Q0 = 2 * block;
         if ((qb0 + block) * BS + 32 * wave >= hb.S) {
@@ -697,9 +699,9 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
           e_cur = e_nxt;
         };
         // A tile that one block only visits runs for that block's column groups: what the other one did not select stays out of
-        // its rows, whatever its values.  About every eleventh tile is of that kind at 4k .. 32k, one in a hundred at 128k (with zero probabilities
-        // for the other two groups instead -> this: MeanPooling 16k 1648 -> 1583 us, 32k 6.11 -> 5.93 ms, 64k layer 23.97 -> 23.05 ms; 128k
-        // 86.0 ms either way).
+        // its rows, whatever its values.  The second blocks' diagonal tiles included, 9 to 14 % of all tiles are of that kind at 4k .. 64k,
+        // 1.4 % at 128k (zero probabilities for the other two groups instead -> this: MeanPooling 16k 1648 -> 1583 us, 32k
+        // 6.11 -> 5.93 ms, 64k layer 23.97 -> 23.05 ms; 128k 86.0 ms either way).
         auto visit = [&](auto masked, auto v_rows) __attribute__((always_inline)) {
           constexpr int MASKED = decltype(masked)::value;
           constexpr bool V_ROWS = decltype(v_rows)::value;
