@@ -62,23 +62,25 @@ struct AttnArgs {
   const uint16_t* pvt;   // (B*Hq, nb, 128, 128) permuted V blocks, transposed
   const uint16_t* k;     // original K at the KV heads, caller's strides
   const uint16_t* v;     // original V at the KV heads, caller's strides
-  const uint16_t* plist; // (B*Hq * npair, cap) merged visit lists, in item order
+  const uint16_t* plist; // (B*Hq * n_items, cap) merged visit lists, in item order
   int* queue;            // 8 work counters, one per XCD
   int cap;               // entries per list row (multiple of 8); 0: no lists in memory and no counters (see own_list)
   uint16_t* o;
   int BH, Hq, Hkv, S, nb, bps;
+  int span, n_items;  // query blocks of an item (two, or one: see item_span), items of a head
   uint32_t k_ss, v_ss;   // key / value row strides in elements (< 2^22)
   int xcd_start[9];   // work items (head-major, long rows first) of XCD x: [xcd_start[x], xcd_start[x + 1])
-  int interleave;     // 0, or 1 + log2(whole heads per XCD range) of a small launch whose tickets go pair-major (see ticket_item)
+  int deal_heads;     // 0, or the heads over which the tickets of a small launch are dealt, longest items first (see ticket_item)
+  uint32_t deal_magic;   // quotients by deal_heads: high word of a product
   int64_t q_sb, q_sh, q_ss, k_sb, k_sh, v_sb, v_sh, o_sb, o_sh, o_ss;
   float scale_log2;
 };
 
 typedef const __attribute__((address_space(4))) struct AttnArgs* ArgsPtr;
 
-// ---- merged visit list of a pair of query blocks, built once per pass by its own kernel.  Row `item` of `plist` (items
-// are numbered head by head, the long pairs of a head first) starts with a header that saves the attention kernel its
-// divisions -- [0] number of tiles, [1] batch, [2] query head, [3] KV head, [4] first query block -- and holds from
+// ---- merged visit list of an item (a pair of query blocks, or one), built once per pass by its own kernel.  Row `item` of `plist` (items
+// are numbered head by head, the long ones of a head first) starts with a header that saves the attention kernel its
+// divisions -- [0] number of tiles, [1] batch, [2] query head, [3] KV head, [4] first query block, [5] how many -- and holds from
 // LIST_HEADER on entries kb | ENT_ORIG? | use_first << 14 |
 // use_second << 15: the union of the two visit lists (ascending), then the own segments in ORIGINAL key order
 // (blocks first-of-segment .. query block, shared where the two blocks share a segment).  Without `cols` every block of
@@ -87,21 +89,22 @@ typedef const __attribute__((address_space(4))) struct AttnArgs* ArgsPtr;
 constexpr int MERGE_THREADS = 256;
 __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const int32_t* __restrict__ cols, const int32_t* __restrict__ cnt,
                                                                uint16_t* __restrict__ plist, int* __restrict__ queue, int nb,
-                                                               int bps, int cap, int Hq, int group, int first_tickets,
+                                                               int span, int bps, int cap, int Hq, int group, int first_tickets,
                                                                const uint8_t* __restrict__ own_needed) {
   __shared__ uint8_t flags0[4096], flags1[4096];
   __shared__ int wsum[MERGE_THREADS / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int npair = (nb + 1) >> 1;
-  const int bh = blockIdx.x / npair, pair = blockIdx.x % npair;
+  const int n_items = (nb + span - 1) / span;
+  const int bh = blockIdx.x / n_items, item = blockIdx.x % n_items;
   if (blockIdx.x == 0 && tid < 8) queue[tid] = first_tickets;
-  const bool second = 2 * pair + 1 < nb;
-  const int qb0 = 2 * pair, qb1 = second ? qb0 + 1 : qb0;
+  const int qb0 = span * item;
+  const bool second = span == 2 && qb0 + 1 < nb;
+  const int qb1 = second ? qb0 + 1 : qb0;
   const int sf0 = (qb0 / bps) * bps, sf1 = (qb1 / bps) * bps;
-  const int32_t* l0 = cols + ((int64_t)bh * nb + 2 * pair) * nb;
+  const int32_t* l0 = cols + ((int64_t)bh * nb + qb0) * nb;
   const int32_t* l1 = l0 + (second ? nb : 0);
-  const int n0 = cols ? cnt[(int64_t)bh * nb + 2 * pair] : 0;
-  const int n1 = cols && second ? cnt[(int64_t)bh * nb + 2 * pair + 1] : 0;
+  const int n0 = cols ? cnt[(int64_t)bh * nb + qb0] : 0;
+  const int n1 = cols && second ? cnt[(int64_t)bh * nb + qb1] : 0;
   constexpr int MAX_PER = 4096 / MERGE_THREADS;
   int c0[MAX_PER], c1[MAX_PER];
 #pragma unroll
@@ -142,13 +145,14 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
     if (x < wave) w += ws;
     total += ws;
   }
-  uint16_t* out = plist + ((int64_t)bh * npair + (npair - 1 - pair)) * cap;
+  uint16_t* out = plist + ((int64_t)bh * n_items + (n_items - 1 - item)) * cap;
   if (tid == 0) {
     const int h = bh % Hq;
     out[1] = (uint16_t)(bh / Hq);
     out[2] = (uint16_t)h;
     out[3] = (uint16_t)(h / group);
-    out[4] = (uint16_t)(2 * pair);
+    out[4] = (uint16_t)qb0;
+    out[5] = (uint16_t)(second ? 2 : 1);
   }
   uint16_t* const header = out;
   out += LIST_HEADER;
@@ -180,22 +184,24 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
   if (tid == 0) header[0] = (uint16_t)(total + n_own);
 }
 
-// Ticket t of the counter of a range of `count` items starting at `begin` -> work item.  Items are numbered head by
-// head, long rows first, and normally handed out in that order (an XCD walks one head at a time: its workgroups
-// share that head's K / V stream in L2).  A launch with only a few items per workgroup cannot balance that way: a
-// workgroup that starts with a short item of one head is handed a long item of the next and finishes last.  There
-// (`il` = 1 + log2 of the whole heads per range, a power of two) the same row pair of every head of the range goes
-// out before the next shorter pair: longest items first across the range.
-// Takes and returns begin + ticket (wave-uniform values: scalar arithmetic only); a ticket past the range is left alone.
-__device__ __forceinline__ int ticket_item(int begin, int end, int item, int il, int npair) {
-  if (il > 0 && item < end) {
-    const int t = item - begin;
-    item = begin + (t & ((1 << (il - 1)) - 1)) * npair + (t >> (il - 1));
-  }
-  return item;
+// Ticket `ticket` (counted from the range's first) of XCD range x, [begin, end) -> work item, or NO_ITEM past the range's end.  Items
+// are numbered head by head, long ones first, and normally handed out in that order (an XCD walks one head at a time: its
+// workgroups share that head's K / V stream in L2).  A launch with only a few items per workgroup cannot balance that way: a
+// workgroup that starts with a short item of one head is handed a long item of the next and finishes last.  There the
+// same item of every head goes out before the next shorter one, longest first: the heads of the range, where
+// every range is of whole heads, or all heads, dealt to the XCDs in turn.  Whole pass, head by head -> dealt: 28 / 4 heads x 4096
+// 199 -> 164 us, x 5120 250 -> 222, x 10240 675 -> 641; 32 / 8 x 4352 219 -> 200, x 5120 260 -> 248, x 10240 731 -> 711.  (Wave-uniform
+// values: scalar arithmetic only.)
+constexpr int NO_ITEM = 1 << 28;
+__device__ __forceinline__ int ticket_item(ArgsPtr a, int x, int begin, int end, int ticket) {
+  if (begin + ticket >= end) return NO_ITEM;
+  const int m = a->deal_heads;
+  if (m == 0) return begin + ticket;
+  const bool all = m == a->BH;
+  const uint32_t r = (uint32_t)(all ? 8 * ticket + x : ticket);
+  const int len = m == 1 ? (int)r : (int)(((uint64_t)r * a->deal_magic) >> 32);
+  return (all ? 0 : begin) + ((int)r - len * m) * a->n_items + len;
 }
-
-constexpr int NO_ITEM = 1 << 28;   // a ticket past every range (a launch has fewer items)
 
 // asynchronous copy of one list row (`chunks` 16-byte pieces) into LDS at byte offset `lds_byte`
 __device__ __forceinline__ void stage_list_async(const uint16_t* src, int chunks, uint32_t lds_byte, int wave, int tid) {
@@ -229,7 +235,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   // registers for the whole kernel.
 #define PBS_ARGS() ({ ArgsPtr p_ = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(); asm volatile("" : "+s"(p_)); p_; })
   ArgsPtr a0 = PBS_ARGS();
-  const int npair = (a0->nb + 1) >> 1;
+  const int n_items = a0->n_items;
   const int xcd = blockIdx.x & 7;
   int q_begin = a0->xcd_start[xcd], q_end = a0->xcd_start[xcd + 1];   // the range being served: this XCD's, later others'
   int vic = xcd, vic_tried = a0->cap ? 0 : 7;   // (no counters: every item is some workgroup's first)
@@ -259,22 +265,22 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       q_begin = as->xcd_start[vic];
       q_end = as->xcd_start[vic + 1];
       __syncthreads();   // everyone has read the previous ticket
-      if (wave == 0 && lane_id_here() == 0) misc[4] = q_begin + atomicAdd(as->queue + vic, 1);
+      if (wave == 0 && lane_id_here() == 0) misc[4] = atomicAdd(as->queue + vic, 1);
       __syncthreads();
-      found = ticket_item(q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]), as->interleave, npair);
-      if (found < q_end) return true;
+      found = ticket_item(as, vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
+      if (found < NO_ITEM) return true;
     }
     return false;
   };
   // The first item: workgroup n of an XCD takes ticket n, without asking (the counters start behind these tickets); where the
   // range is shorter than that, an item of another one.
   if (threadIdx.x == 0) misc[1] = 0;
-  int cur = ticket_item(q_begin, q_end, q_begin + ((int)blockIdx.x >> 3), a0->interleave, npair);
-  if (PBS_UNLIKELY(cur >= q_end)) {
+  int cur = ticket_item(a0, xcd, q_begin, q_end, (int)blockIdx.x >> 3);
+  if (PBS_UNLIKELY(cur == NO_ITEM)) {
     if (!claim_elsewhere()) return;
     cur = found;
   }
-  int nxt = q_end;   // the next item is claimed late in the current one: an item claimed early waits for this
+  int nxt = NO_ITEM;   // the next item is claimed late in the current one: an item claimed early waits for this
                      // workgroup while others may be idle
   bool has_nxt = false;
 
@@ -284,7 +290,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     int n_tiles, b, h, qb0;
     const uint16_t *pk, *pvt, *korig, *vorig;
     uint32_t k_ss, v_ss;
-    int S;
+    int S, q_end;   // q_end: end of the item's queries
   };
   auto read_item = [&](ArgsPtr ap, const uint16_t* list) __attribute__((always_inline)) {
     Item t;
@@ -293,7 +299,8 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     t.n_tiles = (int)(w0 & 0xffffu);
     t.b = (int)(w0 >> 16);
     t.h = (int)(w1 & 0xffffu);
-    t.qb0 = (int)__builtin_amdgcn_readfirstlane((int)hd[2]) & 0xffff;
+    const uint32_t w2 = (uint32_t)__builtin_amdgcn_readfirstlane((int)hd[2]);
+    t.qb0 = (int)(w2 & 0xffffu);
     const int64_t tiles = (int64_t)(t.b * ap->Hq + t.h) * ap->nb * (BS * D), kvh = (int)(w1 >> 16);
     t.pk = ap->pk + tiles;
     t.pvt = ap->pvt + tiles;
@@ -302,6 +309,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     t.k_ss = ap->k_ss;
     t.v_ss = ap->v_ss;
     t.S = ap->S;
+    t.q_end = min(t.S, (t.qb0 + (int)(w2 >> 16)) * BS);
     return t;
   };
   auto first_entry = [&](const uint16_t* list) __attribute__((always_inline)) {
@@ -337,12 +345,12 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   };
   auto list_row = [&](ArgsPtr ap, int item) __attribute__((always_inline)) { return ap->plist + (int64_t)item * ap->cap; };
   // an item's Q^T fragments (B operand): column i16 of group qg is query 32 wave + 16 (qg % 2) + i16 of block qg / 2,
-  // d = 32 kd + 8 g4 + 0..7.  Rows past the end of the sequence compute on the last row's values and are never stored.
+  // d = 32 kd + 8 g4 + 0..7.  Rows past the end of the item's queries compute on the last row's values and are never stored.
   auto load_q = [&](ArgsPtr aq, const Item& t, auto set) __attribute__((always_inline)) {
     const int ln = lane_id_here();
     const int64_t q_ss = aq->q_ss;
     const uint16_t* qhead = aq->q + t.b * aq->q_sb + t.h * aq->q_sh + 8 * (ln >> 4);
-    const int last = t.S - 1, pos0 = t.qb0 * BS + 32 * wave + (ln & 15);
+    const int last = t.q_end - 1, pos0 = t.qb0 * BS + 32 * wave + (ln & 15);
     static_for<QG>([&](auto qc) __attribute__((always_inline)) {
       constexpr int qg = decltype(qc)::value, st = decltype(set)::value;
       const uint16_t* qrow = qhead + (int64_t)min(pos0 + (qg >> 1) * BS + (qg & 1) * 16, last) * q_ss;
@@ -357,8 +365,8 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   // has a workgroup of its own, so that nothing is left of the list kernel (counters, further items).
   auto own_list = [&](ArgsPtr ap, int item) __attribute__((always_inline)) {
     uint16_t* list = reinterpret_cast<uint16_t*>(smem + LDS_LIST);
-    const int bh = item / npair, qb0 = 2 * (npair - 1 - (item - bh * npair));
-    const bool second = qb0 + 1 < ap->nb;
+    const int bh = item / n_items, qb0 = ap->span * (n_items - 1 - (item - bh * n_items));
+    const bool second = ap->span == 2 && qb0 + 1 < ap->nb;
     const int n_own = second ? qb0 + 2 : qb0 + 1;
     for (int kb = (int)threadIdx.x; kb < n_own; kb += THREADS)
       list[LIST_HEADER + kb] = (uint16_t)((uint32_t)kb | ENT_ORIG | (kb <= qb0 ? 1u << 14 : 0u) | (second ? 2u << 14 : 0u));
@@ -369,6 +377,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       list[2] = (uint16_t)h;
       list[3] = (uint16_t)(h / (ap->Hq / ap->Hkv));
       list[4] = (uint16_t)qb0;
+      list[5] = (uint16_t)(second ? 2 : 1);
     }
   };
 
@@ -420,11 +429,11 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     // tile.  Items of fewer than three tiles finish these steps after their loop.
     const int claim_it = careful_only ? -8 : max(n_tiles - 3, 0);
     auto publish_and_fetch = [&]() __attribute__((always_inline)) {   // between the wait for this thread's loads and the barrier ...
-      if (wave == 0 && lane_id_here() == 0) misc[4] = q_begin + claim;
+      if (wave == 0 && lane_id_here() == 0) misc[4] = claim;
     };
     auto adopt_next = [&]() __attribute__((always_inline)) {          // ... and after the barrier
-      nxt = ticket_item(q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]), PBS_ARGS()->interleave, npair);
-      has_nxt = nxt < q_end;
+      nxt = ticket_item(PBS_ARGS(), vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
+      has_nxt = nxt < NO_ITEM;
       if (has_nxt)
         stage_list_async(list_row(PBS_ARGS(), nxt), PBS_ARGS()->cap >> 3, LDS_LIST + (li ^ 1u) * LIST_BYTES, wave, wave * 64 + lane_id_here());
     };
@@ -618,7 +627,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       // the careful tile above 77 tokens took 13.0 and 256 about 18.)
       auto first_diagonal_tile = [&](auto bc) __attribute__((always_inline)) {
         constexpr int block = decltype(bc)::value, Q0 = 2 * block;
-        if ((qb0 + block) * BS + 32 * wave >= hb.S) {
+        if ((qb0 + block) * BS + 32 * wave >= hb.q_end) {
           copy_tile_now(copy);
           return;
         }
@@ -827,12 +836,12 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       const int pos0 = qb0 * BS + 32 * wave + (lane_e >> 4);      // this lane's first row
       uint16_t* obase = ae->o + hb.b * ae->o_sb + hb.h * ae->o_sh + pos0 * o_ss + (lane_e & 15) * 8;
       const uint8_t* rd = smem + stage + (lane_e >> 4) * 256;
-      const bool full = (qb0 + 2) * BS <= hb.S;
+      const bool full = (qb0 + 2) * BS <= hb.q_end;
       auto out_rows = [&](auto all) __attribute__((always_inline)) {
 #pragma unroll
         for (int n = 0; n < 16; ++n) {              // rows 4 n .. 4 n + 3 of the wave's 64: n < 8 of the first block
           const int row = 4 * n + (lane_e >> 4), rel = (n >> 3) * BS + 4 * (n & 7);
-          if (decltype(all)::value || pos0 + rel < hb.S)
+          if (decltype(all)::value || pos0 + rel < hb.q_end)
             *reinterpret_cast<u32x4*>(obase + rel * o_ss) = *reinterpret_cast<const u32x4*>(rd + n * 1024 + (((lane_e & 15) ^ (row & 15)) * 16));
         }
       };
@@ -861,7 +870,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     par ^= (n_tiles & 1) ? 0x8000u : 0u;
     li ^= 1u;
     cur = nxt;
-    nxt = q_end;
+    nxt = NO_ITEM;
     has_nxt = false;
     // (nobody is still to read it: it was zero when this item's last barrier had been passed, or the item was a repetition, which
     // does not read it; the next item's barriers lie before it can be set again)
@@ -878,11 +887,23 @@ std::atomic<int> g_cu_count[64];           // CUs of device d (0: not looked up 
 // earlier segments, at most bps + 1 own-segment blocks
 static int list_cap(int nb, int bps) { return (LIST_HEADER + nb + std::min(bps, nb) + 1 + 7) / 8 * 8; }
 
-// workspace: 256 bytes of work counters, then one merged visit list per pair of query blocks
+// Query blocks per work item: two, which share every tile and each of its fragments, or, in a short pass, one.  A pass of few blocks
+// leaves CUs idle or waits for its longest pair, and a tile for one block takes 2950 cycles against 5100 for two.  Whole pass,
+// pairs -> single blocks, us: 32 / 8 heads x 1024 70.5 -> 67.8, x 1536 85.9 -> 81.8; 28 / 4 x 1000 74.3 -> 69.7; 4 / 1 x 8192 191 -> 146;
+// in one segment 32 / 8 x 512 18.4 -> 14.9, x 1024 28.7 -> 21.5, 8 / 2 x 4096 84.7 -> 58.4.  Up to 512 blocks (two items a
+// workgroup) few, long heads still gain: 8 / 2 x 8192 198 -> 169, 4 / 1 x 16384 343 -> 278; many short ones do not on every input (32 / 8 x
+// 2048 99.6 -> 97.5, concentrated 86.4 -> 88.9).  With 560 blocks and more pairs are better everywhere (32 / 8 x 2560 116 -> 128).
+constexpr int SINGLE_BLOCK_ITEMS = 384;
+constexpr int SINGLE_FEW_HEADS = 512;
+constexpr int DEAL_ITEMS = 2048;
+static int item_span(int rows, int nb) { return (int64_t)rows * nb <= (rows <= 16 ? SINGLE_FEW_HEADS : SINGLE_BLOCK_ITEMS) ? 1 : 2; }
+static int items_of(int nb, int span) { return (nb + span - 1) / span; }
+
+// workspace: 256 bytes of work counters, then one merged visit list per item
 
 extern "C" size_t pbs_sparse_attn_workspace_bytes(int B, int Hq, int S, int segment_size) {
-  const int64_t nb = (S + BS - 1) / BS, npair = (nb + 1) / 2, cap = list_cap((int)nb, segment_size / BS);
-  return 256 + (size_t)B * Hq * npair * cap * 2;
+  const int64_t nb = (S + BS - 1) / BS, n_items = items_of((int)nb, item_span(B * Hq, (int)nb)), cap = list_cap((int)nb, segment_size / BS);
+  return 256 + (size_t)B * Hq * n_items * cap * 2;
 }
 
 extern "C" int pbs_sparse_attn_fwd(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,
@@ -912,34 +933,44 @@ extern "C" int pbs_sparse_attn_fwd_optional_diagonal(const void* q, const void* 
 
 // the eight ranges of work items (AttnArgs::xcd_start) and the ticket order; returns the items of the longest range
 static int plan_ranges(AttnArgs& a) {
-  // eight ranges of equal estimated work: the row pair p of a head costs about p + 1 (causal length)
-  const int64_t npair = (a.nb + 1) / 2;
-  const double head_work = 0.5 * (double)npair * (double)(npair + 1);
+  // eight ranges of equal estimated work: item p of a head costs about p + 1 (causal length)
+  a.span = item_span(a.BH, a.nb);
+  a.n_items = items_of(a.nb, a.span);
+  const int64_t n = a.n_items;
+  const double head_work = 0.5 * (double)n * (double)(n + 1);
   int max_items = 0;
   for (int x = 0; x <= 8; ++x) {
     const double target = head_work * a.BH * x / 8.0;
     int64_t head = (int64_t)(target / head_work);
     if (head > a.BH) head = a.BH;
     const double rem = target - head * head_work;
-    // items of a head in launch order are pairs npair - 1, npair - 2, ...: the first i of them cost
-    // i * npair - i (i - 1) / 2
-    int64_t lo = 0, hi = npair;
+    // items of a head in launch order are n - 1, n - 2, ...: the first i of them cost
+    // i * n - i (i - 1) / 2
+    int64_t lo = 0, hi = n;
     while (lo < hi) {
       const int64_t mid = (lo + hi) / 2;
-      if ((double)mid * npair - 0.5 * (double)mid * (mid - 1) >= rem - 1e-6) hi = mid; else lo = mid + 1;
+      if ((double)mid * n - 0.5 * (double)mid * (mid - 1) >= rem - 1e-6) hi = mid; else lo = mid + 1;
     }
-    int64_t start = head * npair + (head < a.BH ? lo : 0);
-    if (x == 8) start = (int64_t)a.BH * npair;
+    int64_t start = head * n + (head < a.BH ? lo : 0);
+    if (x == 8) start = (int64_t)a.BH * n;
     a.xcd_start[x] = (int)start;
     if (x > 0) max_items = std::max(max_items, a.xcd_start[x] - a.xcd_start[x - 1]);
   }
-  // at most two items per workgroup and ranges of whole heads: hand the tickets out pair-major (see ticket_item;
-  // with four and more items per workgroup the head-by-head order balances well enough and is 1-3 % faster)
-  a.interleave = 0;
-  const int nh = a.BH / 8;
-  if (a.BH % 8 == 0 && (nh & (nh - 1)) == 0 && (int64_t)a.BH * npair <= (int64_t)2 * 256) {
-    for (a.interleave = 1; (1 << (a.interleave - 1)) < nh; ++a.interleave) {}
-    for (int x = 0; x <= 8; ++x) a.xcd_start[x] = (int)(x * (int64_t)nh * npair);
+  // at most eight items per workgroup: longest items first (see ticket_item).  With sixteen the head-by-head order balances well enough, and
+  // where attention is near-uniform it is faster by what an XCD's workgroups share of a head in L2: 32 / 8 x 32768 5.78 against
+  // 6.00 ms.  (Concentrated inputs would gain 1 % there and 7 % at 2 x 28 / 4 heads x 13333.)
+  a.deal_heads = 0;
+  a.deal_magic = 0;
+  const int64_t total = (int64_t)a.BH * n;
+  if (total <= DEAL_ITEMS) {
+    const bool whole_heads = a.BH % 8 == 0;
+    a.deal_heads = whole_heads ? a.BH / 8 : a.BH;
+    a.deal_magic = (uint32_t)((1ull << 32) / a.deal_heads + 1);   // exact for numbers and divisors up to DEAL_ITEMS, 1 apart
+    max_items = 0;
+    for (int x = 0; x <= 8; ++x) {
+      a.xcd_start[x] = whole_heads ? (int)(x * total / 8) : (int)(x * (total / 8) + std::min<int64_t>(x, total % 8));   // (items 8 t + x < total)
+      if (x > 0) max_items = std::max(max_items, a.xcd_start[x] - a.xcd_start[x - 1]);
+    }
   }
   return max_items;
 }
@@ -968,6 +999,7 @@ PairLists pbs_pair_lists(int B, int Hq, int Hkv, int S, int block_size, int segm
   l.Hq = Hq;
   l.group = Hq / Hkv;
   l.first_tickets = (int)(workgroups(plan_ranges(a)) / 8);
+  l.span = a.span;
   return l;
 }
 
@@ -999,8 +1031,7 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
   a.q_sb = q_sb; a.q_sh = q_sh; a.q_ss = q_ss; a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = (uint32_t)k_ss; a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = (uint32_t)v_ss; a.o_sb = o_sb; a.o_sh = o_sh; a.o_ss = o_ss;
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   PBS_REQUIRE(a.nb <= 4096, "pbs_sparse_attn_fwd: more than 4096 blocks per sequence (%d)", a.nb);
-  const int64_t npair = (a.nb + 1) / 2;
-  PBS_REQUIRE((int64_t)a.BH * npair < (1ll << 28) && B < 65536 && Hq < 65536, "pbs_sparse_attn_fwd: launch too large");
+  PBS_REQUIRE((int64_t)a.BH * ((a.nb + 1) / 2) < (1ll << 28) && B < 65536 && Hq < 65536, "pbs_sparse_attn_fwd: launch too large");
   const int max_items = plan_ranges(a);
   a.cap = list_cap(a.nb, a.bps);
   PBS_REQUIRE((uint32_t)a.cap * 2 <= LIST_BYTES, "pbs_sparse_attn_fwd: visit list too long");
@@ -1025,8 +1056,8 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
   const bool own_lists = !lists_built && !csr_cols && !own_block_needed && a.bps >= a.nb && max_items <= n_wg / 8;
   if (own_lists) a.cap = 0;
   else if (!lists_built)
-    hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * npair)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
-                     (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.bps, a.cap, Hq, Hq / Hkv, (int)(n_wg / 8), own_block_needed);
+    hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * a.n_items)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
+                     (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.span, a.bps, a.cap, Hq, Hq / Hkv, (int)(n_wg / 8), own_block_needed);
   hipLaunchKernelGGL(sparse_attn_kernel, dim3((unsigned)n_wg), dim3(THREADS), LDS_TOTAL, (hipStream_t)stream, a);
   return pbs_check_launch("pbs_sparse_attn_fwd");
 }

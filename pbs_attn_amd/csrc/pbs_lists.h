@@ -4,16 +4,17 @@
 #include "pbs_common.h"
 
 constexpr int LIST_HEADER = 8;              // uint16 entries in front of a row's tiles: [0] number of tiles, [1] batch, [2] query head,
-                                            // [3] KV head, [4] first query block of the pair
+                                            // [3] KV head, [4] first query block of the item, [5] how many (two, or one)
 constexpr uint32_t ENT_KB = 0x1fffu;        // visit-list entry: key block ...
 constexpr uint32_t ENT_ORIG = 0x2000u;      // ... | tile of the un-permuted K / V (own segment) | use bits 14, 15
 
-// Where the lists go: row `bh * npair + (npair - 1 - pair)` of `plist`, `cap` entries each, and the attention kernel's eight
+// Where the lists go: row `bh * n + (n - 1 - item)` of `plist` for the n items of a head, `span` query blocks each (the last one
+// may have fewer), `cap` entries a row, and the attention kernel's eight
 // work counters, which start at `first_tickets`.
 struct PairLists {
   uint16_t* plist;
   int* queue;
-  int cap, Hq, group, first_tickets;   // group: query heads per KV head
+  int cap, Hq, group, first_tickets, span;   // group: query heads per KV head
 };
 // of the lists that pbs_sparse_attn_launch expects in `workspace` with lists_built set
 PairLists pbs_pair_lists(int B, int Hq, int Hkv, int S, int block_size, int segment_size, void* workspace);

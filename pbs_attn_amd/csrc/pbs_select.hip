@@ -590,7 +590,7 @@ __global__ __launch_bounds__(256) void select_blocks_groups_kernel(SelectArgs a,
 
 // ---- the single-call path: selection straight into the merged lists that the attention kernel reads (pbs_lists.h).
 // A workgroup decides the rows of two pairs of query blocks, one wave each, into flags in LDS; then the first wave of a
-// pair writes the pair's list and the second one the gather's flags.  No CSR rows (4 bytes per visited block and row, written
+// pair writes the pair's list and the second one the gather's flags (items of one query block: every wave those of its row).  No CSR rows (4 bytes per visited block and row, written
 // here and read back) and no launch that merges them.  Groups are in pairs here: qb_lo / qb_hi are pair numbers.
 // LONG: rows of 1025 .. 2048 candidates, in a kernel of their own: the register need of 32 entries per lane would cost the shorter
 // rows two thirds of their waves.
@@ -623,12 +623,14 @@ __global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, Pa
     }
   }
   __syncthreads();
-  if (!live) return;
-  const bool second = qb0 + 1 < nb;
-  const int qb1 = second ? qb0 + 1 : qb0;
-  const int sf0 = (qb0 / a.bps) * a.bps, sf1 = (qb1 / a.bps) * a.bps;
+  const bool pairs = l.span == 2;
+  if (!live || (!pairs && qb >= nb)) return;
+  const int first = pairs ? qb0 : qb;   // of the item
+  const bool second = pairs && first + 1 < nb;
+  const int qb1 = second ? first + 1 : first;
+  const int sf0 = (first / a.bps) * a.bps, sf1 = (qb1 / a.bps) * a.bps;
   const int end1 = second ? sf1 : 0, end = max(sf0, end1);   // a row's flags count up to its own segment
-  const uint32_t* f0 = reinterpret_cast<const uint32_t*>(smem_w + (wave & 2) * nb_pad);
+  const uint32_t* f0 = reinterpret_cast<const uint32_t*>(smem_w + (pairs ? wave & 2 : wave) * nb_pad);
   const uint32_t* f1 = reinterpret_cast<const uint32_t*>(smem_w + ((wave & 2) + 1) * nb_pad);
   // the flags of blocks 4 x .. 4 x + 3, a byte each: bit 0 visited by the first query block, bit 1 by the second
   auto visited = [&](int x) __attribute__((always_inline)) {
@@ -639,7 +641,7 @@ __global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, Pa
     const uint32_t m0 = below(sf0), m1 = below(end1);
     return (m0 ? f0[x] & m0 : 0u) | (m1 ? f1[x] & m1 : 0u) << 1;
   };
-  if (wave & 1) {
+  if (!pairs || (wave & 1)) {
     if (a.needed)
       for (int x = lane; 4 * x < end; x += 64) {
         const uint32_t v = visited(x);
@@ -647,9 +649,10 @@ __global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, Pa
         for (int e = 0; e < 4; ++e)
           if (v >> (8 * e) & 3u) a.needed[(int64_t)row * nb + 4 * x + e] = 1;   // every writer stores the same value
       }
-    return;
+    if (pairs) return;
   }
-  uint16_t* header = l.plist + ((int64_t)row * npair + (npair - 1 - pair)) * l.cap;
+  const int n_items = pairs ? npair : nb;
+  uint16_t* header = l.plist + ((int64_t)row * n_items + (n_items - 1 - (pairs ? pair : qb))) * l.cap;
   uint16_t* out = header + LIST_HEADER;
   int base = 0;
   for (int x0 = 0; 4 * x0 < end; x0 += 64) {
@@ -670,7 +673,7 @@ __global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, Pa
   const int n_own = qb1 - sf0 + 1;
   for (int t = lane; t < n_own; t += 64) {
     const int kb = sf0 + t;
-    const uint32_t use = (kb <= qb0 ? 1u : 0u) | (second && kb >= sf1 ? 2u : 0u);
+    const uint32_t use = (kb <= first ? 1u : 0u) | (second && kb >= sf1 ? 2u : 0u);
     out[base + t] = (uint16_t)((uint32_t)kb | ENT_ORIG | use << 14);
   }
   if (lane == 0) {
@@ -678,7 +681,8 @@ __global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, Pa
     header[1] = (uint16_t)(row / l.Hq);
     header[2] = (uint16_t)(row % l.Hq);
     header[3] = (uint16_t)(row % l.Hq / l.group);
-    header[4] = (uint16_t)qb0;
+    header[4] = (uint16_t)first;
+    header[5] = (uint16_t)(second ? 2 : 1);
   }
 }
 
