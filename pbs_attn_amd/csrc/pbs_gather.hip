@@ -13,7 +13,7 @@
 //   * filtered: the permuted blocks whose "needed" flag (set by the block selection for every block some query
 //     block visits) is zero are skipped; their perm_k / perm_vt tiles stay unwritten.
 // The pooled values of the two forms are the same bits: same loads, same order of additions.
-#include "pbs_common.h"
+#include "pbs_lists.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 
 namespace {
@@ -253,7 +253,42 @@ __global__ __launch_bounds__(256) void pool_qk_kernel(GatherArgs a, PoolQArgs p,
   else gather_block<true>(a, vt, pool, blk, bh);
 }
 
+// Full gather and query pooling in one launch, for short passes.
+__global__ __launch_bounds__(256) void gather_pool_kernel(GatherArgs a, PoolQArgs p, TaskGroups t) {
+  __shared__ uint16_t vt[BS * VT_PITCH];
+  __shared__ float pool[16][D];
+  int kind, bh, blk;
+  if (!my_task(t, a.nb, kind, bh, blk)) return;
+  if (kind) pool_q_block(pool, p.q, p.pooled_q, a.Hq, a.S, a.nb, p.q_sb, p.q_sh, p.q_ss, p.pool_max, blk, bh);
+  else gather_block<false>(a, vt, pool, blk, bh);
+}
+
 }  // namespace
+
+int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const int32_t* key_indices, void* pooled_q, void* pooled_k,
+                           void* perm_k, void* perm_vt, int B, int Hq, int Hkv, int S, int head_dim, int block_size, int64_t q_sb,
+                           int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
+                           int query_pool_max, int key_pool_max, void* stream) {
+  PBS_REQUIRE(q && k && v && key_indices && pooled_q && pooled_k && perm_k && perm_vt, "pbs_gather_pool: null tensor pointer");
+  PBS_REQUIRE(head_dim == D && block_size == BS, "pbs_gather_pool: head_dim and block_size must be 128 (got %d, %d)", head_dim, block_size);
+  PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0, "pbs_gather_pool: bad shape");
+  PBS_REQUIRE(q_sb % 8 == 0 && q_sh % 8 == 0 && q_ss % 8 == 0 && k_sb % 8 == 0 && k_sh % 8 == 0 && k_ss % 8 == 0 && v_sb % 8 == 0 &&
+                  v_sh % 8 == 0 && v_ss % 8 == 0 && ((uintptr_t)q % 16) == 0 && ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0,
+              "pbs_gather_pool: rows must be 16-byte aligned");
+  GatherArgs a = {};
+  a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.idx = key_indices;
+  a.perm_k = (uint16_t*)perm_k; a.perm_vt = (uint16_t*)perm_vt; a.pooled_k = (uint16_t*)pooled_k;
+  a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.S = S; a.nb = (S + BS - 1) / BS;
+  a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = k_ss; a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = v_ss;
+  a.pool_max = key_pool_max;
+  PoolQArgs p;
+  p.q = (const uint16_t*)q; p.pooled_q = (uint16_t*)pooled_q; p.q_sb = q_sb; p.q_sh = q_sh; p.q_ss = q_ss;
+  p.pool_max = query_pool_max;
+  const TaskGroups t = task_groups(B, Hq, Hkv, a.nb, 2);
+  PBS_REQUIRE(t.grid.y <= 65535 && t.grid.z <= 65535, "pbs_gather_pool: too many heads or blocks");
+  hipLaunchKernelGGL(gather_pool_kernel, t.grid, dim3(256), 0, (hipStream_t)stream, a, p, t);
+  return pbs_check_launch("pbs_gather_pool");
+}
 
 extern "C" int pbs_gather_kv(const void* k, const void* v, const int32_t* key_indices, void* perm_k, void* perm_vt,
                              void* pooled_k, int B, int Hq, int Hkv, int S, int head_dim, int block_size, int64_t k_sb,

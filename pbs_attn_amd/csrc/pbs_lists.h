@@ -40,3 +40,8 @@ int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold
 // to be a complete segment)
 int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,
                                int S_pad, int segment_size, void* stream);
+// pbs_pool_blocks and an unfiltered pbs_gather_kv in one launch (the pooled key blocks have the bits of both)
+int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const int32_t* key_indices, void* pooled_q, void* pooled_k,
+                           void* perm_k, void* perm_vt, int B, int Hq, int Hkv, int S, int head_dim, int block_size, int64_t q_sb,
+                           int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
+                           int query_pool_max, int key_pool_max, void* stream);

@@ -11,6 +11,14 @@ __global__ void identity_indices_kernel(int32_t* idx, int S_pad, int64_t total) 
   if (i < total) idx[i] = (int32_t)(i % S_pad);
 }
 
+// Passes of few, short rows gather every block at once, in the launch that pools: a launch and a read of K less.  Whole pass, filtered gather
+// after the selection -> this, us: 32 / 8 heads x 512 54.3 -> 51.1, x 1024 68.9 -> 64.4, x 4096 181 -> 175, x 8192 499 -> 488, on
+// concentrated inputs 64.0 -> 59.8, 141 -> 139, 339 -> 333; 28 / 4 x 8192 218 -> 216.5.  Longer rows leave more of the blocks unvisited: 8 / 2
+// heads x 16384, concentrated, 154.9 against 156.7, x 32768 263 against 279.
+constexpr int SHORT_PASS_BLOCKS = 2048, SHORT_PASS_ROW = 64;
+bool short_pass(int rows, int nb) { return nb <= SHORT_PASS_ROW && rows * nb <= SHORT_PASS_BLOCKS; }
+
+
 struct Layout {
   size_t scores, score_ws, idx, perm_k, perm_vt, pooled_k, pooled_q, probs, cols, cnt, needed, select_ws, attn_ws, total;
 };
@@ -119,16 +127,22 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
     if ((rc = pbs_segment_argsort_launch((const float*)(w + L.scores), (int32_t*)(w + L.idx), (int32_t*)(w + L.select_ws), block_size,
                                          rows, S, s_pad, segment_size, stream))) return rc;
   }
+  const bool is_short = !threshold_is_int_one && short_pass(rows, nb);
   // With a real threshold the permuted K / V are gathered AFTER the selection, and only the blocks some query
   // block visits: the estimate needs no more than the pooled permuted key blocks, which come straight from K.
+  // (Short passes: see short_pass.)
   // (Every candidate selected: everything is visited, one full gather.)
-  uint8_t* needed = threshold_is_int_one ? nullptr : w + L.needed;
+  uint8_t* needed = threshold_is_int_one || is_short ? nullptr : w + L.needed;
   const bool pair_lists = !threshold_is_int_one && nb <= PBS_PAIR_SELECT_MAX_BLOCKS;
   if (threshold_is_int_one) {
     if ((rc = pbs_gather_kv(k, v, (const int32_t*)(w + L.idx), w + L.perm_k, w + L.perm_vt, nullptr, B, Hq, Hkv,
                             S, head_dim, block_size, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, key_pool_max, nullptr, stream))) return rc;
   } else {
-    if ((rc = pbs_pool_blocks(q, k, (const int32_t*)(w + L.idx), w + L.pooled_q, w + L.pooled_k, needed, B, Hq, Hkv, S,
+    if (is_short) {
+      if ((rc = pbs_gather_pool_launch(q, k, v, (const int32_t*)(w + L.idx), w + L.pooled_q, w + L.pooled_k, w + L.perm_k, w + L.perm_vt, B, Hq,
+                                       Hkv, S, head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss,
+                                       query_pool_max, key_pool_max, stream))) return rc;
+    } else if ((rc = pbs_pool_blocks(q, k, (const int32_t*)(w + L.idx), w + L.pooled_q, w + L.pooled_k, needed, B, Hq, Hkv, S,
                               head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, query_pool_max, key_pool_max,
                               stream))) return rc;
     // (the selection into pair lists reads a row's candidate entries only: the others are not written)
@@ -147,8 +161,9 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
                                   segment_size, nullptr, nullptr, (int32_t*)(w + L.cols), (int32_t*)(w + L.cnt), needed,
                                   w + L.select_ws, L.attn_ws - L.select_ws, stream))) return rc;
     }
-    if ((rc = pbs_gather_kv(k, v, (const int32_t*)(w + L.idx), w + L.perm_k, w + L.perm_vt, nullptr, B, Hq, Hkv,
-                            S, head_dim, block_size, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, key_pool_max, needed, stream))) return rc;
+    if (!is_short)
+      if ((rc = pbs_gather_kv(k, v, (const int32_t*)(w + L.idx), w + L.perm_k, w + L.perm_vt, nullptr, B, Hq, Hkv,
+                              S, head_dim, block_size, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, key_pool_max, needed, stream))) return rc;
   }
   // (every candidate selected: the lists follow from the block numbers)
   const int32_t* cols = threshold_is_int_one || pair_lists ? nullptr : (const int32_t*)(w + L.cols);
