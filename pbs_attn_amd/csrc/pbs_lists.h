@@ -36,6 +36,11 @@ constexpr int PBS_PAIR_SELECT_MAX_BLOCKS = 2048;
 int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold_per_row, float threshold, const int32_t* first_blk,
                           int rows, int S, int block_size, int segment_size, uint8_t* block_needed, const PairLists& lists,
                           void* stream);
+// pbs_block_logits_softmax and that selection in one launch, for rows of up to PBS_ESTIMATE_SELECT_MAX_BLOCKS blocks
+constexpr int PBS_ESTIMATE_SELECT_MAX_BLOCKS = 64;
+int pbs_estimate_select_pair_lists(const void* pooled_q, const void* pooled_k, const float* threshold_per_row, float threshold,
+                                   const int32_t* first_blk, int rows, int S, int head_dim, int block_size, int segment_size,
+                                   uint8_t* block_needed, const PairLists& lists, void* stream);
 // pbs_segment_argsort; first_blk, if not null, receives per row the block of `block_size` that holds original key 0 (there has
 // to be a complete segment)
 int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,

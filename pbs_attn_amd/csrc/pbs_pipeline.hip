@@ -15,7 +15,8 @@ __global__ void identity_indices_kernel(int32_t* idx, int S_pad, int64_t total) 
 // after the selection -> this, us: 32 / 8 heads x 512 54.3 -> 51.1, x 1024 68.9 -> 64.4, x 4096 181 -> 175, x 8192 499 -> 488, on
 // concentrated inputs 64.0 -> 59.8, 141 -> 139, 339 -> 333; 28 / 4 x 8192 218 -> 216.5.  Longer rows leave more of the blocks unvisited: 8 / 2
 // heads x 16384, concentrated, 154.9 against 156.7, x 32768 263 against 279.
-constexpr int SHORT_PASS_BLOCKS = 2048, SHORT_PASS_ROW = 64;
+// (The same passes take estimate and selection in one launch: see estimate_select_kernel.)
+constexpr int SHORT_PASS_BLOCKS = 2048, SHORT_PASS_ROW = PBS_ESTIMATE_SELECT_MAX_BLOCKS;
 bool short_pass(int rows, int nb) { return nb <= SHORT_PASS_ROW && rows * nb <= SHORT_PASS_BLOCKS; }
 
 
@@ -145,8 +146,13 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
     } else if ((rc = pbs_pool_blocks(q, k, (const int32_t*)(w + L.idx), w + L.pooled_q, w + L.pooled_k, needed, B, Hq, Hkv, S,
                               head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, query_pool_max, key_pool_max,
                               stream))) return rc;
+    if (is_short) {
+      if ((rc = pbs_estimate_select_pair_lists(w + L.pooled_q, w + L.pooled_k, threshold_per_row, threshold,
+                                               force_select_first_block ? (const int32_t*)(w + L.select_ws) : nullptr, rows, S, head_dim,
+                                               block_size, segment_size, needed,
+                                               pbs_pair_lists(B, Hq, Hkv, S, block_size, segment_size, w + L.attn_ws), stream))) return rc;
     // (the selection into pair lists reads a row's candidate entries only: the others are not written)
-    if (pair_lists) {
+    } else if (pair_lists) {
       if ((rc = pbs_block_logits_softmax_candidates_only(w + L.pooled_q, w + L.pooled_k, (float*)(w + L.probs), rows, nb,
                                                          head_dim, segment_size / block_size, stream))) return rc;
       if ((rc = pbs_select_pair_lists((const float*)(w + L.probs), threshold_per_row, threshold,

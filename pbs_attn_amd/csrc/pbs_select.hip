@@ -12,6 +12,7 @@
 // Rows of up to 1024 blocks (2048 on the single-call path, which writes the attention kernel's merged lists instead of
 // CSR rows) take the wave-level variant further down (one wave per row, the row in registers).
 #include "pbs_lists.h"
+#include "pbs_estimate.h"
 #include "pbs_wave.h"
 #include <utility>
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
@@ -319,20 +320,18 @@ __device__ __forceinline__ void wave_bitonic_sort_u32(uint32_t (&k)[NPL], int la
   }
 }
 
-// One wave decides row (head `row`, query block qb): flag[0 .. nb) (this wave's, in LDS) becomes the selection.
+// One wave decides row (head `row`, query block qb) with the probabilities p[0 .. nb): flag[0 .. nb) (this wave's, in LDS) becomes the selection.
 template <int NPL>
-__device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb, uint8_t* flag) {
+__device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb, const float* p, uint8_t* flag) {
   const int lane = threadIdx.x & 63;
   const int nb = a.nb;
   const int seg_first = (qb / a.bps) * a.bps;
-  const int64_t row_off = ((int64_t)row * nb + qb) * nb;
 
   for (int kb = lane; kb < nb; kb += 64) flag[kb] = 0;
 
   if (a.thr_is_int_one) {
     for (int kb = lane; kb < seg_first; kb += 64) flag[kb] = 1;
   } else {
-    const float* p = a.P + row_off;
     // entries that are zero by construction sort behind every candidate (ties keep index order) and add nothing
     // to the running sum: the row is sorted up to its last candidate only (the launch is sized for that)
     const int count = a.cand_rule == 1 ? seg_first : a.cand_rule == 2 ? min(qb + 1, nb) : nb;
@@ -340,7 +339,7 @@ __device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb,
     // (lane, register) is the order of the indices.  No entry has the key ~0, which stands for "none".
     uint32_t k0v[NPL];
     float raw[NPL];
-    if (NPL >= 4 && (nb & 3) == 0 && ((uintptr_t)a.P & 15) == 0) {
+    if (NPL >= 4 && (nb & 3) == 0 && ((uintptr_t)a.P & 15) == 0) {   // (p is a row of a.P)
       // whole 16-byte pieces: the one that holds the last candidate ends inside the row (nb is a multiple of four)
 #pragma unroll
       for (int r = 0; r < NPL; r += 4) {
@@ -530,7 +529,7 @@ __device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t 
   const int seg_first = (qb / a.bps) * a.bps;
   const int seg_end = min(seg_first + a.bps, nb);
   const int64_t row_off = ((int64_t)row * nb + qb) * nb;
-  decide_row<NPL>(a, row, qb, flag);
+  decide_row<NPL>(a, row, qb, a.P + row_off, flag);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -588,50 +587,20 @@ __global__ __launch_bounds__(256) void select_blocks_groups_kernel(SelectArgs a,
   }
 }
 
-// ---- the single-call path: selection straight into the merged lists that the attention kernel reads (pbs_lists.h).
-// A workgroup decides the rows of two pairs of query blocks, one wave each, into flags in LDS; then the first wave of a
-// pair writes the pair's list and the second one the gather's flags (items of one query block: every wave those of its row).  No CSR rows (4 bytes per visited block and row, written
-// here and read back) and no launch that merges them.  Groups are in pairs here: qb_lo / qb_hi are pair numbers.
-// LONG: rows of 1025 .. 2048 candidates, in a kernel of their own: the register need of 32 entries per lane would cost the shorter
-// rows two thirds of their waves.
-template <bool LONG>
-__global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, PairLists l, SelectGroups gr, int rows) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem_w[];
-  int g = 0;
-  while (g + 1 < gr.n && (int)blockIdx.x >= gr.wg_end[g]) ++g;
-  const int wg0 = g == 0 ? 0 : gr.wg_end[g - 1];
-  const int n_pairs = gr.qb_hi[g] - gr.qb_lo[g], total = rows * n_pairs;
+// Row (`row`, pair) of a workgroup whose waves have decided the rows of two pairs into `flags` (nb rounded up to 16 bytes a wave): the first wave
+// of a pair writes its list, the second one the gather's flags; items of one query block: every wave both.
+__device__ __forceinline__ void write_lists(const SelectArgs& a, const PairLists& l, int row, int pair, const uint8_t* flags) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int unit = ((int)blockIdx.x - wg0) * 2 + (wave >> 1);
-  const bool live = unit < total;
-  const int row = live ? unit / n_pairs : 0, pair = gr.qb_lo[g] + (live ? unit - row * n_pairs : 0);
-  const int nb = a.nb, nb_pad = (nb + 15) & ~15, npair = (nb + 1) >> 1;
-  const int qb0 = 2 * pair, qb = qb0 + (wave & 1);
-  uint8_t* flag = smem_w + wave * nb_pad;
-  if (blockIdx.x == 0 && threadIdx.x < 8) l.queue[threadIdx.x] = l.first_tickets;
-  if (live && qb < nb) {
-    if constexpr (LONG) {
-      decide_row<32>(a, row, qb, flag);
-    } else {
-      switch (gr.npl[g]) {
-        case 1: decide_row<1>(a, row, qb, flag); break;
-        case 2: decide_row<2>(a, row, qb, flag); break;
-        case 4: decide_row<4>(a, row, qb, flag); break;
-        case 8: decide_row<8>(a, row, qb, flag); break;
-        default: decide_row<16>(a, row, qb, flag); break;
-      }
-    }
-  }
-  __syncthreads();
+  const int nb = a.nb, nb_pad = (nb + 15) & ~15, npair = (nb + 1) >> 1, qb0 = 2 * pair, qb = qb0 + (wave & 1);
   const bool pairs = l.span == 2;
-  if (!live || (!pairs && qb >= nb)) return;
+  if (!pairs && qb >= nb) return;
   const int first = pairs ? qb0 : qb;   // of the item
   const bool second = pairs && first + 1 < nb;
   const int qb1 = second ? first + 1 : first;
   const int sf0 = (first / a.bps) * a.bps, sf1 = (qb1 / a.bps) * a.bps;
   const int end1 = second ? sf1 : 0, end = max(sf0, end1);   // a row's flags count up to its own segment
-  const uint32_t* f0 = reinterpret_cast<const uint32_t*>(smem_w + (pairs ? wave & 2 : wave) * nb_pad);
-  const uint32_t* f1 = reinterpret_cast<const uint32_t*>(smem_w + ((wave & 2) + 1) * nb_pad);
+  const uint32_t* f0 = reinterpret_cast<const uint32_t*>(flags + (pairs ? wave & 2 : wave) * nb_pad);
+  const uint32_t* f1 = reinterpret_cast<const uint32_t*>(flags + ((wave & 2) + 1) * nb_pad);
   // the flags of blocks 4 x .. 4 x + 3, a byte each: bit 0 visited by the first query block, bit 1 by the second
   auto visited = [&](int x) __attribute__((always_inline)) {
     auto below = [&](int n) __attribute__((always_inline)) {   // bytes of blocks below n
@@ -684,6 +653,68 @@ __global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, Pa
     header[4] = (uint16_t)first;
     header[5] = (uint16_t)(second ? 2 : 1);
   }
+}
+
+// ---- the single-call path: selection straight into the merged lists that the attention kernel reads (pbs_lists.h).
+// A workgroup decides the rows of two pairs of query blocks, one wave each, into flags in LDS; then the first wave of a
+// pair writes the pair's list and the second one the gather's flags (items of one query block: every wave those of its row).  No CSR rows (4 bytes per visited block and row, written
+// here and read back) and no launch that merges them.  Groups are in pairs here: qb_lo / qb_hi are pair numbers.
+// LONG: rows of 1025 .. 2048 candidates, in a kernel of their own: the register need of 32 entries per lane would cost the shorter
+// rows two thirds of their waves.
+template <bool LONG>
+__global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, PairLists l, SelectGroups gr, int rows) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem_w[];
+  int g = 0;
+  while (g + 1 < gr.n && (int)blockIdx.x >= gr.wg_end[g]) ++g;
+  const int wg0 = g == 0 ? 0 : gr.wg_end[g - 1];
+  const int n_pairs = gr.qb_hi[g] - gr.qb_lo[g], total = rows * n_pairs;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int unit = ((int)blockIdx.x - wg0) * 2 + (wave >> 1);
+  const bool live = unit < total;
+  const int row = live ? unit / n_pairs : 0, pair = gr.qb_lo[g] + (live ? unit - row * n_pairs : 0);
+  const int nb = a.nb, nb_pad = (nb + 15) & ~15, qb = 2 * pair + (wave & 1);
+  uint8_t* flag = smem_w + wave * nb_pad;
+  if (blockIdx.x == 0 && threadIdx.x < 8) l.queue[threadIdx.x] = l.first_tickets;
+  if (live && qb < nb) {
+    const float* p = a.P + ((int64_t)row * nb + qb) * nb;
+    if constexpr (LONG) {
+      decide_row<32>(a, row, qb, p, flag);
+    } else {
+      switch (gr.npl[g]) {
+        case 1: decide_row<1>(a, row, qb, p, flag); break;
+        case 2: decide_row<2>(a, row, qb, p, flag); break;
+        case 4: decide_row<4>(a, row, qb, p, flag); break;
+        case 8: decide_row<8>(a, row, qb, p, flag); break;
+        default: decide_row<16>(a, row, qb, p, flag); break;
+      }
+    }
+  }
+  __syncthreads();
+  if (live) write_lists(a, l, row, pair, smem_w);
+}
+
+// Estimate and selection of four query blocks in one launch, for rows of up to 64 blocks: the workgroup forms the probabilities of
+// the 32 query blocks its own are among (the products are next to nothing) and keeps its own rows in LDS.  A launch and its
+// way to memory and back less: 32 / 8 heads x 512 51.8 -> 48.6 us a pass, 28 / 4 x 1000 63.1 -> 59.4, 32 / 8 x 4096 174.0 -> 169.9, x
+// 8192 482 -> 477.  Above 2048 blocks the repeated products outweigh it: 128 heads x 6144 1159 against 1162, 32 / 8 x
+// 12288 (two entries a lane) 962 against 970.
+__global__ __launch_bounds__(256) void estimate_select_kernel(const uint16_t* pooled_q, const uint16_t* pooled_k, SelectArgs a, PairLists l, Divisor sqrt_d) {
+  __shared__ EstimateStats st;
+  __shared__ float probs[4][PBS_ESTIMATE_SELECT_MAX_BLOCKS];
+  __shared__ __attribute__((aligned(16))) uint8_t flags[4 * PBS_ESTIMATE_SELECT_MAX_BLOCKS];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int four = (int)gridDim.x - 1 - (int)blockIdx.x, row = blockIdx.y;   // the rows with the most candidates start first
+  const int nb = a.nb, nb_pad = (nb + 15) & ~15, qb = 4 * four + wave;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 8) l.queue[threadIdx.x] = l.first_tickets;
+  const int64_t head = (int64_t)row * nb * ESTIMATE_D;
+  estimate_tile<false, true>(pooled_q + head, pooled_k + head, nb, a.bps, sqrt_d, four / 8, st, [&](int ql, int kb, float p) __attribute__((always_inline)) {
+    if (ql >> 2 == (four & 7)) probs[ql & 3][kb] = p;
+  });
+  __syncthreads();
+  if (qb < nb) decide_row<1>(a, row, qb, probs[wave], flags + wave * nb_pad);
+  __syncthreads();
+  const int pair = 2 * four + (wave >> 1);
+  if (2 * pair < nb) write_lists(a, l, row, pair, flags);
 }
 
 // Visit lists from a given block mask: one wave per (row, query block), the set bits of strictly earlier segments
@@ -819,6 +850,7 @@ int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold
                           void* stream) {
   const int nb = (S + block_size - 1) / block_size, npair = (nb + 1) / 2;
   PBS_REQUIRE(rows > 0 && rows <= 65535 && nb <= PBS_PAIR_SELECT_MAX_BLOCKS, "pbs_select_pair_lists: bad shape");
+  PBS_REQUIRE(block_attn_scores, "pbs_select_pair_lists: null score pointer");
   SelectArgs a = {};
   a.P = block_attn_scores; a.thr_rows = threshold_per_row; a.thr = threshold;
   a.force_first = first_blk != nullptr;
@@ -857,4 +889,24 @@ int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold
   if (wgs)
     hipLaunchKernelGGL(select_pair_lists_kernel<false>, dim3((unsigned)wgs), dim3(256), lds, (hipStream_t)stream, a, lists, gr, rows);
   return pbs_check_launch("pbs_select_pair_lists");
+}
+
+int pbs_estimate_select_pair_lists(const void* pooled_q, const void* pooled_k, const float* threshold_per_row, float threshold,
+                                   const int32_t* first_blk, int rows, int S, int head_dim, int block_size, int segment_size,
+                                   uint8_t* block_needed, const PairLists& lists, void* stream) {
+  const int nb = (S + block_size - 1) / block_size;
+  PBS_REQUIRE(pooled_q && pooled_k && head_dim == ESTIMATE_D, "pbs_estimate_select: bad pooled tensors");
+  PBS_REQUIRE(rows > 0 && rows <= 65535 && nb <= PBS_ESTIMATE_SELECT_MAX_BLOCKS, "pbs_estimate_select: bad shape");
+  SelectArgs a = {};
+  a.thr_rows = threshold_per_row; a.thr = threshold;
+  a.force_first = first_blk != nullptr;
+  a.first_blk = const_cast<int32_t*>(first_blk);
+  a.nb = nb; a.bs = block_size; a.bps = segment_size / block_size; a.S = S;
+  a.needed = block_needed;
+  a.cand_rule = 1;
+  const dim3 grid((unsigned)((nb + 3) / 4), (unsigned)rows);
+  const Divisor sqrt_d = pbs_sqrt_divisor(head_dim);
+  hipLaunchKernelGGL(estimate_select_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)pooled_q, (const uint16_t*)pooled_k, a,
+                     lists, sqrt_d);
+  return pbs_check_launch("pbs_estimate_select");
 }
