@@ -50,6 +50,7 @@
 //   An item's tiles come in the order permuted tiles, own-segment tiles before the diagonal, diagonal tile, and
 //   each kind has a loop of its own (see the loops).
 #include "pbs_attn_tile.h"
+#include "pbs_wave.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 #include <atomic>
 #include <type_traits>
@@ -70,8 +71,8 @@ struct AttnArgs {
   int span, n_items;  // query blocks of an item (two, or one: see item_span), items of a head
   uint32_t k_ss, v_ss;   // key / value row strides in elements (< 2^22)
   int xcd_start[9];   // work items (head-major, long rows first) of XCD x: [xcd_start[x], xcd_start[x + 1])
-  int deal_heads;     // 0, or the heads over which the tickets of a small launch are dealt, longest items first (see ticket_item)
-  uint32_t deal_magic;   // quotients by deal_heads: high word of a product
+  int deal;           // how tickets become items (see ticket_item)
+  uint32_t deal_magic;   // quotients by DEAL_HEADS * n_items or by BH: high word of a product
   int64_t q_sb, q_sh, q_ss, k_sb, k_sh, v_sb, v_sh, o_sb, o_sh, o_ss;
   float scale_log2;
 };
@@ -185,22 +186,51 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
 }
 
 // Ticket `ticket` (counted from the range's first) of XCD range x, [begin, end) -> work item, or NO_ITEM past the range's end.  Items
-// are numbered head by head, long ones first, and normally handed out in that order (an XCD walks one head at a time: its
+// are numbered head by head, long ones first, and in a large launch handed out in that order (an XCD walks one head at a time: its
 // workgroups share that head's K / V stream in L2).  A launch with only a few items per workgroup cannot balance that way: a
 // workgroup that starts with a short item of one head is handed a long item of the next and finishes last.  There the
-// same item of every head goes out before the next shorter one, longest first: the heads of the range, where
-// every range is of whole heads, or all heads, dealt to the XCDs in turn.  Whole pass, head by head -> dealt: 28 / 4 heads x 4096
-// 199 -> 164 us, x 5120 250 -> 222, x 10240 675 -> 641; 32 / 8 x 4352 219 -> 200, x 5120 260 -> 248, x 10240 731 -> 711.  (Wave-uniform
-// values: scalar arithmetic only.)
-constexpr int NO_ITEM = 1 << 28;
-__device__ __forceinline__ int ticket_item(ArgsPtr a, int x, int begin, int end, int ticket) {
+// same item of several heads goes out before the next shorter one.  DEAL_GROUPS (every range is of whole heads): DEAL_HEADS heads
+// of the range at a time, since an XCD's L2 holds the tiles of a few (4 x 28 / 4 heads x 2513, over the range's fourteen: 285 -> 291 us).
+// DEAL_ALL: all heads, dealt to the XCDs in turn.  Whole pass, head by head -> dealt: 28 / 4 heads x 4096
+// 199 -> 164 us, x 5120 250 -> 222, x 10240 675 -> 641; 32 / 8 x 4352 219 -> 200, x 5120 260 -> 248, x 10240 731 -> 711.
+// DEAL_BY_LISTS: DEAL_GROUPS where the visit lists are short, else DEAL_NONE (see lists_are_short).
+// (Wave-uniform values: scalar arithmetic only.)
+constexpr int NO_ITEM = 1 << 28, DEAL_NONE = 0, DEAL_GROUPS = 1, DEAL_ALL = 2, DEAL_BY_LISTS = 3, DEAL_HEADS = 4;
+__device__ __forceinline__ int quotient(uint32_t r, uint32_t magic) { return (int)(((uint64_t)r * magic) >> 32); }
+__device__ __forceinline__ int ticket_item(ArgsPtr a, int deal, int x, int begin, int end, int ticket) {
   if (begin + ticket >= end) return NO_ITEM;
-  const int m = a->deal_heads;
-  if (m == 0) return begin + ticket;
-  const bool all = m == a->BH;
-  const uint32_t r = (uint32_t)(all ? 8 * ticket + x : ticket);
-  const int len = m == 1 ? (int)r : (int)(((uint64_t)r * a->deal_magic) >> 32);
-  return (all ? 0 : begin) + ((int)r - len * m) * a->n_items + len;
+  const int n = a->n_items;
+  if (deal == DEAL_NONE) return begin + ticket;
+  if (deal == DEAL_ALL) {
+    const int r = 8 * ticket + x, len = a->BH == 1 ? r : quotient((uint32_t)r, a->deal_magic);
+    return (r - len * a->BH) * n + len;
+  }
+  const int group = quotient((uint32_t)ticket, a->deal_magic) * (DEAL_HEADS * n), r = ticket - group;
+  const int left = end - begin - group;   // items of this group of heads and those after it
+  const int len = left >= 4 * n ? r >> 2 : left >= 3 * n ? quotient((uint32_t)r, 0x55555556u) : left >= 2 * n ? r >> 1 : r;
+  const int heads = left >= 4 * n ? 4 : left >= 3 * n ? 3 : left >= 2 * n ? 2 : 1;
+  return begin + group + (r - len * heads) * n + len;
+}
+
+// Whether an item visits few tiles, from 64 lists across the launch: every workgroup reads the same ones.  Such a launch gains by
+// the dealt order at any length: 2 x 32 / 8 heads x 13333 concentrated 947 -> 877 us a pass, 32 / 8 x 30000 1449 -> 1416, x 131072 2780 ->
+// 2690.  Where lists are long it loses what an XCD's workgroups share of a head in L2: 32 / 8 x 64000 with 100 tiles an item
+// 9.75 -> 10.11 ms, near-uniform 2 x 32 / 8 x 13333 (0.8 of an item's causal tiles and more) 2276 -> 2312 us.  (A round trip to memory
+// at the kernel's start, 2 us.)
+constexpr int SHORT_LIST = 40;
+__device__ __forceinline__ bool lists_are_short(ArgsPtr a) {
+  const int n = a->n_items, lane = lane_id_here();
+  // one of every 64th part of the items, at another place in each: lists grow shorter towards a head's end (65 * 63 < 4096: never past the last)
+  const int64_t item = ((int64_t)a->BH * n * (65 * lane)) >> 12;
+  uint32_t tiles = a->plist[item * a->cap];
+  auto add = [&](auto t) __attribute__((always_inline)) { return t.a + t.b; };
+  tiles = add(with_lane_xor<1>(tiles));
+  tiles = add(with_lane_xor<2>(tiles));
+  tiles = add(with_lane_xor<4>(tiles));
+  tiles = add(with_lane_xor<8>(tiles));
+  tiles = add(with_lane_xor<16>(tiles));
+  tiles = add(with_lane_xor<32>(tiles));
+  return __builtin_amdgcn_readfirstlane((int)tiles) <= min(46 * n, 64 * SHORT_LIST);   // (64 times 0.72)
 }
 
 // asynchronous copy of one list row (`chunks` 16-byte pieces) into LDS at byte offset `lds_byte`
@@ -236,6 +266,8 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
 #define PBS_ARGS() ({ ArgsPtr p_ = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(); asm volatile("" : "+s"(p_)); p_; })
   ArgsPtr a0 = PBS_ARGS();
   const int n_items = a0->n_items;
+  int deal = a0->deal;
+  if (deal == DEAL_BY_LISTS) deal = lists_are_short(a0) ? DEAL_GROUPS : DEAL_NONE;
   const int xcd = blockIdx.x & 7;
   int q_begin = a0->xcd_start[xcd], q_end = a0->xcd_start[xcd + 1];   // the range being served: this XCD's, later others'
   int vic = xcd, vic_tried = a0->cap ? 0 : 7;   // (no counters: every item is some workgroup's first)
@@ -267,7 +299,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       __syncthreads();   // everyone has read the previous ticket
       if (wave == 0 && lane_id_here() == 0) misc[4] = atomicAdd(as->queue + vic, 1);
       __syncthreads();
-      found = ticket_item(as, vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
+      found = ticket_item(as, deal, vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
       if (found < NO_ITEM) return true;
     }
     return false;
@@ -275,7 +307,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   // The first item: workgroup n of an XCD takes ticket n, without asking (the counters start behind these tickets); where the
   // range is shorter than that, an item of another one.
   if (threadIdx.x == 0) misc[1] = 0;
-  int cur = ticket_item(a0, xcd, q_begin, q_end, (int)blockIdx.x >> 3);
+  int cur = ticket_item(a0, deal, xcd, q_begin, q_end, (int)blockIdx.x >> 3);
   if (PBS_UNLIKELY(cur == NO_ITEM)) {
     if (!claim_elsewhere()) return;
     cur = found;
@@ -432,7 +464,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       if (wave == 0 && lane_id_here() == 0) misc[4] = claim;
     };
     auto adopt_next = [&]() __attribute__((always_inline)) {          // ... and after the barrier
-      nxt = ticket_item(PBS_ARGS(), vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
+      nxt = ticket_item(PBS_ARGS(), deal, vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
       has_nxt = nxt < NO_ITEM;
       if (has_nxt)
         stage_list_async(list_row(PBS_ARGS(), nxt), PBS_ARGS()->cap >> 3, LDS_LIST + (li ^ 1u) * LIST_BYTES, wave, wave * 64 + lane_id_here());
@@ -895,14 +927,22 @@ static int list_cap(int nb, int bps) { return (LIST_HEADER + nb + std::min(bps, 
 // 2048 99.6 -> 97.5, concentrated 86.4 -> 88.9).  With 560 blocks and more pairs are better everywhere (32 / 8 x 2560 116 -> 128).
 constexpr int SINGLE_BLOCK_ITEMS = 384;
 constexpr int SINGLE_FEW_HEADS = 512;
-constexpr int DEAL_ITEMS = 2048;
-static int item_span(int rows, int nb) { return (int64_t)rows * nb <= (rows <= 16 ? SINGLE_FEW_HEADS : SINGLE_BLOCK_ITEMS) ? 1 : 2; }
+constexpr int DEAL_ROW = 44;
+constexpr int DEAL_ITEMS = 1400;
+// A sequence inside one segment with more single blocks than workgroups would need the list kernel besides (see pbs_sparse_attn_launch): only from
+// ONE_SEGMENT_ROW blocks a row on (128 heads x 295 tokens 29 against 40 us, 32 heads x 1536 38.9 against 37.0).
+constexpr int ONE_SEGMENT_ROW = 12, ITEMS_WITHOUT_LISTS = 256;
+static int item_span(int rows, int nb, int bps) {
+  const int64_t blocks = (int64_t)rows * nb;
+  if (blocks > (rows <= 16 ? SINGLE_FEW_HEADS : SINGLE_BLOCK_ITEMS)) return 2;
+  return bps < nb || blocks <= ITEMS_WITHOUT_LISTS || nb >= ONE_SEGMENT_ROW ? 1 : 2;
+}
 static int items_of(int nb, int span) { return (nb + span - 1) / span; }
 
 // workspace: 256 bytes of work counters, then one merged visit list per item
 
 extern "C" size_t pbs_sparse_attn_workspace_bytes(int B, int Hq, int S, int segment_size) {
-  const int64_t nb = (S + BS - 1) / BS, n_items = items_of((int)nb, item_span(B * Hq, (int)nb)), cap = list_cap((int)nb, segment_size / BS);
+  const int64_t nb = (S + BS - 1) / BS, n_items = items_of((int)nb, item_span(B * Hq, (int)nb, segment_size / BS)), cap = list_cap((int)nb, segment_size / BS);
   return 256 + (size_t)B * Hq * n_items * cap * 2;
 }
 
@@ -934,7 +974,7 @@ extern "C" int pbs_sparse_attn_fwd_optional_diagonal(const void* q, const void* 
 // the eight ranges of work items (AttnArgs::xcd_start) and the ticket order; returns the items of the longest range
 static int plan_ranges(AttnArgs& a) {
   // eight ranges of equal estimated work: item p of a head costs about p + 1 (causal length)
-  a.span = item_span(a.BH, a.nb);
+  a.span = item_span(a.BH, a.nb, a.bps);
   a.n_items = items_of(a.nb, a.span);
   const int64_t n = a.n_items;
   const double head_work = 0.5 * (double)n * (double)(n + 1);
@@ -956,16 +996,16 @@ static int plan_ranges(AttnArgs& a) {
     a.xcd_start[x] = (int)start;
     if (x > 0) max_items = std::max(max_items, a.xcd_start[x] - a.xcd_start[x - 1]);
   }
-  // at most eight items per workgroup: longest items first (see ticket_item).  With sixteen the head-by-head order balances well enough, and
-  // where attention is near-uniform it is faster by what an XCD's workgroups share of a head in L2: 32 / 8 x 32768 5.78 against
-  // 6.00 ms.  (Concentrated inputs would gain 1 % there and 7 % at 2 x 28 / 4 heads x 13333.)
-  a.deal_heads = 0;
-  a.deal_magic = 0;
+  // Few items a head: longest first (see ticket_item).  With more of them the head-by-head order balances well enough,
+  // and where attention is near-uniform it is faster by what an XCD's workgroups share of a head in L2: 32 / 8 heads x 16384 1616 against
+  // 1644 us, x 32768 5.78 against 6.00 ms; 16 / 16 x 22016 1427 against 1435.
   const int64_t total = (int64_t)a.BH * n;
-  if (total <= DEAL_ITEMS) {
-    const bool whole_heads = a.BH % 8 == 0;
-    a.deal_heads = whole_heads ? a.BH / 8 : a.BH;
-    a.deal_magic = (uint32_t)((1ull << 32) / a.deal_heads + 1);   // exact for numbers and divisors up to DEAL_ITEMS, 1 apart
+  const bool whole_heads = a.BH % 8 == 0;
+  a.deal = whole_heads ? (a.BH == 8 ? DEAL_NONE : n <= DEAL_ROW ? DEAL_GROUPS : DEAL_BY_LISTS) : total <= DEAL_ITEMS ? DEAL_ALL : DEAL_NONE;
+  const int64_t by = whole_heads ? DEAL_HEADS * n : a.BH;
+  a.deal_magic = (uint32_t)((1ull << 32) / by + 1);   // (by > 1, or not used) quotients are exact below 2^32 / by
+  if (total / 8 >= (1ll << 32) / by) a.deal = DEAL_NONE;
+  if (a.deal != DEAL_NONE) {
     max_items = 0;
     for (int x = 0; x <= 8; ++x) {
       a.xcd_start[x] = whole_heads ? (int)(x * total / 8) : (int)(x * (total / 8) + std::min<int64_t>(x, total % 8));   // (items 8 t + x < total)
@@ -992,6 +1032,7 @@ PairLists pbs_pair_lists(int B, int Hq, int Hkv, int S, int block_size, int segm
   AttnArgs a;
   a.BH = B * Hq;
   a.nb = (S + block_size - 1) / block_size;
+  a.bps = segment_size / block_size;
   PairLists l;
   l.plist = (uint16_t*)((char*)workspace + 256);
   l.queue = (int*)workspace;
@@ -1054,7 +1095,10 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
   // A sequence inside one segment with an item or less per workgroup: the attention kernel forms the lists itself (77 tokens, 32 / 8
   // heads: 19.9 -> 17.1 us, one launch instead of two; the host needs about 17).
   const bool own_lists = !lists_built && !csr_cols && !own_block_needed && a.bps >= a.nb && max_items <= n_wg / 8;
-  if (own_lists) a.cap = 0;
+  if (own_lists) {
+    a.cap = 0;
+    if (a.deal == DEAL_BY_LISTS) a.deal = DEAL_NONE;
+  }
   else if (!lists_built)
     hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * a.n_items)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
                      (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.span, a.bps, a.cap, Hq, Hq / Hkv, (int)(n_wg / 8), own_block_needed);

@@ -17,8 +17,11 @@ pytestmark = pytest.mark.gpu
     (28, 4, 13 * 128 + 77, 128, 0.5, 3, "local_window", "mean"),  # 392 in pairs, dealt over all heads; 84 heads
     (7, 7, 9 * 128, 128, 0.0, 9, "uniform_heavy", "mean"),      # rows without selected blocks, items of one tile
     (1, 1, 300 * 128, 1024, 0.9, 5, "strong_heavy", "mean"),    # one head: 300 single blocks; 750 pairs of five
-    (8, 2, 512 * 128, 1024, 0.9, 2, "strong_heavy", "mean"),    # 2048 items, dealt; 4096, head by head
-    (5, 5, 818 * 128, 1024, 0.9, 2, "strong_uniform", "mean"),  # 2045 items dealt over all heads; 4090 head by head
+    (8, 2, 350 * 128, 1024, 0.9, 2, "strong_heavy", "mean"),    # 1400 items, dealt; 2800, head by head
+    (8, 8, 89 * 128, 128, 0.9, 3, "uniform_heavy", "mean"),     # 45 items a head: one head a range; three, the long lists head by head
+    (16, 16, 89 * 128, 512, 0.9, 2, "strong_heavy", "mean"),    # the same length, short lists: dealt
+    (8, 4, 87 * 128, 256, 0.9, 7, "local_window", "mean"),      # 44 items a head, seven heads a range: a group of four and one of three
+    (5, 5, 559 * 128, 1024, 0.9, 2, "strong_uniform", "mean"),  # 1400 items dealt over all heads; 2800 head by head
 ])
 def test_the_same_heads_in_launches_of_other_sizes(dev, Hq, Hkv, S, seg, thr, reps, kind, pool):
     q, k, v = (x.to(dev) for x in small_case(1, Hq, Hkv, S, kind=kind, seed=S + Hq))
@@ -33,7 +36,7 @@ def test_the_same_heads_in_launches_of_other_sizes(dev, Hq, Hkv, S, seg, thr, re
         assert torch.equal(alone[:, :g], one)
 
 
-@pytest.mark.parametrize("Hq,Hkv,S,reps", [(32, 8, 77, 1), (16, 4, 2048, 3), (3, 1, 128, 40), (1, 1, 511 * 128, 2), (28, 4, 1500, 2), (9, 3, 40 * 128 - 1, 2)])
+@pytest.mark.parametrize("Hq,Hkv,S,reps", [(32, 8, 77, 1), (16, 4, 2048, 3), (32, 8, 295, 4), (32, 8, 1536, 2), (3, 1, 128, 40), (1, 1, 511 * 128, 2), (28, 4, 1500, 2), (9, 3, 40 * 128 - 1, 2)])
 def test_one_segment_in_launches_of_other_sizes(dev, Hq, Hkv, S, reps):
     q, k, v = (x.to(dev) for x in small_case(1, Hq, Hkv, S, seed=S))
     run = lambda a, b, c: P.permuted_block_sparse_attn_fwd(a, b, c, 128, 65536, 0.9, True)
