@@ -203,6 +203,15 @@ int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v, void* out,
                          int key_pool_max, float softmax_scale, void* workspace, size_t workspace_bytes,
                          void* stream);
 
+/* The same for a short sequence inside one segment (S <= segment_size: plain causal attention, whatever the threshold): one
+ * launch, no workspace.  PBS_NOT_ONE_LAUNCH, and nothing enqueued, where the sequence is longer or the heads are too
+ * many: pbs_prefill_attn_fwd takes those (and these, with the same bits). */
+#define PBS_NOT_ONE_LAUNCH (-3)
+int pbs_one_segment_attn_fwd(const void* q, const void* k, const void* v, void* out, int B, int Hq, int Hkv, int S,
+                             int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                             int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
+                             int64_t o_sb, int64_t o_sh, int64_t o_ss, float softmax_scale, void* stream);
+
 /* Rotary position embedding of Q and K in one pass: out = bf16(bf16(x * cos) + bf16(rotate_half(x) * sin)),
  * bit-identical to the bf16 tensor expression of pbs_attn/patch/huggingface.py:14-25 (called at :203).
  * q (B, Hq, S, 128) and k (B, Hkv, S, 128) with their strides (e.g. the (B, S, H, D) memory of the

@@ -1028,6 +1028,16 @@ static int64_t workgroups(int max_items) {
   return std::min<int64_t>((int64_t)8 * max_items, (int64_t)(n_cu + 7) / 8 * 8);
 }
 
+bool pbs_sparse_attn_forms_lists(int B, int Hq, int S, int block_size) {
+  AttnArgs a;
+  a.BH = B * Hq;
+  a.nb = (S + block_size - 1) / block_size;
+  a.bps = a.nb;
+  if ((int64_t)a.BH * a.nb > 4 * 256) return false;   // (two blocks an item, 256 workgroups or fewer)
+  const int max_items = plan_ranges(a);
+  return max_items <= workgroups(max_items) / 8;
+}
+
 PairLists pbs_pair_lists(int B, int Hq, int Hkv, int S, int block_size, int segment_size, void* workspace) {
   AttnArgs a;
   a.BH = B * Hq;
@@ -1051,7 +1061,7 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
                               int64_t o_sh, int64_t o_ss, float softmax_scale, const uint8_t* own_block_needed, void* workspace,
                               void* stream) {
   PBS_REQUIRE(q && perm_k && perm_vt && k && v && out, "pbs_sparse_attn_fwd: null tensor pointer");
-  PBS_REQUIRE(workspace && ((uintptr_t)workspace % 256) == 0, "pbs_sparse_attn_fwd: workspace must be a 256-byte aligned device buffer of pbs_sparse_attn_workspace_bytes()");
+  PBS_REQUIRE(((uintptr_t)workspace % 256) == 0, "pbs_sparse_attn_fwd: workspace must be a 256-byte aligned device buffer of pbs_sparse_attn_workspace_bytes()");
   PBS_REQUIRE(head_dim == D && block_size == BS, "pbs_sparse_attn_fwd: head_dim and block_size must be 128 (got %d, %d)", head_dim, block_size);
   PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0, "pbs_sparse_attn_fwd: bad shape");
   PBS_REQUIRE(segment_size > 0 && segment_size % block_size == 0, "pbs_sparse_attn_fwd: segment_size must be a multiple of block_size");
@@ -1079,6 +1089,10 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
   a.queue = (int*)workspace;
   a.plist = (const uint16_t*)((char*)workspace + 256);
   const int64_t n_wg = workgroups(max_items);
+  // A sequence inside one segment with an item or less per workgroup: the attention kernel forms the lists itself (77 tokens, 32 / 8
+  // heads: 19.9 -> 17.1 us, one launch instead of two; the host needs about 17) and needs no workspace.
+  const bool own_lists = !lists_built && !csr_cols && !own_block_needed && a.bps >= a.nb && max_items <= n_wg / 8;
+  PBS_REQUIRE(workspace || own_lists, "pbs_sparse_attn_fwd: workspace must be a 256-byte aligned device buffer of pbs_sparse_attn_workspace_bytes()");
   int dev = 0;
   hipError_t attr = hipGetDevice(&dev);
   const bool tracked = attr == hipSuccess && dev >= 0 && dev < 64;
@@ -1092,9 +1106,6 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
     pbs_set_error("pbs_sparse_attn_fwd: cannot reserve %u bytes of LDS: %s", LDS_TOTAL, hipGetErrorString(attr));
     return (int)attr;
   }
-  // A sequence inside one segment with an item or less per workgroup: the attention kernel forms the lists itself (77 tokens, 32 / 8
-  // heads: 19.9 -> 17.1 us, one launch instead of two; the host needs about 17).
-  const bool own_lists = !lists_built && !csr_cols && !own_block_needed && a.bps >= a.nb && max_items <= n_wg / 8;
   if (own_lists) {
     a.cap = 0;
     if (a.deal == DEAL_BY_LISTS) a.deal = DEAL_NONE;

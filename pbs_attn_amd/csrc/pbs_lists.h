@@ -19,6 +19,9 @@ struct PairLists {
 // of the lists that pbs_sparse_attn_launch expects in `workspace` with lists_built set
 PairLists pbs_pair_lists(int B, int Hq, int Hkv, int S, int block_size, int segment_size, void* workspace);
 
+// Whether the launch below forms the lists of a sequence inside one segment by itself, and then needs no workspace
+bool pbs_sparse_attn_forms_lists(int B, int Hq, int S, int block_size);
+
 // pbs_sparse_attn_fwd (and its optional-diagonal form, with own_block_needed) after their null checks.  lists_built: the
 // visit lists and counters are in the workspace already.  Otherwise they are merged from the CSR rows or, with csr_cols
 // null (csr_cnt is not read), hold every block of every earlier segment.

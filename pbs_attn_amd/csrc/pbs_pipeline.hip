@@ -78,6 +78,22 @@ extern "C" size_t pbs_prefill_attn_workspace_bytes(int B, int Hq, int Hkv, int S
   return make_layout(B, Hq, Hkv, S, head_dim, block_size, segment_size).total;
 }
 
+extern "C" int pbs_one_segment_attn_fwd(const void* q, const void* k, const void* v, void* out, int B, int Hq, int Hkv, int S,
+                                        int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
+                                        int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
+                                        int64_t o_sb, int64_t o_sh, int64_t o_ss, float softmax_scale, void* stream) {
+  PBS_REQUIRE(q && k && v && out, "pbs_one_segment_attn_fwd: null tensor pointer");
+  PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0, "pbs_one_segment_attn_fwd: bad shape");
+  PBS_REQUIRE(block_size > 0 && segment_size > 0 && segment_size % block_size == 0,
+              "pbs_one_segment_attn_fwd: segment_size must be a multiple of block_size");
+  if (S > segment_size || (S + block_size - 1) / block_size > 511 || !pbs_sparse_attn_forms_lists(B, Hq, S, block_size))
+    return PBS_NOT_ONE_LAUNCH;
+  // (permuted tiles: none is listed, any aligned address will do)
+  return pbs_sparse_attn_launch(q, q, q, k, v, nullptr, nullptr, false, out, B, Hq, Hkv, S, head_dim, block_size,
+                                one_segment_size(S, block_size), q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss,
+                                softmax_scale, nullptr, nullptr, stream);
+}
+
 extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v, void* out, int B, int Hq, int Hkv, int S,
                                     int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh,
                                     int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh,

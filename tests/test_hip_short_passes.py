@@ -33,3 +33,31 @@ def test_short_pass_of_projection_shaped_tensors(dev):
     qt = q.transpose(1, 2).contiguous().transpose(1, 2)
     got = P.permuted_block_sparse_attn_fwd(qt, kv[..., 8:136].transpose(1, 2), kv[..., 264:392].transpose(1, 2), 128, 256, 0.9, True)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,seg,one_launch", [
+    (1, 32, 8, 77, 256, True), (1, 2, 1, 1, 128, True), (4, 64, 8, 128, 128, True), (1, 257, 257, 100, 256, False),
+    (2, 128, 8, 256, 256, True), (2, 129, 3, 256, 256, False), (1, 1, 1, 511 * 128, 65536, False), (1, 4, 4, 300, 256, False),
+])
+def test_one_launch_entry_point(dev, B, Hq, Hkv, S, seg, one_launch):
+    """pbs_one_segment_attn_fwd against pbs_prefill_attn_fwd on the same tensors, and where it hands the call back, without a trace in the output."""
+    from pbs_attn_amd import _lib
+    lib = _lib.load()
+    q, k, v = (x.to(dev) for x in small_case(B, Hq, Hkv, S, seed=S))
+    out = torch.full_like(q, 7.0)
+    common = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Hq, Hkv, S, 128, 128, seg, *q.stride()[:3], *k.stride()[:3],
+              *v.stride()[:3], *out.stride()[:3])
+    st = torch.cuda.current_stream().cuda_stream
+    rc = lib.pbs_one_segment_attn_fwd(*common, 128 ** -0.5, st)
+    got = out.clone()
+    if not one_launch:
+        assert rc == _lib.NOT_ONE_LAUNCH and torch.equal(got, torch.full_like(q, 7.0))
+        return
+    assert rc == 0
+    n = lib.pbs_prefill_attn_workspace_bytes(B, Hq, Hkv, S, 128, 128, seg)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    assert lib.pbs_prefill_attn_fwd(*common, 0.9, None, 0, 1, 0, 0, 128 ** -0.5, ws.data_ptr(), n, st) == 0
+    assert torch.equal(got, out)
+    assert lib.pbs_prefill_attn_fwd(*common, 0.9, None, 0, 1, 0, 0, 128 ** -0.5, None, 0, st) == -1   # refused as before
+    assert lib.pbs_one_segment_attn_fwd(*common[:8], 64, *common[9:], 128 ** -0.5, st) == -1
+    assert lib.pbs_one_segment_attn_fwd(*common[:10], 200, *common[11:], 128 ** -0.5, st) == -1
