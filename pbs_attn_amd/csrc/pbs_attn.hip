@@ -72,7 +72,8 @@ struct AttnArgs {
   uint32_t k_ss, v_ss;   // key / value row strides in elements (< 2^22)
   int xcd_start[9];   // work items (head-major, long rows first) of XCD x: [xcd_start[x], xcd_start[x + 1])
   int deal;           // how tickets become items (see ticket_item)
-  uint32_t deal_magic;   // quotients by DEAL_HEADS * n_items or by BH: high word of a product
+  int deal_heads;     // heads dealt together
+  uint32_t group_magic, heads_magic;   // quotients by deal_heads * n_items and by deal_heads: high word of a product
   int64_t q_sb, q_sh, q_ss, k_sb, k_sh, v_sb, v_sh, o_sb, o_sh, o_ss;
   float scale_log2;
 };
@@ -190,25 +191,31 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
 // workgroups share that head's K / V stream in L2).  A launch with only a few items per workgroup cannot balance that way: a
 // workgroup that starts with a short item of one head is handed a long item of the next and finishes last.  There the
 // same item of several heads goes out before the next shorter one.  DEAL_GROUPS (every range is of whole heads): DEAL_HEADS heads
-// of the range at a time, since an XCD's L2 holds the tiles of a few (4 x 28 / 4 heads x 2513, over the range's fourteen: 285 -> 291 us).
+// of the range at a time, since an XCD's L2 holds the tiles of a few (4 x 28 / 4 heads x 2513, over the range's fourteen: 285 -> 291 us);
+// at two items a workgroup and fewer, all of the range's (4 x 32 / 8 heads x 1021 in one segment 49 us, four at a time 55).
 // DEAL_ALL: all heads, dealt to the XCDs in turn.  Whole pass, head by head -> dealt: 28 / 4 heads x 4096
 // 199 -> 164 us, x 5120 250 -> 222, x 10240 675 -> 641; 32 / 8 x 4352 219 -> 200, x 5120 260 -> 248, x 10240 731 -> 711.
 // DEAL_BY_LISTS: DEAL_GROUPS where the visit lists are short, else DEAL_NONE (see lists_are_short).
 // (Wave-uniform values: scalar arithmetic only.)
 constexpr int NO_ITEM = 1 << 28, DEAL_NONE = 0, DEAL_GROUPS = 1, DEAL_ALL = 2, DEAL_BY_LISTS = 3, DEAL_HEADS = 4;
-__device__ __forceinline__ int quotient(uint32_t r, uint32_t magic) { return (int)(((uint64_t)r * magic) >> 32); }
+__device__ __forceinline__ int quotient(int r, int divisor, uint32_t magic) { return divisor == 1 ? r : (int)(((uint64_t)(uint32_t)r * magic) >> 32); }
 __device__ __forceinline__ int ticket_item(ArgsPtr a, int deal, int x, int begin, int end, int ticket) {
   if (begin + ticket >= end) return NO_ITEM;
-  const int n = a->n_items;
   if (deal == DEAL_NONE) return begin + ticket;
+  const int n = a->n_items, m = a->deal_heads;
   if (deal == DEAL_ALL) {
-    const int r = 8 * ticket + x, len = a->BH == 1 ? r : quotient((uint32_t)r, a->deal_magic);
-    return (r - len * a->BH) * n + len;
+    const int r = 8 * ticket + x, len = quotient(r, m, a->heads_magic);
+    return (r - len * m) * n + len;
   }
-  const int group = quotient((uint32_t)ticket, a->deal_magic) * (DEAL_HEADS * n), r = ticket - group;
+  const int group = quotient(ticket, m * n, a->group_magic) * (m * n), r = ticket - group;
   const int left = end - begin - group;   // items of this group of heads and those after it
-  const int len = left >= 4 * n ? r >> 2 : left >= 3 * n ? quotient((uint32_t)r, 0x55555556u) : left >= 2 * n ? r >> 1 : r;
-  const int heads = left >= 4 * n ? 4 : left >= 3 * n ? 3 : left >= 2 * n ? 2 : 1;
+  int heads = m, len;
+  if (left >= m * n) {
+    len = quotient(r, m, a->heads_magic);
+  } else {   // the last DEAL_HEADS - 1 heads of a range and fewer
+    heads = left >= 3 * n ? 3 : left >= 2 * n ? 2 : 1;
+    len = heads == 3 ? quotient(r, 3, 0x55555556u) : r >> (heads - 1);
+  }
   return begin + group + (r - len * heads) * n + len;
 }
 
@@ -996,19 +1003,22 @@ static int plan_ranges(AttnArgs& a) {
     a.xcd_start[x] = (int)start;
     if (x > 0) max_items = std::max(max_items, a.xcd_start[x] - a.xcd_start[x - 1]);
   }
-  // Few items a head: longest first (see ticket_item).  With more of them the head-by-head order balances well enough,
-  // and where attention is near-uniform it is faster by what an XCD's workgroups share of a head in L2: 32 / 8 heads x 16384 1616 against
-  // 1644 us, x 32768 5.78 against 6.00 ms; 16 / 16 x 22016 1427 against 1435.
+  // An item a workgroup: as they are numbered.  Few items a head: longest first (see ticket_item).  With more of them the head-by-head order
+  // balances well enough, and where attention is near-uniform it is faster by what an XCD's workgroups share of a head in L2: 32 / 8
+  // heads x 16384 1616 against 1644 us, x 32768 5.78 against 6.00 ms; 16 / 16 x 22016 1427 against 1435.
   const int64_t total = (int64_t)a.BH * n;
-  const bool whole_heads = a.BH % 8 == 0;
-  a.deal = whole_heads ? (a.BH == 8 ? DEAL_NONE : n <= DEAL_ROW ? DEAL_GROUPS : DEAL_BY_LISTS) : total <= DEAL_ITEMS ? DEAL_ALL : DEAL_NONE;
-  const int64_t by = whole_heads ? DEAL_HEADS * n : a.BH;
-  a.deal_magic = (uint32_t)((1ull << 32) / by + 1);   // (by > 1, or not used) quotients are exact below 2^32 / by
-  if (total / 8 >= (1ll << 32) / by) a.deal = DEAL_NONE;
-  if (a.deal != DEAL_NONE) {
+  const bool whole_heads = a.BH % 8 == 0, one_each = total <= 256;
+  a.deal = one_each ? DEAL_NONE : whole_heads ? (a.BH == 8 ? DEAL_NONE : n <= DEAL_ROW ? DEAL_GROUPS : DEAL_BY_LISTS) : total <= DEAL_ITEMS ? DEAL_ALL : DEAL_NONE;
+  a.deal_heads = !whole_heads ? a.BH : total <= 2 * 256 ? a.BH / 8 : DEAL_HEADS;
+  const int64_t group = a.deal_heads * n;
+  // (divisors of 1 are not used) quotients are exact below 2^32 / divisor
+  a.group_magic = (uint32_t)((1ull << 32) / group + 1);
+  a.heads_magic = (uint32_t)((1ull << 32) / a.deal_heads + 1);
+  if (total / 8 >= (1ll << 32) / group) a.deal = DEAL_NONE;
+  if (one_each || a.deal != DEAL_NONE) {
     max_items = 0;
     for (int x = 0; x <= 8; ++x) {
-      a.xcd_start[x] = whole_heads ? (int)(x * total / 8) : (int)(x * (total / 8) + std::min<int64_t>(x, total % 8));   // (items 8 t + x < total)
+      a.xcd_start[x] = !one_each && whole_heads ? (int)(x * total / 8) : (int)(x * (total / 8) + std::min<int64_t>(x, total % 8));   // (DEAL_ALL: items 8 t + x < total)
       if (x > 0) max_items = std::max(max_items, a.xcd_start[x] - a.xcd_start[x - 1]);
     }
   }

@@ -36,7 +36,7 @@ def test_the_same_heads_in_launches_of_other_sizes(dev, Hq, Hkv, S, seg, thr, re
         assert torch.equal(alone[:, :g], one)
 
 
-@pytest.mark.parametrize("Hq,Hkv,S,reps", [(32, 8, 77, 1), (16, 4, 2048, 3), (32, 8, 295, 4), (32, 8, 1536, 2), (3, 1, 128, 40), (1, 1, 511 * 128, 2), (28, 4, 1500, 2), (9, 3, 40 * 128 - 1, 2)])
+@pytest.mark.parametrize("Hq,Hkv,S,reps", [(32, 8, 77, 1), (16, 4, 2048, 3), (32, 8, 295, 4), (32, 8, 1536, 2), (32, 8, 1021, 4), (8, 8, 4096 - 1, 3), (24, 8, 1400, 1), (3, 1, 128, 40), (1, 1, 511 * 128, 2), (28, 4, 1500, 2), (9, 3, 40 * 128 - 1, 2)])
 def test_one_segment_in_launches_of_other_sizes(dev, Hq, Hkv, S, reps):
     q, k, v = (x.to(dev) for x in small_case(1, Hq, Hkv, S, seed=S))
     run = lambda a, b, c: P.permuted_block_sparse_attn_fwd(a, b, c, 128, 65536, 0.9, True)
