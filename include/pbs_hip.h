@@ -212,6 +212,17 @@ int pbs_one_segment_attn_fwd(const void* q, const void* k, const void* v, void* 
                              int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
                              int64_t o_sb, int64_t o_sh, int64_t o_ss, float softmax_scale, void* stream);
 
+/* The un-permuted MeanPooling mode in one call: mean-pooled blocks, candidates up to and including the diagonal block, which is
+ * always selected, up to 2048 blocks per sequence; K and V are read in place.  Replaces
+ * pbs_attn/baselines/MeanPooling.py:7-99 (with force_select_current_block). */
+size_t pbs_meanpooling_attn_workspace_bytes(int B, int Hq, int Hkv, int S, int head_dim, int block_size);
+int pbs_meanpooling_attn_fwd(const void* q, const void* k, const void* v, void* out, int B, int Hq, int Hkv, int S,
+                             int head_dim, int block_size, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
+                             int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
+                             int64_t o_sh, int64_t o_ss, float threshold, const float* threshold_per_row,
+                             int force_select_first_block, float softmax_scale, void* workspace,
+                             size_t workspace_bytes, void* stream);
+
 /* Rotary position embedding of Q and K in one pass: out = bf16(bf16(x * cos) + bf16(rotate_half(x) * sin)),
  * bit-identical to the bf16 tensor expression of pbs_attn/patch/huggingface.py:14-25 (called at :203).
  * q (B, Hq, S, 128) and k (B, Hkv, S, 128) with their strides (e.g. the (B, S, H, D) memory of the

@@ -34,6 +34,8 @@ SIGNATURES = {
     "pbs_rope_qk": (c_int, [_P] * 6 + [_I] * 5 + [_L] * 8 + [_P]),
     "pbs_identity_indices": (c_int, [_P, _I, _I, _P]),
     "pbs_prefill_attn_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I, _I]),
+    "pbs_meanpooling_attn_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I]),
+    "pbs_meanpooling_attn_fwd": (c_int, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I] + [_L] * 12 + [_F, _P, _I, _F, _P, _Z, _P]),
     "pbs_one_segment_attn_fwd": (c_int, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I] + [_L] * 12 + [_F, _P]),
     "pbs_prefill_attn_fwd": (c_int, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I] + [_L] * 12 +
                              [_F, _P, _I, _I, _I, _I, _F, _P, _Z, _P]),

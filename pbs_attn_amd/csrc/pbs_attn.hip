@@ -756,7 +756,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
           if (PBS_UNLIKELY(e_cur & unseen)) first_reference(std::integral_constant<int, 0>{}, e_cur);
           if (PBS_LIKELY((e_cur & (USE0 | USE1)) == (USE0 | USE1)))
             fast_tile<0, 4, MASKED, V_ROWS>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
-          else if (V_ROWS || (e_cur & USE0))   // (of own-segment tiles the second block alone visits its diagonal one only)
+          else if ((MASKED && V_ROWS) || (e_cur & USE0))   // (a diagonal tile is one of its own block)
             fast_tile<0, 2, MASKED, V_ROWS>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);
           else
             fast_tile<2, 2, MASKED, V_ROWS>(ka, va, c_log2, m_ref, l_row, poisoned, wave, copy);

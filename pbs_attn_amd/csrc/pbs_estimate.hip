@@ -8,6 +8,7 @@
 // waves split the key-block tiles, first to find each row's (max, sum), then to
 // recompute the logits and write P with 128-byte row segments per store.
 #include "pbs_estimate.h"
+#include "pbs_lists.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 
 namespace {
@@ -36,7 +37,10 @@ int launch_block_logits(const char* who, bool causal, bool candidates_only, cons
   PBS_REQUIRE(rows > 0 && rows <= 65535 && nb > 0 && blocks_per_segment > 0, "%s: bad shape", who);
   const dim3 grid((nb + 31) / 32, rows);
   const Divisor sqrt_d = pbs_sqrt_divisor(head_dim);
-  if (candidates_only)
+  if (candidates_only && causal)
+    hipLaunchKernelGGL((block_logits_softmax_kernel<true, true>), grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)pooled_q,
+                       (const uint16_t*)pooled_k, block_attn_scores, nb, blocks_per_segment, sqrt_d);
+  else if (candidates_only)
     hipLaunchKernelGGL((block_logits_softmax_kernel<false, true>), grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)pooled_q,
                        (const uint16_t*)pooled_k, block_attn_scores, nb, blocks_per_segment, sqrt_d);
   else if (causal)
@@ -59,6 +63,11 @@ extern "C" int pbs_block_logits_softmax_causal(const void* pooled_q, const void*
                                                int rows, int nb, int head_dim, void* stream) {
   return launch_block_logits("pbs_block_logits_softmax_causal", true, false, pooled_q, pooled_k, block_attn_scores, rows, nb,
                              head_dim, 1, stream);
+}
+
+int pbs_block_logits_softmax_causal_candidates(const void* pooled_q, const void* pooled_k, float* block_attn_scores, int rows, int nb,
+                                               int head_dim, void* stream) {
+  return launch_block_logits("pbs_block_logits_softmax_causal", true, true, pooled_q, pooled_k, block_attn_scores, rows, nb, head_dim, 1, stream);
 }
 
 extern "C" int pbs_block_logits_softmax_candidates_only(const void* pooled_q, const void* pooled_k, float* block_attn_scores, int rows,

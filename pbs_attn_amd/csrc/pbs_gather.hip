@@ -25,7 +25,7 @@ constexpr int VT_PITCH = 130;  // bf16 elements per staged V row (padded: bank s
 struct GatherArgs {
   const uint16_t* k;
   const uint16_t* v;
-  const int32_t* idx;  // (B*Hq, S_pad)
+  const int32_t* idx;  // (B*Hq, S_pad), or null: every key in its own place (POOL_ONLY)
   uint16_t* perm_k;
   uint16_t* perm_vt;
   uint16_t* pooled_k;
@@ -55,7 +55,7 @@ __device__ __forceinline__ void gather_block(GatherArgs& a, uint16_t* vt, float 
   // row 0 and are zeroed afterwards, so that no load sits behind a branch.
   int src[8];
 #pragma unroll
-  for (int pass = 0; pass < 8; ++pass) src[pass] = idx[pass * 16 + rg];
+  for (int pass = 0; pass < 8; ++pass) src[pass] = POOL_ONLY && !a.idx ? kb * BS + pass * 16 + rg : idx[pass * 16 + rg];
   u32x4 kv[8], vv[8];
 #pragma unroll
   for (int pass = 0; pass < 8; ++pass) {
@@ -336,7 +336,16 @@ extern "C" int pbs_pool_blocks(const void* q, const void* k, const int32_t* key_
                                uint8_t* block_needed, int B, int Hq, int Hkv, int S, int head_dim, int block_size,
                                int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss,
                                int query_pool_max, int key_pool_max, void* stream) {
-  PBS_REQUIRE(q && k && key_indices && pooled_q && pooled_k, "pbs_pool_blocks: null tensor pointer");
+  PBS_REQUIRE(key_indices, "pbs_pool_blocks: null tensor pointer");
+  return pbs_pool_blocks_launch(q, k, key_indices, pooled_q, pooled_k, block_needed, B, Hq, Hkv, S, head_dim, block_size, q_sb, q_sh, q_ss,
+                                k_sb, k_sh, k_ss, query_pool_max, key_pool_max, stream);
+}
+
+int pbs_pool_blocks_launch(const void* q, const void* k, const int32_t* key_indices, void* pooled_q, void* pooled_k,
+                           uint8_t* block_needed, int B, int Hq, int Hkv, int S, int head_dim, int block_size,
+                           int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss,
+                           int query_pool_max, int key_pool_max, void* stream) {
+  PBS_REQUIRE(q && k && pooled_q && pooled_k, "pbs_pool_blocks: null tensor pointer");
   PBS_REQUIRE(head_dim == D && block_size == BS, "pbs_pool_blocks: head_dim and block_size must be 128 (got %d, %d)", head_dim, block_size);
   PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0, "pbs_pool_blocks: bad shape");
   PBS_REQUIRE(q_sb % 8 == 0 && q_sh % 8 == 0 && q_ss % 8 == 0 && k_sb % 8 == 0 && k_sh % 8 == 0 && k_ss % 8 == 0 &&

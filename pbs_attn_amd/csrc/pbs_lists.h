@@ -32,22 +32,33 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
                            int64_t o_sh, int64_t o_ss, float softmax_scale, const uint8_t* own_block_needed, void* workspace,
                            void* stream);
 
-// The selection of pbs_select_blocks for rows of block probabilities that are non-zero in the blocks of earlier segments
-// only, up to PBS_PAIR_SELECT_MAX_BLOCKS blocks, straight into the merged lists.  first_blk: the block that holds original
-// key 0, per row, or null.
+// The selection of pbs_select_blocks for rows of block probabilities that are non-zero in the candidates of `rule` only, up to
+// PBS_PAIR_SELECT_MAX_BLOCKS blocks, straight into the merged lists.  EARLIER_SEGMENTS: the blocks of earlier segments are candidates,
+// permuted tiles, and the own segment comes besides.  UP_TO_DIAGONAL: every block up to the diagonal one is, all of them tiles of the
+// un-permuted K and V, the diagonal one always visited.  force_first: so is the block that holds original key 0, first_blk[row] or,
+// with first_blk null, block 0.
 constexpr int PBS_PAIR_SELECT_MAX_BLOCKS = 2048;
-int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold_per_row, float threshold, const int32_t* first_blk,
-                          int rows, int S, int block_size, int segment_size, uint8_t* block_needed, const PairLists& lists,
+enum class Candidates { EARLIER_SEGMENTS = 1, UP_TO_DIAGONAL = 2 };   // candidate_rule of pbs_select_blocks
+int pbs_select_pair_lists(const float* block_attn_scores, Candidates rule, const float* threshold_per_row, float threshold, bool force_first,
+                          const int32_t* first_blk, int rows, int S, int block_size, int segment_size, uint8_t* block_needed, const PairLists& lists,
                           void* stream);
 // pbs_block_logits_softmax and that selection in one launch, for rows of up to PBS_ESTIMATE_SELECT_MAX_BLOCKS blocks
 constexpr int PBS_ESTIMATE_SELECT_MAX_BLOCKS = 64;
-int pbs_estimate_select_pair_lists(const void* pooled_q, const void* pooled_k, const float* threshold_per_row, float threshold,
-                                   const int32_t* first_blk, int rows, int S, int head_dim, int block_size, int segment_size,
+int pbs_estimate_select_pair_lists(const void* pooled_q, const void* pooled_k, Candidates rule, const float* threshold_per_row,
+                                   float threshold, bool force_first, const int32_t* first_blk, int rows, int S, int head_dim, int block_size, int segment_size,
                                    uint8_t* block_needed, const PairLists& lists, void* stream);
 // pbs_segment_argsort; first_blk, if not null, receives per row the block of `block_size` that holds original key 0 (there has
 // to be a complete segment)
 int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,
                                int S_pad, int segment_size, void* stream);
+// pbs_block_logits_softmax_causal without the entries that are no candidates
+int pbs_block_logits_softmax_causal_candidates(const void* pooled_q, const void* pooled_k, float* block_attn_scores, int rows, int nb,
+                                               int head_dim, void* stream);
+// pbs_pool_blocks; key_indices null: every key in its own place
+int pbs_pool_blocks_launch(const void* q, const void* k, const int32_t* key_indices, void* pooled_q, void* pooled_k,
+                           uint8_t* block_needed, int B, int Hq, int Hkv, int S, int head_dim, int block_size,
+                           int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss,
+                           int query_pool_max, int key_pool_max, void* stream);
 // pbs_pool_blocks and an unfiltered pbs_gather_kv in one launch (the pooled key blocks have the bits of both)
 int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const int32_t* key_indices, void* pooled_q, void* pooled_k,
                            void* perm_k, void* perm_vt, int B, int Hq, int Hkv, int S, int head_dim, int block_size, int64_t q_sb,

@@ -163,16 +163,16 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
                               head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, query_pool_max, key_pool_max,
                               stream))) return rc;
     if (is_short) {
-      if ((rc = pbs_estimate_select_pair_lists(w + L.pooled_q, w + L.pooled_k, threshold_per_row, threshold,
-                                               force_select_first_block ? (const int32_t*)(w + L.select_ws) : nullptr, rows, S, head_dim,
+      if ((rc = pbs_estimate_select_pair_lists(w + L.pooled_q, w + L.pooled_k, Candidates::EARLIER_SEGMENTS, threshold_per_row, threshold,
+                                               force_select_first_block != 0, (const int32_t*)(w + L.select_ws), rows, S, head_dim,
                                                block_size, segment_size, needed,
                                                pbs_pair_lists(B, Hq, Hkv, S, block_size, segment_size, w + L.attn_ws), stream))) return rc;
     // (the selection into pair lists reads a row's candidate entries only: the others are not written)
     } else if (pair_lists) {
       if ((rc = pbs_block_logits_softmax_candidates_only(w + L.pooled_q, w + L.pooled_k, (float*)(w + L.probs), rows, nb,
                                                          head_dim, segment_size / block_size, stream))) return rc;
-      if ((rc = pbs_select_pair_lists((const float*)(w + L.probs), threshold_per_row, threshold,
-                                      force_select_first_block ? (const int32_t*)(w + L.select_ws) : nullptr, rows, S, block_size,
+      if ((rc = pbs_select_pair_lists((const float*)(w + L.probs), Candidates::EARLIER_SEGMENTS, threshold_per_row, threshold,
+                                      force_select_first_block != 0, (const int32_t*)(w + L.select_ws), rows, S, block_size,
                                       segment_size, needed,
                                       pbs_pair_lists(B, Hq, Hkv, S, block_size, segment_size, w + L.attn_ws), stream))) return rc;
     } else {
@@ -192,4 +192,64 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
   return pbs_sparse_attn_launch(q, w + L.perm_k, w + L.perm_vt, k, v, cols, (const int32_t*)(w + L.cnt), pair_lists, out, B, Hq, Hkv, S,
                                 head_dim, block_size, segment_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb,
                                 o_sh, o_ss, softmax_scale, nullptr, w + L.attn_ws, stream);
+}
+
+// ---- the un-permuted MeanPooling mode (pbs_attn/baselines/MeanPooling.py) in one call: pooled blocks in their own order, every block up to
+// the diagonal one a candidate, all tiles read in place from K and V
+namespace {
+
+struct MeanPoolingLayout {
+  size_t pooled_k, pooled_q, probs, attn_ws, total;
+};
+MeanPoolingLayout meanpooling_layout(int B, int Hq, int S, int D, int block_size) {
+  MeanPoolingLayout L;
+  const size_t rows = (size_t)B * Hq, nb = (size_t)(S + block_size - 1) / block_size;
+  size_t off = 0;
+  auto take = [&](size_t bytes) { const size_t o = off; off = align256(off + bytes); return o; };
+  L.pooled_k = take(rows * nb * D * 2);
+  L.pooled_q = take(rows * nb * D * 2);
+  L.probs = take(short_pass((int)rows, (int)nb) ? 0 : rows * nb * nb * 4);
+  L.attn_ws = off;
+  L.total = align256(off + pbs_sparse_attn_workspace_bytes(B, Hq, S, block_size));
+  return L;
+}
+
+}  // namespace
+
+extern "C" size_t pbs_meanpooling_attn_workspace_bytes(int B, int Hq, int Hkv, int S, int head_dim, int block_size) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || S <= 0 || head_dim <= 0 || block_size <= 0) return 0;
+  return meanpooling_layout(B, Hq, S, head_dim, block_size).total;
+}
+
+extern "C" int pbs_meanpooling_attn_fwd(const void* q, const void* k, const void* v, void* out, int B, int Hq, int Hkv, int S,
+                                        int head_dim, int block_size, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
+                                        int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t o_sb,
+                                        int64_t o_sh, int64_t o_ss, float threshold, const float* threshold_per_row,
+                                        int force_select_first_block, float softmax_scale, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
+  PBS_REQUIRE(q && k && v && out, "pbs_meanpooling_attn_fwd: null tensor pointer");
+  PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0 && block_size > 0, "pbs_meanpooling_attn_fwd: bad shape");
+  const int rows = B * Hq, nb = (S + block_size - 1) / block_size;
+  PBS_REQUIRE(rows <= 65535, "pbs_meanpooling_attn_fwd: too many heads (%d)", rows);
+  PBS_REQUIRE(nb <= PBS_PAIR_SELECT_MAX_BLOCKS, "pbs_meanpooling_attn_fwd: more than %d blocks per sequence (%d)", PBS_PAIR_SELECT_MAX_BLOCKS, nb);
+  const MeanPoolingLayout L = meanpooling_layout(B, Hq, S, head_dim, block_size);
+  PBS_REQUIRE(workspace && workspace_bytes >= L.total && ((uintptr_t)workspace % 256) == 0,
+              "pbs_meanpooling_attn_fwd: workspace must be a 256-byte aligned device buffer of %zu bytes", L.total);
+  uint8_t* w = (uint8_t*)workspace;
+  int rc;
+  if ((rc = pbs_pool_blocks_launch(q, k, nullptr, w + L.pooled_q, w + L.pooled_k, nullptr, B, Hq, Hkv, S, head_dim, block_size, q_sb, q_sh,
+                                   q_ss, k_sb, k_sh, k_ss, 0, 0, stream))) return rc;
+  const PairLists lists = pbs_pair_lists(B, Hq, Hkv, S, block_size, block_size, w + L.attn_ws);
+  if (short_pass(rows, nb)) {
+    if ((rc = pbs_estimate_select_pair_lists(w + L.pooled_q, w + L.pooled_k, Candidates::UP_TO_DIAGONAL, threshold_per_row, threshold,
+                                             force_select_first_block != 0, nullptr, rows, S, head_dim, block_size, block_size, nullptr,
+                                             lists, stream))) return rc;
+  } else {
+    if ((rc = pbs_block_logits_softmax_causal_candidates(w + L.pooled_q, w + L.pooled_k, (float*)(w + L.probs), rows, nb, head_dim, stream))) return rc;
+    if ((rc = pbs_select_pair_lists((const float*)(w + L.probs), Candidates::UP_TO_DIAGONAL, threshold_per_row, threshold,
+                                    force_select_first_block != 0, nullptr, rows, S, block_size, block_size, nullptr, lists, stream))) return rc;
+  }
+  // (permuted tiles: none is listed, any aligned address will do)
+  return pbs_sparse_attn_launch(q, q, q, k, v, nullptr, nullptr, true, out, B, Hq, Hkv, S, head_dim, block_size, block_size, q_sb, q_sh, q_ss,
+                                k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale, nullptr, w + L.attn_ws, stream);
 }

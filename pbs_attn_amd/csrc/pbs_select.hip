@@ -36,6 +36,7 @@ struct SelectArgs {
   uint8_t* needed;         // (rows, nb) or null: set to 1 for every key block on some query block's visit list
   int cand_rule;           // which entries of a row can be non-zero: 0 any, 1 kb < first block of qb's segment, 2 kb <= qb
   int qb_lo, qb_hi;        // wave kernel: the query blocks this launch covers
+  int in_place;            // merged lists of un-permuted blocks up to the diagonal one, which is always visited
 };
 
 // Block that holds original key 0.  A segment-wise permutation keeps it inside the first segment, so that
@@ -511,9 +512,10 @@ __device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb,
   }
   __builtin_amdgcn_wave_barrier();
   if (a.force_first && lane == 0) {
-    const int fb = a.first_blk[row];
+    const int fb = a.first_blk ? a.first_blk[row] : 0;
     if (fb >= 0 && fb < nb) flag[fb] = 1;
   }
+  if (a.in_place && lane == 0) flag[qb] = 1;
 }
 
 // one wave decides row `rq` ((row, qb - qb_lo) flattened) of the group of rows [qb_lo, qb_hi) x all heads
@@ -598,7 +600,9 @@ __device__ __forceinline__ void write_lists(const SelectArgs& a, const PairLists
   const bool second = pairs && first + 1 < nb;
   const int qb1 = second ? first + 1 : first;
   const int sf0 = (first / a.bps) * a.bps, sf1 = (qb1 / a.bps) * a.bps;
-  const int end1 = second ? sf1 : 0, end = max(sf0, end1);   // a row's flags count up to its own segment
+  // a row's flags count up to its own segment, or up to its own block
+  const int end0 = a.in_place ? first + 1 : sf0, end1 = second ? (a.in_place ? qb1 + 1 : sf1) : 0, end = max(end0, end1);
+  const uint32_t kind = a.in_place ? ENT_ORIG : 0u;
   const uint32_t* f0 = reinterpret_cast<const uint32_t*>(flags + (pairs ? wave & 2 : wave) * nb_pad);
   const uint32_t* f1 = reinterpret_cast<const uint32_t*>(flags + ((wave & 2) + 1) * nb_pad);
   // the flags of blocks 4 x .. 4 x + 3, a byte each: bit 0 visited by the first query block, bit 1 by the second
@@ -607,7 +611,7 @@ __device__ __forceinline__ void write_lists(const SelectArgs& a, const PairLists
       const int valid = n - 4 * x;
       return valid >= 4 ? ~0u : valid <= 0 ? 0u : (1u << (8 * valid)) - 1u;
     };
-    const uint32_t m0 = below(sf0), m1 = below(end1);
+    const uint32_t m0 = below(end0), m1 = below(end1);
     return (m0 ? f0[x] & m0 : 0u) | (m1 ? f1[x] & m1 : 0u) << 1;
   };
   if (!pairs || (wave & 1)) {
@@ -635,11 +639,11 @@ __device__ __forceinline__ void write_lists(const SelectArgs& a, const PairLists
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const uint32_t use = v >> (8 * e) & 3u;
-      if (use) out[w++] = (uint16_t)((uint32_t)(4 * x + e) | use << 14);
+      if (use) out[w++] = (uint16_t)((uint32_t)(4 * x + e) | kind | use << 14);
     }
     base += __popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2);
   }
-  const int n_own = qb1 - sf0 + 1;
+  const int n_own = a.in_place ? 0 : qb1 - sf0 + 1;
   for (int t = lane; t < n_own; t += 64) {
     const int kb = sf0 + t;
     const uint32_t use = (kb <= first ? 1u : 0u) | (second && kb >= sf1 ? 2u : 0u);
@@ -698,6 +702,7 @@ __global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, Pa
 // way to memory and back less: 32 / 8 heads x 512 51.8 -> 48.6 us a pass, 28 / 4 x 1000 63.1 -> 59.4, 32 / 8 x 4096 174.0 -> 169.9, x
 // 8192 482 -> 477.  Above 2048 blocks the repeated products outweigh it: 128 heads x 6144 1159 against 1162, 32 / 8 x
 // 12288 (two entries a lane) 962 against 970.
+template <bool CAUSAL>
 __global__ __launch_bounds__(256) void estimate_select_kernel(const uint16_t* pooled_q, const uint16_t* pooled_k, SelectArgs a, PairLists l, Divisor sqrt_d) {
   __shared__ EstimateStats st;
   __shared__ float probs[4][PBS_ESTIMATE_SELECT_MAX_BLOCKS];
@@ -707,7 +712,7 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(const uint16_t* po
   const int nb = a.nb, nb_pad = (nb + 15) & ~15, qb = 4 * four + wave;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 8) l.queue[threadIdx.x] = l.first_tickets;
   const int64_t head = (int64_t)row * nb * ESTIMATE_D;
-  estimate_tile<false, true>(pooled_q + head, pooled_k + head, nb, a.bps, sqrt_d, four / 8, st, [&](int ql, int kb, float p) __attribute__((always_inline)) {
+  estimate_tile<CAUSAL, true>(pooled_q + head, pooled_k + head, nb, a.bps, sqrt_d, four / 8, st, [&](int ql, int kb, float p) __attribute__((always_inline)) {
     if (ql >> 2 == (four & 7)) probs[ql & 3][kb] = p;
   });
   __syncthreads();
@@ -845,23 +850,24 @@ extern "C" int pbs_select_blocks(const float* block_attn_scores, const float* th
   return pbs_check_launch("pbs_select_blocks");
 }
 
-int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold_per_row, float threshold, const int32_t* first_blk,
-                          int rows, int S, int block_size, int segment_size, uint8_t* block_needed, const PairLists& lists,
+int pbs_select_pair_lists(const float* block_attn_scores, Candidates rule, const float* threshold_per_row, float threshold, bool force_first,
+                          const int32_t* first_blk, int rows, int S, int block_size, int segment_size, uint8_t* block_needed, const PairLists& lists,
                           void* stream) {
   const int nb = (S + block_size - 1) / block_size, npair = (nb + 1) / 2;
   PBS_REQUIRE(rows > 0 && rows <= 65535 && nb <= PBS_PAIR_SELECT_MAX_BLOCKS, "pbs_select_pair_lists: bad shape");
   PBS_REQUIRE(block_attn_scores, "pbs_select_pair_lists: null score pointer");
   SelectArgs a = {};
   a.P = block_attn_scores; a.thr_rows = threshold_per_row; a.thr = threshold;
-  a.force_first = first_blk != nullptr;
+  a.force_first = force_first;
   a.first_blk = const_cast<int32_t*>(first_blk);
   a.nb = nb; a.bs = block_size; a.bps = segment_size / block_size; a.S = S;
   a.needed = block_needed;
-  a.cand_rule = 1;
+  a.cand_rule = (int)rule;
+  a.in_place = rule == Candidates::UP_TO_DIAGONAL;
   // groups of pairs whose second row's candidates fit 64 * npl sorted entries, longest first
   int npl[6], lo[6], hi[6], n = 0, from = 0;
   for (int x = 1; x <= 32 && from < npair; x *= 2) {
-    const int64_t blocks = (64 * x / a.bps + 1) * (int64_t)a.bps;   // query blocks with at most 64 x candidates
+    const int64_t blocks = a.in_place ? 64 * x : (64 * x / a.bps + 1) * (int64_t)a.bps;   // query blocks with at most 64 x candidates
     const int to = blocks >= nb ? npair : (int)(blocks / 2);
     if (to > from) {
       npl[n] = x; lo[n] = from; hi[n] = to;
@@ -891,22 +897,23 @@ int pbs_select_pair_lists(const float* block_attn_scores, const float* threshold
   return pbs_check_launch("pbs_select_pair_lists");
 }
 
-int pbs_estimate_select_pair_lists(const void* pooled_q, const void* pooled_k, const float* threshold_per_row, float threshold,
-                                   const int32_t* first_blk, int rows, int S, int head_dim, int block_size, int segment_size,
+int pbs_estimate_select_pair_lists(const void* pooled_q, const void* pooled_k, Candidates rule, const float* threshold_per_row,
+                                   float threshold, bool force_first, const int32_t* first_blk, int rows, int S, int head_dim, int block_size, int segment_size,
                                    uint8_t* block_needed, const PairLists& lists, void* stream) {
   const int nb = (S + block_size - 1) / block_size;
   PBS_REQUIRE(pooled_q && pooled_k && head_dim == ESTIMATE_D, "pbs_estimate_select: bad pooled tensors");
   PBS_REQUIRE(rows > 0 && rows <= 65535 && nb <= PBS_ESTIMATE_SELECT_MAX_BLOCKS, "pbs_estimate_select: bad shape");
   SelectArgs a = {};
   a.thr_rows = threshold_per_row; a.thr = threshold;
-  a.force_first = first_blk != nullptr;
+  a.force_first = force_first;
   a.first_blk = const_cast<int32_t*>(first_blk);
   a.nb = nb; a.bs = block_size; a.bps = segment_size / block_size; a.S = S;
   a.needed = block_needed;
-  a.cand_rule = 1;
+  a.cand_rule = (int)rule;
+  a.in_place = rule == Candidates::UP_TO_DIAGONAL;
   const dim3 grid((unsigned)((nb + 3) / 4), (unsigned)rows);
   const Divisor sqrt_d = pbs_sqrt_divisor(head_dim);
-  hipLaunchKernelGGL(estimate_select_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)pooled_q, (const uint16_t*)pooled_k, a,
+  hipLaunchKernelGGL(a.in_place ? estimate_select_kernel<true> : estimate_select_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)pooled_q, (const uint16_t*)pooled_k, a,
                      lists, sqrt_d);
   return pbs_check_launch("pbs_estimate_select");
 }

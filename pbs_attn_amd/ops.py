@@ -330,6 +330,28 @@ def prefill_attn_fwd(q, k, v, block_size, segment_size, threshold, force_select_
     return out
 
 
+def meanpooling_attn_fwd(q, k, v, threshold, force_select_first_block=True):
+    """The un-permuted MeanPooling mode in one library call, K and V read in place (up to MEANPOOLING_MAX_BLOCKS blocks)."""
+    _check_bf16_cuda(q, k, v)
+    lib = _lib.load()
+    q, k, v = _rows16(q), _rows16(k), _rows16(v)
+    B, Hq, S, D = q.shape
+    Hkv = k.shape[1]
+    _, thr_rows, thr = _threshold_args(threshold, B, Hq, q.device)
+    out = q.new_empty(B, Hq, S, D)
+    ws_bytes = lib.pbs_meanpooling_attn_workspace_bytes(B, Hq, Hkv, S, D, BLOCK)
+    ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=q.device)
+    _lib.check(lib.pbs_meanpooling_attn_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Hq, Hkv, S, D, BLOCK,
+        *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], Hq * S * D, S * D, D,
+        thr, _ptr(thr_rows), int(bool(force_select_first_block)), 1.0 / math.sqrt(D), ws.data_ptr(), max(ws_bytes, 256), _stream()),
+        "pbs_meanpooling_attn_fwd")
+    return out
+
+
+MEANPOOLING_MAX_BLOCKS = 2048
+
+
 def rope_qk(q, k, cos, sin):
     """Rotary embedding of q (B, Hq, S, D) and k (B, Hkv, S, D) with cos / sin (B or 1, S, D): the bits of
     ``x * cos + rotate_half(x) * sin`` in bf16 (pbs_attn/patch/huggingface.py:14-25), in one pass, returned
