@@ -51,6 +51,11 @@ int pbs_estimate_select_pair_lists(const void* pooled_q, const void* pooled_k, C
 // to be a complete segment)
 int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,
                                int S_pad, int segment_size, void* stream);
+// pbs_score_keys and pbs_segment_argsort_launch in one: the final scoring pass of short sequences of short segments sorts
+bool pbs_score_sorts(int B, int Hq, int Hkv, int S, int segment_size);
+int pbs_score_sort_launch(const void* q, const void* k, int32_t* key_indices, int32_t* first_blk, int B, int Hq, int Hkv, int S, int S_pad,
+                          int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
+                          int64_t k_sh, int64_t k_ss, void* workspace, size_t workspace_bytes, void* stream);
 // pbs_block_logits_softmax_causal without the entries that are no candidates
 int pbs_block_logits_softmax_causal_candidates(const void* pooled_q, const void* pooled_k, float* block_attn_scores, int rows, int nb,
                                                int head_dim, void* stream);

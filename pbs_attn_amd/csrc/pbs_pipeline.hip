@@ -138,6 +138,9 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
                                   w + L.attn_ws, stream);
   if (one_segment || nseg == 0 || (nseg == 1 && rem == 0)) {
     if ((rc = pbs_identity_indices((int32_t*)(w + L.idx), rows, s_pad, stream))) return rc;
+  } else if (pbs_score_sorts(B, Hq, Hkv, S, segment_size)) {
+    if ((rc = pbs_score_sort_launch(q, k, (int32_t*)(w + L.idx), (int32_t*)(w + L.select_ws), B, Hq, Hkv, S, s_pad, head_dim, block_size,
+                                    segment_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;
   } else {
     if ((rc = pbs_score_keys(q, k, (float*)(w + L.scores), B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh,
                              q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;

@@ -8,7 +8,8 @@
 //   3. score_final   : recompute the logits and emit the per-key mean probability
 // Logits reproduce the rounding points of a bf16 matmul followed by a bf16
 // divide: fp32 accumulate -> bf16 -> / sqrt(D) -> bf16.
-#include "pbs_common.h"
+#include "pbs_lists.h"
+#include "pbs_sort.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 #include <atomic>
 #include <mutex>
@@ -32,6 +33,9 @@ struct ScoreArgs {
   float* scores;  // (B*Hq, Sc)
   int nchunk;
   int chunk_keys;
+  int32_t* idx;        // (SORT) order of the keys (B*Hq, S_pad) and the block that holds key 0 (B*Hq)
+  int32_t* first_blk;
+  int S_pad, block_size;
 };
 
 __device__ __forceinline__ bf16x8 load_frag(const uint16_t* row_ptr, int t, int half) {
@@ -88,7 +92,9 @@ __device__ __forceinline__ void stage_keys_async(const uint16_t* rows, int64_t k
 // One wave per query head of the KV group; the waves of a workgroup share the staged key rows.  SPLIT (short sequences, see
 // score_plan): the four waves take 32 queries each of ONE head.
 // Waves per SIMD: the final pass of the split form needs 147 registers and would spill 18 of them at four.
-template <bool FINAL, bool SPLIT>
+// SORT: a workgroup of the final split pass takes a whole segment, keeps its scores in LDS, and its first wave sorts them, SORT keys a
+// lane: no launch, and no way to memory and back, for the sort.
+template <bool FINAL, bool SPLIT, int SORT = 0>
 __global__ __launch_bounds__(256, SPLIT ? (FINAL ? 3 : 4) : 2) void score_kernel(ScoreArgs a) {
   constexpr int QT = SPLIT ? 1 : NQ / 32;   // query tiles of a wave
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // starts at LDS offset 0: this kernel has no static LDS
@@ -105,6 +111,7 @@ __global__ __launch_bounds__(256, SPLIT ? (FINAL ? 3 : 4) : 2) void score_kernel
   const uint16_t* kbase = a.k + b * a.k_sb + kvh * a.k_sh;
   float* s_stats = reinterpret_cast<float*>(smem + LDS_STATS) + wave * (32 * QT);   // p = exp2(logit - stat)
   float* s_sums = reinterpret_cast<float*>(smem + LDS_STATS) + NQ;   // SPLIT: a wave's sums of the stage's keys
+  float* s_scores = reinterpret_cast<float*>(smem + LDS_SCORE_TOTAL);   // SORT: the segment's scores
   // LDS byte offset of fragment 0 of key row j inside a stage buffer; fragment t lies at frag0 ^ (t << 5),
   // rows 32 .. 63 of the stage 8 KB further on
   const uint32_t frag0 = (uint32_t)(j * 256 + ((half ^ (j & 15)) * 16));
@@ -244,9 +251,21 @@ __global__ __launch_bounds__(256, SPLIT ? (FINAL ? 3 : 4) : 2) void score_kernel
         __syncthreads();   // (the next stage's sums are written behind its first barrier)
         if (wave == 0) {
           const float* s = s_sums + lane;
-          a.scores[(int64_t)bh * a.Sc + key_lo + st * STAGE_KEYS + lane] =
-              ((s[0] + s[STAGE_KEYS]) + (s[2 * STAGE_KEYS] + s[3 * STAGE_KEYS])) * (1.0f / NQ);
+          const float score = ((s[0] + s[STAGE_KEYS]) + (s[2 * STAGE_KEYS] + s[3 * STAGE_KEYS])) * (1.0f / NQ);
+          if (SORT) s_scores[st * STAGE_KEYS + lane] = score;
+          else a.scores[(int64_t)bh * a.Sc + key_lo + st * STAGE_KEYS + lane] = score;
         }
+      }
+    }
+    if constexpr (SORT > 0) {
+      int32_t* row = a.idx + (int64_t)bh * a.S_pad;
+      if (wave == 0) {   // (its own stores, in order)
+        double k[SORT];
+#pragma unroll
+        for (int r = 0; r < SORT; ++r) k[r] = sort_key_of<SORT>(s_scores, 64 * r + lane, a.chunk_keys);
+        sort_and_store<SORT>(k, lane, a.chunk_keys, key_lo, chunk, row + key_lo, a.first_blk ? a.first_blk + bh : nullptr, a.block_size);
+      } else if (chunk == 0) {   // the remainder of the sequence and the block padding keep their places
+        for (int i = a.Sc + (int)threadIdx.x - 64; i < a.S_pad; i += 192) row[i] = i;
       }
     }
     if (!FINAL && active) {
@@ -316,8 +335,17 @@ int chunks_for(int Sc, int chunk_keys) { return (Sc + chunk_keys - 1) / chunk_ke
 //   * groups that leave waves of the grouped form idle: 28 / 4 x 9000 601 -> 567, 16 / 16 x 20000 783 -> 763 and x 131072 1485 ->
 //     1409, 8 / 8 x 131072 790 -> 760, 16 / 8 x 32768 460 -> 430, 14 / 2 x 65536 632 -> 624; at 28 / 4 x 65536, where an eighth is
 //     idle, the two are equal (1193, 1196), hence the limit for groups with less than a quarter idle.
+// A short sequence's workgroups all run at once, three a CU: one more round costs more than the longer chunk (a stage of 64 keys 1.2 us a
+// pass).  Whole pass: 32 / 8 heads x 2048, 1024 workgroups of 64 keys -> 512 of 128, 93.9 -> 90.7 us; x 4096, 1024 of 128 -> 512 of 256,
+// 167.5 -> 165.8; 28 / 4 x 4096 153.3 -> 151.5; fewer than they have to be: 16 / 16 x 2048, 512 -> 256, 65.5 -> 69.4.
+constexpr int SPLIT_WORKGROUPS = 3 * 256;
+// The final pass sorts where a segment is at most two chunks long, so that a workgroup's serial part hardly grows, and its workgroups still
+// run at once.  Whole pass, sort kernel -> this: segments of 128, 32 / 8 heads x 512 45.3 -> 42.9 us, 28 / 4 x 1019 59.8 -> 56.7, 4 / 1 x
+// 16384 257.7 -> 249.6; of 256, 32 / 8 x 4096 166.1 -> 163.8, 28 / 4 x 4091 153.5 -> 150.8, 4 / 1 x 16384 160.5 -> 152.4.  Outside: segments of
+// four chunks 8 / 2 x 2048 58.9 against 60.4, 1024 workgroups 32 / 8 x 4096 164.9 against 165.7.
+constexpr int SORT_IN_PASS_KEYS = 256;
 struct ScorePlan {
-  bool split;
+  bool split, small;
   int chunk_keys, nchunk;
 };
 ScorePlan score_plan(int B, int Hq, int Hkv, int Sc) {
@@ -331,8 +359,8 @@ ScorePlan score_plan(int B, int Hq, int Hkv, int Sc) {
   const bool uneven = idle > 0 && heads >= 8 && (4 * idle >= slots || keys <= 1 << 20);
   const bool split = (small || uneven) && heads <= 65535;
   if (split)
-    while (chunks_for(Sc, chunk) > SPLIT_MAX_CHUNKS) chunk *= 2;
-  return {split, chunk, chunks_for(Sc, chunk)};
+    while (chunks_for(Sc, chunk) > SPLIT_MAX_CHUNKS || (small && chunks_for(Sc, chunk) * heads > SPLIT_WORKGROUPS)) chunk *= 2;
+  return {split, small, chunk, chunks_for(Sc, chunk)};
 }
 
 }  // namespace
@@ -350,8 +378,9 @@ namespace {
 // partials and the folded row statistics.
 int score_keys_launch(const char* who, const void* q, const void* k, float* scores, int B, int Hq, int Hkv, int S,
                       int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss,
-                      int64_t k_sb, int64_t k_sh, int64_t k_ss, void* workspace, size_t workspace_bytes, void* stream) {
-  PBS_REQUIRE(q && k && scores, "%s: null tensor pointer", who);
+                      int64_t k_sb, int64_t k_sh, int64_t k_ss, void* workspace, size_t workspace_bytes, void* stream,
+                      int32_t* idx = nullptr, int32_t* first_blk = nullptr, int S_pad = 0) {
+  PBS_REQUIRE(q && k && (scores || idx), "%s: null tensor pointer", who);
   PBS_REQUIRE(head_dim == D, "%s: head_dim must be 128, got %d", who, head_dim);
   PBS_REQUIRE(block_size == NQ, "%s: block_size must be 128, got %d", who, block_size);
   PBS_REQUIRE(B > 0 && Hkv > 0 && Hq > 0 && Hq % Hkv == 0, "%s: bad head counts Hq=%d Hkv=%d", who, Hq, Hkv);
@@ -380,18 +409,29 @@ int score_keys_launch(const char* who, const void* q, const void* k, float* scor
   a.part = (float*)workspace;
   a.stats = a.part + (size_t)B * Hq * a.nchunk * NQ * 2;
   a.scores = scores;
+  a.idx = idx; a.first_blk = first_blk; a.S_pad = S_pad; a.block_size = block_size;
   static std::atomic<bool> lds_checked{false};   // once per process: a property of the code object
   if (!lds_checked.load(std::memory_order_acquire)) {
     if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<false, false>, who)) return rc;
     if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, false>, who)) return rc;
     if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<false, true>, who)) return rc;
     if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, true>, who)) return rc;
+    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, true, 2>, who)) return rc;
+    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, true, 4>, who)) return rc;
     lds_checked.store(true, std::memory_order_release);
   }
   hipStream_t st = (hipStream_t)stream;
   if (plan.split) {
     const dim3 grid(a.nchunk, B * Hq);
     hipLaunchKernelGGL((score_kernel<false, true>), grid, dim3(256), LDS_SCORE_TOTAL, st, a);
+    if (idx) {
+      a.chunk_keys = segment_size;
+      const dim3 segments(Sc / segment_size, B * Hq);
+      const size_t lds = LDS_SCORE_TOTAL + segment_size * sizeof(float);
+      if (segment_size <= 128) hipLaunchKernelGGL((score_kernel<true, true, 2>), segments, dim3(256), lds, st, a);
+      else hipLaunchKernelGGL((score_kernel<true, true, 4>), segments, dim3(256), lds, st, a);
+      return pbs_check_launch(who);
+    }
     hipLaunchKernelGGL((score_kernel<true, true>), grid, dim3(256), LDS_SCORE_TOTAL, st, a);
     return pbs_check_launch(who);
   }
@@ -404,6 +444,21 @@ int score_keys_launch(const char* who, const void* q, const void* k, float* scor
 }
 
 }  // namespace
+
+bool pbs_score_sorts(int B, int Hq, int Hkv, int S, int segment_size) {
+  const int Sc = (S / segment_size) * segment_size;
+  if (Sc == 0 || segment_size > SORT_IN_PASS_KEYS || segment_size % STAGE_KEYS) return false;
+  const ScorePlan plan = score_plan(B, Hq, Hkv, Sc);
+  return plan.split && plan.small && segment_size <= 2 * plan.chunk_keys && (int64_t)B * Hq * (Sc / segment_size) <= SPLIT_WORKGROUPS;
+}
+
+int pbs_score_sort_launch(const void* q, const void* k, int32_t* key_indices, int32_t* first_blk, int B, int Hq, int Hkv, int S, int S_pad,
+                          int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
+                          int64_t k_sh, int64_t k_ss, void* workspace, size_t workspace_bytes, void* stream) {
+  PBS_REQUIRE(key_indices && pbs_score_sorts(B, Hq, Hkv, S, segment_size), "pbs_score_sort: bad arguments");
+  return score_keys_launch("pbs_score_keys", q, k, nullptr, B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh, q_ss, k_sb,
+                           k_sh, k_ss, workspace, workspace_bytes, stream, key_indices, first_blk, S_pad);
+}
 
 extern "C" int pbs_score_keys(const void* q, const void* k, float* scores, int B, int Hq, int Hkv, int S, int head_dim,
                               int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,

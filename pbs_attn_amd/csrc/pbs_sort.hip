@@ -5,7 +5,7 @@
 // trailing partial segment and the padding up to a whole block keep identity order.
 // Segments of up to 2048 keys are sorted by one wave in registers, longer ones by a workgroup in LDS.
 #include "pbs_lists.h"
-#include "pbs_wave.h"
+#include "pbs_sort.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 #include <algorithm>
 
@@ -34,73 +34,6 @@ __global__ __launch_bounds__(256) void segment_argsort_kernel(const float* score
       if ((uint32_t)keys[i] == 0) first_blk[row] = i / block_size;
 }
 
-// ---- one wave per segment, NPL keys per lane in registers.
-// The 32 score bits and an 11-bit index make a 43-bit integer.  As the mantissa of a double in [1, 2) it keeps its order, and
-// a compare-exchange inside a lane is one minimum and one maximum of doubles (64-bit integers take a comparison and four
-// selects); descending runs carry the keys negated.  Between lanes: two moves, a comparison, two selects, no LDS.
-// Segments of 1024, 32 heads x 128k keys: 87 -> 37 us (the LDS network moved each key through memory in all 55 stages);
-// segments of 256 at 4k: 10.2 -> 7.2 us.
-__device__ __forceinline__ double sort_key(float score, uint32_t index) {
-  const uint64_t u = (uint64_t)(~f32_orderable(score)) << 11 | index;
-  return __builtin_bit_cast(double, 0x3ff0000000000000ull | u);
-}
-__device__ __forceinline__ uint32_t sort_key_index(double key) { return (uint32_t)__builtin_bit_cast(uint64_t, key) & 2047u; }
-
-// lane distance LS: the lower lane keeps the smaller key
-template <int NPL, int LS>
-__device__ __forceinline__ void cross_lane_sort_stage(double (&k)[NPL], int lane) {
-  const bool upper = (lane & LS) != 0;
-#pragma unroll
-  for (int r = 0; r < NPL; ++r) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, k[r]);
-    const TwoOf lo = with_lane_xor<LS>((uint32_t)u), hi = with_lane_xor<LS>((uint32_t)(u >> 32));
-    const double a = __builtin_bit_cast(double, (uint64_t)hi.a << 32 | lo.a), b = __builtin_bit_cast(double, (uint64_t)hi.b << 32 | lo.b);
-    const bool first = (a < b) != upper;
-    const uint32_t rl = first ? lo.a : lo.b, rh = first ? hi.a : hi.b;
-    k[r] = __builtin_bit_cast(double, (uint64_t)rh << 32 | rl);
-  }
-}
-template <int NPL>
-__device__ __forceinline__ void local_sort_stages(double (&k)[NPL], int size) {
-#pragma unroll
-  for (int stride = min(size, NPL) >> 1; stride > 0; stride >>= 1) {
-#pragma unroll
-    for (int r = 0; r < NPL; ++r) {
-      if ((r & stride) == 0) {
-        const int p = r | stride;
-        const bool up = size >= NPL || (r & size) == 0;
-        const double lo = fmin(k[r], k[p]), hi = fmax(k[r], k[p]);
-        k[r] = up ? lo : hi;
-        k[p] = up ? hi : lo;
-      }
-    }
-  }
-}
-// ascending; the result's element lane * NPL + r is in register r.  The phases that reach across lanes are a loop over one
-// copy of each stage (the unrolled network of a long segment does not fit the instruction cache).
-template <int NPL>
-__device__ __forceinline__ void wave_sort(double (&k)[NPL], int lane) {
-#pragma unroll
-  for (int size = 2; size < NPL; size <<= 1) local_sort_stages<NPL>(k, size);
-  double sign = 1.0;   // what the keys are multiplied with
-#pragma nounroll
-  for (int lanes = 1; lanes <= 64; lanes <<= 1) {   // runs of NPL * lanes keys
-    const double want = (lane & lanes) ? -1.0 : 1.0, change = want * sign;
-#pragma unroll
-    for (int r = 0; r < NPL; ++r) k[r] *= change;
-    sign = want;
-    switch (lanes) {   // strides from lanes / 2 lanes down to one
-      case 64: cross_lane_sort_stage<NPL, 32>(k, lane); [[fallthrough]];
-      case 32: cross_lane_sort_stage<NPL, 16>(k, lane); [[fallthrough]];
-      case 16: cross_lane_sort_stage<NPL, 8>(k, lane); [[fallthrough]];
-      case 8: cross_lane_sort_stage<NPL, 4>(k, lane); [[fallthrough]];
-      case 4: cross_lane_sort_stage<NPL, 2>(k, lane); [[fallthrough]];
-      case 2: cross_lane_sort_stage<NPL, 1>(k, lane); [[fallthrough]];
-      default: local_sort_stages<NPL>(k, NPL); break;
-    }
-  }
-}
-
 template <int NPL>
 __global__ __launch_bounds__(256) void segment_argsort_wave_kernel(const float* scores, int32_t* idx, int Sc, int S_pad, int seg, int n_units,
                                                                    int rows, int32_t* first_blk, int block_size) {
@@ -118,32 +51,8 @@ __global__ __launch_bounds__(256) void segment_argsort_wave_kernel(const float* 
   const float* src = scores + (int64_t)row * Sc + base;
   double k[NPL];
 #pragma unroll
-  for (int r = 0; r < NPL; ++r) {
-    const int i = 64 * r + lane;   // (where a key starts does not matter: its index goes with it)
-    const double none = __builtin_bit_cast(double, 0x3ff0000000000000ull | (uint64_t)0xffffffffu << 11 | (uint32_t)i);
-    k[r] = i < seg ? sort_key(src[i], (uint32_t)i) : none;
-  }
-  wave_sort<NPL>(k, lane);
-  const int at = lane * NPL;   // a segment is a multiple of the block size or not: the last lanes may hold padding
-  int32_t o[NPL];
-  int zero_at = -1;
-#pragma unroll
-  for (int r = 0; r < NPL; ++r) {
-    const uint32_t i = sort_key_index(k[r]);
-    zero_at = i == 0 ? at + r : zero_at;
-    o[r] = base + (int32_t)i;
-  }
-  if (first_blk && s == 0 && zero_at >= 0) first_blk[row] = zero_at / block_size;
-  if (NPL >= 4 && (seg & 3) == 0 && ((uintptr_t)out & 15) == 0) {
-    typedef __attribute__((ext_vector_type(4))) int32_t i32x4;
-#pragma unroll
-    for (int r = 0; r < NPL; r += 4)
-      if (at + r < seg) *reinterpret_cast<i32x4*>(out + at + r) = (i32x4){o[r], o[(r + 1) % NPL], o[(r + 2) % NPL], o[(r + 3) % NPL]};
-  } else {
-#pragma unroll
-    for (int r = 0; r < NPL; ++r)
-      if (at + r < seg) out[at + r] = o[r];
-  }
+  for (int r = 0; r < NPL; ++r) k[r] = sort_key_of<NPL>(src, 64 * r + lane, seg);   // (where a key starts does not matter: its index goes with it)
+  sort_and_store<NPL>(k, lane, seg, base, s, out, first_blk ? first_blk + row : nullptr, block_size);
 }
 
 }  // namespace

@@ -18,6 +18,9 @@ pytestmark = pytest.mark.gpu
     (2, 4, 4, 31 * 128, 256, 0.8, "strong_heavy", dict(key_pool_mode="max")),
     (1, 3, 1, 129, 128, 0.9, "uniform_heavy", {}),                   # two blocks, one candidate
     (1, 2, 2, 7 * 128 + 64, 384, 0.0, "local_window", {}),           # rows without candidates are selected too; ragged last block
+    # scoring passes that sort, and their neighbours: 768 and 792 segments, segments of two chunks and of four, a partial last segment
+    (1, 32, 8, 24 * 128, 128, 0.9, "strong_uniform", {}), (1, 33, 11, 24 * 128, 128, 0.9, "strong_uniform", {}),
+    (1, 4, 1, 4096 + 77, 256, "rows", "strong_heavy", {}), (1, 8, 2, 2048, 256, 0.9, "strong_heavy", {}), (2, 3, 3, 300, 128, 0.9, "uniform_heavy", {}),
     (1, 28, 4, 1000, 256, 1.0, "strong_heavy", dict(force_select_first_block=False)),   # sums that may never reach the threshold
 ])
 def test_short_passes(dev, B, Hq, Hkv, S, seg, thr, kind, kw):
