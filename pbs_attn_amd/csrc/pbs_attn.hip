@@ -68,12 +68,15 @@ struct AttnArgs {
   int cap;               // entries per list row (multiple of 8); 0: no lists in memory and no counters (see own_list)
   uint16_t* o;
   int BH, Hq, Hkv, S, nb, bps;
-  int span, n_items;  // query blocks of an item (two, or one: see item_span), items of a head
+  int span;           // query blocks of an item (two, or one: see item_span)
   uint32_t k_ss, v_ss;   // key / value row strides in elements (< 2^22)
   int xcd_start[9];   // work items (head-major, long rows first) of XCD x: [xcd_start[x], xcd_start[x + 1])
-  int deal;           // how tickets become items (see ticket_item)
-  int deal_heads;     // heads dealt together
-  uint32_t group_magic, heads_magic;   // quotients by deal_heads * n_items and by deal_heads: high word of a product
+  struct Deal {
+    int how;     // how tickets become items (see ticket_item)
+    int n;       // items of a head
+    int heads;   // heads dealt together
+    uint32_t group_magic, heads_magic;   // quotients by heads * n and by heads: high word of a product
+  } deal;
   int64_t q_sb, q_sh, q_ss, k_sb, k_sh, v_sb, v_sh, o_sb, o_sh, o_ss;
   float scale_log2;
 };
@@ -199,19 +202,19 @@ __global__ __launch_bounds__(MERGE_THREADS) void merge_pair_lists_kernel(const i
 // (Wave-uniform values: scalar arithmetic only.)
 constexpr int NO_ITEM = 1 << 28, DEAL_NONE = 0, DEAL_GROUPS = 1, DEAL_ALL = 2, DEAL_BY_LISTS = 3, DEAL_HEADS = 4;
 __device__ __forceinline__ int quotient(int r, int divisor, uint32_t magic) { return divisor == 1 ? r : (int)(((uint64_t)(uint32_t)r * magic) >> 32); }
-__device__ __forceinline__ int ticket_item(ArgsPtr a, int deal, int x, int begin, int end, int ticket) {
+__device__ __forceinline__ int ticket_item(const AttnArgs::Deal& d, int how, int x, int begin, int end, int ticket) {
   if (begin + ticket >= end) return NO_ITEM;
-  if (deal == DEAL_NONE) return begin + ticket;
-  const int n = a->n_items, m = a->deal_heads;
-  if (deal == DEAL_ALL) {
-    const int r = 8 * ticket + x, len = quotient(r, m, a->heads_magic);
+  if (how == DEAL_NONE) return begin + ticket;
+  const int n = d.n, m = d.heads;
+  if (how == DEAL_ALL) {
+    const int r = 8 * ticket + x, len = quotient(r, m, d.heads_magic);
     return (r - len * m) * n + len;
   }
-  const int group = quotient(ticket, m * n, a->group_magic) * (m * n), r = ticket - group;
+  const int group = quotient(ticket, m * n, d.group_magic) * (m * n), r = ticket - group;
   const int left = end - begin - group;   // items of this group of heads and those after it
   int heads = m, len;
   if (left >= m * n) {
-    len = quotient(r, m, a->heads_magic);
+    len = quotient(r, m, d.heads_magic);
   } else {   // the last DEAL_HEADS - 1 heads of a range and fewer
     heads = left >= 3 * n ? 3 : left >= 2 * n ? 2 : 1;
     len = heads == 3 ? quotient(r, 3, 0x55555556u) : r >> (heads - 1);
@@ -226,7 +229,7 @@ __device__ __forceinline__ int ticket_item(ArgsPtr a, int deal, int x, int begin
 // at the kernel's start, 2 us.)
 constexpr int SHORT_LIST = 40;
 __device__ __forceinline__ bool lists_are_short(ArgsPtr a) {
-  const int n = a->n_items, lane = lane_id_here();
+  const int n = a->deal.n, lane = lane_id_here();
   // one of every 64th part of the items, at another place in each: lists grow shorter towards a head's end (65 * 63 < 4096: never past the last)
   const int64_t item = ((int64_t)a->BH * n * (65 * lane)) >> 12;
   uint32_t tiles = a->plist[item * a->cap];
@@ -272,8 +275,13 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   // registers for the whole kernel.
 #define PBS_ARGS() ({ ArgsPtr p_ = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(); asm volatile("" : "+s"(p_)); p_; })
   ArgsPtr a0 = PBS_ARGS();
-  const int n_items = a0->n_items;
-  int deal = a0->deal;
+  auto deal_of = [](ArgsPtr p) __attribute__((always_inline)) {
+    return AttnArgs::Deal{p->deal.how, p->deal.n, p->deal.heads, p->deal.group_magic, p->deal.heads_magic};
+  };
+  AttnArgs::Deal d0 = deal_of(a0);
+  // (loaded together, ahead of the branches that use them: one round trip at the kernel's start)
+  asm volatile("" : "+s"(d0.how), "+s"(d0.n), "+s"(d0.heads), "+s"(d0.group_magic), "+s"(d0.heads_magic));
+  int deal = d0.how;
   if (deal == DEAL_BY_LISTS) deal = lists_are_short(a0) ? DEAL_GROUPS : DEAL_NONE;
   const int xcd = blockIdx.x & 7;
   int q_begin = a0->xcd_start[xcd], q_end = a0->xcd_start[xcd + 1];   // the range being served: this XCD's, later others'
@@ -306,7 +314,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       __syncthreads();   // everyone has read the previous ticket
       if (wave == 0 && lane_id_here() == 0) misc[4] = atomicAdd(as->queue + vic, 1);
       __syncthreads();
-      found = ticket_item(as, deal, vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
+      found = ticket_item(deal_of(as), deal, vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
       if (found < NO_ITEM) return true;
     }
     return false;
@@ -314,7 +322,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   // The first item: workgroup n of an XCD takes ticket n, without asking (the counters start behind these tickets); where the
   // range is shorter than that, an item of another one.
   if (threadIdx.x == 0) misc[1] = 0;
-  int cur = ticket_item(a0, deal, xcd, q_begin, q_end, (int)blockIdx.x >> 3);
+  int cur = ticket_item(d0, deal, xcd, q_begin, q_end, (int)blockIdx.x >> 3);
   if (PBS_UNLIKELY(cur == NO_ITEM)) {
     if (!claim_elsewhere()) return;
     cur = found;
@@ -404,7 +412,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   // has a workgroup of its own, so that nothing is left of the list kernel (counters, further items).
   auto own_list = [&](ArgsPtr ap, int item) __attribute__((always_inline)) {
     uint16_t* list = reinterpret_cast<uint16_t*>(smem + LDS_LIST);
-    const int bh = item / n_items, qb0 = ap->span * (n_items - 1 - (item - bh * n_items));
+    const int n_items = ap->deal.n, bh = item / n_items, qb0 = ap->span * (n_items - 1 - (item - bh * n_items));
     const bool second = ap->span == 2 && qb0 + 1 < ap->nb;
     const int n_own = second ? qb0 + 2 : qb0 + 1;
     for (int kb = (int)threadIdx.x; kb < n_own; kb += THREADS)
@@ -471,7 +479,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       if (wave == 0 && lane_id_here() == 0) misc[4] = claim;
     };
     auto adopt_next = [&]() __attribute__((always_inline)) {          // ... and after the barrier
-      nxt = ticket_item(PBS_ARGS(), deal, vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
+      nxt = ticket_item(deal_of(PBS_ARGS()), deal, vic, q_begin, q_end, __builtin_amdgcn_readfirstlane(misc[4]));
       has_nxt = nxt < NO_ITEM;
       if (has_nxt)
         stage_list_async(list_row(PBS_ARGS(), nxt), PBS_ARGS()->cap >> 3, LDS_LIST + (li ^ 1u) * LIST_BYTES, wave, wave * 64 + lane_id_here());
@@ -982,8 +990,7 @@ extern "C" int pbs_sparse_attn_fwd_optional_diagonal(const void* q, const void* 
 static int plan_ranges(AttnArgs& a) {
   // eight ranges of equal estimated work: item p of a head costs about p + 1 (causal length)
   a.span = item_span(a.BH, a.nb, a.bps);
-  a.n_items = items_of(a.nb, a.span);
-  const int64_t n = a.n_items;
+  const int64_t n = a.deal.n = items_of(a.nb, a.span);
   const double head_work = 0.5 * (double)n * (double)(n + 1);
   int max_items = 0;
   for (int x = 0; x <= 8; ++x) {
@@ -1003,22 +1010,22 @@ static int plan_ranges(AttnArgs& a) {
     a.xcd_start[x] = (int)start;
     if (x > 0) max_items = std::max(max_items, a.xcd_start[x] - a.xcd_start[x - 1]);
   }
-  // An item a workgroup: as they are numbered.  Few items a head: longest first (see ticket_item).  With more of them the head-by-head order
-  // balances well enough, and where attention is near-uniform it is faster by what an XCD's workgroups share of a head in L2: 32 / 8
+  // Few items a head: longest first (see ticket_item; also at an item a workgroup, since the workgroups start one after the other).  With
+  // more of them the head-by-head order balances well enough, and where attention is near-uniform it is faster by what an XCD's workgroups share of a head in L2: 32 / 8
   // heads x 16384 1616 against 1644 us, x 32768 5.78 against 6.00 ms; 16 / 16 x 22016 1427 against 1435.
   const int64_t total = (int64_t)a.BH * n;
-  const bool whole_heads = a.BH % 8 == 0, one_each = total <= 256;
-  a.deal = one_each ? DEAL_NONE : whole_heads ? (a.BH == 8 ? DEAL_NONE : n <= DEAL_ROW ? DEAL_GROUPS : DEAL_BY_LISTS) : total <= DEAL_ITEMS ? DEAL_ALL : DEAL_NONE;
-  a.deal_heads = !whole_heads ? a.BH : total <= 2 * 256 ? a.BH / 8 : DEAL_HEADS;
-  const int64_t group = a.deal_heads * n;
+  const bool whole_heads = a.BH % 8 == 0;
+  a.deal.how = whole_heads ? (a.BH == 8 ? DEAL_NONE : n <= DEAL_ROW ? DEAL_GROUPS : DEAL_BY_LISTS) : total <= DEAL_ITEMS ? DEAL_ALL : DEAL_NONE;
+  a.deal.heads = !whole_heads ? a.BH : total <= 2 * 256 ? a.BH / 8 : DEAL_HEADS;
+  const int64_t group = a.deal.heads * n;
   // (divisors of 1 are not used) quotients are exact below 2^32 / divisor
-  a.group_magic = (uint32_t)((1ull << 32) / group + 1);
-  a.heads_magic = (uint32_t)((1ull << 32) / a.deal_heads + 1);
-  if (total / 8 >= (1ll << 32) / group) a.deal = DEAL_NONE;
-  if (one_each || a.deal != DEAL_NONE) {
+  a.deal.group_magic = (uint32_t)((1ull << 32) / group + 1);
+  a.deal.heads_magic = (uint32_t)((1ull << 32) / a.deal.heads + 1);
+  if (total / 8 >= (1ll << 32) / group) a.deal.how = DEAL_NONE;
+  if (a.deal.how != DEAL_NONE) {
     max_items = 0;
     for (int x = 0; x <= 8; ++x) {
-      a.xcd_start[x] = !one_each && whole_heads ? (int)(x * total / 8) : (int)(x * (total / 8) + std::min<int64_t>(x, total % 8));   // (DEAL_ALL: items 8 t + x < total)
+      a.xcd_start[x] = whole_heads ? (int)(x * total / 8) : (int)(x * (total / 8) + std::min<int64_t>(x, total % 8));   // (DEAL_ALL: items 8 t + x < total)
       if (x > 0) max_items = std::max(max_items, a.xcd_start[x] - a.xcd_start[x - 1]);
     }
   }
@@ -1118,10 +1125,10 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
   }
   if (own_lists) {
     a.cap = 0;
-    if (a.deal == DEAL_BY_LISTS) a.deal = DEAL_NONE;
+    if (a.deal.how == DEAL_BY_LISTS) a.deal.how = DEAL_NONE;
   }
   else if (!lists_built)
-    hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * a.n_items)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
+    hipLaunchKernelGGL(merge_pair_lists_kernel, dim3((unsigned)(a.BH * a.deal.n)), dim3(MERGE_THREADS), 0, (hipStream_t)stream, csr_cols, csr_cnt,
                      (uint16_t*)((char*)workspace + 256), a.queue, a.nb, a.span, a.bps, a.cap, Hq, Hq / Hkv, (int)(n_wg / 8), own_block_needed);
   hipLaunchKernelGGL(sparse_attn_kernel, dim3((unsigned)n_wg), dim3(THREADS), LDS_TOTAL, (hipStream_t)stream, a);
   return pbs_check_launch("pbs_sparse_attn_fwd");
