@@ -14,6 +14,7 @@
 //     block visits) is zero are skipped; their perm_k / perm_vt tiles stay unwritten.
 // The pooled values of the two forms are the same bits: same loads, same order of additions.
 #include "pbs_lists.h"
+#include "pbs_pool.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 
 namespace {
@@ -179,87 +180,30 @@ __global__ __launch_bounds__(256) void gather_kv_kernel(GatherArgs a, TaskGroups
 }
 
 
-// Mean / max pooling of Q blocks (rows past S count as zeros, the divisor stays 128).
-__device__ __forceinline__ void pool_q_block(float (&pool)[16][D], const uint16_t* q, uint16_t* pooled, int Hq, int S, int nb,
-                                             int64_t q_sb, int64_t q_sh, int64_t q_ss, int pool_max, int qb, int bh) {
-  const int b = bh / Hq, h = bh % Hq;
-  const int rg = threadIdx.x >> 4, c = threadIdx.x & 15;
-  const uint16_t* src = q + b * q_sb + h * q_sh;
-  // all eight loads in flight before the first is used; rows past the end read the last row and count as zeros
-  u32x4 x[8];
-#pragma unroll
-  for (int pass = 0; pass < 8; ++pass) {
-    const int pos = qb * BS + pass * 16 + rg;
-    x[pass] = *reinterpret_cast<const u32x4*>(src + (int64_t)min(pos, S - 1) * q_ss + c * 8);
-  }
-#pragma unroll
-  for (int pass = 0; pass < 8; ++pass)
-    if (qb * BS + pass * 16 + rg >= S) x[pass] = (u32x4){0, 0, 0, 0};
-  float acc[8];
-  if (pool_max) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = -INFINITY;
-#pragma unroll
-    for (int pass = 0; pass < 8; ++pass)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[2 * e] = fmaxf(acc[2 * e], bf16_bits_to_f32(x[pass][e] & 0xffffu));
-        acc[2 * e + 1] = fmaxf(acc[2 * e + 1], bf16_bits_to_f32(x[pass][e] >> 16));
-      }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-#pragma unroll
-    for (int pass = 0; pass < 8; ++pass)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[2 * e] += bf16_bits_to_f32(x[pass][e] & 0xffffu);
-        acc[2 * e + 1] += bf16_bits_to_f32(x[pass][e] >> 16);
-      }
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) pool[rg][c * 8 + e] = acc[e];
-  __syncthreads();
-  if (threadIdx.x < D) {
-    float s = pool[0][threadIdx.x];
-    for (int r = 1; r < 16; ++r) s = pool_max ? fmaxf(s, pool[r][threadIdx.x]) : s + pool[r][threadIdx.x];
-    if (!pool_max) s = s / (float)BS;
-    pooled[((int64_t)bh * nb + qb) * D + threadIdx.x] = (uint16_t)f32_to_bf16_bits(s);
-  }
-}
-
-__global__ __launch_bounds__(256) void pool_q_kernel(const uint16_t* q, uint16_t* pooled, int Hq, int S, int nb,
-                                                     int64_t q_sb, int64_t q_sh, int64_t q_ss, int pool_max) {
+__global__ __launch_bounds__(256) void pool_q_kernel(PoolQ p) {
   __shared__ float pool[16][D];
-  pool_q_block(pool, q, pooled, Hq, S, nb, q_sb, q_sh, q_ss, pool_max, blockIdx.x, blockIdx.y);
+  pool_q_block(pool, p, blockIdx.x, blockIdx.y);
 }
 
 // Both poolings of the block estimate in one launch: the pooling of permuted key blocks waits on scattered 256-byte
 // rows, the pooling of query blocks streams Q from HBM; side by side each fills what the other leaves idle.  A task
 // group's key poolings come first, then the query poolings of the same heads and blocks.
-struct PoolQArgs {
-  const uint16_t* q;
-  uint16_t* pooled_q;
-  int64_t q_sb, q_sh, q_ss;
-  int pool_max;
-};
-
-__global__ __launch_bounds__(256) void pool_qk_kernel(GatherArgs a, PoolQArgs p, TaskGroups t) {
+__global__ __launch_bounds__(256) void pool_qk_kernel(GatherArgs a, PoolQ p, TaskGroups t) {
   __shared__ uint16_t vt[2];
   __shared__ float pool[16][D];
   int kind, bh, blk;
   if (!my_task(t, a.nb, kind, bh, blk)) return;
-  if (kind) pool_q_block(pool, p.q, p.pooled_q, a.Hq, a.S, a.nb, p.q_sb, p.q_sh, p.q_ss, p.pool_max, blk, bh);
+  if (kind) pool_q_block(pool, p, blk, bh);
   else gather_block<true>(a, vt, pool, blk, bh);
 }
 
 // Full gather and query pooling in one launch, for short passes.
-__global__ __launch_bounds__(256) void gather_pool_kernel(GatherArgs a, PoolQArgs p, TaskGroups t) {
+__global__ __launch_bounds__(256) void gather_pool_kernel(GatherArgs a, PoolQ p, TaskGroups t) {
   __shared__ uint16_t vt[BS * VT_PITCH];
   __shared__ float pool[16][D];
   int kind, bh, blk;
   if (!my_task(t, a.nb, kind, bh, blk)) return;
-  if (kind) pool_q_block(pool, p.q, p.pooled_q, a.Hq, a.S, a.nb, p.q_sb, p.q_sh, p.q_ss, p.pool_max, blk, bh);
+  if (kind) pool_q_block(pool, p, blk, bh);
   else gather_block<false>(a, vt, pool, blk, bh);
 }
 
@@ -281,9 +225,7 @@ int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const in
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.S = S; a.nb = (S + BS - 1) / BS;
   a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = k_ss; a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = v_ss;
   a.pool_max = key_pool_max;
-  PoolQArgs p;
-  p.q = (const uint16_t*)q; p.pooled_q = (uint16_t*)pooled_q; p.q_sb = q_sb; p.q_sh = q_sh; p.q_ss = q_ss;
-  p.pool_max = query_pool_max;
+  const PoolQ p = {(const uint16_t*)q, (uint16_t*)pooled_q, q_sb, q_sh, q_ss, query_pool_max, Hq, S, a.nb};
   const TaskGroups t = task_groups(B, Hq, Hkv, a.nb, 2);
   PBS_REQUIRE(t.grid.y <= 65535 && t.grid.z <= 65535, "pbs_gather_pool: too many heads or blocks");
   hipLaunchKernelGGL(gather_pool_kernel, t.grid, dim3(256), 0, (hipStream_t)stream, a, p, t);
@@ -356,9 +298,7 @@ int pbs_pool_blocks_launch(const void* q, const void* k, const int32_t* key_indi
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.S = S; a.nb = (S + BS - 1) / BS;
   a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = k_ss;
   a.pool_max = key_pool_max;
-  PoolQArgs p;
-  p.q = (const uint16_t*)q; p.pooled_q = (uint16_t*)pooled_q; p.q_sb = q_sb; p.q_sh = q_sh; p.q_ss = q_ss;
-  p.pool_max = query_pool_max;
+  const PoolQ p = {(const uint16_t*)q, (uint16_t*)pooled_q, q_sb, q_sh, q_ss, query_pool_max, Hq, S, a.nb};
   const TaskGroups t = task_groups(B, Hq, Hkv, a.nb, 2);
   PBS_REQUIRE(t.grid.y <= 65535 && t.grid.z <= 65535, "pbs_pool_blocks: too many heads or blocks");
   hipLaunchKernelGGL(pool_qk_kernel, t.grid, dim3(256), 0, (hipStream_t)stream, a, p, t);
@@ -373,7 +313,7 @@ extern "C" int pbs_pool_q(const void* q, void* pooled_q, int B, int Hq, int S, i
   PBS_REQUIRE(q_sb % 8 == 0 && q_sh % 8 == 0 && q_ss % 8 == 0 && ((uintptr_t)q % 16) == 0,
               "pbs_pool_q: rows must be 16-byte aligned");
   const int nb = (S + BS - 1) / BS;
-  hipLaunchKernelGGL(pool_q_kernel, dim3(nb, B * Hq), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)q,
-                     (uint16_t*)pooled_q, Hq, S, nb, q_sb, q_sh, q_ss, query_pool_max);
+  const PoolQ p = {(const uint16_t*)q, (uint16_t*)pooled_q, q_sb, q_sh, q_ss, query_pool_max, Hq, S, nb};
+  hipLaunchKernelGGL(pool_q_kernel, dim3(nb, B * Hq), dim3(256), 0, (hipStream_t)stream, p);
   return pbs_check_launch("pbs_pool_q");
 }

@@ -47,10 +47,18 @@ constexpr int PBS_ESTIMATE_SELECT_MAX_BLOCKS = 64;
 int pbs_estimate_select_pair_lists(const void* pooled_q, const void* pooled_k, Candidates rule, const float* threshold_per_row,
                                    float threshold, bool force_first, const int32_t* first_blk, int rows, int S, int head_dim, int block_size, int segment_size,
                                    uint8_t* block_needed, const PairLists& lists, void* stream);
+// A pooling of query blocks (pbs_pool_q): all of it is a workgroup of 256 threads per block, so that it can ride in another launch
+struct PoolQ {
+  const uint16_t* q;
+  uint16_t* pooled_q;
+  int64_t q_sb, q_sh, q_ss;
+  int pool_max, Hq, S, nb;   // nb 0: none
+};
 // pbs_segment_argsort; first_blk, if not null, receives per row the block of `block_size` that holds original key 0 (there has
-// to be a complete segment)
+// to be a complete segment).  `ride`: a query pooling in the same launch, of which the sort by waves alone can take one
 int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,
-                               int S_pad, int segment_size, void* stream);
+                               int S_pad, int segment_size, void* stream, const PoolQ& ride = {});
+bool pbs_segment_argsort_takes_ride(int segment_size);
 // pbs_score_keys and pbs_segment_argsort_launch in one: the final scoring pass of short sequences of short segments sorts
 bool pbs_score_sorts(int B, int Hq, int Hkv, int S, int segment_size);
 int pbs_score_sort_launch(const void* q, const void* k, int32_t* key_indices, int32_t* first_blk, int B, int Hq, int Hkv, int S, int S_pad,

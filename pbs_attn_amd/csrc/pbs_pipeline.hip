@@ -136,6 +136,8 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
     return pbs_sparse_attn_launch(q, w, w, k, v, nullptr, nullptr, false, out, B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb,
                                   q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale, nullptr,
                                   w + L.attn_ws, stream);
+  const bool is_short = !threshold_is_int_one && short_pass(rows, nb);
+  bool q_pooled = false;   // the query blocks' pooling is under way
   if (one_segment || nseg == 0 || (nseg == 1 && rem == 0)) {
     if ((rc = pbs_identity_indices((int32_t*)(w + L.idx), rows, s_pad, stream))) return rc;
   } else if (pbs_score_sorts(B, Hq, Hkv, S, segment_size)) {
@@ -144,10 +146,13 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
   } else {
     if ((rc = pbs_score_keys(q, k, (float*)(w + L.scores), B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh,
                              q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;
+    // the query pooling rides with the sort, which leaves the memory idle
+    const bool ride = !threshold_is_int_one && !is_short && pbs_segment_argsort_takes_ride(segment_size);
+    const PoolQ pooling = {(const uint16_t*)q, (uint16_t*)(w + L.pooled_q), q_sb, q_sh, q_ss, query_pool_max, Hq, S, nb};
     if ((rc = pbs_segment_argsort_launch((const float*)(w + L.scores), (int32_t*)(w + L.idx), (int32_t*)(w + L.select_ws), block_size,
-                                         rows, S, s_pad, segment_size, stream))) return rc;
+                                         rows, S, s_pad, segment_size, stream, ride ? pooling : PoolQ{}))) return rc;
+    q_pooled = ride;
   }
-  const bool is_short = !threshold_is_int_one && short_pass(rows, nb);
   // With a real threshold the permuted K / V are gathered AFTER the selection, and only the blocks some query
   // block visits: the estimate needs no more than the pooled permuted key blocks, which come straight from K.
   // (Short passes: see short_pass.)
@@ -162,9 +167,12 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
       if ((rc = pbs_gather_pool_launch(q, k, v, (const int32_t*)(w + L.idx), w + L.pooled_q, w + L.pooled_k, w + L.perm_k, w + L.perm_vt, B, Hq,
                                        Hkv, S, head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss,
                                        query_pool_max, key_pool_max, stream))) return rc;
+    } else if (q_pooled) {
+      if ((rc = pbs_pool_k_permuted(k, (const int32_t*)(w + L.idx), w + L.pooled_k, needed, B, Hq, Hkv, S, head_dim, block_size, k_sb, k_sh,
+                                    k_ss, key_pool_max, stream))) return rc;
     } else if ((rc = pbs_pool_blocks(q, k, (const int32_t*)(w + L.idx), w + L.pooled_q, w + L.pooled_k, needed, B, Hq, Hkv, S,
-                              head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, query_pool_max, key_pool_max,
-                              stream))) return rc;
+                                     head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, query_pool_max, key_pool_max,
+                                     stream))) return rc;
     if (is_short) {
       if ((rc = pbs_estimate_select_pair_lists(w + L.pooled_q, w + L.pooled_k, Candidates::EARLIER_SEGMENTS, threshold_per_row, threshold,
                                                force_select_first_block != 0, (const int32_t*)(w + L.select_ws), rows, S, head_dim,

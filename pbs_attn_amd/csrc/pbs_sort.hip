@@ -5,6 +5,7 @@
 // trailing partial segment and the padding up to a whole block keep identity order.
 // Segments of up to 2048 keys are sorted by one wave in registers, longer ones by a workgroup in LDS.
 #include "pbs_lists.h"
+#include "pbs_pool.h"
 #include "pbs_sort.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 #include <algorithm>
@@ -34,12 +35,23 @@ __global__ __launch_bounds__(256) void segment_argsort_kernel(const float* score
       if ((uint32_t)keys[i] == 0) first_blk[row] = i / block_size;
 }
 
+// The workgroups behind the first `sort_wgs` do the ride's pooling: the sort waits on its lanes and leaves the memory idle.
+// Whole pass, pooling with the key blocks -> here, us: 32 / 8 heads x 20000 in segments of 2048 671 -> 654, 16 / 16 x 60000 875 -> 868, 28 / 4 x
+// 13333 twice 778 -> 776.  (In the first pass of the split scoring, which leaves half of a CU free, it took more than it saved: 16 / 16 x
+// 60000 854 -> 880, 32 / 8 x 2048 88.7 -> 91.1.)
 template <int NPL>
 __global__ __launch_bounds__(256) void segment_argsort_wave_kernel(const float* scores, int32_t* idx, int Sc, int S_pad, int seg, int n_units,
-                                                                   int rows, int32_t* first_blk, int block_size) {
+                                                                   int rows, int32_t* first_blk, int block_size, int64_t sort_wgs, PoolQ ride) {
+  __shared__ float pool[16][POOL_D];
   const int lane = threadIdx.x & 63;
+  const int64_t wg = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  if (wg >= sort_wgs) {
+    const int64_t blk = wg - sort_wgs;
+    if (blk < (int64_t)rows * ride.nb) pool_q_block(pool, ride, (int)(blk % ride.nb), (int)(blk / ride.nb));
+    return;
+  }
   // a segment of a row, or a piece of its identity tail
-  const int64_t unit = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int64_t unit = wg * 4 + (threadIdx.x >> 6);
   const int row = (int)(unit / n_units), s = (int)(unit - (int64_t)row * n_units);
   if (row >= rows) return;
   const int base = s * seg;
@@ -57,8 +69,11 @@ __global__ __launch_bounds__(256) void segment_argsort_wave_kernel(const float* 
 
 }  // namespace
 
+bool pbs_segment_argsort_takes_ride(int segment_size) { return segment_size <= 2048; }
+
 int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,
-                               int S_pad, int segment_size, void* stream) {
+                               int S_pad, int segment_size, void* stream, const PoolQ& ride) {
+  PBS_REQUIRE(!ride.nb || pbs_segment_argsort_takes_ride(segment_size), "pbs_segment_argsort: no pooling with segments of %d", segment_size);
   PBS_REQUIRE(key_indices, "pbs_segment_argsort: null index pointer");
   PBS_REQUIRE(rows > 0 && S > 0 && S_pad >= S, "pbs_segment_argsort: bad shape rows=%d S=%d S_pad=%d", rows, S, S_pad);
   PBS_REQUIRE(segment_size > 0 && segment_size <= 8192, "pbs_segment_argsort: segment_size %d outside (0, 8192]", segment_size);
@@ -71,13 +86,13 @@ int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_
   if (segment_size <= 2048) {
     const int n_units = nseg + tail_blocks;
     // a launch holds fewer than 2^32 work-items along a dimension: rows of very many segments go on along y
-    const int64_t wgs = ((int64_t)rows * n_units + 3) / 4, gx = std::min<int64_t>(wgs, 1 << 23);
+    const int64_t sort_wgs = ((int64_t)rows * n_units + 3) / 4, wgs = sort_wgs + (int64_t)rows * ride.nb, gx = std::min<int64_t>(wgs, 1 << 23);
     const int64_t gy = (wgs + gx - 1) / gx;
     PBS_REQUIRE(gy <= 65535, "pbs_segment_argsort: launch too large");
     const dim3 grid((unsigned)gx, (unsigned)gy);
     auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, scores, key_indices, Sc, S_pad, segment_size, n_units, rows,
-                         first_blk, block_size);
+                         first_blk, block_size, sort_wgs, ride);
     };
     if (segment_size <= 128) launch(segment_argsort_wave_kernel<2>);
     else if (segment_size <= 256) launch(segment_argsort_wave_kernel<4>);
