@@ -20,6 +20,10 @@ constexpr int SHORT_PASS_BLOCKS = 2048, SHORT_PASS_ROW = PBS_ESTIMATE_SELECT_MAX
 bool short_pass(int rows, int nb) { return nb <= SHORT_PASS_ROW && rows * nb <= SHORT_PASS_BLOCKS; }
 
 
+// Sort with the query pooling + key pooling, against sort + both poolings, us: 32768 tokens, 32 / 8 heads 52 + 23 against 20 + 60; 13333 tokens twice
+// 51 + 19 against 13 + 57; 131072 tokens 208 + 91 against 36 + 247, where the key pooling alone has too little to do while it waits for its rows.
+constexpr int RIDE_BLOCKS = 16384;
+
 struct Layout {
   size_t scores, score_ws, idx, perm_k, perm_vt, pooled_k, pooled_q, probs, cols, cnt, needed, select_ws, attn_ws, total;
 };
@@ -146,8 +150,8 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
   } else {
     if ((rc = pbs_score_keys(q, k, (float*)(w + L.scores), B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh,
                              q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;
-    // the query pooling rides with the sort, which leaves the memory idle
-    const bool ride = !threshold_is_int_one && !is_short && pbs_segment_argsort_takes_ride(segment_size);
+    // the query pooling rides with the sort, which leaves the memory idle (see RIDE_BLOCKS)
+    const bool ride = !threshold_is_int_one && !is_short && rows * nb <= RIDE_BLOCKS && pbs_segment_argsort_takes_ride(segment_size);
     const PoolQ pooling = {(const uint16_t*)q, (uint16_t*)(w + L.pooled_q), q_sb, q_sh, q_ss, query_pool_max, Hq, S, nb};
     if ((rc = pbs_segment_argsort_launch((const float*)(w + L.scores), (int32_t*)(w + L.idx), (int32_t*)(w + L.select_ws), block_size,
                                          rows, S, s_pad, segment_size, stream, ride ? pooling : PoolQ{}))) return rc;
