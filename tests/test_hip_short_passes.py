@@ -1,5 +1,5 @@
 """GPU: short passes (rows of up to 64 blocks, up to 2048 blocks in all) take launches of their own for the gather with the pooling and for the
-estimate with the selection.  Against the stage-by-stage calls, bit for bit, at the edges of the rule and of their tiles."""
+estimate with the selection, scoring passes of short segments sort, and longer passes pool their query blocks in the sort's launch.  Against the stage-by-stage calls, bit for bit, at the edges of the rule and of their tiles."""
 import pytest
 import torch
 
@@ -21,6 +21,9 @@ pytestmark = pytest.mark.gpu
     # scoring passes that sort, and their neighbours: 768 and 792 segments, segments of two chunks and of four, a partial last segment
     (1, 32, 8, 24 * 128, 128, 0.9, "strong_uniform", {}), (1, 33, 11, 24 * 128, 128, 0.9, "strong_uniform", {}),
     (1, 4, 1, 4096 + 77, 256, "rows", "strong_heavy", {}), (1, 8, 2, 2048, 256, 0.9, "strong_heavy", {}), (2, 3, 3, 300, 128, 0.9, "uniform_heavy", {}),
+    # query poolings that ride with the sort: 16384 blocks, the last; one block a head more; segments too long for the sort by waves
+    (1, 64, 8, 32768, 1024, 0.9, "strong_heavy", {}), (1, 64, 8, 32769, 1024, 0.9, "strong_heavy", {}),
+    (1, 3, 1, 70 * 128 + 5, 2048, 0.9, "strong_uniform", dict(query_pool_mode="max")), (1, 3, 1, 9000, 4096, 0.9, "uniform_heavy", {}),
     (1, 28, 4, 1000, 256, 1.0, "strong_heavy", dict(force_select_first_block=False)),   # sums that may never reach the threshold
 ])
 def test_short_passes(dev, B, Hq, Hkv, S, seg, thr, kind, kw):
