@@ -337,6 +337,7 @@ def meanpooling_attn_fwd(q, k, v, threshold, force_select_first_block=True):
     q, k, v = _rows16(q), _rows16(k), _rows16(v)
     B, Hq, S, D = q.shape
     Hkv = k.shape[1]
+    assert k.shape == (B, Hkv, S, D) and v.shape == (B, Hkv, S, D)
     _, thr_rows, thr = _threshold_args(threshold, B, Hq, q.device)
     out = q.new_empty(B, Hq, S, D)
     ws_bytes = lib.pbs_meanpooling_attn_workspace_bytes(B, Hq, Hkv, S, D, BLOCK)

@@ -49,3 +49,11 @@ def test_single_call_refuses_what_it_cannot_take(dev):
     assert call(S=2048 * 128 + 1, size=1 << 40) == -1
     with pytest.raises(_lib.PbsHipError):
         MeanPooling_prefill(q.cpu(), q.cpu(), q.cpu())
+
+
+def test_single_call_refuses_mismatched_shapes(dev):
+    q = torch.zeros(2, 4, 256, 128, dtype=torch.bfloat16, device=dev)
+    k = q[:, :2]
+    for bad_k, bad_v in ((k, k[:, :, :128]), (k, k[:, :1]), (k, k[:1]), (k[:1], k), (k[..., :64], k)):
+        with pytest.raises(AssertionError):   # the stage-by-stage form's own host checks refuse the same
+            MeanPooling_prefill(q, bad_k, bad_v)
