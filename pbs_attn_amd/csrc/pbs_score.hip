@@ -337,7 +337,8 @@ int chunks_for(int Sc, int chunk_keys) { return (Sc + chunk_keys - 1) / chunk_ke
 //     idle, the two are equal (1193, 1196), hence the limit for groups with less than a quarter idle.
 // A short sequence's workgroups all run at once, three a CU: one more round costs more than the longer chunk (a stage of 64 keys 1.2 us a
 // pass).  Whole pass: 32 / 8 heads x 2048, 1024 workgroups of 64 keys -> 512 of 128, 93.9 -> 90.7 us; x 4096, 1024 of 128 -> 512 of 256,
-// 167.5 -> 165.8; 28 / 4 x 4096 153.3 -> 151.5; fewer than they have to be: 16 / 16 x 2048, 512 -> 256, 65.5 -> 69.4.
+// 167.5 -> 165.8; 28 / 4 x 4096 153.3 -> 151.5; fewer than they have to be: 16 / 16 x 2048, 512 -> 256, 65.5 -> 69.4.  More heads than
+// that do not run at once even with one chunk each: theirs stay short (and the doubling would have no end).
 constexpr int SPLIT_WORKGROUPS = 3 * 256;
 // The final pass sorts where a segment is at most two chunks long, so that a workgroup's serial part hardly grows, and its workgroups still
 // run at once.  Whole pass, sort kernel -> this: segments of 128, 32 / 8 heads x 512 45.3 -> 42.9 us, 28 / 4 x 1019 59.8 -> 56.7, 4 / 1 x
@@ -358,8 +359,9 @@ ScorePlan score_plan(int B, int Hq, int Hkv, int Sc) {
   const bool small = keys <= 3 << 16 && Sc <= 16384;
   const bool uneven = idle > 0 && heads >= 8 && (4 * idle >= slots || keys <= 1 << 20);
   const bool split = (small || uneven) && heads <= 65535;
+  const bool at_once = small && heads <= SPLIT_WORKGROUPS;
   if (split)
-    while (chunks_for(Sc, chunk) > SPLIT_MAX_CHUNKS || (small && chunks_for(Sc, chunk) * heads > SPLIT_WORKGROUPS)) chunk *= 2;
+    while (chunks_for(Sc, chunk) > SPLIT_MAX_CHUNKS || (at_once && chunks_for(Sc, chunk) * heads > SPLIT_WORKGROUPS)) chunk *= 2;
   return {split, small, chunk, chunks_for(Sc, chunk)};
 }
 

@@ -112,6 +112,7 @@ def test_segment_sort_of_more_work_items_than_one_grid_dimension_holds(dev):
 @pytest.mark.parametrize("B,Hq,Hkv,S,seg", [
     (1, 1, 1, 130, 128), (2, 7, 1, 1000, 128), (1, 4, 1, 2048, 128), (1, 4, 1, 2190, 128),   # 2 .. 32 chunks of 64, 17 of 128 keys
     (1, 12, 3, 16384, 128), (1, 12, 3, 16512, 128),   # the longest sequence of the split scoring, and one block more
+    (25, 32, 8, 200, 128), (12, 64, 8, 200, 128),     # 800 heads of one segment in two chunks; 768 in one
     (1, 8, 4, 26880, 256), (3, 5, 5, 1111, 256),      # groups that would leave waves idle: 27 chunks of 1024, and a ragged batch
 ])
 def test_key_scores_at_the_edges_of_the_split_form(dev, B, Hq, Hkv, S, seg):

@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
     # scoring passes that sort, and their neighbours: 768 and 792 segments, segments of two chunks and of four, a partial last segment
     (1, 32, 8, 24 * 128, 128, 0.9, "strong_uniform", {}), (1, 33, 11, 24 * 128, 128, 0.9, "strong_uniform", {}),
     (1, 4, 1, 4096 + 77, 256, "rows", "strong_heavy", {}), (1, 8, 2, 2048, 256, 0.9, "strong_heavy", {}), (2, 3, 3, 300, 128, 0.9, "uniform_heavy", {}),
+    (25, 32, 8, 200, 128, 0.9, "strong_uniform", {}),   # 800 heads of one segment: more than run at once, two chunks a head
     # query poolings that ride with the sort: 16384 blocks, the last; one block a head more; segments too long for the sort by waves
     (1, 64, 8, 32768, 1024, 0.9, "strong_heavy", {}), (1, 64, 8, 32769, 1024, 0.9, "strong_heavy", {}),
     (1, 3, 1, 70 * 128 + 5, 2048, 0.9, "strong_uniform", dict(query_pool_mode="max")), (1, 3, 1, 9000, 4096, 0.9, "uniform_heavy", {}),
