@@ -153,7 +153,9 @@ int pbs_block_mask_to_csr(const uint8_t* block_mask, int32_t* csr_cols, int32_t*
  * (a segment's permuted blocks hold the same keys as its original blocks).
  * out: (B, Hq, S, 128) bf16 with its own strides, original query order.
  * workspace: pbs_sparse_attn_workspace_bytes(B, Hq, S, segment_size) bytes of device memory, 256-byte
- * aligned (work counters and the merged visit list of every pair of query blocks, rewritten by each call).
+ * aligned (work counters and the merged visit list of every work item, one or two query blocks, rewritten by each
+ * call).  The size never falls as B, Hq, S or segment_size grow: a workspace for the largest call serves the smaller
+ * ones.
  * Two launches: the list merge, then one persistent workgroup per CU.
  * Replaces pbs_attn/src/kernels/permuted_block_sparse_attention.py:134-311
  * (launch at pbs_attn/src/pbs.py:220-246). */

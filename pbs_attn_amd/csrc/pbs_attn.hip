@@ -954,11 +954,15 @@ static int item_span(int rows, int nb, int bps) {
 }
 static int items_of(int nb, int span) { return (nb + span - 1) / span; }
 
-// workspace: 256 bytes of work counters, then one merged visit list per item
+// workspace: 256 bytes of work counters, then one merged visit list per item.  Room for the lists of every call of fewer heads, a shorter
+// sequence or a shorter segment as well, whose items may be single blocks: callers make one workspace for their largest call, and
+// pbs_sparse_attn_fwd is not told its size.
 
 extern "C" size_t pbs_sparse_attn_workspace_bytes(int B, int Hq, int S, int segment_size) {
-  const int64_t nb = (S + BS - 1) / BS, n_items = items_of((int)nb, item_span(B * Hq, (int)nb, segment_size / BS)), cap = list_cap((int)nb, segment_size / BS);
-  return 256 + (size_t)B * Hq * n_items * cap * 2;
+  const int64_t rows = (int64_t)B * Hq, nb = (S + BS - 1) / BS, cap = list_cap((int)nb, segment_size / BS);
+  static_assert(SINGLE_BLOCK_ITEMS <= SINGLE_FEW_HEADS, "the most single-block items of a launch");
+  const int64_t lists = std::max<int64_t>(rows * items_of((int)nb, 2), std::min<int64_t>(rows * nb, SINGLE_FEW_HEADS));
+  return 256 + (size_t)lists * cap * 2;
 }
 
 extern "C" int pbs_sparse_attn_fwd(const void* q, const void* perm_k, const void* perm_vt, const void* k, const void* v,

@@ -30,3 +30,35 @@ def test_scoring_chunks_of_more_heads_than_run_at_once():
     """One segment of 128 keys: up to 768 heads one chunk or two, so that all workgroups run at once; more heads never do, and keep two."""
     lib = _lib.load()
     assert [_chunks(lib, heads, 4, 200, 128) for heads in (384, 388, 768, 772, 800, 1536)] == [2, 1, 1, 2, 2, 2]
+
+
+LENGTHS = sorted({*range(1, 140), *range(140, 1100, 7), 384, 512, 513, 1024, 2047, 2048, 2049, 4095, 4096})   # in blocks
+HEADS = [1, 2, 3, 4, 5, 8, 15, 16, 17, 24, 28, 32, 33, 64, 96, 128, 129, 256, 384, 385, 512, 513, 1000, 4096]
+
+
+def _not_growing(sizes):
+    return [(a, b) for a, b in zip(sizes, sizes[1:]) if a[1] > b[1]]
+
+
+@pytest.mark.parametrize("segment", [128, 256, 384, 1024, 8192])
+def test_attention_workspace_grows_with_the_shape(segment):
+    """pbs_sparse_attn_fwd is not told how large its workspace is: one that was made for the longest sequence and the most heads
+    has to hold the lists of every smaller call too."""
+    lib = _lib.load()
+    size = lambda heads, blocks, tail=0, seg=segment: lib.pbs_sparse_attn_workspace_bytes(1, heads, blocks * 128 - tail, seg)
+    for heads in HEADS:
+        assert not _not_growing([(n, size(heads, n)) for n in LENGTHS]), heads
+        assert all(size(heads, n, 127) == size(heads, n) for n in LENGTHS)   # (whole blocks)
+    for n in LENGTHS:
+        assert not _not_growing([(heads, size(heads, n)) for heads in HEADS]), n
+        assert size(6, n) == lib.pbs_sparse_attn_workspace_bytes(3, 2, n * 128, segment)
+        assert not _not_growing([(seg, size(32, n, seg=seg)) for seg in (128, 256, 384, 1024, 8192, 65536)]), n
+
+
+def test_single_call_workspaces_grow_with_the_length():
+    """A sequence inside one segment needs the lists alone; the MeanPooling mode its pooled blocks, probabilities and lists."""
+    lib = _lib.load()
+    for heads in HEADS:
+        one_segment = [(n, lib.pbs_prefill_attn_workspace_bytes(1, heads, heads, n * 128, 128, 128, 511 * 128)) for n in LENGTHS if n <= 511]
+        assert not _not_growing(one_segment), heads
+        assert not _not_growing([(n, lib.pbs_meanpooling_attn_workspace_bytes(1, heads, heads, n * 128, 128, 128)) for n in LENGTHS]), heads
