@@ -30,7 +30,8 @@ const char* pbs_last_error(void);
 /* Key scoring: scores[b,h,k] = mean over the last 128 queries of
  * softmax_k(bf16(bf16(q.k) / sqrt(D))) over the keys of the complete segments.
  * scores: (B, Hq, Sc) float32, Sc = (S / segment_size) * segment_size.  Strides in elements, rows 16-byte
- * aligned, key row stride in [128, 2^28).
+ * aligned, key row stride in [128, 2^28).  The workspace size is this call's: a shorter sequence may be cut into
+ * more chunks and need more.
  * Replaces pbs_attn/src/permute_states.py:44-50. */
 size_t pbs_score_keys_workspace_bytes(int B, int Hq, int Hkv, int S, int segment_size);
 int pbs_score_keys(const void* q, const void* k, float* scores, int B, int Hq, int Hkv, int S, int head_dim,
@@ -193,8 +194,9 @@ int pbs_identity_indices(int32_t* key_indices, int rows, int S_pad, void* stream
 
 /* The whole path in one call: key scoring, segment sort, gather, estimation, selection and sparse
  * attention enqueued back to back on `stream`, intermediates in `workspace` (256-byte aligned,
- * pbs_prefill_attn_workspace_bytes).  S <= segment_size gives plain causal attention, as the
- * reference does.  Replaces pbs_attn/src/pbs.py:132-257 as a whole. */
+ * pbs_prefill_attn_workspace_bytes, which never falls as S grows: a workspace for the longest sequence serves the
+ * shorter ones).  S <= segment_size gives plain causal attention, as the reference does.
+ * Replaces pbs_attn/src/pbs.py:132-257 as a whole. */
 size_t pbs_prefill_attn_workspace_bytes(int B, int Hq, int Hkv, int S, int head_dim, int block_size,
                                         int segment_size);
 int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v, void* out, int B, int Hq, int Hkv, int S,

@@ -59,6 +59,8 @@ struct PoolQ {
 int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_t* first_blk, int block_size, int rows, int S,
                                int S_pad, int segment_size, void* stream, const PoolQ& ride = {});
 bool pbs_segment_argsort_takes_ride(int segment_size);
+// pbs_score_keys_workspace_bytes of this sequence or of any shorter one (which may be cut into more chunks), the largest
+size_t pbs_score_keys_workspace_bound(int B, int Hq, int Hkv, int S, int segment_size);
 // pbs_score_keys and pbs_segment_argsort_launch in one: the final scoring pass of short sequences of short segments sorts
 bool pbs_score_sorts(int B, int Hq, int Hkv, int S, int segment_size);
 int pbs_score_sort_launch(const void* q, const void* k, int32_t* key_indices, int32_t* first_blk, int B, int Hq, int Hkv, int S, int S_pad,

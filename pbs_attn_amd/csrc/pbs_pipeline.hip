@@ -40,7 +40,7 @@ Layout make_layout(int B, int Hq, int Hkv, int S, int D, int block_size, int seg
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t o = off; off = align256(off + (own_tiles_only ? 0 : bytes)); return o; };
   L.scores = take(rows * sc * 4);
-  L.score_ws = take(pbs_score_keys_workspace_bytes(B, Hq, Hkv, S, segment_size));
+  L.score_ws = take(pbs_score_keys_workspace_bound(B, Hq, Hkv, S, segment_size));
   L.idx = take(rows * s_pad * 4);
   L.perm_k = take(rows * s_pad * D * 2);
   L.perm_vt = take(rows * s_pad * D * 2);

@@ -11,6 +11,7 @@
 #include "pbs_lists.h"
 #include "pbs_sort.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -349,10 +350,12 @@ struct ScorePlan {
   bool split, small;
   int chunk_keys, nchunk;
 };
+int longest_chunk(bool grouped) { return grouped ? KEYS_PER_WG : KEYS_PER_WG / 4; }
+int64_t workgroups_wanted(bool grouped) { return grouped ? 512 : 2048; }
 ScorePlan score_plan(int B, int Hq, int Hkv, int Sc) {
   const bool grouped = Hq / Hkv > 1;
-  int chunk = grouped ? KEYS_PER_WG : KEYS_PER_WG / 4;
-  const int64_t want = grouped ? 512 : 2048;
+  int chunk = longest_chunk(grouped);
+  const int64_t want = workgroups_wanted(grouped);
   while (chunk > 64 && (int64_t)chunks_for(Sc, chunk) * B * Hkv < want) chunk /= 2;
   const int64_t heads = (int64_t)B * Hq, keys = heads * Sc;
   const int G = Hq / Hkv, slots = (G + 3) / 4 * 4, idle = slots - G;
@@ -372,6 +375,16 @@ extern "C" size_t pbs_score_keys_workspace_bytes(int B, int Hq, int Hkv, int S, 
   const int Sc = (S / segment_size) * segment_size;
   if (Sc == 0) return 0;
   return (size_t)B * Hq * ((size_t)score_plan(B, Hq, Hkv, Sc).nchunk + 1) * NQ * 2 * sizeof(float);
+}
+
+size_t pbs_score_keys_workspace_bound(int B, int Hq, int Hkv, int S, int segment_size) {
+  const int Sc = (S / segment_size) * segment_size;
+  if (Sc == 0) return 0;
+  // A chunk is the longest one, or half of one that gave fewer workgroups than wanted, or longer (score_plan); 64 keys and more.
+  const bool grouped = Hq / Hkv > 1;
+  const int64_t halved = 2 * ((workgroups_wanted(grouped) - 1) / ((int64_t)B * Hkv));
+  const int64_t chunks = std::min<int64_t>(chunks_for(Sc, 64), std::max<int64_t>(chunks_for(Sc, longest_chunk(grouped)), halved));
+  return (size_t)B * Hq * ((size_t)chunks + 1) * NQ * 2 * sizeof(float);
 }
 
 namespace {

@@ -62,3 +62,13 @@ def test_single_call_workspaces_grow_with_the_length():
         one_segment = [(n, lib.pbs_prefill_attn_workspace_bytes(1, heads, heads, n * 128, 128, 128, 511 * 128)) for n in LENGTHS if n <= 511]
         assert not _not_growing(one_segment), heads
         assert not _not_growing([(n, lib.pbs_meanpooling_attn_workspace_bytes(1, heads, heads, n * 128, 128, 128)) for n in LENGTHS]), heads
+
+
+@pytest.mark.parametrize("B,Hq,Hkv", [(1, 1, 1), (1, 4, 1), (1, 8, 2), (1, 12, 3), (1, 16, 16), (1, 28, 4), (1, 32, 8), (2, 32, 8), (4, 28, 4),
+                                      (25, 32, 8), (8, 128, 8)])
+def test_prefill_workspace_grows_with_the_length(B, Hq, Hkv):
+    """The space for the chunk partials of the key scoring covers those of a shorter sequence, which may be cut into more chunks."""
+    lib = _lib.load()
+    lengths = sorted({*range(1, 6000, 61), *range(6000, 70000, 997), *range(128, 6016, 128), *range(6016, 70000, 896), 131072, 262144})
+    for segment in (128, 256, 384, 512, 1024, 4096, 65408):
+        assert not _not_growing([(S, lib.pbs_prefill_attn_workspace_bytes(B, Hq, Hkv, S, 128, 128, segment)) for S in lengths]), segment
