@@ -36,6 +36,7 @@ def MeanPooling_prefill(
     _, num_kv_heads, kv_len, _ = key_states.shape
     assert num_q_heads % num_kv_heads == 0
     assert q_len == kv_len, "Only support prefilling for now, q_len: {}, kv_len: {}".format(q_len, kv_len)
+    assert key_states.shape == (batch_size, num_kv_heads, kv_len, head_dim) and value_states.shape == key_states.shape
     assert causal
     # MeanPooling.py:50 hands the threshold to select_blocks as it is: there is no "int 1 = everything" rule here
     thr = threshold if isinstance(threshold, torch.Tensor) else float(threshold)

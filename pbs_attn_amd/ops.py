@@ -293,14 +293,18 @@ def prefill_attn_fwd(q, k, v, block_size, segment_size, threshold, force_select_
                      query_pool_mode="mean", key_pool_mode="mean", softmax_scale=None):
     """Every stage in one library call (pbs.py:132-257): one workspace allocation, one
     host round trip.  Returns (B, Hq, S, D)."""
+    B, Hq, S, D = q.shape
+    kv_shape = k.shape
+    Hkv = kv_shape[1]
+    # (the kernels take K's and V's sizes from here: smaller ones would be read past their end)
+    assert kv_shape == (B, Hkv, S, D) and v.shape == kv_shape
     _check_bf16_cuda(q, k, v)
     for mode, what in ((query_pool_mode, "query_pool_mode"), (key_pool_mode, "key_pool_mode")):
         if mode not in ("mean", "max"):
             raise ValueError(f"Invalid {what}: {mode}")
     lib = _lib.load()
     q, k, v = _rows16(q), _rows16(k), _rows16(v)
-    B, Hq, S, D = q.shape
-    Hkv, device = k.shape[1], q.device
+    device = q.device
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
     is_int_one, thr_rows, thr = _threshold_args(threshold, B, Hq, device)

@@ -179,6 +179,7 @@ def permuted_block_sparse_attn_fwd(
         return ops.prefill_attn_fwd(query_states, key_states, value_states, block_size, segment_size, threshold,
                                     force_select_first_block, query_pool_mode, key_pool_mode)
 
+    assert key_states.shape == (batch_size, num_kv_heads, q_len, head_dim) and value_states.shape == key_states.shape
     one_segment = q_len <= segment_size
     if one_segment:
         # pbs.py:175-182: plain causal attention.  Same kernel, identity order, every causal block visited: one

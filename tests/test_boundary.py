@@ -190,6 +190,38 @@ def test_product_path_has_no_cpu_fallback():
         permuted_block_sparse_attn_fwd(q, q, q, 128, 256, 0.9, True)
 
 
+@pytest.mark.parametrize("S", [77, 256, 700])   # inside one segment; several
+@pytest.mark.parametrize("staged", [False, True])
+def test_mismatched_key_and_value_shapes_are_refused_before_anything_else(S, staged):
+    """The kernels take K's and V's sizes from Q: a smaller K or V would be read past its end."""
+    from pbs_attn_amd import ops
+    from pbs_attn_amd import pbs as P
+    from pbs_attn_amd._lib import PbsHipError
+    from pbs_attn_amd.meanpooling import MeanPooling_prefill
+
+    class Timer:
+        def mark(self, name):
+            pass
+
+    q = torch.zeros((2, 4, S, 128), dtype=torch.bfloat16)
+    k = q[:, :2]
+    bad = [(k[:1], k), (k, k[:1]), (k, k[:, :1]), (k[:, :1], k), (k, k[:, :, :S - 1]), (k, k[..., :64]), (k[..., :64], k), (k[..., :64], k[..., :64])]
+    P.stage_timer = Timer() if staged else None
+    try:
+        for bad_k, bad_v in bad:
+            with pytest.raises(AssertionError):
+                P.permuted_block_sparse_attn_fwd(q, bad_k, bad_v, 128, 256, 0.9, True)
+        with pytest.raises(PbsHipError, match="GPU"):   # (shapes that fit get as far as the check of the device)
+            P.permuted_block_sparse_attn_fwd(q, k, k, 128, 256, 0.9, True)
+    finally:
+        P.stage_timer = None
+    for bad_k, bad_v in [*bad, (k[:, :, :S - 1], k)]:
+        with pytest.raises(AssertionError):
+            ops.prefill_attn_fwd(q, bad_k, bad_v, 128, 256, 0.9)
+        with pytest.raises(AssertionError):
+            MeanPooling_prefill(q, bad_k, bad_v, force_select_current_block=not staged)   # (without: stage by stage)
+
+
 # ------------------------------------------------------------------ patcher on tiny models
 def _tiny(kind, layers=2):
     from transformers import LlamaConfig, LlamaForCausalLM, Qwen2Config, Qwen2ForCausalLM
