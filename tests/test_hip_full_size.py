@@ -8,7 +8,7 @@ import torch.nn.functional as F
 from pbs_attn_amd import ops
 from pbs_attn_amd import pbs as P
 from pbs_attn_amd.synth import make_qkv
-from tests.util import assert_attn_close
+from tests.util import assert_attn_close, heads_for_items
 
 pytestmark = pytest.mark.gpu
 
@@ -118,15 +118,17 @@ def test_ones_value_and_linearity_at_32k(dev):
     assert torch.equal(fwd(v), fwd(v))
 
 
+@pytest.mark.parametrize("pairs", [False, True])   # work items of one query block, of two
 @pytest.mark.parametrize("gain,what", [(3.0, "lazy rescale"), (12.0, "rescale by many octaves"), (60.0, "overflow -> redo without speculation")])
-def test_late_dominant_keys_take_the_rare_paths(dev, gain, what):
+def test_late_dominant_keys_take_the_rare_paths(dev, gain, what, pairs):
     # keys far stronger than everything seen before them show up late in the visit list: the fast
     # tiles' fixed reference maximum must be moved (exactly), or the row redone when exp2 overflowed
     S, seg = 4096, 256
+    H = heads_for_items(dev, pairs, S, seg, few=2)
     g = torch.Generator().manual_seed(7)
-    q = torch.randn((1, 2, S, 128), generator=g)
-    k = torch.randn((1, 2, S, 128), generator=g)
-    v = torch.randn((1, 2, S, 128), generator=g)
+    q = torch.randn((1, H, S, 128), generator=g)
+    k = torch.randn((1, H, S, 128), generator=g)
+    v = torch.randn((1, H, S, 128), generator=g)
     u = torch.zeros(128)
     u[0] = 1.0
     q = q + 4.0 * u
@@ -139,22 +141,24 @@ def test_late_dominant_keys_take_the_rare_paths(dev, gain, what):
     assert_attn_close(out, ref, what=what)
 
 
+@pytest.mark.parametrize("pairs", [False, True])
 @pytest.mark.parametrize("gain,what", [(3.0, "lazy rescale inside the first tile"), (12.0, "many octaves inside the first tile"),
                                        (60.0, "overflow inside the first tile -> redo")])
-def test_first_tile_reference_from_its_first_keys(dev, gain, what):
+def test_first_tile_reference_from_its_first_keys(dev, gain, what, pairs):
     # the first tile of a row takes its reference maximum from its first 32 keys only; keys 40..127 of
     # that tile are far stronger here (identity key order is forced through injected scores)
     S, seg = 2048, 256
+    H = heads_for_items(dev, pairs, S, seg, few=2)
     g = torch.Generator().manual_seed(11)
-    q = torch.randn((1, 2, S, 128), generator=g)
-    k = torch.randn((1, 2, S, 128), generator=g)
-    v = torch.randn((1, 2, S, 128), generator=g)
+    q = torch.randn((1, H, S, 128), generator=g)
+    k = torch.randn((1, H, S, 128), generator=g)
+    v = torch.randn((1, H, S, 128), generator=g)
     u = torch.zeros(128)
     u[3] = 1.0
     q = q + 4.0 * u
     k[:, :, 40:128] += gain * 4.0 * u
     q, k, v = (t.to(torch.bfloat16).to(dev) for t in (q, k, v))
-    scores = -torch.arange(S, device=dev, dtype=torch.float32).view(1, 1, S).expand(1, 2, S).contiguous()
+    scores = -torch.arange(S, device=dev, dtype=torch.float32).view(1, 1, S).expand(1, H, S).contiguous()
     perm = P.apply_permutation(q, k, v, 128, seg, scores=scores)
     assert torch.equal(perm.key_indices[0, 0, :S].cpu(), torch.arange(S, dtype=torch.int32))
     sel = P.permuted_block_selection(q, perm, 128, seg, 1, want_masks=False)

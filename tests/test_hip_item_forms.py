@@ -28,12 +28,15 @@ def test_the_same_heads_in_launches_of_other_sizes(dev, Hq, Hkv, S, seg, thr, re
     kw = dict(query_pool_mode=pool, key_pool_mode=pool)
     whole = P.permuted_block_sparse_attn_fwd(q.repeat(reps, 1, 1, 1), k.repeat(reps, 1, 1, 1), v.repeat(reps, 1, 1, 1), 128, seg, thr, True, **kw)
     alone = P.permuted_block_sparse_attn_fwd(q, k, v, 128, seg, thr, True, **kw)
-    g = Hq // Hkv
-    one = P.permuted_block_sparse_attn_fwd(q[:, :g], k[:, :1], v[:, :1], 128, seg, thr, True, **kw)
     assert torch.equal(whole, alone.expand(reps, -1, -1, -1))
-    # (scores of other head counts come from another split of the keys: their sums may differ in the last bit, and with them the order)
-    if Hkv > 1 and thr == 0.0:
-        assert torch.equal(alone[:, :g], one)
+    # one KV head's query heads by themselves, on the key order and the visit lists of all of them (scores of other head counts come from
+    # another split of the keys: their sums may differ in the last bit, and with them the order)
+    perm = P.apply_permutation(q, k, v, 128, seg, pool)
+    sel = P.permuted_block_selection(q, perm, 128, seg, thr, want_masks=False, **kw)
+    together = perm.attention(q, sel["csr_cols"], sel["csr_cnt"], seg)
+    g = Hq // Hkv
+    part = P.PermutedKV(*(x[:, :g].contiguous() for x in (perm.key_indices, perm.perm_k, perm.perm_vt, perm.pooled_k)), S, k[:, :1], v[:, :1])
+    assert torch.equal(part.attention(q[:, :g], *(sel[x][:, :g].contiguous() for x in ("csr_cols", "csr_cnt")), seg), together[:, :g])
 
 
 @pytest.mark.parametrize("Hq,Hkv,S,reps", [(32, 8, 77, 1), (16, 4, 2048, 3), (32, 8, 295, 4), (32, 8, 1536, 2), (32, 8, 1021, 4), (8, 8, 4096 - 1, 3), (24, 8, 1400, 1), (3, 1, 128, 40), (1, 1, 511 * 128, 2), (28, 4, 1500, 2), (9, 3, 40 * 128 - 1, 2)])

@@ -6,7 +6,7 @@ import torch
 from oracle import pbs_oracle as O
 from pbs_attn_amd import compat, ops
 from pbs_attn_amd.meanpooling import MeanPooling_prefill
-from tests.util import assert_attn_close, expand_kv, small_case
+from tests.util import assert_attn_close, blocks_of_an_item, expand_kv, small_case
 
 pytestmark = pytest.mark.gpu
 
@@ -61,11 +61,14 @@ def test_meanpooling_through_the_factory_and_patch(dev):
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,S,thr,ff", [(1, 4, 2, 2048, 0.3, True), (2, 2, 2, 1000, 0.5, True), (1, 7, 1, 1536, 0.2, False),
-                                               (1, 2, 2, 1280, 0.9, True)])
+                                               (1, 2, 2, 1280, 0.9, True),
+                                               # launches in pairs of query blocks (the ones above: single ones)
+                                               (4, 33, 11, 500, 0.3, True), (4, 27, 9, 600, 0.2, False), (1, 33, 33, 2048, 0.3, True)])
 def test_meanpooling_with_an_optional_diagonal_block(dev, B, Hq, Hkv, S, thr, ff):
     """force_select_current_block=False (MeanPooling.py:54-58 skipped): a query block attends to its diagonal block
     only where the threshold selected it.  Masks bit-exact on the oracle's block probabilities, output against dense
     attention on that mask; low thresholds so that many diagonals are in fact dropped."""
+    assert blocks_of_an_item(dev, B * Hq, S, 128) == (2 if Hq >= 27 else 1)
     q, k, v = small_case(B, Hq, Hkv, S, seed=S + Hq + 1)
     ke, ve = expand_kv(q, k), expand_kv(q, v)
     ref_out, mid = O.meanpooling_prefill(q, ke, ve, 128, 1024, thr, True, ff, False, return_intermediates=True)
@@ -124,12 +127,16 @@ def test_stage_adapters_with_the_reference_signatures(dev):
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,S,thr", [(1, 4, 2, 2048, 1.5), (2, 2, 2, 1000, 1.0), (1, 3, 1, 1536, 1.0), (1, 2, 2, 128, 2.0),
-                                            (1, 1, 1, 4096, 1.5)])
+                                            (1, 1, 1, 4096, 1.5),
+                                            # launches in pairs of query blocks (the ones above: single ones)
+                                            (4, 33, 11, 500, 1.5), (4, 27, 9, 600, 1.0), (1, 33, 33, 2048, 1.0)])
 def test_query_blocks_that_select_nothing_give_zeros(dev, B, Hq, Hkv, S, thr):
     """force_select_first_block=False and force_select_current_block=False with a threshold the running sum never
     reaches (above 1, or 1.0 against a float32 sum that tops out below it): select_blocks picks nothing for such a
     row (utils.py:74-84) and the attention gives zeros for it (kernels/...:340-343).  Whole launches without a single
     tile, pairs of query blocks where one or both visit nothing, and rows that do reach the threshold, side by side."""
+    if S > 128:
+        assert blocks_of_an_item(dev, B * Hq, S, 128) == (2 if Hq >= 27 else 1)
     q, k, v = small_case(B, Hq, Hkv, S, seed=S + Hq + 5)
     ke, ve = expand_kv(q, k), expand_kv(q, v)
     ref_out, mid = O.meanpooling_prefill(q, ke, ve, 128, 1024, thr, True, False, False, return_intermediates=True)

@@ -5,7 +5,7 @@ import torch
 
 from pbs_attn_amd import ops
 from pbs_attn_amd import pbs as P
-from tests.util import small_case
+from tests.util import heads_for_items, small_case
 
 pytestmark = pytest.mark.gpu
 
@@ -52,6 +52,7 @@ def _check(dev, Hq, S, seg, token, bad_k, bad_v, seed, scale=1):
         assert torch.isnan(got[0][sees & (rows >= token)]).all()
 
 
+@pytest.mark.parametrize("pairs", [False, True])   # work items of one query block, of two
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
 @pytest.mark.parametrize("S,seg,token", [
     (128, 128, 127), (128, 128, 33), (77, 128, 64),                  # one diagonal tile
@@ -59,10 +60,11 @@ def _check(dev, Hq, S, seg, token, bad_k, bad_v, seed, scale=1):
     (896, 256, 800),                                                 # a pair of one block
     (1024, 128, 991), (1024, 384, 1000),                             # segments of an odd number of blocks
 ])
-def test_later_keys_of_the_diagonal_block(dev, S, seg, token, bad):
-    _check(dev, 3, S, seg, token, bad, None, S + token)
+def test_later_keys_of_the_diagonal_block(dev, S, seg, token, bad, pairs):
+    _check(dev, heads_for_items(dev, pairs, S, seg), S, seg, token, bad, None, S + token)
 
 
+@pytest.mark.parametrize("pairs", [False, True])
 @pytest.mark.parametrize("scale", [1, 20])   # 20: exponents that overflow, the item is repeated
 @pytest.mark.parametrize("bad_k,bad_v", [(float("nan"), None), (float("inf"), None), (None, float("nan")), (None, float("inf"))])
 @pytest.mark.parametrize("S,seg,token", [
@@ -70,9 +72,9 @@ def test_later_keys_of_the_diagonal_block(dev, S, seg, token, bad):
     (1100, 384, 300),                   # the first block's own segment ends inside the pair; a last pair of one block
     (2048, 384, 130),                   # ... a tile before its diagonal
 ])
-def test_blocks_that_did_not_select_the_token(dev, S, seg, token, bad_k, bad_v, scale):
-    seed = S + seg
-    mask = _random_lists(3, (S + 127) // 128, seg // 128, seed)[0][..., token // 128]
+def test_blocks_that_did_not_select_the_token(dev, S, seg, token, bad_k, bad_v, scale, pairs):
+    seed, heads = S + seg, heads_for_items(dev, pairs, S, seg)
+    mask = _random_lists(heads, (S + 127) // 128, seg // 128, seed)[0][..., token // 128]
     first, second = mask[..., :-1:2], mask[..., 1::2]
     assert (first & ~second).any() and (second & ~first).any()
-    _check(dev, 3, S, seg, token, bad_k, bad_v, seed, scale)
+    _check(dev, heads, S, seg, token, bad_k, bad_v, seed, scale)

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from pbs_attn_amd import pbs as P
-from tests.util import small_case
+from tests.util import blocks_of_an_item, small_case
 
 pytestmark = pytest.mark.gpu
 
@@ -42,10 +42,13 @@ def test_routes_without_a_selection(dev, B, Hq, Hkv, S, seg, thr):
     (1, 32, 8, 77, 1), (3, 5, 5, 700, 1), (1, 28, 4, 1000, 1), (1, 32, 8, 2048, 1),   # an item or less per workgroup
     (1, 33, 3, 2048, 1), (1, 64, 8, 1100, 1),                                         # more items: the list kernel
     (1, 4, 2, 900, 20), (1, 2, 1, 2048, 20),   # exponents that overflow: the item is repeated from the same list
+    (3, 16, 4, 1100, 20), (8, 16, 4, 900, 20),   # the same in pairs of query blocks: 240 items, 512 (the list kernel)
 ])
 def test_one_segment_with_lists_formed_by_the_attention_kernel(dev, B, Hq, Hkv, S, scale):
     q, k, v = (x.to(dev) for x in small_case(B, Hq, Hkv, S, seed=S))
     q, k = q * scale, k * scale
+    if scale > 1:
+        assert blocks_of_an_item(dev, B * Hq, S, (S + 127) // 128 * 128) == (1 if B == 1 else 2)
     single = P.permuted_block_sparse_attn_fwd(q, k, v, 128, 2048, 0.9, True)
     P.stage_timer = _NullTimer()
     try:

@@ -1,15 +1,15 @@
 """GPU: the attention kernel's work distribution (one persistent workgroup per CU, items claimed from per-XCD
 counters, other XCDs' items taken at the end, the next item's list / queries / first tiles requested during the
 current item).  Shapes chosen for the corners of that machinery: items of one and two tiles (their look-ahead
-steps run after the tile loop), an odd number of query blocks (the last item has one query block), fewer items
-than workgroups, head counts that leave XCD ranges uneven, many short items per workgroup."""
+steps run after the tile loop), pairs of an odd number of query blocks (the last item has one query block), fewer items
+than workgroups, head counts that leave XCD ranges uneven, several items per workgroup."""
 import math
 
 import pytest
 import torch
 
 from pbs_attn_amd import pbs as P
-from tests.util import assert_attn_close, small_case
+from tests.util import assert_attn_close, blocks_of_an_item, small_case
 
 pytestmark = pytest.mark.gpu
 
@@ -32,17 +32,21 @@ def test_short_sequences_every_block_selected(dev, S, seg):
     assert_attn_close(out, _dense_causal(qd, kd, vd), what=f"S={S} seg={seg}")
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,seg,thr", [
-    (3, 5, 1, 640, 256, 0.5),        # 45 items of 1-5 tiles: fewer items than workgroups
-    (1, 3, 3, 8192, 1024, 0.9),      # 96 items in eight uneven ranges
-    (2, 7, 1, 4096 + 77, 512, 0.8),  # ragged length, odd head count
-    (4, 8, 2, 2048, 256, 0.3),       # 256 short items
-    (1, 1, 1, 16384 + 128, 256, 0.9),  # one head, odd block count: the last item is a single query block
-    (1, 32, 8, 4096, 256, 0.9),      # few items per workgroup, 4 whole heads per range: tickets handed out pair-major
-    (2, 8, 8, 2048 + 300, 512, 0.7),   # same with 2 heads per range, ragged length, odd block count (160 items)
-    (1, 8, 2, 1024, 256, 0.9),       # one head per range: pair-major is head-major
+@pytest.mark.parametrize("B,Hq,Hkv,S,seg,thr,span", [   # span: query blocks of an item
+    (3, 5, 1, 640, 256, 0.5, 1),        # 75 items of 1-5 tiles: fewer items than workgroups
+    (1, 3, 3, 8192, 1024, 0.9, 1),      # 192 items dealt over three heads
+    (2, 7, 1, 4096 + 77, 512, 0.8, 1),  # 462 items, ragged length, odd head count
+    (4, 8, 2, 2048, 256, 0.3, 2),       # 256 short items, four heads per range
+    (1, 1, 1, 16384 + 128, 256, 0.9, 1),  # 129 items of one head
+    (1, 32, 8, 4096, 256, 0.9, 2),      # 512 items, two a workgroup; four whole heads per range, dealt together
+    (2, 8, 8, 2048 + 300, 512, 0.7, 1),   # 304 items, two heads per range, ragged length
+    (1, 8, 2, 1024, 256, 0.9, 1),       # one head per range
+    (5, 7, 1, 2048 + 52, 256, 0.7, 2),  # 315 items of 35 heads dealt over all of them; odd block count: a head's last item is one query block
+    (9, 8, 2, 1000, 384, 0.5, 2),       # 288 items, nine whole heads per range
+    (1, 4, 1, 16384 + 128, 1024, 0.9, 2),   # 260 items of four heads, odd block count
 ])
-def test_work_distribution_shapes_against_dense_attention_on_the_mask(dev, B, Hq, Hkv, S, seg, thr):
+def test_work_distribution_shapes_against_dense_attention_on_the_mask(dev, B, Hq, Hkv, S, seg, thr, span):
+    assert blocks_of_an_item(dev, B * Hq, S, seg) == span
     q, k, v = small_case(B, Hq, Hkv, S, kind="strong_heavy", seed=B * 100 + Hq)
     qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
     out = P.permuted_block_sparse_attn_fwd(qd, kd, vd, 128, seg, thr, True)
