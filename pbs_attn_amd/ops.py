@@ -31,6 +31,16 @@ def _rows16(t: torch.Tensor) -> torch.Tensor:
     return t
 
 
+def _rows16_args(t: torch.Tensor):
+    """``_rows16`` of a (B, H, S, D) tensor with its address and strides, each read once: (tensor, address, (B, H, S) strides)."""
+    sb, sh, ss, last = t.stride()
+    address = t.data_ptr()
+    if last != 1 or address % 16 or sb % 8 or sh % 8 or ss % 8:
+        t = t.contiguous()
+        return t, t.data_ptr(), t.stride()[:3]
+    return t, address, (sb, sh, ss)
+
+
 def _check_bf16_cuda(*ts):
     for t in ts:
         if t.is_cuda and t.dtype is torch.bfloat16:
@@ -303,7 +313,9 @@ def prefill_attn_fwd(q, k, v, block_size, segment_size, threshold, force_select_
         if mode not in ("mean", "max"):
             raise ValueError(f"Invalid {what}: {mode}")
     lib = _lib.load()
-    q, k, v = _rows16(q), _rows16(k), _rows16(v)
+    q, q_ptr, q_strides = _rows16_args(q)
+    k, k_ptr, k_strides = _rows16_args(k)
+    v, v_ptr, v_strides = _rows16_args(v)
     device = q.device
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
@@ -317,8 +329,8 @@ def prefill_attn_fwd(q, k, v, block_size, segment_size, threshold, force_select_
         # a short sequence inside one segment: one launch, and the host's share of it (a workspace and its size, thirteen more
         # arguments) is what bounds the call: 77 tokens 12.5 -> 10.1 us
         rc = lib.pbs_one_segment_attn_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Hq, Hkv, S, D, block_size, segment_size,
-            *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], Hq * S * D, S * D, D, softmax_scale, _stream())
+            q_ptr, k_ptr, v_ptr, out.data_ptr(), B, Hq, Hkv, S, D, block_size, segment_size,
+            *q_strides, *k_strides, *v_strides, Hq * S * D, S * D, D, softmax_scale, _stream())
         if rc != _lib.NOT_ONE_LAUNCH:
             if rc:
                 _lib.check(rc, "pbs_one_segment_attn_fwd")
@@ -326,8 +338,8 @@ def prefill_attn_fwd(q, k, v, block_size, segment_size, threshold, force_select_
     ws_bytes = lib.pbs_prefill_attn_workspace_bytes(B, Hq, Hkv, S, D, block_size, segment_size)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=device)
     _lib.check(lib.pbs_prefill_attn_fwd(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Hq, Hkv, S, D, block_size, segment_size,
-        *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], Hq * S * D, S * D, D,
+        q_ptr, k_ptr, v_ptr, out.data_ptr(), B, Hq, Hkv, S, D, block_size, segment_size,
+        *q_strides, *k_strides, *v_strides, Hq * S * D, S * D, D,
         thr, _ptr(thr_rows), int(is_int_one), int(bool(force_select_first_block)),
         int(query_pool_mode == "max"), int(key_pool_mode == "max"), softmax_scale,
         ws.data_ptr(), max(ws_bytes, 256), _stream()), "pbs_prefill_attn_fwd")
