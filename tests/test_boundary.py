@@ -222,6 +222,24 @@ def test_mismatched_key_and_value_shapes_are_refused_before_anything_else(S, sta
             MeanPooling_prefill(q, bad_k, bad_v, force_select_current_block=not staged)   # (without: stage by stage)
 
 
+def test_addresses_and_strides_of_the_prefill_call():
+    """Read once for the alignment check and the library call: those of the tensor that _rows16 gives, copied where rows are not 16-byte aligned."""
+    from pbs_attn_amd import ops
+    x = torch.zeros(4 * 64 * 160 + 64, dtype=torch.bfloat16)
+    x = x[(-x.data_ptr() % 64) // 2:]   # the strided views start on a 64-byte boundary
+    views = [x.as_strided((2, 3, 5, 128), st, off) for off in (0, 8, 4) for st in [
+        (1920, 640, 128, 1), (1920, 128, 384, 1), (2400, 800, 160, 1), (0, 640, 128, 1),    # contiguous, token-major, padded rows, one batch for all
+        (1924, 640, 128, 1), (1920, 644, 128, 1), (1920, 640, 132, 1), (1920, 640, 2, 5)]]
+    copied = 0
+    for t in views:
+        want = ops._rows16(t)
+        got, address, strides = ops._rows16_args(t)
+        assert got.shape == t.shape and got.stride() == want.stride() and tuple(strides) == want.stride()[:3]
+        assert address == got.data_ptr() and (got is t) == (want is t)
+        copied += got is not t
+    assert copied == 4 + 4 + 7   # (a contiguous tensor that starts off the boundary stays as it is: the library refuses it)
+
+
 # ------------------------------------------------------------------ patcher on tiny models
 def _tiny(kind, layers=2):
     from transformers import LlamaConfig, LlamaForCausalLM, Qwen2Config, Qwen2ForCausalLM
