@@ -8,12 +8,12 @@
 //     on key order, so this is the reference's "every block of the own segment, element mask original key
 //     position > query position" with half the tiles and one masked tile instead of all.
 // Work decomposition
-//   A work item is TWO adjacent 128-query blocks of one head, served by one workgroup (4 waves, one per
-//   SIMD): wave w takes queries 32 w .. 32 w + 31 of either block, so that the waves finish a tile together also where
-//   only one block visits it, as always the item's last tile, the second block's diagonal one; such a tile takes half a
-//   tile's time.  The two visit lists of every item come merged into one list in HBM (ascending key-block indices, own-segment blocks appended),
+//   A work item is two adjacent 128-query blocks of one head, or in a short pass one (item_span), served by one workgroup
+//   (4 waves, one per SIMD): wave w takes queries 32 w .. 32 w + 31 of either block, so that the waves finish a tile together
+//   also where only one block visits it, as the last tile of a pair, the second block's diagonal one; such a tile takes half a
+//   tile's time.  A pair's two visit lists come merged into one list in HBM (ascending key-block indices, own-segment blocks appended),
 //   written by the block selection, by the list kernel below from CSR rows, or, for a sequence inside one segment, formed in
-//   LDS by the workgroup itself; every merged tile is copied ONCE into LDS for both query blocks, which
+//   LDS by the workgroup itself; every merged tile is copied ONCE into LDS for both query blocks of a pair, which
 //   halves the L2 -> LDS traffic and doubles the time a tile stays in flight.  K and V tiles are
 //   double-buffered (2 x 64 KB) and fetched one tile ahead with asynchronous global -> LDS copies (no
 //   registers), one workgroup barrier per tile.
@@ -225,8 +225,9 @@ __device__ __forceinline__ int ticket_item(const AttnArgs::Deal& d, int how, int
 // Whether an item visits few tiles, from 64 lists across the launch: every workgroup reads the same ones.  Such a launch gains by
 // the dealt order at any length: 2 x 32 / 8 heads x 13333 concentrated 947 -> 877 us a pass, 32 / 8 x 30000 1449 -> 1416, x 131072 2780 ->
 // 2690.  Where lists are long it loses what an XCD's workgroups share of a head in L2: 32 / 8 x 64000 with 100 tiles an item
-// 9.75 -> 10.11 ms, near-uniform 2 x 32 / 8 x 13333 (0.8 of an item's causal tiles and more) 2276 -> 2312 us.  (A round trip to memory
-// at the kernel's start, 2 us.)
+// 9.75 -> 10.11 ms, near-uniform 2 x 32 / 8 x 13333 (0.8 of an item's causal tiles and more) 2276 -> 2312 us.  Around the line, 32 / 8 x
+// 64000 in segments of 512, head by head -> dealt: 35 tiles an item 3976 -> 3928 us, 40 4465 -> 4421, 47 5101 -> 5023, 56 5955 -> 5895, by about as
+// much as runs differ (1 - 2 %): it lies at the lower end of where dealing stops to gain.  (A round trip to memory at the kernel's start, 2 us.)
 constexpr int SHORT_LIST = 40;
 __device__ __forceinline__ bool lists_are_short(ArgsPtr a) {
   const int n = a->deal.n, lane = lane_id_here();
@@ -264,10 +265,11 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   RESERVE_ACC_REGS();
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 
-  // Work items = (head, pair of query blocks), ordered head by head with the long rows of a head first and cut
-  // into eight contiguous ranges of about equal work, one per XCD (blockIdx % 8): an XCD works through one
-  // head at a time, so its resident workgroups walk the same permuted K/V stream at about the same pace and
-  // share its tiles in that XCD's L2.  The launch holds one workgroup per CU; each takes the next item of its
+  // Work items = (head, one or two query blocks), numbered head by head with the long rows of a head first and cut
+  // into eight contiguous ranges, one per XCD (blockIdx % 8).  Handed out in that order (ranges of about equal work) an XCD works
+  // through one head at a time, so its resident workgroups walk the same permuted K/V stream at about the same pace and
+  // share its tiles in that XCD's L2; passes of few items a head or of short lists deal several heads' items in turn instead
+  // (ticket_item).  The launch holds one workgroup per CU; each takes the next item of its
   // XCD's range from a counter until the range is used up, so that the copies of an item's first tiles, the
   // fetch of its list and of its queries overlap the previous item's last tile and epilogue.
   // The arguments are read through the kernel-argument pointer where they are needed, and that pointer is made
@@ -942,7 +944,13 @@ static int list_cap(int nb, int bps) { return (LIST_HEADER + nb + std::min(bps, 
 // 2048 99.6 -> 97.5, concentrated 86.4 -> 88.9).  With 560 blocks and more pairs are better everywhere (32 / 8 x 2560 116 -> 128).
 constexpr int SINGLE_BLOCK_ITEMS = 384;
 constexpr int SINGLE_FEW_HEADS = 512;
+// Limits of the dealt ticket orders (plan_ranges), near-uniform passes, head by head -> dealt.
+// Items a head up to which whole heads are dealt whatever their lists: 2 x 28 / 4 heads, 32 items 859 -> 827 us, 40 1221 -> 1204, 44 1459 ->
+// 1437, 48 1703 -> 1687, 56 2234 -> 2231, 64 2822 -> 2845; 32 / 8, 40 items 745 -> 729, 44 869 -> 846, 48 994 -> 978, 52 1142 -> 1138, 64 1639 -> 1642; 16 / 16 equal
+// from 32 to 64.  Above 44 the lists decide (DEAL_BY_LISTS).
 constexpr int DEAL_ROW = 44;
+// Items of a launch of other head counts: 28 / 4 heads, 1176 items 750 -> 700 us, 1400 989 -> 949, 1596 1258 -> 1213, 1988 1829 -> 1794, 2576 2833 -> 2916;
+// 12 / 4, 1392 2144 -> 1988, 1992 4048 -> 3927, 2592 6319 -> 6474.  (The gain ends between 2000 and 2600.)
 constexpr int DEAL_ITEMS = 1400;
 // A sequence inside one segment with more single blocks than workgroups would need the list kernel besides (see pbs_sparse_attn_launch): only from
 // ONE_SEGMENT_ROW blocks a row on (128 heads x 295 tokens 29 against 40 us, 32 heads x 1536 38.9 against 37.0).
@@ -1111,7 +1119,7 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
   a.plist = (const uint16_t*)((char*)workspace + 256);
   const int64_t n_wg = workgroups(max_items);
   // A sequence inside one segment with an item or less per workgroup: the attention kernel forms the lists itself (77 tokens, 32 / 8
-  // heads: 19.9 -> 17.1 us, one launch instead of two; the host needs about 17) and needs no workspace.
+  // heads: 19.9 -> 17.1 us when this came in, one launch instead of two) and needs no workspace.
   const bool own_lists = !lists_built && !csr_cols && !own_block_needed && a.bps >= a.nb && max_items <= n_wg / 8;
   PBS_REQUIRE(workspace || own_lists, "pbs_sparse_attn_fwd: workspace must be a 256-byte aligned device buffer of pbs_sparse_attn_workspace_bytes()");
   int dev = 0;
