@@ -12,7 +12,7 @@ LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libpbs_hip.so")
 
 SOURCES = ["pbs_abi.hip", "pbs_score.hip", "pbs_sort.hip", "pbs_gather.hip", "pbs_estimate.hip",
-           "pbs_select.hip", "pbs_attn.hip", "pbs_pipeline.hip", "pbs_rope.hip"]
+           "pbs_select.hip", "pbs_attn.hip", "pbs_attn_block.hip", "pbs_pipeline.hip", "pbs_rope.hip"]
 # measurement kernels for bench.py, in a library of their own: not part of the operator's ABI
 PROBE_SOURCES = ["pbs_probe.hip"]
 PROBE_LIB_PATH = os.path.join(LIB_DIR, "libpbs_probe.so")

@@ -50,6 +50,7 @@
 //   An item's tiles come in the order permuted tiles, own-segment tiles before the diagonal, diagonal tile, and
 //   each kind has a loop of its own (see the loops).
 #include "pbs_attn_tile.h"
+#include "pbs_attn_block.h"
 #include "pbs_wave.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 #include <atomic>
@@ -1114,6 +1115,11 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
   a.scale_log2 = softmax_scale * 1.4426950408889634f;
   PBS_REQUIRE(a.nb <= 4096, "pbs_sparse_attn_fwd: more than 4096 blocks per sequence (%d)", a.nb);
   PBS_REQUIRE((int64_t)a.BH * ((a.nb + 1) / 2) < (1ll << 28) && B < 65536 && Hq < 65536, "pbs_sparse_attn_fwd: launch too large");
+  // A sequence of one block needs no list and has a kernel of its own, which is faster for any number of heads (launches in a graph, this kernel ->
+  // that one, us: 32 / 8 heads x 77 9.6 -> 4.7, x 128 10.5 -> 6.0, 28 / 4 x 33 8.7 -> 3.8, 16 x 32 / 8 x 128 28.7 -> 20.8, 256 x 32 / 8 x 128 333 -> 258).
+  if (a.nb == 1 && !lists_built && !csr_cols && !own_block_needed)
+    return pbs_one_block_attn_launch(OneBlockArgs{a.q, a.k, a.v, a.o, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, S, 0,
+                                                  a.scale_log2}, B, Hq, Hkv, stream);
   const int max_items = plan_ranges(a);
   a.cap = list_cap(a.nb, a.bps);
   PBS_REQUIRE((uint32_t)a.cap * 2 <= LIST_BYTES, "pbs_sparse_attn_fwd: visit list too long");

@@ -252,6 +252,10 @@ extern "C" int pbs_meanpooling_attn_fwd(const void* q, const void* k, const void
   PBS_REQUIRE(workspace && workspace_bytes >= L.total && ((uintptr_t)workspace % 256) == 0,
               "pbs_meanpooling_attn_fwd: workspace must be a 256-byte aligned device buffer of %zu bytes", L.total);
   uint8_t* w = (uint8_t*)workspace;
+  // one block a row: its own, always selected (32 / 8 heads x 100 tokens 20.6 -> 5.3 us, 16 x 32 / 8 x 128 42.9 -> 20.8)
+  if (nb == 1)
+    return pbs_sparse_attn_launch(q, q, q, k, v, nullptr, nullptr, false, out, B, Hq, Hkv, S, head_dim, block_size, block_size, q_sb, q_sh, q_ss,
+                                  k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale, nullptr, w + L.attn_ws, stream);
   int rc;
   if ((rc = pbs_pool_blocks_launch(q, k, nullptr, w + L.pooled_q, w + L.pooled_k, nullptr, B, Hq, Hkv, S, head_dim, block_size, q_sb, q_sh,
                                    q_ss, k_sb, k_sh, k_ss, 0, 0, stream))) return rc;
