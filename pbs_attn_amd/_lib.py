@@ -6,6 +6,7 @@ import ctypes
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
+HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_pbs_host.so")
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libpbs_hip.so")
 
 # name -> (restype, argtypes); mirrors include/pbs_hip.h
@@ -44,6 +45,7 @@ SIGNATURES = {
 NOT_ONE_LAUNCH = -3   # PBS_NOT_ONE_LAUNCH
 
 _lib = None
+_one_segment = None
 
 
 class PbsHipError(RuntimeError):
@@ -68,6 +70,25 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def one_segment():
+    """The native call of short prompts (csrc/pbs_host.c): (q, k, v, block_size, segment_size, threshold, causal, use_triton,
+    query_pool_mode, key_pool_mode) -> the output, or None where the general path has to take the call."""
+    global _one_segment
+    if _one_segment is None:
+        import importlib.util
+
+        import torch
+        if not os.path.exists(HOST_PATH):
+            raise PbsHipError(f"{HOST_PATH} is missing: build it with `python -m pbs_attn_amd.build`")
+        address = ctypes.cast(load().pbs_one_segment_attn_fwd, c_void_p).value
+        spec = importlib.util.spec_from_file_location("_pbs_host", HOST_PATH)
+        host = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(host)
+        host.setup(torch.Tensor, torch.bfloat16, torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, check, address)
+        _one_segment = host.one_segment
+    return _one_segment
 
 
 def check(code: int, what: str):

@@ -4,6 +4,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sysconfig
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -58,6 +59,18 @@ def build_library(verbose: bool = False) -> str:
     return LIB_PATH
 
 
+HOST_SRC = os.path.join(CSRC, "pbs_host.c")
+HOST_PATH = os.path.join(LIB_DIR, "_pbs_host.so")
+
+
+def build_host_module() -> str:
+    """Compiles the CPython module of the native call of short prompts (it is handed the library's function, not linked to it)."""
+    os.makedirs(LIB_DIR, exist_ok=True)
+    subprocess.run(["gcc", "-std=c99", "-O2", "-Wall", "-fPIC", "-shared", "-I" + sysconfig.get_path("include"), HOST_SRC, "-o", HOST_PATH, "-lm"],
+                   check=True)
+    return HOST_PATH
+
+
 C_SMOKE_SRC = os.path.join(os.path.dirname(HERE), "tests", "c_abi", "smoke.c")
 C_SMOKE_BIN = os.path.join(os.path.dirname(HERE), "tests", "c_abi", "smoke")
 
@@ -76,4 +89,5 @@ def build_c_smoke() -> str:
 
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_host_module())
     print(build_c_smoke())

@@ -25,7 +25,7 @@ from typing import Optional, Union
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 _warned_use_triton = False
 
@@ -163,6 +163,12 @@ def permuted_block_sparse_attn_fwd(
     query_states (B, Hq, S, D); key/value_states (B, Hkv or Hq, S, D); bf16 on the
     GPU.  Returns (B, Hq, S, D) in original query order."""
     global _warned_use_triton
+    if stage_timer is None and query_states.is_cuda:
+        # a short prompt inside one segment, which the host's share bounds: natively, from tensors to launch (None: not such a call)
+        out = (_lib._one_segment or _lib.one_segment())(query_states, key_states, value_states, block_size, segment_size, threshold, causal,
+                                                        use_triton, query_pool_mode, key_pool_mode)
+        if out is not None:
+            return out
     batch_size, num_q_heads, q_len, head_dim = query_states.shape
     _, num_kv_heads, kv_len, _ = key_states.shape
     assert num_q_heads % num_kv_heads == 0
