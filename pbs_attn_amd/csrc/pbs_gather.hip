@@ -15,6 +15,7 @@
 // The pooled values of the two forms are the same bits: same loads, same order of additions.
 #include "pbs_lists.h"
 #include "pbs_pool.h"
+#include "pbs_sort.h"
 #include "../../include/pbs_hip.h"   // the definitions below are checked against the public declarations
 
 namespace {
@@ -36,8 +37,9 @@ struct GatherArgs {
   int pool_max;
 };
 
-template <bool POOL_ONLY>
-__device__ __forceinline__ void gather_block(GatherArgs& a, uint16_t* vt, float (&pool)[16][D], int kb, int grid_row) {
+// `order(i)`: the key at place i of the block
+template <bool POOL_ONLY, class Order>
+__device__ __forceinline__ void gather_block(GatherArgs& a, uint16_t* vt, float (&pool)[16][D], int kb, int grid_row, Order order) {
   const int bh = grid_row;
   if (POOL_ONLY) {
     if (a.needed && threadIdx.x == 0) a.needed[(int64_t)bh * a.nb + kb] = 0;
@@ -48,7 +50,6 @@ __device__ __forceinline__ void gather_block(GatherArgs& a, uint16_t* vt, float 
   const int rg = threadIdx.x >> 4, c = threadIdx.x & 15;  // row group, 16-byte chunk
   const uint16_t* ksrc = a.k + b * a.k_sb + kvh * a.k_sh;
   const uint16_t* vsrc = a.v + b * a.v_sb + kvh * a.v_sh;
-  const int32_t* idx = a.idx + (int64_t)bh * a.nb * BS + kb * BS;
   uint16_t* kdst = a.perm_k + ((int64_t)bh * a.nb + kb) * BS * D;
 
   // Every load of the block is requested before the first is used: a workgroup's rows are then in flight together
@@ -56,7 +57,7 @@ __device__ __forceinline__ void gather_block(GatherArgs& a, uint16_t* vt, float 
   // row 0 and are zeroed afterwards, so that no load sits behind a branch.
   int src[8];
 #pragma unroll
-  for (int pass = 0; pass < 8; ++pass) src[pass] = POOL_ONLY && !a.idx ? kb * BS + pass * 16 + rg : idx[pass * 16 + rg];
+  for (int pass = 0; pass < 8; ++pass) src[pass] = order(pass * 16 + rg);
   u32x4 kv[8], vv[8];
 #pragma unroll
   for (int pass = 0; pass < 8; ++pass) {
@@ -133,6 +134,12 @@ __device__ __forceinline__ void gather_block(GatherArgs& a, uint16_t* vt, float 
   }
 }
 
+template <bool POOL_ONLY>
+__device__ __forceinline__ void gather_block(GatherArgs& a, uint16_t* vt, float (&pool)[16][D], int kb, int bh) {
+  const int32_t* idx = a.idx + (int64_t)bh * a.nb * BS + kb * BS;
+  gather_block<POOL_ONLY>(a, vt, pool, kb, bh, [&](int i) { return POOL_ONLY && !a.idx ? kb * BS + i : idx[i]; });
+}
+
 // Launch order.  The query heads of a KV group read the same keys (and values) in different orders, and a permuted
 // block only holds rows of its own segment.  Workgroups are handed to the XCDs round-robin in launch order (x
 // fastest), so the grid is (8, members of a task group, groups / 8): the workgroups of one task group -- CHUNK
@@ -207,13 +214,54 @@ __global__ __launch_bounds__(256) void gather_pool_kernel(GatherArgs a, PoolQ p,
   else gather_block<false>(a, vt, pool, blk, bh);
 }
 
+// The same from the scores: a workgroup's first wave sorts the block's segment, NPL keys a lane (the order of the sort kernel, key by key).  A
+// segment is sorted once per block of it; what bounds it is the latency of one sort, and where all the sorting workgroups are in flight at once
+// (41 KB of LDS, three a CU) that costs less than the launch and the way to memory it saves.
+template <int NPL>
+__global__ __launch_bounds__(256) void sort_gather_pool_kernel(GatherArgs a, PoolQ p, TaskGroups t, SegmentScores s) {
+  __shared__ uint16_t vt[BS * VT_PITCH];
+  __shared__ float pool[16][D];
+  __shared__ int32_t keys[BS];
+  int kind, bh, blk;
+  if (!my_task(t, a.nb, kind, bh, blk)) return;
+  if (kind) {
+    pool_q_block(pool, p, blk, bh);
+    return;
+  }
+  const int segment = blk * BS / s.seg, base = segment * s.seg;
+  if (base >= s.Sc) {   // the remainder of the sequence keeps its places
+    gather_block<false>(a, vt, pool, blk, bh, [&](int i) { return blk * BS + i; });
+    return;
+  }
+  if (threadIdx.x < PBS_WAVE) {
+    const int lane = threadIdx.x, first = blk * BS - base;
+    const float* src = s.scores + (int64_t)bh * s.Sc + base;
+    double k[NPL];
+#pragma unroll
+    for (int r = 0; r < NPL; ++r) k[r] = sort_key_of<NPL>(src, 64 * r + lane, s.seg);
+    wave_sort<NPL>(k, lane);
+#pragma unroll
+    for (int r = 0; r < NPL; ++r) {
+      const int at = lane * NPL + r - first, i = (int)sort_key_index(k[r]);
+      if (at >= 0 && at < BS) {
+        keys[at] = base + i;
+        if (segment == 0 && i == 0) s.first_blk[bh] = blk;
+      }
+    }
+  }
+  __syncthreads();
+  gather_block<false>(a, vt, pool, blk, bh, [&](int i) { return keys[i]; });
+}
+
 }  // namespace
 
 int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const int32_t* key_indices, void* pooled_q, void* pooled_k,
                            void* perm_k, void* perm_vt, int B, int Hq, int Hkv, int S, int head_dim, int block_size, int64_t q_sb,
                            int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
-                           int query_pool_max, int key_pool_max, void* stream) {
-  PBS_REQUIRE(q && k && v && key_indices && pooled_q && pooled_k && perm_k && perm_vt, "pbs_gather_pool: null tensor pointer");
+                           int query_pool_max, int key_pool_max, void* stream, const SegmentScores& scores) {
+  PBS_REQUIRE(!scores.scores || (scores.first_blk && scores.seg <= PBS_SORT_IN_GATHER_KEYS && scores.seg % BS == 0 && scores.Sc % scores.seg == 0),
+              "pbs_gather_pool: bad scores");
+  PBS_REQUIRE(q && k && v && (key_indices || scores.scores) && pooled_q && pooled_k && perm_k && perm_vt, "pbs_gather_pool: null tensor pointer");
   PBS_REQUIRE(head_dim == D && block_size == BS, "pbs_gather_pool: head_dim and block_size must be 128 (got %d, %d)", head_dim, block_size);
   PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0, "pbs_gather_pool: bad shape");
   PBS_REQUIRE(q_sb % 8 == 0 && q_sh % 8 == 0 && q_ss % 8 == 0 && k_sb % 8 == 0 && k_sh % 8 == 0 && k_ss % 8 == 0 && v_sb % 8 == 0 &&
@@ -228,6 +276,14 @@ int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const in
   const PoolQ p = {(const uint16_t*)q, (uint16_t*)pooled_q, q_sb, q_sh, q_ss, query_pool_max, Hq, S, a.nb};
   const TaskGroups t = task_groups(B, Hq, Hkv, a.nb, 2);
   PBS_REQUIRE(t.grid.y <= 65535 && t.grid.z <= 65535, "pbs_gather_pool: too many heads or blocks");
+  if (scores.scores) {
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, t.grid, dim3(256), 0, (hipStream_t)stream, a, p, t, scores); };
+    if (scores.seg <= 128) launch(sort_gather_pool_kernel<2>);
+    else if (scores.seg <= 256) launch(sort_gather_pool_kernel<4>);
+    else if (scores.seg <= 512) launch(sort_gather_pool_kernel<8>);
+    else launch(sort_gather_pool_kernel<16>);
+    return pbs_check_launch("pbs_gather_pool");
+  }
   hipLaunchKernelGGL(gather_pool_kernel, t.grid, dim3(256), 0, (hipStream_t)stream, a, p, t);
   return pbs_check_launch("pbs_gather_pool");
 }

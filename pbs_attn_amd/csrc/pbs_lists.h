@@ -61,8 +61,9 @@ int pbs_segment_argsort_launch(const float* scores, int32_t* key_indices, int32_
 bool pbs_segment_argsort_takes_ride(int segment_size);
 // pbs_score_keys_workspace_bytes of this sequence or of any shorter one (which may be cut into more chunks), the largest
 size_t pbs_score_keys_workspace_bound(int B, int Hq, int Hkv, int S, int segment_size);
-// pbs_score_keys and pbs_segment_argsort_launch in one: the final scoring pass of short sequences of short segments sorts
-bool pbs_score_sorts(int B, int Hq, int Hkv, int S, int segment_size);
+// pbs_score_keys and pbs_segment_argsort_launch in one: the final scoring pass of short sequences of short segments sorts.  Where it can,
+// the keys that a workgroup of it would take if it did not (it then takes a segment); else 0.
+int pbs_score_sort_chunk(int B, int Hq, int Hkv, int S, int segment_size);
 int pbs_score_sort_launch(const void* q, const void* k, int32_t* key_indices, int32_t* first_blk, int B, int Hq, int Hkv, int S, int S_pad,
                           int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
                           int64_t k_sh, int64_t k_ss, void* workspace, size_t workspace_bytes, void* stream);
@@ -74,8 +75,16 @@ int pbs_pool_blocks_launch(const void* q, const void* k, const int32_t* key_indi
                            uint8_t* block_needed, int B, int Hq, int Hkv, int S, int head_dim, int block_size,
                            int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss,
                            int query_pool_max, int key_pool_max, void* stream);
-// pbs_pool_blocks and an unfiltered pbs_gather_kv in one launch (the pooled key blocks have the bits of both)
+// Scores of the keys of the complete segments (rows, Sc), for a launch that sorts them; first_blk as in pbs_segment_argsort_launch
+struct SegmentScores {
+  const float* scores;   // null: none
+  int32_t* first_blk;
+  int Sc, seg;
+};
+constexpr int PBS_SORT_IN_GATHER_KEYS = 1024;
+// pbs_pool_blocks and an unfiltered pbs_gather_kv in one launch (the pooled key blocks have the bits of both), by key_indices or, for
+// segments of up to PBS_SORT_IN_GATHER_KEYS keys, by the order of `scores`
 int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const int32_t* key_indices, void* pooled_q, void* pooled_k,
                            void* perm_k, void* perm_vt, int B, int Hq, int Hkv, int S, int head_dim, int block_size, int64_t q_sb,
                            int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
-                           int query_pool_max, int key_pool_max, void* stream);
+                           int query_pool_max, int key_pool_max, void* stream, const SegmentScores& scores = {});

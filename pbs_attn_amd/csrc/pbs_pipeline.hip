@@ -19,6 +19,18 @@ __global__ void identity_indices_kernel(int32_t* idx, int S_pad, int64_t total) 
 constexpr int SHORT_PASS_BLOCKS = 2048, SHORT_PASS_ROW = PBS_ESTIMATE_SELECT_MAX_BLOCKS;
 bool short_pass(int rows, int nb) { return nb <= SHORT_PASS_ROW && rows * nb <= SHORT_PASS_BLOCKS; }
 
+// Short passes whose gather sorts: those whose gathering workgroups are in flight at once, three a CU.  Whole pass, sort kernel -> this, us: 28 / 4
+// heads x 1000 in segments of 256 60.8 -> 57.7, x 1100 of 512 66.7 -> 62.7; 32 / 8 x 2200 of 1024 110.7 -> 105.4, x 3000 (768 blocks) of 1024 133.8 ->
+// 129.1, of 512 127.7 -> 122.0, x 3500 (896 blocks) of 1024 159.5 against 168.7, x 4096 of 1024 184.4 against 194.7; 8 / 2 x 2048 of 256 66.1 -> 64.1;
+// 28 / 4 x 2500 of 2048, thirty-two keys a lane, 126 against 147, hence the limit of the segment.
+// Where the final scoring pass can sort: that loses workgroups if a segment is longer than their chunks (segments of 128, 32 / 8 x 600
+// 42.8 -> 41.4 here; of 256, 4 / 1 x 4096 94.1 -> 91.7), up to some 512 blocks (28 / 4 x 2800 of 256, 616 blocks, 111.6 against 112.9; 8 x 32 / 8 x 300
+// of 256 81.1 against 83.5), and costs little if not (4 / 1 x 8192 of 128 134.2 against 137.4, of 256 99.6 against 101.0).
+constexpr int SORT_IN_GATHER_BLOCKS = 3 * 256;
+bool sorts_in_gather(int blocks, int segment_size, int score_sort_chunk) {
+  if (segment_size > PBS_SORT_IN_GATHER_KEYS) return false;
+  return blocks <= (score_sort_chunk == 0 ? SORT_IN_GATHER_BLOCKS : score_sort_chunk < segment_size ? 512 : 0);
+}
 
 // Sort with the query pooling + key pooling, against sort + both poolings, us: 32768 tokens, 32 / 8 heads 52 + 23 against 20 + 60; 13333 tokens twice
 // 51 + 19 against 13 + 57; 131072 tokens 208 + 91 against 36 + 247, where the key pooling alone has too little to do while it waits for its rows.
@@ -142,10 +154,15 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
                                   q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, o_sb, o_sh, o_ss, softmax_scale, nullptr,
                                   w + L.attn_ws, stream);
   const bool is_short = !threshold_is_int_one && short_pass(rows, nb);
+  SegmentScores scores = {};   // of a gather that sorts
   bool q_pooled = false;   // the query blocks' pooling is under way
   if (one_segment || nseg == 0 || (nseg == 1 && rem == 0)) {
     if ((rc = pbs_identity_indices((int32_t*)(w + L.idx), rows, s_pad, stream))) return rc;
-  } else if (pbs_score_sorts(B, Hq, Hkv, S, segment_size)) {
+  } else if (is_short && sorts_in_gather(rows * nb, segment_size, pbs_score_sort_chunk(B, Hq, Hkv, S, segment_size))) {
+    scores = {(const float*)(w + L.scores), (int32_t*)(w + L.select_ws), nseg * segment_size, segment_size};
+    if ((rc = pbs_score_keys(q, k, (float*)(w + L.scores), B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh,
+                             q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;
+  } else if (pbs_score_sort_chunk(B, Hq, Hkv, S, segment_size)) {
     if ((rc = pbs_score_sort_launch(q, k, (int32_t*)(w + L.idx), (int32_t*)(w + L.select_ws), B, Hq, Hkv, S, s_pad, head_dim, block_size,
                                     segment_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;
   } else {
@@ -171,7 +188,7 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
     if (is_short) {
       if ((rc = pbs_gather_pool_launch(q, k, v, (const int32_t*)(w + L.idx), w + L.pooled_q, w + L.pooled_k, w + L.perm_k, w + L.perm_vt, B, Hq,
                                        Hkv, S, head_dim, block_size, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss,
-                                       query_pool_max, key_pool_max, stream))) return rc;
+                                       query_pool_max, key_pool_max, stream, scores))) return rc;
     } else if (q_pooled) {
       if ((rc = pbs_pool_k_permuted(k, (const int32_t*)(w + L.idx), w + L.pooled_k, needed, B, Hq, Hkv, S, head_dim, block_size, k_sb, k_sh,
                                     k_ss, key_pool_max, stream))) return rc;

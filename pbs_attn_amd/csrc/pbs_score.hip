@@ -460,17 +460,18 @@ int score_keys_launch(const char* who, const void* q, const void* k, float* scor
 
 }  // namespace
 
-bool pbs_score_sorts(int B, int Hq, int Hkv, int S, int segment_size) {
+int pbs_score_sort_chunk(int B, int Hq, int Hkv, int S, int segment_size) {
   const int Sc = (S / segment_size) * segment_size;
-  if (Sc == 0 || segment_size > SORT_IN_PASS_KEYS || segment_size % STAGE_KEYS) return false;
+  if (Sc == 0 || segment_size > SORT_IN_PASS_KEYS || segment_size % STAGE_KEYS) return 0;
   const ScorePlan plan = score_plan(B, Hq, Hkv, Sc);
-  return plan.split && plan.small && segment_size <= 2 * plan.chunk_keys && (int64_t)B * Hq * (Sc / segment_size) <= SPLIT_WORKGROUPS;
+  const bool sorts = plan.split && plan.small && segment_size <= 2 * plan.chunk_keys && (int64_t)B * Hq * (Sc / segment_size) <= SPLIT_WORKGROUPS;
+  return sorts ? plan.chunk_keys : 0;
 }
 
 int pbs_score_sort_launch(const void* q, const void* k, int32_t* key_indices, int32_t* first_blk, int B, int Hq, int Hkv, int S, int S_pad,
                           int head_dim, int block_size, int segment_size, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb,
                           int64_t k_sh, int64_t k_ss, void* workspace, size_t workspace_bytes, void* stream) {
-  PBS_REQUIRE(key_indices && pbs_score_sorts(B, Hq, Hkv, S, segment_size), "pbs_score_sort: bad arguments");
+  PBS_REQUIRE(key_indices && pbs_score_sort_chunk(B, Hq, Hkv, S, segment_size), "pbs_score_sort: bad arguments");
   return score_keys_launch("pbs_score_keys", q, k, nullptr, B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh, q_ss, k_sb,
                            k_sh, k_ss, workspace, workspace_bytes, stream, key_indices, first_blk, S_pad);
 }
