@@ -66,7 +66,8 @@ struct AttnArgs {
   const uint16_t* v;     // original V at the KV heads, caller's strides
   const uint16_t* plist; // (B*Hq * n_items, cap) merged visit lists, in item order
   int* queue;            // 8 work counters, one per XCD
-  int cap;               // entries per list row (multiple of 8); 0: no lists in memory and no counters (see own_list)
+  int cap;               // entries per list row (multiple of 8); 0: no lists in memory (see own_list)
+  int one_each;          // every item is some workgroup's first: nobody asks for a further one
   uint16_t* o;
   int BH, Hq, Hkv, S, nb, bps;
   int span;           // query blocks of an item (two, or one: see item_span)
@@ -288,12 +289,13 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
   if (deal == DEAL_BY_LISTS) deal = lists_are_short(a0) ? DEAL_GROUPS : DEAL_NONE;
   const int xcd = blockIdx.x & 7;
   int q_begin = a0->xcd_start[xcd], q_end = a0->xcd_start[xcd + 1];   // the range being served: this XCD's, later others'
-  int vic = xcd, vic_tried = a0->cap ? 0 : 7;   // (no counters: every item is some workgroup's first)
+  int vic = xcd, vic_tried = a0->one_each ? 7 : 0;
   int* misc = reinterpret_cast<int*>(smem + LDS_MISC);   // [1] redo flag, [4] next item, [5] ranges with items left
   // Another range that still has items, once this one is used up: true with the item in `found` and the range in
   // vic / q_begin / q_end.  All eight counters are read at once, and a range whose counter has passed its end is skipped
   // without asking for a ticket (counters only grow): at the end of a launch, when every range is used up, that is one round
-  // trip to memory instead of seven.
+  // trip to memory instead of seven.  (Read ahead, during the last item, they are out of date when they are looked at, and the
+  // tickets asked for in vain cost more than the round trip: 32 / 8 heads x 4096 166.6 -> 169.0 us.)
   int found = 0;
   auto claim_elsewhere = [&]() __attribute__((always_inline)) {
     if (vic_tried >= 7) return false;
@@ -477,7 +479,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
     // the next item: claimed three tiles before the end of this one (the counter's latency passes under a
     // tile), published and its list requested one tile later, its queries and its first tile requested at the last
     // tile.  Items of fewer than three tiles finish these steps after their loop.
-    const int claim_it = careful_only ? -8 : max(n_tiles - 3, 0);
+    const int claim_it = careful_only || ap->one_each ? -8 : max(n_tiles - 3, 0);
     auto publish_and_fetch = [&]() __attribute__((always_inline)) {   // between the wait for this thread's loads and the barrier ...
       if (wave == 0 && lane_id_here() == 0) misc[4] = claim;
     };
@@ -548,10 +550,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
         __syncthreads();                      // every wave's share of tile `it` has landed; every wave is done with tile it - 1
         if (PBS_UNLIKELY((unsigned)(it - claim_it) < 2u)) {
           if (it != claim_it) adopt_next();
-          else if (wave == 0 && lane_id_here() == 0) {
-            ArgsPtr ac = PBS_ARGS();
-            claim = ac->cap ? atomicAdd(ac->queue + vic, 1) : NO_ITEM;
-          }
+          else if (wave == 0 && lane_id_here() == 0) claim = atomicAdd(PBS_ARGS()->queue + vic, 1);
         }
         // the list entries are read from LDS one tile ahead of their use (the read's latency would otherwise sit in
         // front of the copy requests of every tile): `e_ahead` holds entry it + 1, requested at the tile before
@@ -834,7 +833,7 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
           next_tile();
         }
       }
-      if (!careful_only && n_tiles < 3) {
+      if (claim_it >= 0 && n_tiles < 3) {
         if (n_tiles < 2) {
           __builtin_amdgcn_s_waitcnt(0x0f70);
           publish_and_fetch();
@@ -916,7 +915,10 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
         copy_tile_now(copy);
       }
     }
-    if (!has_nxt) break;
+    if (!has_nxt) {
+      __builtin_amdgcn_s_waitcnt(0x0f70);   // the last tile's copies, which nobody waits for, do not outlive the workgroup's LDS
+      break;
+    }
     q_ready = !stolen;
     careful_only = false;
     par ^= (n_tiles & 1) ? 0x8000u : 0u;
@@ -1143,6 +1145,10 @@ int pbs_sparse_attn_launch(const void* q, const void* perm_k, const void* perm_v
     pbs_set_error("pbs_sparse_attn_fwd: cannot reserve %u bytes of LDS: %s", LDS_TOTAL, hipGetErrorString(attr));
     return (int)attr;
   }
+  // Then nobody claims a further item, and above all nobody asks the other ranges for one before he ends, a round trip to memory behind the longest
+  // item: whole pass, 28 / 4 heads x 1000 57.7 -> 55.6 us, 8 / 2 x 2000 63.2 -> 62.1, 32 / 8 x 600 43.7 -> 43.1, in one segment 32 / 8 x 256 10.3 -> 10.0.
+  // (Launches without lists in memory have no counters either, and are of this kind.)
+  a.one_each = max_items <= n_wg / 8;
   if (own_lists) {
     a.cap = 0;
     if (a.deal.how == DEAL_BY_LISTS) a.deal.how = DEAL_NONE;
