@@ -214,12 +214,12 @@ __global__ __launch_bounds__(256) void gather_pool_kernel(GatherArgs a, PoolQ p,
   else gather_block<false>(a, vt, pool, blk, bh);
 }
 
-// The same from the scores: a workgroup's first wave sorts the block's segment, NPL keys a lane (the order of the sort kernel, key by key).  A
-// segment is sorted once per block of it; what bounds it is the latency of one sort, and where all the sorting workgroups are in flight at once
-// (41 KB of LDS, three a CU) that costs less than the launch and the way to memory it saves.
+// The same from the scores: a workgroup orders the block's segment itself, key by key as the sort kernel does: up to PBS_RANKED_KEYS keys by ranks,
+// longer ones by its first wave, NPL keys a lane.  A segment is ordered once per block of it; what bounds that is latency, and it costs less
+// than the launch and the way to memory and back that it saves (the rules, with both sides measured, stand at sorts_in_gather).
 template <int NPL>
 __global__ __launch_bounds__(256) void sort_gather_pool_kernel(GatherArgs a, PoolQ p, TaskGroups t, SegmentScores s) {
-  __shared__ uint16_t vt[BS * VT_PITCH];
+  __shared__ __attribute__((aligned(16))) uint16_t vt[BS * VT_PITCH];
   __shared__ float pool[16][D];
   __shared__ int32_t keys[BS];
   int kind, bh, blk;
@@ -233,21 +233,30 @@ __global__ __launch_bounds__(256) void sort_gather_pool_kernel(GatherArgs a, Poo
     gather_block<false>(a, vt, pool, blk, bh, [&](int i) { return blk * BS + i; });
     return;
   }
-  if (threadIdx.x < PBS_WAVE) {
-    const int lane = threadIdx.x, first = blk * BS - base;
-    const float* src = s.scores + (int64_t)bh * s.Sc + base;
+  const int first = blk * BS - base;
+  const float* src = s.scores + (int64_t)bh * s.Sc + base;
+  auto place = [&](int at, int i) {   // key i of the segment
+    at -= first;
+    if (at >= 0 && at < BS) {
+      keys[at] = base + i;
+      if (segment == 0 && i == 0) s.first_blk[bh] = blk;
+    }
+  };
+  if constexpr (64 * NPL <= PBS_RANKED_KEYS) {
+    double* const s_keys = reinterpret_cast<double*>(vt);
+    const int i = threadIdx.x;
+    const double own = i < s.seg ? sort_key(src[i], (uint32_t)i) : 0.0;
+    if (i < s.seg) s_keys[i] = own;
+    __syncthreads();
+    if (i < s.seg) place(rank_of(own, s_keys, s.seg), i);
+  } else if (threadIdx.x < PBS_WAVE) {
+    const int lane = threadIdx.x;
     double k[NPL];
 #pragma unroll
     for (int r = 0; r < NPL; ++r) k[r] = sort_key_of<NPL>(src, 64 * r + lane, s.seg);
     wave_sort<NPL>(k, lane);
 #pragma unroll
-    for (int r = 0; r < NPL; ++r) {
-      const int at = lane * NPL + r - first, i = (int)sort_key_index(k[r]);
-      if (at >= 0 && at < BS) {
-        keys[at] = base + i;
-        if (segment == 0 && i == 0) s.first_blk[bh] = blk;
-      }
-    }
+    for (int r = 0; r < NPL; ++r) place(lane * NPL + r, (int)sort_key_index(k[r]));
   }
   __syncthreads();
   gather_block<false>(a, vt, pool, blk, bh, [&](int i) { return keys[i]; });

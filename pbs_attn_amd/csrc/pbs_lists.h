@@ -81,7 +81,7 @@ struct SegmentScores {
   int32_t* first_blk;
   int Sc, seg;
 };
-constexpr int PBS_SORT_IN_GATHER_KEYS = 1024;
+constexpr int PBS_SORT_IN_GATHER_KEYS = 1024, PBS_RANKED_KEYS = 256;   // (up to the latter a workgroup ranks them)
 // pbs_pool_blocks and an unfiltered pbs_gather_kv in one launch (the pooled key blocks have the bits of both), by key_indices or, for
 // segments of up to PBS_SORT_IN_GATHER_KEYS keys, by the order of `scores`
 int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const int32_t* key_indices, void* pooled_q, void* pooled_k,

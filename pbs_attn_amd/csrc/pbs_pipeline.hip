@@ -19,17 +19,18 @@ __global__ void identity_indices_kernel(int32_t* idx, int S_pad, int64_t total) 
 constexpr int SHORT_PASS_BLOCKS = 2048, SHORT_PASS_ROW = PBS_ESTIMATE_SELECT_MAX_BLOCKS;
 bool short_pass(int rows, int nb) { return nb <= SHORT_PASS_ROW && rows * nb <= SHORT_PASS_BLOCKS; }
 
-// Short passes whose gather sorts: those whose gathering workgroups are in flight at once, three a CU.  Whole pass, sort kernel -> this, us: 28 / 4
-// heads x 1000 in segments of 256 60.8 -> 57.7, x 1100 of 512 66.7 -> 62.7; 32 / 8 x 2200 of 1024 110.7 -> 105.4, x 3000 (768 blocks) of 1024 133.8 ->
-// 129.1, of 512 127.7 -> 122.0, x 3500 (896 blocks) of 1024 159.5 against 168.7, x 4096 of 1024 184.4 against 194.7; 8 / 2 x 2048 of 256 66.1 -> 64.1;
-// 28 / 4 x 2500 of 2048, thirty-two keys a lane, 126 against 147, hence the limit of the segment.
-// Where the final scoring pass can sort: that loses workgroups if a segment is longer than their chunks (segments of 128, 32 / 8 x 600
-// 42.8 -> 41.4 here; of 256, 4 / 1 x 4096 94.1 -> 91.7), up to some 512 blocks (28 / 4 x 2800 of 256, 616 blocks, 111.6 against 112.9; 8 x 32 / 8 x 300
-// of 256 81.1 against 83.5), and costs little if not (4 / 1 x 8192 of 128 134.2 against 137.4, of 256 99.6 against 101.0).
-constexpr int SORT_IN_GATHER_BLOCKS = 3 * 256;
-bool sorts_in_gather(int blocks, int segment_size, int score_sort_chunk) {
-  if (segment_size > PBS_SORT_IN_GATHER_KEYS) return false;
-  return blocks <= (score_sort_chunk == 0 ? SORT_IN_GATHER_BLOCKS : score_sort_chunk < segment_size ? 512 : 0);
+// Short passes whose gather sorts its blocks' segments.
+// Up to 256 keys, which a workgroup ranks.  Whole pass, sort kernel -> this, us: 28 / 4 heads x 1000 in segments of 256 61.0 -> 52.9, 32 / 8 x 1500
+// 73.8 -> 67.5, x 8192 472.1 -> 468.7, of 128 474.5 -> 471.8, 28 / 4 x 300 41.7 -> 37.2, 8 x 16 / 16 x 600 84.2 -> 82.9.  From 256 heads on the other
+// routes win: 32 x 8 / 2 x 300 79.5 against 80.6, 16 x 32 / 8 x 200 of 128 88.7 against 91.4.  Where the final scoring pass could sort: 28 / 4 x 3400 of 256
+// 124.2 -> 121.3, 32 / 8 x 4096 162.4 -> 160.6, but not where a segment is less than what its workgroups take otherwise, so that it gains workgroups by
+// sorting (4 / 1 x 6000 of 128 106.9 against 109.6).
+// Longer ones, by the first wave, as long as the gathering workgroups are in flight at once, three a CU: 28 / 4 x 1100 of 512 66.7 -> 62.7; 32 / 8 x 2200 of
+// 1024 110.7 -> 105.4, x 3000 (768 blocks) 133.8 -> 129.1, x 3500 (896) 159.5 against 168.7; 28 / 4 x 2500 of 2048, thirty-two keys a lane, 126 against 147.
+constexpr int SORT_IN_GATHER_BLOCKS = 3 * 256, RANK_IN_GATHER_HEADS = 255;
+bool sorts_in_gather(int rows, int nb, int segment_size, int score_sort_chunk) {
+  if (segment_size <= PBS_RANKED_KEYS) return rows <= RANK_IN_GATHER_HEADS && score_sort_chunk <= segment_size;
+  return segment_size <= PBS_SORT_IN_GATHER_KEYS && rows * nb <= SORT_IN_GATHER_BLOCKS;
 }
 
 // Sort with the query pooling + key pooling, against sort + both poolings, us: 32768 tokens, 32 / 8 heads 52 + 23 against 20 + 60; 13333 tokens twice
@@ -158,7 +159,7 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
   bool q_pooled = false;   // the query blocks' pooling is under way
   if (one_segment || nseg == 0 || (nseg == 1 && rem == 0)) {
     if ((rc = pbs_identity_indices((int32_t*)(w + L.idx), rows, s_pad, stream))) return rc;
-  } else if (is_short && sorts_in_gather(rows * nb, segment_size, pbs_score_sort_chunk(B, Hq, Hkv, S, segment_size))) {
+  } else if (is_short && sorts_in_gather(rows, nb, segment_size, pbs_score_sort_chunk(B, Hq, Hkv, S, segment_size))) {
     scores = {(const float*)(w + L.scores), (int32_t*)(w + L.select_ws), nseg * segment_size, segment_size};
     if ((rc = pbs_score_keys(q, k, (float*)(w + L.scores), B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh,
                              q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;

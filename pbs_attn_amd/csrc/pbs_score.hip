@@ -93,9 +93,9 @@ __device__ __forceinline__ void stage_keys_async(const uint16_t* rows, int64_t k
 // One wave per query head of the KV group; the waves of a workgroup share the staged key rows.  SPLIT (short sequences, see
 // score_plan): the four waves take 32 queries each of ONE head.
 // Waves per SIMD: the final pass of the split form needs 147 registers and would spill 18 of them at four.
-// SORT: a workgroup of the final split pass takes a whole segment, keeps its scores in LDS, and its first wave sorts them, SORT keys a
-// lane: no launch, and no way to memory and back, for the sort.
-template <bool FINAL, bool SPLIT, int SORT = 0>
+// SORT: a workgroup of the final split pass takes a whole segment of up to 256 keys, keeps its scores in LDS, and ranks them: no launch, and
+// no way to memory and back, for the sort.
+template <bool FINAL, bool SPLIT, bool SORT = false>
 __global__ __launch_bounds__(256, SPLIT ? (FINAL ? 3 : 4) : 2) void score_kernel(ScoreArgs a) {
   constexpr int QT = SPLIT ? 1 : NQ / 32;   // query tiles of a wave
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // starts at LDS offset 0: this kernel has no static LDS
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256, SPLIT ? (FINAL ? 3 : 4) : 2) void score_kernel
   const uint16_t* kbase = a.k + b * a.k_sb + kvh * a.k_sh;
   float* s_stats = reinterpret_cast<float*>(smem + LDS_STATS) + wave * (32 * QT);   // p = exp2(logit - stat)
   float* s_sums = reinterpret_cast<float*>(smem + LDS_STATS) + NQ;   // SPLIT: a wave's sums of the stage's keys
-  float* s_scores = reinterpret_cast<float*>(smem + LDS_SCORE_TOTAL);   // SORT: the segment's scores
+  double* s_keys = reinterpret_cast<double*>(smem + LDS_SCORE_TOTAL);   // SORT: the segment's sort keys
   // LDS byte offset of fragment 0 of key row j inside a stage buffer; fragment t lies at frag0 ^ (t << 5),
   // rows 32 .. 63 of the stage 8 KB further on
   const uint32_t frag0 = (uint32_t)(j * 256 + ((half ^ (j & 15)) * 16));
@@ -253,20 +253,22 @@ __global__ __launch_bounds__(256, SPLIT ? (FINAL ? 3 : 4) : 2) void score_kernel
         if (wave == 0) {
           const float* s = s_sums + lane;
           const float score = ((s[0] + s[STAGE_KEYS]) + (s[2 * STAGE_KEYS] + s[3 * STAGE_KEYS])) * (1.0f / NQ);
-          if (SORT) s_scores[st * STAGE_KEYS + lane] = score;
+          if (SORT) s_keys[st * STAGE_KEYS + lane] = sort_key(score, (uint32_t)(st * STAGE_KEYS + lane));
           else a.scores[(int64_t)bh * a.Sc + key_lo + st * STAGE_KEYS + lane] = score;
         }
       }
     }
-    if constexpr (SORT > 0) {
+    if constexpr (SORT) {
       int32_t* row = a.idx + (int64_t)bh * a.S_pad;
-      if (wave == 0) {   // (its own stores, in order)
-        double k[SORT];
-#pragma unroll
-        for (int r = 0; r < SORT; ++r) k[r] = sort_key_of<SORT>(s_scores, 64 * r + lane, a.chunk_keys);
-        sort_and_store<SORT>(k, lane, a.chunk_keys, key_lo, chunk, row + key_lo, a.first_blk ? a.first_blk + bh : nullptr, a.block_size);
-      } else if (chunk == 0) {   // the remainder of the sequence and the block padding keep their places
-        for (int i = a.Sc + (int)threadIdx.x - 64; i < a.S_pad; i += 192) row[i] = i;
+      __syncthreads();
+      const int i = threadIdx.x;
+      if (i < a.chunk_keys) {
+        const int rank = rank_of(s_keys[i], s_keys, a.chunk_keys);
+        row[key_lo + rank] = key_lo + i;
+        if (chunk == 0 && i == 0 && a.first_blk) a.first_blk[bh] = rank / a.block_size;
+      }
+      if (chunk == 0) {   // the remainder of the sequence and the block padding keep their places
+        for (int i = a.Sc + (int)threadIdx.x; i < a.S_pad; i += 256) row[i] = i;
       }
     }
     if (!FINAL && active) {
@@ -342,7 +344,7 @@ int chunks_for(int Sc, int chunk_keys) { return (Sc + chunk_keys - 1) / chunk_ke
 // that do not run at once even with one chunk each: theirs stay short (and the doubling would have no end).
 constexpr int SPLIT_WORKGROUPS = 3 * 256;
 // The final pass sorts where a segment is at most two chunks long, so that a workgroup's serial part hardly grows, and its workgroups still
-// run at once.  Whole pass, sort kernel -> this: segments of 128, 32 / 8 heads x 512 45.3 -> 42.9 us, 28 / 4 x 1019 59.8 -> 56.7, 4 / 1 x
+// run at once (and the gather does not: short passes mostly leave it to that).  Whole pass, sort kernel -> this, with a sort by one wave: segments of 128, 32 / 8 heads x 512 45.3 -> 42.9 us, 28 / 4 x 1019 59.8 -> 56.7, 4 / 1 x
 // 16384 257.7 -> 249.6; of 256, 32 / 8 x 4096 166.1 -> 163.8, 28 / 4 x 4091 153.5 -> 150.8, 4 / 1 x 16384 160.5 -> 152.4.  Outside: segments of
 // four chunks 8 / 2 x 2048 58.9 against 60.4, 1024 workgroups 32 / 8 x 4096 164.9 against 165.7.
 constexpr int SORT_IN_PASS_KEYS = 256;
@@ -431,8 +433,7 @@ int score_keys_launch(const char* who, const void* q, const void* k, float* scor
     if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, false>, who)) return rc;
     if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<false, true>, who)) return rc;
     if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, true>, who)) return rc;
-    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, true, 2>, who)) return rc;
-    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, true, 4>, who)) return rc;
+    if (const int rc = pbs_require_no_static_lds((const void*)score_kernel<true, true, true>, who)) return rc;
     lds_checked.store(true, std::memory_order_release);
   }
   hipStream_t st = (hipStream_t)stream;
@@ -442,9 +443,7 @@ int score_keys_launch(const char* who, const void* q, const void* k, float* scor
     if (idx) {
       a.chunk_keys = segment_size;
       const dim3 segments(Sc / segment_size, B * Hq);
-      const size_t lds = LDS_SCORE_TOTAL + segment_size * sizeof(float);
-      if (segment_size <= 128) hipLaunchKernelGGL((score_kernel<true, true, 2>), segments, dim3(256), lds, st, a);
-      else hipLaunchKernelGGL((score_kernel<true, true, 4>), segments, dim3(256), lds, st, a);
+      hipLaunchKernelGGL((score_kernel<true, true, true>), segments, dim3(256), LDS_SCORE_TOTAL + segment_size * sizeof(double), st, a);
       return pbs_check_launch(who);
     }
     hipLaunchKernelGGL((score_kernel<true, true>), grid, dim3(256), LDS_SCORE_TOTAL, st, a);

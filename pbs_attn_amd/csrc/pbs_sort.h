@@ -97,6 +97,32 @@ __device__ __forceinline__ void sort_and_store(double (&k)[NPL], int lane, int s
       if (at + r < seg) out[at + r] = o[r];
   }
 }
+// ---- a workgroup ranks the keys of a segment of up to 256: `keys` (LDS, 16-byte aligned) are its sort keys, and the place of the one
+// that is `own` is the number of smaller ones.  Quadratic, a comparison and an addition with carry per pair, and yet the shorter chain where
+// a workgroup waits for its order (a segment of 256 by one wave's network -> this, whole pass: 28 / 4 heads x 1000 55.8 -> 52.9 us, 32 / 8 x 4096
+// 160.8 -> 159.4, 4 / 1 x 16384 164.8 -> 162.2; of 512, two keys a thread, 28 / 4 x 1100 60.8 -> 61.4); launches of nothing but
+// sorts, which are bound by the instructions, keep the network.
+__device__ __forceinline__ int rank_of(double own, const double* keys, int seg) {
+  typedef __attribute__((ext_vector_type(2))) double f64x2;
+  constexpr int AT_ONCE = 16;   // pairs of keys requested before the first is looked at
+  int n = 0;
+  for (int j = 0; j < seg; j += 2 * AT_ONCE) {   // a segment is a multiple of 64
+    f64x2 k[AT_ONCE];
+#pragma unroll
+    for (int x = 0; x < AT_ONCE; ++x) k[x] = *reinterpret_cast<const f64x2*>(keys + j + 2 * x);
+#pragma unroll
+    for (int x = 0; x < AT_ONCE; x += 2) {
+      uint64_t m0, m1, m2, m3;   // (a comparison's mask may be read two instructions later)
+      asm("v_cmp_lt_f64_e64 %1, %5, %9\n\tv_cmp_lt_f64_e64 %2, %6, %9\n\tv_cmp_lt_f64_e64 %3, %7, %9\n\tv_cmp_lt_f64_e64 %4, %8, %9\n\t"
+          "v_addc_co_u32_e64 %0, %1, %0, 0, %1\n\tv_addc_co_u32_e64 %0, %2, %0, 0, %2\n\tv_addc_co_u32_e64 %0, %3, %0, 0, %3\n\t"
+          "v_addc_co_u32_e64 %0, %4, %0, 0, %4"
+          : "+v"(n), "=&s"(m0), "=&s"(m1), "=&s"(m2), "=&s"(m3)
+          : "v"(k[x].x), "v"(k[x].y), "v"(k[x + 1].x), "v"(k[x + 1].y), "v"(own));
+    }
+  }
+  return n;
+}
+
 template <int NPL>
 __device__ __forceinline__ double sort_key_of(const float* scores, int i, int seg) {
   const double none = __builtin_bit_cast(double, 0x3ff0000000000000ull | (uint64_t)0xffffffffu << 11 | (uint32_t)i);

@@ -19,7 +19,9 @@ pytestmark = pytest.mark.gpu
     (1, 2, 1, 3 * 1152 + 1, 1152, 0.9, "uniform_heavy", {}),                       # segments too long for it
     (1, 32, 8, 24 * 128, 512, 0.9, "uniform_heavy", {}), (1, 33, 11, 24 * 128, 512, 0.9, "uniform_heavy", {}),   # 768 blocks, the last; 792
     (8, 8, 2, 1024, 128, 0.9, "strong_uniform", {}), (9, 8, 2, 1024, 128, 0.9, "strong_uniform", {}),   # 512 blocks where the scoring pass could sort; 576
-    (1, 1, 1, 64 * 128, 256, 0.9, "strong_heavy", {}),
+    (1, 1, 1, 64 * 128, 256, 0.9, "strong_heavy", {}), (1, 32, 8, 64 * 128, 256, "rows", "strong_uniform", {}),
+    (1, 255, 51, 300, 128, 0.9, "uniform_heavy", {}), (1, 256, 64, 300, 128, 0.9, "uniform_heavy", {}),   # the most heads of ranked segments; one more
+    (1, 4, 1, 6000, 128, 0.9, "strong_heavy", {}), (1, 4, 1, 6000, 256, 0.9, "strong_heavy", {}),         # segments shorter than a scoring chunk; as long as one
 ])
 def test_against_the_stages(dev, B, Hq, Hkv, S, seg, thr, kind, kw):
     assert torch.equal(*_single_and_staged(dev, B, Hq, Hkv, S, seg, thr, kind, **kw))
@@ -43,3 +45,18 @@ def test_equal_scores_and_strided_tensors(dev, seg):
     finally:
         P.stage_timer = None
     assert all(torch.equal(o, staged) for o in outs)
+
+
+@pytest.mark.parametrize("S,seg,value", [(300, 128, float("nan")), (700, 256, float("inf")), (1300, 512, float("nan"))])
+def test_scores_that_are_not_finite(dev, S, seg, value):
+    """Every score of a row is NaN once one of its logits is: keys keep their order."""
+    q, k, v = (x.to(dev) for x in small_case(1, 4, 2, S, seed=seg))
+    k[:, 0, seg // 3] = value
+    single = P.permuted_block_sparse_attn_fwd(q, k, v, 128, seg, 0.9, True)
+    P.stage_timer = _NullTimer()
+    try:
+        staged = P.permuted_block_sparse_attn_fwd(q, k, v, 128, seg, 0.9, True)
+    finally:
+        P.stage_timer = None
+    nan = torch.isnan(single)
+    assert torch.equal(nan, torch.isnan(staged)) and torch.equal(single[~nan], staged[~nan])
