@@ -302,7 +302,12 @@ __device__ __forceinline__ void mfma_o(const bf16x8& v, const bf16x8& p) {
 struct MfmaOp { int kind, k, T, x, q, frag; };   // kind 0: S (sub-tile k, row tile T, d-step x); 1: P.V (k, d tile x); 2: row sums (k)
 constexpr int N_FRAG = 64, UNITS_PER_COMBO = 7;
 constexpr int FRAG_BUFS = 6, FRAG_AHEAD = 11;   // fragment registers; how many matrix instructions ahead of its use a fragment is read
-constexpr int COPY_FIRST_GAP = 2, COPY_GAP_STEP = 8;
+constexpr int COPY_FIRST_GAP = 2;
+// A piece of the next tile's copy every so many matrix instructions: all of them are on their way before the middle of a tile, which leaves its second
+// half to the memory's latency.  In a tile of two column groups pieces 8 apart end with the tile, and its wait was a round trip to L2: passes of single
+// blocks, 8 apart -> 4, 4 / 1 heads x 8192 96.3 -> 92.0 us, 129.1 -> 124.3 in segments of 128, 8 / 2 x 2048 60.5 -> 59.2, 28 / 4 x 1000 53.5 -> 52.7;
+// 3 apart 93.7, 127.7, 59.7 and 52.8, 2 apart no better than 8.
+constexpr int copy_gap_step(int nq) { return 2 * nq; }
 // NQ: the column groups the tile is worked on for, four or (a tile that only one of the pair's blocks sees) two
 template <int NQ>
 struct TileSchedule {
@@ -413,7 +418,7 @@ constexpr int check_schedule() {
     if (s.read_after[f] >= 0 && s.first_use[f] < s.read_after[f] + 6) return 5;
     if (f >= FRAG_BUFS && s.read_after[f] < s.last_use[f - FRAG_BUFS]) return 6;
   }
-  if (s.unit_gap(8 * NQ - 1, 6) >= s.N_MFMA || COPY_FIRST_GAP + 15 * COPY_GAP_STEP >= s.N_MFMA) return 7;
+  if (s.unit_gap(8 * NQ - 1, 6) >= s.N_MFMA || COPY_FIRST_GAP + 15 * copy_gap_step(NQ) >= s.N_MFMA) return 7;
   return 0;
 }
 static_assert(check_schedule<4>() == 0 && check_schedule<2>() == 0, "tile schedule");
@@ -449,7 +454,7 @@ constexpr int lds_reads_younger(int f, int i, bool v_rows) {
 // Exponentials are taken against a LAZY reference maximum (see pbs_attn.hip).  Row sums
 // come from one more matrix instruction per sub-tile and column group, ones x P, whose every output row is the sum over
 // the sub-tile's 32 keys of the probabilities as the P.V product sees them (rounded to bf16).
-// `copy`: the next tile's copies, a piece every COPY_GAP_STEP matrix instructions.
+// `copy`: the next tile's copies, a piece every copy_gap_step matrix instructions.
 template <int Q0, int NQ, int MASKED, bool V_ROWS, bool COPIES = true>
 __device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_t (&va)[4], float c_log2, float (&m_ref)[QG],
                                           float (&l_row)[QG], bool& poisoned, int wave, const TileCopy& copy) {
@@ -530,8 +535,9 @@ __device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_
       __builtin_amdgcn_sched_barrier(0);
     }
     read_frag(std::integral_constant<int, frag_read_after<NQ>(i)>{});
-    if constexpr (COPIES && i >= COPY_FIRST_GAP && (i - COPY_FIRST_GAP) % COPY_GAP_STEP == 0 && (i - COPY_FIRST_GAP) / COPY_GAP_STEP < 16) {
-      copy_piece<(i - COPY_FIRST_GAP) / COPY_GAP_STEP>(copy);
+    constexpr int past = i - COPY_FIRST_GAP, step = copy_gap_step(NQ);
+    if constexpr (COPIES && past >= 0 && past % step == 0 && past / step < 16) {
+      copy_piece<past / step>(copy);
       __builtin_amdgcn_sched_barrier(0);
     }
     constexpr int u = i - Sched::FIRST_UNIT_GAP;
