@@ -38,8 +38,9 @@ struct EstimateStats {   // in LDS
 };
 // The probabilities of query blocks 32 qt .. 32 qt + 31, one after the other to sink(query block in the tile, key block, probability).
 // CANDIDATES_ONLY: only those of candidates; otherwise of all nb key blocks, zeros outside the candidates and NaN rows where
-// there are none.  pq, pk: the head's pooled query and key blocks.
-template <bool CAUSAL, bool CANDIDATES_ONLY, class Sink>
+// there are none.  pq, pk: the head's pooled query and key blocks.  ONE_TILE: up to 128 key blocks, a tile of 32 a wave, whose fragments
+// serve both passes.
+template <bool CAUSAL, bool CANDIDATES_ONLY, bool ONE_TILE = false, class Sink>
 __device__ __forceinline__ void estimate_tile(const uint16_t* pq, const uint16_t* pk, int nb, int bps, Divisor sqrt_d, int qt,
                                               EstimateStats& st, Sink sink) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -49,7 +50,12 @@ __device__ __forceinline__ void estimate_tile(const uint16_t* pq, const uint16_t
   const int n_kt_cand = (cand_max + 31) / 32;
   const int n_kt_all = (nb + 31) / 32;
 
-  bf16x8 qf[8];
+  bf16x8 qf[8], kf[8];
+  auto load_keys = [&](int kt) __attribute__((always_inline)) {
+    const uint16_t* row = pk + (int64_t)min(32 * kt + j, nb - 1) * ESTIMATE_D;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) kf[t] = load_frag(row, t, half);
+  };
   {
     const uint16_t* row = pq + (int64_t)min(32 * qt + j, nb - 1) * ESTIMATE_D;
 #pragma unroll
@@ -61,10 +67,10 @@ __device__ __forceinline__ void estimate_tile(const uint16_t* pq, const uint16_t
   const int cand_col = qb_col < nb ? candidate_count<CAUSAL>(qb_col, bps) : 0;
   float m_run = -INFINITY, l_run = 0.f;
   for (int kt = wave; kt < n_kt_cand; kt += 4) {
-    const uint16_t* row = pk + (int64_t)min(32 * kt + j, nb - 1) * ESTIMATE_D;
+    load_keys(kt);
     f32x16 acc = {0};
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load_frag(row, t, half), qf[t], acc, 0, 0, 0);
+    for (int t = 0; t < 8; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t], qf[t], acc, 0, 0, 0);
     float v[16], mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
@@ -105,16 +111,13 @@ __device__ __forceinline__ void estimate_tile(const uint16_t* pq, const uint16_t
   __syncthreads();
 
   // ---- pass B: rows = query blocks, column = key block j of tile kt
-  bf16x8 qa[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) qa[t] = qf[t];
   for (int kt = wave; kt < (CANDIDATES_ONLY ? n_kt_cand : n_kt_all); kt += 4) {
     const int kb = 32 * kt + j;
     f32x16 acc = {0};
     if (kt < n_kt_cand) {
-      const uint16_t* row = pk + (int64_t)min(kb, nb - 1) * ESTIMATE_D;
+      if (!ONE_TILE) load_keys(kt);
 #pragma unroll
-      for (int t = 0; t < 8; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[t], load_frag(row, t, half), acc, 0, 0, 0);
+      for (int t = 0; t < 8; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[t], kf[t], acc, 0, 0, 0);
     }
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {

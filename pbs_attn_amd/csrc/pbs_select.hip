@@ -69,6 +69,37 @@ __device__ __forceinline__ double readlane_f64(double v, int lane) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+// ---- sums over the lanes of a wave without LDS: a shuffle is a trip through it, and what follows waits for it; a row's decision had 24 of
+// them in a chain (whole pass, with them -> this and the key fragments and the threshold read once, ahead: 32 / 8 heads x 600 40.9 -> 39.4 us, 28 / 4 x 1000
+// 52.5 -> 51.5, 8 / 2 x 8192 110.0 -> 108.7).
+// the lane above's value of an inclusive prefix, zero for the first lane; and the prefix itself: inside rows of sixteen lanes, then
+// rows 0 and 2 to the next, then the first two rows to the others
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero_f64(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xf, false);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double wave_prefix_f64(double v) {
+  v += dpp_or_zero_f64<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+  v += dpp_or_zero_f64<0x112, 0xf>(v);
+  v += dpp_or_zero_f64<0x114, 0xf>(v);
+  v += dpp_or_zero_f64<0x118, 0xf>(v);
+  v += dpp_or_zero_f64<0x142, 0xa>(v);   // row_bcast 15 into rows 1 and 3
+  v += dpp_or_zero_f64<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ double lane_before_f64(double v) { return dpp_or_zero_f64<0x138, 0xf>(v); }   // wave_shr 1
+// numbers of up to `BITS` bits: their sum over the wave, and over the lanes before
+template <int BITS>
+__device__ __forceinline__ int wave_sum_of(int n, uint64_t lanes = ~0ull) {
+  int sum = 0;
+#pragma unroll
+  for (int b = 0; b < BITS; ++b) sum += __popcll(__ballot(n >> b & 1) & lanes) << b;
+  return sum;
+}
+
 __global__ __launch_bounds__(256) void select_blocks_kernel(SelectArgs a) {
   extern __shared__ uint64_t keys[];
   uint8_t* flag = reinterpret_cast<uint8_t*>(keys + a.n_pow2);
@@ -321,11 +352,20 @@ __device__ __forceinline__ void wave_bitonic_sort_u32(uint32_t (&k)[NPL], int la
   }
 }
 
-// One wave decides row (head `row`, query block qb) with the probabilities p[0 .. nb): flag[0 .. nb) (this wave's, in LDS) becomes the selection.
+// what a row's decision reads besides its probabilities: the threshold, and the block to be selected in any case (-1: none)
+struct RowRule {
+  float thr;
+  int first_blk;
+};
+__device__ __forceinline__ RowRule row_rule(const SelectArgs& a, int row) {
+  return {a.thr_rows ? a.thr_rows[row] : a.thr, a.force_first ? (a.first_blk ? a.first_blk[row] : 0) : -1};
+}
+// One wave decides a head's row of query block qb with the probabilities p[0 .. nb): flag[0 .. nb) (this wave's, in LDS) becomes the selection.
 template <int NPL>
-__device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb, const float* p, uint8_t* flag) {
+__device__ __forceinline__ void decide_row(const SelectArgs& a, RowRule rule, int qb, const float* p, uint8_t* flag) {
   const int lane = threadIdx.x & 63;
   const int nb = a.nb;
+  const float thr = rule.thr;
   const int seg_first = (qb / a.bps) * a.bps;
 
   for (int kb = lane; kb < nb; kb += 64) flag[kb] = 0;
@@ -366,8 +406,6 @@ __device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb,
       else if (v == -INFINITY) v = -FLT_MAX;
       k0v[r] = lane * NPL + r < count ? ~f32_orderable(v) : ~0u;
     }
-    const float thr = a.thr_rows ? a.thr_rows[row] : a.thr;
-
     // Rows whose mass sits in a few blocks need no sort: the largest remaining entry is taken out of the row
     // (value descending, ties by index -- the order of the sort) and added to the
     // sequential float64 sum until float32(sum) reaches the threshold: the reference's decision, term by term.
@@ -428,14 +466,7 @@ __device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb,
     double c = 0.0;
 #pragma unroll
     for (int r = 0; r < NPL; ++r) c += (double)value(r);
-    double incl = c;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const double t = shfl_up_f64(incl, d);
-      if (lane >= d) incl += t;
-    }
-    double excl = shfl_up_f64(incl, 1);
-    if (lane == 0) excl = 0.0;
+    const double excl = lane_before_f64(wave_prefix_f64(c));
     // float32 rounding boundary of the threshold (midpoint to its predecessor), as a double
     const double mid = 0.5 * ((double)thr + (double)nextafterf(thr, -INFINITY));
     const double tol = 1e-11 * fmax(1.0, fabs(mid));
@@ -448,9 +479,12 @@ __device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb,
       reach |= ((float)cp >= thr ? 1u : 0u) << r;
       amb |= (fabs(cp - mid) <= tol ? 1u : 0u) << r;
     }
-    int first = reach ? lane * NPL + __builtin_ctz(reach) : INT_MAX;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) first = min(first, __shfl_xor(first, off, 64));
+    const uint64_t reached = __ballot(reach != 0);   // the first rank is the lowest lane's lowest
+    int first = INT_MAX;
+    if (reached) {
+      const int owner = __builtin_ctzll(reached);
+      first = owner * NPL + __builtin_ctz((uint32_t)__builtin_amdgcn_readlane((int)reach, owner));
+    }
     // ambiguous prefixes at or before the first hit?
     bool my_amb = false;
 #pragma unroll
@@ -489,16 +523,9 @@ __device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb,
         above += k0v[r] < kstar ? 1 : 0;
         ties += k0v[r] == kstar ? 1 : 0;
       }
-      int ties_incl = ties;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int t = __shfl_up(ties_incl, d, 64);
-        if (lane >= d) ties_incl += t;
-      }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) above += __shfl_xor(above, off, 64);
-      const int m = first + 1 - above;
-      int tie_rank = ties_incl - ties;   // ties at lower indices
+      constexpr int BITS = NPL == 1 ? 1 : NPL <= 2 ? 2 : NPL <= 4 ? 3 : NPL <= 8 ? 4 : NPL <= 16 ? 5 : 6;   // of 0 .. NPL
+      const int m = first + 1 - wave_sum_of<BITS>(above);
+      int tie_rank = wave_sum_of<BITS>(ties, (1ull << lane) - 1ull);   // ties at lower indices
 #pragma unroll
       for (int r = 0; r < NPL; ++r) {
         const bool tie = k0v[r] == kstar;
@@ -511,10 +538,7 @@ __device__ __forceinline__ void decide_row(const SelectArgs& a, int row, int qb,
     if (count == 0 && 0.0f >= thr && lane == 0) flag[0] = 1;
   }
   __builtin_amdgcn_wave_barrier();
-  if (a.force_first && lane == 0) {
-    const int fb = a.first_blk ? a.first_blk[row] : 0;
-    if (fb >= 0 && fb < nb) flag[fb] = 1;
-  }
+  if (lane == 0 && rule.first_blk >= 0 && rule.first_blk < nb) flag[rule.first_blk] = 1;
   if (a.in_place && lane == 0) flag[qb] = 1;
 }
 
@@ -531,7 +555,7 @@ __device__ __forceinline__ void select_row_by_wave(const SelectArgs& a, int64_t 
   const int seg_first = (qb / a.bps) * a.bps;
   const int seg_end = min(seg_first + a.bps, nb);
   const int64_t row_off = ((int64_t)row * nb + qb) * nb;
-  decide_row<NPL>(a, row, qb, a.P + row_off, flag);
+  decide_row<NPL>(a, row_rule(a, row), qb, a.P + row_off, flag);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -681,15 +705,16 @@ __global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, Pa
   if (blockIdx.x == 0 && threadIdx.x < 8) l.queue[threadIdx.x] = l.first_tickets;
   if (live && qb < nb) {
     const float* p = a.P + ((int64_t)row * nb + qb) * nb;
+    const RowRule rule = row_rule(a, row);
     if constexpr (LONG) {
-      decide_row<32>(a, row, qb, p, flag);
+      decide_row<32>(a, rule, qb, p, flag);
     } else {
       switch (gr.npl[g]) {
-        case 1: decide_row<1>(a, row, qb, p, flag); break;
-        case 2: decide_row<2>(a, row, qb, p, flag); break;
-        case 4: decide_row<4>(a, row, qb, p, flag); break;
-        case 8: decide_row<8>(a, row, qb, p, flag); break;
-        default: decide_row<16>(a, row, qb, p, flag); break;
+        case 1: decide_row<1>(a, rule, qb, p, flag); break;
+        case 2: decide_row<2>(a, rule, qb, p, flag); break;
+        case 4: decide_row<4>(a, rule, qb, p, flag); break;
+        case 8: decide_row<8>(a, rule, qb, p, flag); break;
+        default: decide_row<16>(a, rule, qb, p, flag); break;
       }
     }
   }
@@ -712,11 +737,13 @@ __global__ __launch_bounds__(256) void estimate_select_kernel(const uint16_t* po
   const int nb = a.nb, nb_pad = (nb + 15) & ~15, qb = 4 * four + wave;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 8) l.queue[threadIdx.x] = l.first_tickets;
   const int64_t head = (int64_t)row * nb * ESTIMATE_D;
-  estimate_tile<CAUSAL, true>(pooled_q + head, pooled_k + head, nb, a.bps, sqrt_d, four / 8, st, [&](int ql, int kb, float p) __attribute__((always_inline)) {
+  const RowRule rule = row_rule(a, row);   // (on its way while the probabilities are formed)
+  static_assert(PBS_ESTIMATE_SELECT_MAX_BLOCKS <= 4 * 32, "a tile of key blocks a wave");
+  estimate_tile<CAUSAL, true, true>(pooled_q + head, pooled_k + head, nb, a.bps, sqrt_d, four / 8, st, [&](int ql, int kb, float p) __attribute__((always_inline)) {
     if (ql >> 2 == (four & 7)) probs[ql & 3][kb] = p;
   });
   __syncthreads();
-  if (qb < nb) decide_row<1>(a, row, qb, probs[wave], flags + wave * nb_pad);
+  if (qb < nb) decide_row<1>(a, rule, qb, probs[wave], flags + wave * nb_pad);
   __syncthreads();
   const int pair = 2 * four + (wave >> 1);
   if (2 * pair < nb) write_lists(a, l, row, pair, flags);
