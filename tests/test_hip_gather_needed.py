@@ -1,0 +1,32 @@
+"""GPU: the filtered gather of long calls, four blocks of a head a workgroup, against the unfiltered one: marked tiles bit for bit, the others untouched."""
+import pytest
+import torch
+
+from pbs_attn_amd import _lib, ops
+from tests.util import small_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S", [
+    (8, 64, 8, 33 * 128 - 5),      # 16896 blocks, an odd number a head, the last one ragged: chunks of one block
+    (1, 512, 512, 32 * 128),       # 16384, the fewest
+    (3, 28, 4, 196 * 128 + 1),     # 16548, seven heads a group
+])
+@pytest.mark.parametrize("share", [0.0, 0.03, 0.6, 1.0])
+def test_against_the_unfiltered_gather(dev, B, Hq, Hkv, S, share):
+    nb = (S + 127) // 128
+    assert B * Hq * nb >= 16384
+    _, k, v = (x.to(dev) for x in small_case(B, Hkv, Hkv, S, seed=S))
+    g = torch.Generator(device=dev).manual_seed(S)
+    idx = torch.rand(B, Hq, S, device=dev, generator=g).argsort(-1).to(torch.int32)
+    idx = torch.cat((idx, torch.arange(S, nb * 128, device=dev, dtype=torch.int32).expand(B, Hq, -1)), -1).contiguous()
+    needed = (torch.rand(B, Hq, nb, device=dev, generator=g) < share).to(torch.uint8)
+    full_k, full_vt, _ = ops.gather_kv(k, v, idx, Hq, want_pooled=False)
+    got_k, got_vt = torch.full_like(full_k, 7.0), torch.full_like(full_vt, 7.0)
+    _lib.check(_lib.load().pbs_gather_kv(k.data_ptr(), v.data_ptr(), idx.data_ptr(), got_k.data_ptr(), got_vt.data_ptr(), None, B, Hq, Hkv, S, 128, 128,
+                                         *k.stride()[:3], *v.stride()[:3], 0, needed.data_ptr(), torch.cuda.current_stream().cuda_stream), "pbs_gather_kv")
+    on = needed.bool()
+    for got, full in ((got_k, full_k), (got_vt, full_vt)):
+        got, full = got.view(B, Hq, nb, -1), full.view(B, Hq, nb, -1)
+        assert torch.equal(got[on], full[on]) and bool((got[~on] == 7.0).all())
