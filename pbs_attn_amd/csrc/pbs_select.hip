@@ -689,8 +689,10 @@ __device__ __forceinline__ void write_lists(const SelectArgs& a, const PairLists
 // here and read back) and no launch that merges them.  Groups are in pairs here: qb_lo / qb_hi are pair numbers.
 // LONG: rows of 1025 .. 2048 candidates, in a kernel of their own: the register need of 32 entries per lane would cost the shorter
 // rows two thirds of their waves.
+// Waves per SIMD: left to itself the compiler gives the long rows one (8 / 2 heads x 262144 7.39 against 7.21 ms a pass) and the others, a register too many,
+// three (32 / 8 x 131072 concentrated 2584 against 2572 us).
 template <bool LONG>
-__global__ __launch_bounds__(256) void select_pair_lists_kernel(SelectArgs a, PairLists l, SelectGroups gr, int rows) {
+__global__ __launch_bounds__(256, LONG ? 2 : 4) void select_pair_lists_kernel(SelectArgs a, PairLists l, SelectGroups gr, int rows) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_w[];
   int g = 0;
   while (g + 1 < gr.n && (int)blockIdx.x >= gr.wg_end[g]) ++g;
