@@ -857,7 +857,8 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       // ---- epilogue: normalise and store from the registers.  Lane group g holds d 4 g .. 4 g + 3 of each d tile of its query; once the
       // odd and even groups have exchanged between two d tiles it is eight consecutive ones of the first (groups 0 and 2) or the
       // second (1 and 3): 16-byte stores, 64 consecutive bytes a row, the line's other half by the next store.  (Through LDS, in whole
-      // rows of 256 bytes a store, 77 tokens of 32 / 8 heads took 9.89 us a call, now 9.36; 1000 to 128k tokens take the same.)
+      // rows of 256 bytes a store, 77 tokens of 32 / 8 heads took 9.89 us a call, now 9.36, before they had a kernel of their own; 1000 to 128k tokens
+      // take the same: what bounds it either way is the arithmetic of a wave by itself, some 800 instructions, 4240 cycles.)
       // a query block that used no tile (no selected block and no own block: possible only with an optional diagonal)
       // has a zero sum and writes zeros, as the reference does for a row without selected blocks
       MFMA_FENCE();
