@@ -72,20 +72,29 @@ def load():
     return lib
 
 
+def _never_native(*args):
+    return None
+
+
 def one_segment():
     """The native call of short prompts (csrc/pbs_host.c): (q, k, v, block_size, segment_size, threshold, causal, use_triton,
-    query_pool_mode, key_pool_mode) -> the output, or None where the general path has to take the call."""
+    query_pool_mode, key_pool_mode) -> the output, or None where the general path has to take the call.  Where the module is missing or
+    does not fit this interpreter that is every call: the same kernels, 3 us later."""
     global _one_segment
     if _one_segment is None:
         import importlib.util
 
         import torch
-        if not os.path.exists(HOST_PATH):
-            raise PbsHipError(f"{HOST_PATH} is missing: build it with `python -m pbs_attn_amd.build`")
         address = ctypes.cast(load().pbs_one_segment_attn_fwd, c_void_p).value
-        spec = importlib.util.spec_from_file_location("_pbs_host", HOST_PATH)
-        host = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(host)
+        try:
+            spec = importlib.util.spec_from_file_location("_pbs_host", HOST_PATH)
+            host = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(host)
+        except ImportError as e:
+            import warnings
+            _one_segment = _never_native
+            warnings.warn(f"short prompts are called through Python: build the native call with `python -m pbs_attn_amd.build` ({e})")
+            return _one_segment
         host.setup(torch.Tensor, torch.bfloat16, torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, check, address)
         _one_segment = host.one_segment
     return _one_segment

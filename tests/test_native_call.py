@@ -1,10 +1,41 @@
 """The native call of short prompts takes the plain case and hands everything else to the general path, which then serves or refuses it."""
+import os
+import warnings
+
 import pytest
 import torch
 
 from pbs_attn_amd import _lib, ops
 from pbs_attn_amd import pbs as P
 from tests.util import small_case
+
+
+@pytest.fixture(params=["missing", "of another kind"])
+def without_the_module(request, monkeypatch, tmp_path):
+    path = tmp_path / os.path.basename(_lib.HOST_PATH)
+    if request.param != "missing":
+        path.write_bytes(b"no module")
+    monkeypatch.setattr(_lib, "HOST_PATH", str(path))
+    monkeypatch.setattr(_lib, "_one_segment", None)
+
+
+def test_without_the_module_the_general_path_takes_every_call(without_the_module):
+    q, k, v = small_case(1, 4, 2, 77)
+    with pytest.warns(UserWarning, match="through Python"):
+        native = _lib.one_segment()
+    assert native(q, k, v, 128, 256, 0.9, True, True, "mean", "mean") is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.one_segment() is native   # looked for once
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [77, 300, 5000])
+def test_calls_without_the_module(dev, without_the_module, S):
+    q, k, v = (x.to(dev) for x in small_case(1, 4, 2, S, seed=S))
+    with pytest.warns(UserWarning, match="through Python"):
+        out = P.permuted_block_sparse_attn_fwd(q, k, v, 128, 256, 0.9, True)
+    assert torch.equal(out, ops.prefill_attn_fwd(q, k, v, 128, 256, 0.9))
 
 
 def test_tensors_on_the_host_are_not_taken():
