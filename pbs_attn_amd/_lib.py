@@ -4,9 +4,11 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sysconfig
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
-HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_pbs_host.so")
+# named after the interpreter it is built for: another one looks for a file of its own
+HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_pbs_host" + sysconfig.get_config_var("EXT_SUFFIX"))
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libpbs_hip.so")
 
 # name -> (restype, argtypes); mirrors include/pbs_hip.h

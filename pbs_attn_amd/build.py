@@ -60,7 +60,7 @@ def build_library(verbose: bool = False) -> str:
 
 
 HOST_SRC = os.path.join(CSRC, "pbs_host.c")
-HOST_PATH = os.path.join(LIB_DIR, "_pbs_host.so")
+HOST_PATH = os.path.join(LIB_DIR, "_pbs_host" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 def build_host_module() -> str:

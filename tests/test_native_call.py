@@ -1,4 +1,5 @@
 """The native call of short prompts takes the plain case and hands everything else to the general path, which then serves or refuses it."""
+import importlib.machinery
 import os
 import warnings
 
@@ -29,6 +30,12 @@ def test_without_the_module_the_general_path_takes_every_call(without_the_module
         assert _lib.one_segment() is native   # looked for once
 
 
+def test_the_module_is_named_after_its_interpreter():
+    from pbs_attn_amd import build
+    assert build.HOST_PATH == _lib.HOST_PATH
+    assert os.path.basename(_lib.HOST_PATH) == "_pbs_host" + importlib.machinery.EXTENSION_SUFFIXES[0]   # the most specific that is looked for
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("S", [77, 300, 5000])
 def test_calls_without_the_module(dev, without_the_module, S):
@@ -39,6 +46,9 @@ def test_calls_without_the_module(dev, without_the_module, S):
 
 
 def test_tensors_on_the_host_are_not_taken():
+    if not os.path.exists(_lib.HOST_PATH):
+        from pbs_attn_amd.build import build_host_module
+        build_host_module()
     q, k, v = small_case(1, 4, 2, 77)
     native = _lib.one_segment()
     assert native(q, k, v, 128, 256, 0.9, True, True, "mean", "mean") is None
