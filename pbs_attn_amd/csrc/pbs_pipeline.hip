@@ -265,6 +265,8 @@ extern "C" int pbs_meanpooling_attn_fwd(const void* q, const void* k, const void
   PBS_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && S > 0 && block_size > 0, "pbs_meanpooling_attn_fwd: bad shape");
   const int rows = B * Hq, nb = (S + block_size - 1) / block_size;
   PBS_REQUIRE(rows <= 65535, "pbs_meanpooling_attn_fwd: too many heads (%d)", rows);
+  // the launch limit of the pooling, whether or not this call needs it
+  PBS_REQUIRE(Hq / Hkv * 16 <= 65535, "pbs_meanpooling_attn_fwd: too many heads or blocks");
   PBS_REQUIRE(nb <= PBS_PAIR_SELECT_MAX_BLOCKS, "pbs_meanpooling_attn_fwd: more than %d blocks per sequence (%d)", PBS_PAIR_SELECT_MAX_BLOCKS, nb);
   const MeanPoolingLayout L = meanpooling_layout(B, Hq, S, head_dim, block_size);
   PBS_REQUIRE(workspace && workspace_bytes >= L.total && ((uintptr_t)workspace % 256) == 0,

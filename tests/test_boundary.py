@@ -81,6 +81,18 @@ def test_argument_errors_are_reported_without_a_gpu():
     assert rc < 0 and b"key row stride" in lib.pbs_last_error()
 
 
+def test_meanpooling_of_one_block_keeps_the_limit_of_the_general_path():
+    """Refused ahead of any launch, with one block a row as with more: groups of 4096 heads, which the pooling's launch cannot hold."""
+    from pbs_attn_amd import _lib
+    lib = _lib.load()
+    for S in (100, 300):
+        strides = (4096 * S * 128, S * 128, 128)
+        ws = lib.pbs_meanpooling_attn_workspace_bytes(1, 4096, 1, S, 128, 128)
+        rc = lib.pbs_meanpooling_attn_fwd(256, 256, 256, 256, 1, 4096, 1, S, 128, 128, *strides, *strides, *strides, *strides, 0.9, None, 1, 0.1,
+                                          256, ws, None)
+        assert rc == -1 and b"too many heads or blocks" in lib.pbs_last_error()
+
+
 def test_reference_import_paths():
     from pbs_attn import permuted_block_sparse_attn_fwd as a
     from pbs_attn.patch.huggingface import apply_patch_with_prefill, get_permuted_block_sparse_attn_fwd
