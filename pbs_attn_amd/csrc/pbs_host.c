@@ -65,6 +65,7 @@ static int is_pool_mode(PyObject* mode) {
 }
 
 static PyObject* not_taken(void) {
+  if (PyErr_Occurred() && !PyErr_ExceptionMatches(PyExc_Exception)) return NULL;   /* an interrupt, an exit */
   PyErr_Clear();   /* the general path meets the same error again */
   Py_RETURN_NONE;
 }

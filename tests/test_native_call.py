@@ -57,6 +57,26 @@ def test_tensors_on_the_host_are_not_taken():
         native(q, k, v)
 
 
+def test_an_interrupt_is_not_swallowed():
+    """Attributes are read through the modes that are on; what one raises there is met again by the general path, unless it ends the program."""
+    from torch.overrides import TorchFunctionMode
+
+    class Raising(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            raise self.error
+
+    q, k, v = small_case(1, 4, 2, 77)
+    native = _lib.one_segment()
+    for error in (KeyboardInterrupt, RuntimeError("no")):
+        with Raising() as mode:
+            mode.error = error
+            if error is KeyboardInterrupt:
+                with pytest.raises(KeyboardInterrupt):
+                    native(q, k, v, 128, 256, 0.9, True, True, "mean", "mean")
+            else:
+                assert native(q, k, v, 128, 256, 0.9, True, True, "mean", "mean") is None
+
+
 class _Subclass(torch.Tensor):
     pass
 
