@@ -1,4 +1,4 @@
-"""GPU: the filtered gather of long calls, four blocks of a head a workgroup, against the unfiltered one: marked tiles bit for bit, the others untouched."""
+"""GPU: the filtered gather of long calls against the unfiltered one: marked tiles bit for bit, the others untouched."""
 import pytest
 import torch
 
@@ -9,14 +9,13 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,S", [
-    (8, 64, 8, 33 * 128 - 5),      # 16896 blocks, an odd number a head, the last one ragged: chunks of one block
-    (1, 512, 512, 32 * 128),       # 16384, the fewest
-    (3, 28, 4, 196 * 128 + 1),     # 16548, seven heads a group
+    (8, 64, 8, 33 * 128 - 5),      # an odd number of blocks a head, the last one ragged: chunks of one block
+    (1, 512, 512, 32 * 128),       # a head a group, whole chunks
+    (3, 28, 4, 196 * 128 + 1),     # seven heads a group
 ])
 @pytest.mark.parametrize("share", [0.0, 0.03, 0.6, 1.0])
 def test_against_the_unfiltered_gather(dev, B, Hq, Hkv, S, share):
     nb = (S + 127) // 128
-    assert B * Hq * nb >= 16384
     _, k, v = (x.to(dev) for x in small_case(B, Hkv, Hkv, S, seed=S))
     g = torch.Generator(device=dev).manual_seed(S)
     idx = torch.rand(B, Hq, S, device=dev, generator=g).argsort(-1).to(torch.int32)
