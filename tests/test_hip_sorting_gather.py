@@ -18,8 +18,9 @@ pytestmark = pytest.mark.gpu
     (1, 2, 1, 2 * 1024 + 128, 1024, 0.9, "strong_heavy", {}), (1, 2, 2, 2 * 1024, 1024, 0.0, "local_window", {}),
     (1, 2, 1, 3 * 1152 + 1, 1152, 0.9, "uniform_heavy", {}),                       # segments too long for it
     (1, 32, 8, 24 * 128, 512, 0.9, "uniform_heavy", {}), (1, 33, 11, 24 * 128, 512, 0.9, "uniform_heavy", {}),   # 768 blocks, the last; 792
-    (8, 8, 2, 1024, 128, 0.9, "strong_uniform", {}), (9, 8, 2, 1024, 128, 0.9, "strong_uniform", {}),   # 512 blocks where the scoring pass could sort; 576
-    (1, 1, 1, 64 * 128, 256, 0.9, "strong_heavy", {}), (1, 32, 8, 64 * 128, 256, "rows", "strong_uniform", {}),
+    (8, 8, 2, 1024, 128, 0.9, "strong_uniform", {}), (9, 8, 2, 1024, 128, 0.9, "strong_uniform", {}),   # batches
+    (1, 1, 1, 64 * 128, 256, 0.9, "strong_heavy", {}), (1, 32, 8, 64 * 128, 256, "rows", "strong_uniform", {}),   # 64 blocks a row; 2048 blocks, the last
+    (1, 33, 11, 64 * 128, 256, "rows", "strong_uniform", {}),                      # no short pass any more
     (1, 255, 51, 300, 128, 0.9, "uniform_heavy", {}), (1, 256, 64, 300, 128, 0.9, "uniform_heavy", {}),   # the most heads of ranked segments; one more
     (1, 4, 1, 6000, 128, 0.9, "strong_heavy", {}), (1, 4, 1, 6000, 256, 0.9, "strong_heavy", {}),         # segments shorter than a scoring chunk; as long as one
 ])
