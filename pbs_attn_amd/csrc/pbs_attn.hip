@@ -858,7 +858,8 @@ __global__ __launch_bounds__(THREADS, 1) void sparse_attn_kernel(AttnArgs a) {
       // odd and even groups have exchanged between two d tiles it is eight consecutive ones of the first (groups 0 and 2) or the
       // second (1 and 3): 16-byte stores, 64 consecutive bytes a row, the line's other half by the next store.  (Through LDS, in whole
       // rows of 256 bytes a store, 77 tokens of 32 / 8 heads took 9.89 us a call, now 9.36, before they had a kernel of their own; 1000 to 128k tokens
-      // take the same: what bounds it either way is the arithmetic of a wave by itself, some 800 instructions, 4240 cycles.)
+      // take the same.)  What bounds it is the arithmetic of a wave by itself on its SIMD: 400 vector instructions and 56 wait states for its sixteen
+      // stores, 3770 to 3840 cycles, of which 3070 to 3150 remain with the stores masked off; 300 to 400 more pass before the first store.
       // a query block that used no tile (no selected block and no own block: possible only with an optional diagonal)
       // has a zero sum and writes zeros, as the reference does for a row without selected blocks
       MFMA_FENCE();

@@ -146,9 +146,8 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
               "pbs_prefill_attn_fwd: too many heads or blocks");
   int rc;
   // A sequence inside one segment of the kernel's size needs no permuted tile, hence no order, no gather and no
-  // selection: the attention launch, behind the list kernel's where there are more items than workgroups (32 / 8 heads x 77 tokens:
-  // six launches 32.2 us, two 20.7, one 17.1; pbs_one_segment_attn_fwd, which needs no workspace, 10).  (Permuted tiles: none is listed,
-  // any aligned address will do.)
+  // selection: the attention launch, behind the list kernel's where there are more items than workgroups (32 / 8 heads x 77 tokens,
+  // before one block had a kernel of its own: six launches 32.2 us, two 20.7, one 17.1).  (Permuted tiles: none is listed, any aligned address will do.)
   const bool own_tiles_only = segment_size >= s_pad;
   if (own_tiles_only)
     return pbs_sparse_attn_launch(q, w, w, k, v, nullptr, nullptr, false, out, B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb,

@@ -344,9 +344,11 @@ int chunks_for(int Sc, int chunk_keys) { return (Sc + chunk_keys - 1) / chunk_ke
 // that do not run at once even with one chunk each: theirs stay short (and the doubling would have no end).
 constexpr int SPLIT_WORKGROUPS = 3 * 256;
 // The final pass sorts where a segment is at most two chunks long, so that a workgroup's serial part hardly grows, and its workgroups still
-// run at once (and the gather does not: short passes mostly leave it to that).  Whole pass, sort kernel -> this, with a sort by one wave: segments of 128, 32 / 8 heads x 512 45.3 -> 42.9 us, 28 / 4 x 1019 59.8 -> 56.7, 4 / 1 x
-// 16384 257.7 -> 249.6; of 256, 32 / 8 x 4096 166.1 -> 163.8, 28 / 4 x 4091 153.5 -> 150.8, 4 / 1 x 16384 160.5 -> 152.4.  Outside: segments of
-// four chunks 8 / 2 x 2048 58.9 against 60.4, 1024 workgroups 32 / 8 x 4096 164.9 against 165.7.
+// run at once (and the gather does not: short passes mostly leave it to that).  Whole pass, sort kernel -> this, us: segments of 128, 4 / 1 heads x 6000 109.7 -> 102.0, x 16384 267.6 ->
+// 257.8, 32 x 8 / 2 x 300 81.7 -> 78.0, 16 x 32 / 8 x 200 91.7 -> 88.1; of 256, 4 / 1 x 16384 269.2 -> 259.0, 8 / 2 x 12000 195.5 -> 189.0, 16 / 16 x 12000
+// 518 -> 512; everything selected, 28 / 4 x 1019 of 128 52.1 -> 48.0, 32 / 8 x 4096 of 256 164.0 -> 158.8.  Past the limits, measured
+// where everything is selected, there is little left in it: segments of four chunks, 8 / 2 x 2048 61.7 -> 60.6; 1024 workgroups, 32 / 8 x 4096 of 128 162.2 -> 161.4; 1536, 24 / 8 x
+// 8192 386.5 -> 385.7.
 constexpr int SORT_IN_PASS_KEYS = 256;
 struct ScorePlan {
   bool split, small;

@@ -1,4 +1,5 @@
-// The segment sort by one wave in registers: shared by the sort kernel and the final scoring pass of short sequences.
+// The order of a segment's keys: by one wave in registers (the sort kernel, and the gather of short passes for longer segments), and by ranks in a
+// workgroup (that gather and the final scoring pass, segments of up to 256 keys).
 #pragma once
 #include "pbs_wave.h"
 
@@ -71,32 +72,6 @@ __device__ __forceinline__ void wave_sort(double (&k)[NPL], int lane) {
   }
 }
 
-// Sorts the wave's keys of segment `s` of a row (`seg` of them; register r of lane l starts with that of local index 64 r + l) and writes
-// their order, as positions `base` and on, and, of segment 0, the block that holds key 0.
-template <int NPL>
-__device__ __forceinline__ void sort_and_store(double (&k)[NPL], int lane, int seg, int base, int s, int32_t* out, int32_t* first_blk, int block_size) {
-  wave_sort<NPL>(k, lane);
-  const int at = lane * NPL;   // a segment is a multiple of the block size or not: the last lanes may hold padding
-  int32_t o[NPL];
-  int zero_at = -1;
-#pragma unroll
-  for (int r = 0; r < NPL; ++r) {
-    const uint32_t i = sort_key_index(k[r]);
-    zero_at = i == 0 ? at + r : zero_at;
-    o[r] = base + (int32_t)i;
-  }
-  if (first_blk && s == 0 && zero_at >= 0) *first_blk = zero_at / block_size;
-  if (NPL >= 4 && (seg & 3) == 0 && ((uintptr_t)out & 15) == 0) {
-    typedef __attribute__((ext_vector_type(4))) int32_t i32x4;
-#pragma unroll
-    for (int r = 0; r < NPL; r += 4)
-      if (at + r < seg) *reinterpret_cast<i32x4*>(out + at + r) = (i32x4){o[r], o[(r + 1) % NPL], o[(r + 2) % NPL], o[(r + 3) % NPL]};
-  } else {
-#pragma unroll
-    for (int r = 0; r < NPL; ++r)
-      if (at + r < seg) out[at + r] = o[r];
-  }
-}
 // ---- a workgroup ranks the keys of a segment of up to 256: `keys` (LDS, 16-byte aligned) are its sort keys, and the place of the one
 // that is `own` is the number of smaller ones.  Quadratic, a comparison and an addition with carry per pair, and yet the shorter chain where
 // a workgroup waits for its order (a segment of 256 by one wave's network -> this, whole pass: 28 / 4 heads x 1000 55.8 -> 52.9 us, 32 / 8 x 4096

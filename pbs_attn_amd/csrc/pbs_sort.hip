@@ -35,6 +35,33 @@ __global__ __launch_bounds__(256) void segment_argsort_kernel(const float* score
       if ((uint32_t)keys[i] == 0) first_blk[row] = i / block_size;
 }
 
+// Sorts the wave's keys of segment `s` of a row (`seg` of them; register r of lane l starts with that of local index 64 r + l) and writes
+// their order, as positions `base` and on, and, of segment 0, the block that holds key 0.
+template <int NPL>
+__device__ __forceinline__ void sort_and_store(double (&k)[NPL], int lane, int seg, int base, int s, int32_t* out, int32_t* first_blk, int block_size) {
+  wave_sort<NPL>(k, lane);
+  const int at = lane * NPL;   // a segment is a multiple of the block size or not: the last lanes may hold padding
+  int32_t o[NPL];
+  int zero_at = -1;
+#pragma unroll
+  for (int r = 0; r < NPL; ++r) {
+    const uint32_t i = sort_key_index(k[r]);
+    zero_at = i == 0 ? at + r : zero_at;
+    o[r] = base + (int32_t)i;
+  }
+  if (first_blk && s == 0 && zero_at >= 0) *first_blk = zero_at / block_size;
+  if (NPL >= 4 && (seg & 3) == 0 && ((uintptr_t)out & 15) == 0) {
+    typedef __attribute__((ext_vector_type(4))) int32_t i32x4;
+#pragma unroll
+    for (int r = 0; r < NPL; r += 4)
+      if (at + r < seg) *reinterpret_cast<i32x4*>(out + at + r) = (i32x4){o[r], o[(r + 1) % NPL], o[(r + 2) % NPL], o[(r + 3) % NPL]};
+  } else {
+#pragma unroll
+    for (int r = 0; r < NPL; ++r)
+      if (at + r < seg) out[at + r] = o[r];
+  }
+}
+
 // The workgroups behind the first `sort_wgs` do the ride's pooling: the sort waits on its lanes and leaves the memory idle.
 // Whole pass, pooling with the key blocks -> here, us: 32 / 8 heads x 20000 in segments of 2048 671 -> 654, 16 / 16 x 60000 875 -> 868, 28 / 4 x
 // 13333 twice 778 -> 776.  (In the first pass of the split scoring, which leaves half of a CU free, it took more than it saved: 16 / 16 x

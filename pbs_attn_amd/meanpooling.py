@@ -44,7 +44,7 @@ def MeanPooling_prefill(
     if (force_select_current_block and not return_masks and block_size == ops.BLOCK
             and s_pad // block_size <= ops.MEANPOOLING_MAX_BLOCKS):
         # the whole mode in one library call (the stage-by-stage form below gives the same bits): 32 / 8 heads x 128
-        # 76 -> 22 us, x 4096 156 -> 125, x 16384 1.54 -> 1.46 ms, x 32768 5.78 -> 5.57
+        # 75 -> 13 us, x 4096 155 -> 126, x 16384 1.54 -> 1.50 ms, x 32768 5.80 -> 5.74
         return ops.meanpooling_attn_fwd(query_states, key_states, value_states, thr, force_select_first_block)
     idx = torch.arange(s_pad, dtype=torch.int32, device=query_states.device).view(1, 1, -1)
     idx = idx.expand(batch_size, num_q_heads, -1).contiguous()
