@@ -156,12 +156,12 @@ struct TaskGroups {
   dim3 grid;
 };
 
-__host__ inline TaskGroups task_groups(int B, int Hq, int Hkv, int nb, int kinds) {
+__host__ inline TaskGroups task_groups(int B, int Hq, int Hkv, int nb, int kinds, int blocks_each = 1) {
   TaskGroups t;
   t.n_chunks = (nb + CHUNK - 1) / CHUNK;
   t.n_groups = B * Hkv * t.n_chunks;
   t.G = Hq / Hkv;
-  t.grid = dim3(8, (unsigned)(kinds * t.G * CHUNK), (unsigned)((t.n_groups + 7) / 8));
+  t.grid = dim3(8, (unsigned)(kinds * t.G * CHUNK / blocks_each), (unsigned)((t.n_groups + 7) / 8));
   return t;
 }
 
@@ -175,6 +175,34 @@ __device__ __forceinline__ bool my_task(const TaskGroups& t, int nb, int& kind, 
   blk = chunk * CHUNK + (mm & (CHUNK - 1));
   bh = bkv * t.G + mm / CHUNK;   // (b * Hkv + kvh) * G + head in group == b * Hq + h
   return tg < t.n_groups && blk < nb;
+}
+
+// A filtered gather of a long call, where most workgroups would find their block unvisited and handing them out is the launch's time: a workgroup
+// looks after FEW blocks of a head, one after the other.  Whole pass, a workgroup a block -> this, us: concentrated 2 x 32 / 8 heads x 65536 3211 -> 3155,
+// 4 x 28 / 4 x 40000 5567 -> 5472, 32 / 8 x 131072 2952 -> 2950, 4 x 32 / 8 x 32768 3413 -> 3384; a twelfth of the blocks visited (strong_uniform) 32 / 8 x 131072
+// 7798 -> 7736, 4 x 28 / 4 x 40000 8209 -> 8046; near-uniform, inside the spread, 4 x 32 / 8 x 32768 23.41 -> 23.38 ms, 2 x 28 / 4 x 80000 57.55 -> 57.70.
+// In calls of fewer blocks its workgroups, a quarter as many and up to four times as long, end in a last wave that weighs: from 16384 blocks on
+// near-uniform 4 x 32 / 8 x 16384 6508 against 6558, strong_uniform 4 x 28 / 4 x 20000 2269 against 2284 and 28 / 4 x 100000 6212 against 6234, for concentrated 4 x 32 / 8 x
+// 16384 1925 -> 1879, 2 x 32 / 8 x 32768 1615 -> 1605 and 8 / 2 x 262144 6822 -> 6791.
+constexpr int FEW = 4, FEW_EACH_BLOCKS = 32768;
+__global__ __launch_bounds__(256) void gather_needed_kernel(GatherArgs a, TaskGroups t) {
+  __shared__ uint16_t vt[BS * VT_PITCH];
+  __shared__ float pool[16][D];
+  const int tg = blockIdx.z * 8 + blockIdx.x, m = blockIdx.y;
+  if (tg >= t.n_groups) return;
+  const int bkv = tg / t.n_chunks, chunk = tg - bkv * t.n_chunks;
+  const int first = chunk * CHUNK + m % (CHUNK / FEW) * FEW, bh = bkv * t.G + m / (CHUNK / FEW);
+  uint32_t wanted = 0;
+#pragma unroll
+  for (int x = 0; x < FEW; ++x)
+    if (first + x < a.nb && a.needed[(int64_t)bh * a.nb + first + x]) wanted |= 1u << x;
+  wanted = __builtin_amdgcn_readfirstlane(wanted);
+  while (wanted) {
+    const int x = __builtin_ctz(wanted);
+    wanted &= wanted - 1;
+    gather_block<false>(a, vt, pool, first + x, bh);
+    if (wanted) __syncthreads();   // the staged rows have been read
+  }
 }
 
 template <bool POOL_ONLY>
@@ -314,8 +342,13 @@ extern "C" int pbs_gather_kv(const void* k, const void* v, const int32_t* key_in
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.S = S; a.nb = (S + BS - 1) / BS;
   a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = k_ss; a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = v_ss;
   a.pool_max = key_pool_max;
-  const TaskGroups t = task_groups(B, Hq, Hkv, a.nb, 1);
-  PBS_REQUIRE(t.grid.y <= 65535 && t.grid.z <= 65535, "pbs_gather_kv: too many heads or blocks");
+  const bool few_each = block_needed && (int64_t)B * Hq * a.nb >= FEW_EACH_BLOCKS;
+  const TaskGroups t = task_groups(B, Hq, Hkv, a.nb, 1, few_each ? FEW : 1);
+  PBS_REQUIRE(Hq / Hkv * CHUNK <= 65535 && t.grid.z <= 65535, "pbs_gather_kv: too many heads or blocks");
+  if (few_each) {
+    hipLaunchKernelGGL(gather_needed_kernel, t.grid, dim3(256), 0, (hipStream_t)stream, a, t);
+    return pbs_check_launch("pbs_gather_kv");
+  }
   hipLaunchKernelGGL(gather_kv_kernel<false>, t.grid, dim3(256), 0, (hipStream_t)stream, a, t);
   return pbs_check_launch("pbs_gather_kv");
 }

@@ -1,9 +1,9 @@
-"""GPU: the filtered gather of long calls against the unfiltered one: marked tiles bit for bit, the others untouched."""
+"""GPU: the filtered gather against the unfiltered one, on both sides of the 32768 blocks from which on a workgroup takes four of a head: marked tiles bit
+for bit, the others untouched."""
 import pytest
 import torch
 
 from pbs_attn_amd import _lib, ops
-from tests.util import small_case
 
 pytestmark = pytest.mark.gpu
 
@@ -11,13 +11,14 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,Hq,Hkv,S", [
     (8, 64, 8, 33 * 128 - 5),      # an odd number of blocks a head, the last one ragged: chunks of one block
     (1, 512, 512, 32 * 128),       # a head a group, whole chunks
+    (8, 128, 8, 33 * 128 - 5), (1, 1024, 1024, 32 * 128), (3, 56, 8, 196 * 128 + 1),   # the same of four a workgroup: 33792 blocks, 32768, 33096
     (3, 28, 4, 196 * 128 + 1),     # seven heads a group
 ])
 @pytest.mark.parametrize("share", [0.0, 0.03, 0.6, 1.0])
 def test_against_the_unfiltered_gather(dev, B, Hq, Hkv, S, share):
     nb = (S + 127) // 128
-    _, k, v = (x.to(dev) for x in small_case(B, Hkv, Hkv, S, seed=S))
     g = torch.Generator(device=dev).manual_seed(S)
+    k, v = (torch.randn(B, Hkv, S, 128, device=dev, generator=g).bfloat16() for _ in "kv")
     idx = torch.rand(B, Hq, S, device=dev, generator=g).argsort(-1).to(torch.int32)
     idx = torch.cat((idx, torch.arange(S, nb * 128, device=dev, dtype=torch.int32).expand(B, Hq, -1)), -1).contiguous()
     needed = (torch.rand(B, Hq, nb, device=dev, generator=g) < share).to(torch.uint8)

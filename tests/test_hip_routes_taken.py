@@ -15,6 +15,7 @@ SCORES = ["score_kernel", "score_kernel"]
 REST = ["estimate_select_kernel", "sparse_attn_kernel"]
 GATHER_SORTS = SCORES + ["sort_gather_pool_kernel"] + REST
 PASS_SORTS = SCORES + ["gather_pool_kernel"] + REST
+LONG = ["score_kernel", "score_reduce_kernel", "score_kernel", "segment_argsort_wave_kernel", "pool_qk_kernel", "block_logits_softmax_kernel", "select_pair_lists_kernel"]
 KERNEL_SORTS = SCORES + ["segment_argsort_wave_kernel", "gather_pool_kernel"] + REST
 
 
@@ -43,6 +44,8 @@ def _kernels(call):
     (1, 32, 8, 64 * 128, 256, 0.9, ["score_kernel", "score_reduce_kernel", "score_kernel"] + GATHER_SORTS[2:]),
     (1, 33, 11, 64 * 128, 256, 0.9, SCORES + ["segment_argsort_wave_kernel", "gather_kv_kernel", "block_logits_softmax_kernel",   # three heads a group: the split
                                               "select_pair_lists_kernel", "gather_kv_kernel", "sparse_attn_kernel"]),             # scoring, without a reduction
+    # the filtered gather: from 32768 blocks on four a workgroup
+    (1, 1024, 8, 32 * 128, 1024, 0.9, LONG + ["gather_needed_kernel", "sparse_attn_kernel"]), (1, 1016, 8, 32 * 128, 1024, 0.9, LONG + ["gather_kv_kernel", "sparse_attn_kernel"]),
 ])
 def test_prefill(dev, B, Hq, Hkv, S, seg, thr, kernels):
     q, k, v = (x.to(dev) for x in small_case(B, Hq, Hkv, S, seed=S))
