@@ -183,8 +183,11 @@ __device__ __forceinline__ bool my_task(const TaskGroups& t, int nb, int& kind, 
 // 7798 -> 7736, 4 x 28 / 4 x 40000 8209 -> 8046; near-uniform, inside the spread, 4 x 32 / 8 x 32768 23.41 -> 23.38 ms, 2 x 28 / 4 x 80000 57.55 -> 57.70.
 // In calls of fewer blocks its workgroups, a quarter as many and up to four times as long, end in a last wave that weighs: from 16384 blocks on
 // near-uniform 4 x 32 / 8 x 16384 6508 against 6558, strong_uniform 4 x 28 / 4 x 20000 2269 against 2284 and 28 / 4 x 100000 6212 against 6234, for concentrated 4 x 32 / 8 x
-// 16384 1925 -> 1879, 2 x 32 / 8 x 32768 1615 -> 1605 and 8 / 2 x 262144 6822 -> 6791.
-constexpr int FEW = 4, FEW_EACH_BLOCKS = 32768;
+// 16384 1925 -> 1879 and 2 x 32 / 8 x 32768 1615 -> 1605.
+// (The more blocks a row has, the less the gather weighs beside the attention: rows of more than 1024 lose nothing from 16384 blocks on.  strong_uniform 8 / 2 x
+// 262144 6769 -> 6747, 28 / 4 x 140000 8171 -> 8134, 14 / 2 x 160000 5675 -> 5647; near-uniform 8 / 2 x 262144 83.62 -> 83.68 ms, 16 / 16 x 131200 43.60 -> 43.64, inside the spread.)
+constexpr int FEW = 4, LONG_ROW = 1024;
+bool few_each(int64_t blocks, int nb) { return blocks >= (nb > LONG_ROW ? 16384 : 32768); }
 __global__ __launch_bounds__(256) void gather_needed_kernel(GatherArgs a, TaskGroups t) {
   __shared__ uint16_t vt[BS * VT_PITCH];
   __shared__ float pool[16][D];
@@ -342,10 +345,10 @@ extern "C" int pbs_gather_kv(const void* k, const void* v, const int32_t* key_in
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.S = S; a.nb = (S + BS - 1) / BS;
   a.k_sb = k_sb; a.k_sh = k_sh; a.k_ss = k_ss; a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = v_ss;
   a.pool_max = key_pool_max;
-  const bool few_each = block_needed && (int64_t)B * Hq * a.nb >= FEW_EACH_BLOCKS;
-  const TaskGroups t = task_groups(B, Hq, Hkv, a.nb, 1, few_each ? FEW : 1);
+  const bool few = block_needed && few_each((int64_t)B * Hq * a.nb, a.nb);
+  const TaskGroups t = task_groups(B, Hq, Hkv, a.nb, 1, few ? FEW : 1);
   PBS_REQUIRE(Hq / Hkv * CHUNK <= 65535 && t.grid.z <= 65535, "pbs_gather_kv: too many heads or blocks");
-  if (few_each) {
+  if (few) {
     hipLaunchKernelGGL(gather_needed_kernel, t.grid, dim3(256), 0, (hipStream_t)stream, a, t);
     return pbs_check_launch("pbs_gather_kv");
   }
