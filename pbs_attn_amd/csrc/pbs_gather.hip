@@ -295,6 +295,20 @@ __global__ __launch_bounds__(256) void sort_gather_pool_kernel(GatherArgs a, Poo
 
 }  // namespace
 
+int pbs_sorts_of_an_engine(int B, int Hq, int Hkv, int nb, int sorted_blocks) {
+  const int kv_heads = B * Hkv, n_chunks = (nb + CHUNK - 1) / CHUNK;
+  int load[8] = {}, most = 0;
+  for (int r = 0; r < 8; ++r)   // KV heads r, r + 8, ...: the task groups of their chunk c go to XCD (r * n_chunks + c) % 8
+    for (int c = 0; c < n_chunks; ++c) {
+      const int sorted = sorted_blocks - c * CHUNK;   // block m of a chunk goes to engine m % 4
+      if (sorted <= 0) break;
+      int& l = load[(r * n_chunks + c) & 7];
+      l += (kv_heads + 7 - r) / 8 * (Hq / Hkv) * (sorted >= CHUNK ? CHUNK / 4 : (sorted + 3) / 4);
+      if (l > most) most = l;
+    }
+  return most;
+}
+
 int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const int32_t* key_indices, void* pooled_q, void* pooled_k,
                            void* perm_k, void* perm_vt, int B, int Hq, int Hkv, int S, int head_dim, int block_size, int64_t q_sb,
                            int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,

@@ -82,6 +82,9 @@ struct SegmentScores {
   int Sc, seg;
 };
 constexpr int PBS_SORT_IN_GATHER_KEYS = 1024, PBS_RANKED_KEYS = 256;   // (up to the latter a workgroup ranks them)
+// The sorting workgroups of that launch on the shader engine that gets the most of them, where a row's first `sorted_blocks` blocks are sorted
+// (the launch goes round the eight XCDs, and inside one round its four engines)
+int pbs_sorts_of_an_engine(int B, int Hq, int Hkv, int nb, int sorted_blocks);
 // pbs_pool_blocks and an unfiltered pbs_gather_kv in one launch (the pooled key blocks have the bits of both), by key_indices or, for
 // segments of up to PBS_SORT_IN_GATHER_KEYS keys, by the order of `scores`
 int pbs_gather_pool_launch(const void* q, const void* k, const void* v, const int32_t* key_indices, void* pooled_q, void* pooled_k,

@@ -25,12 +25,17 @@ bool short_pass(int rows, int nb) { return nb <= SHORT_PASS_ROW && rows * nb <= 
 // routes win: 32 x 8 / 2 x 300 79.5 against 80.6, 16 x 32 / 8 x 200 of 128 88.7 against 91.4.  Where the final scoring pass could sort: 28 / 4 x 3400 of 256
 // 124.2 -> 121.3, 32 / 8 x 4096 162.4 -> 160.6, but not where a segment is less than what its workgroups take otherwise, so that it gains workgroups by
 // sorting (4 / 1 x 6000 of 128 106.9 against 109.6).
-// Longer ones, by the first wave, as long as the gathering workgroups are in flight at once, three a CU: 28 / 4 x 1100 of 512 66.7 -> 62.7; 32 / 8 x 2200 of
-// 1024 110.7 -> 105.4, x 3000 (768 blocks) 133.8 -> 129.1, x 3500 (896) 159.5 against 168.7; 28 / 4 x 2500 of 2048, thirty-two keys a lane, 126 against 147.
-constexpr int SORT_IN_GATHER_BLOCKS = 3 * 256, RANK_IN_GATHER_HEADS = 255;
-bool sorts_in_gather(int rows, int nb, int segment_size, int score_sort_chunk) {
-  if (segment_size <= PBS_RANKED_KEYS) return rows <= RANK_IN_GATHER_HEADS && score_sort_chunk <= segment_size;
-  return segment_size <= PBS_SORT_IN_GATHER_KEYS && rows * nb <= SORT_IN_GATHER_BLOCKS;
+// Longer ones, by the first wave, as long as the sorting workgroups are in flight at once: a segment's blocks all sort it, so that a second round of them is another
+// sort behind the first.  Three run on a CU, twenty-four on a shader engine of eight, and the launch deals them to the engines in a fixed order, which short rows fill
+// unevenly (pbs_sorts_of_an_engine).  Up to 24 on the fullest, us: 28 / 4 x 1100 of 512 66.7 -> 62.7; 32 / 8 x 2200 of 1024 110.7 -> 105.4, x 3000 133.8 -> 129.1; 365 shapes of up to
+// 768 blocks 1.00 to 1.08 times as fast.  27 and more: 28 / 4 x 2139 of 640 104.6 against 112.4, 2 x 32 / 8 x 1115 of 1024 96.2 against 105.2, 4 x 16 / 16 x 1115 of 512 94.3
+// against 97.2; 116 shapes 0.90 to 1.00.  Thirty-two keys a lane: 28 / 4 x 2500 of 2048 126 against 147.
+constexpr int SORT_IN_GATHER_BLOCKS = 3 * 256, SORTS_OF_AN_ENGINE = 3 * 8, RANK_IN_GATHER_HEADS = 255;
+bool sorts_in_gather(int B, int Hq, int Hkv, int S, int block_size, int segment_size, int score_sort_chunk) {
+  if (segment_size <= PBS_RANKED_KEYS) return B * Hq <= RANK_IN_GATHER_HEADS && score_sort_chunk <= segment_size;
+  const int nb = (S + block_size - 1) / block_size;
+  return segment_size <= PBS_SORT_IN_GATHER_KEYS && B * Hq * nb <= SORT_IN_GATHER_BLOCKS &&
+         pbs_sorts_of_an_engine(B, Hq, Hkv, nb, S / segment_size * (segment_size / block_size)) <= SORTS_OF_AN_ENGINE;
 }
 
 // Sort with the query pooling + key pooling, against sort + both poolings, us: 32768 tokens, 32 / 8 heads 52 + 23 against 20 + 60; 13333 tokens twice
@@ -158,7 +163,7 @@ extern "C" int pbs_prefill_attn_fwd(const void* q, const void* k, const void* v,
   bool q_pooled = false;   // the query blocks' pooling is under way
   if (one_segment || nseg == 0 || (nseg == 1 && rem == 0)) {
     if ((rc = pbs_identity_indices((int32_t*)(w + L.idx), rows, s_pad, stream))) return rc;
-  } else if (is_short && sorts_in_gather(rows, nb, segment_size, pbs_score_sort_chunk(B, Hq, Hkv, S, segment_size))) {
+  } else if (is_short && sorts_in_gather(B, Hq, Hkv, S, block_size, segment_size, pbs_score_sort_chunk(B, Hq, Hkv, S, segment_size))) {
     scores = {(const float*)(w + L.scores), (int32_t*)(w + L.select_ws), nseg * segment_size, segment_size};
     if ((rc = pbs_score_keys(q, k, (float*)(w + L.scores), B, Hq, Hkv, S, head_dim, block_size, segment_size, q_sb, q_sh,
                              q_ss, k_sb, k_sh, k_ss, w + L.score_ws, L.idx - L.score_ws, stream))) return rc;

@@ -37,8 +37,10 @@ def _kernels(call):
     # the gather sorts: ranks up to 256 keys and 255 heads, where the scoring pass would take no more keys than a segment
     (1, 28, 4, 1000, 256, 0.9, GATHER_SORTS), (1, 255, 51, 300, 128, 0.9, GATHER_SORTS), (1, 256, 64, 300, 128, 0.9, PASS_SORTS),
     (1, 4, 1, 6000, 256, 0.9, GATHER_SORTS), (1, 4, 1, 6000, 128, 0.9, PASS_SORTS),
-    # longer segments: up to 1024 keys and 768 blocks
+    # longer segments: up to 1024 keys, 768 blocks and 24 sorting workgroups on a shader engine
     (1, 32, 8, 24 * 128, 512, 0.9, GATHER_SORTS), (1, 33, 11, 24 * 128, 512, 0.9, KERNEL_SORTS),
+    (1, 32, 8, 18 * 128, 1024, 0.9, GATHER_SORTS), (2, 32, 8, 9 * 128, 1024, 0.9, KERNEL_SORTS), (1, 28, 4, 20 * 128, 1024, 0.9, KERNEL_SORTS),   # 24; 32; 28
+    (4, 28, 4, 6 * 128, 512, 0.9, GATHER_SORTS), (4, 28, 4, 6 * 128, 640, 0.9, KERNEL_SORTS),                                             # 14; 28, five blocks of a chunk
     (1, 2, 1, 2 * 1024 + 128, 1024, 0.9, GATHER_SORTS), (1, 2, 1, 3 * 1152 + 1, 1152, 0.9, KERNEL_SORTS),
     # short passes: up to 2048 blocks, 64 a row
     (1, 32, 8, 64 * 128, 256, 0.9, ["score_kernel", "score_reduce_kernel", "score_kernel"] + GATHER_SORTS[2:]),
