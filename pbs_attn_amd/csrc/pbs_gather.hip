@@ -178,14 +178,14 @@ __device__ __forceinline__ bool my_task(const TaskGroups& t, int nb, int& kind, 
 }
 
 // A filtered gather of a long call, where most workgroups would find their block unvisited and handing them out is the launch's time: a workgroup
-// looks after FEW blocks of a head, one after the other.  Whole pass, a workgroup a block -> this, us: concentrated 2 x 32 / 8 heads x 65536 3211 -> 3155,
-// 4 x 28 / 4 x 40000 5567 -> 5472, 32 / 8 x 131072 2952 -> 2950, 4 x 32 / 8 x 32768 3413 -> 3384; a twelfth of the blocks visited (strong_uniform) 32 / 8 x 131072
-// 7798 -> 7736, 4 x 28 / 4 x 40000 8209 -> 8046; near-uniform, inside the spread, 4 x 32 / 8 x 32768 23.41 -> 23.38 ms, 2 x 28 / 4 x 80000 57.55 -> 57.70.
+// looks after FEW blocks of a head, one after the other.  Whole pass, a workgroup a block -> this, us, both in turn and each first once: concentrated 2 x 32 / 8 heads
+// x 65536 3103 -> 3079, 4 x 28 / 4 x 40000 5497 -> 5415, 4 x 32 / 8 x 32768 3345 -> 3320, 32 / 8 x 131072 2881 -> 2880; a twelfth of the blocks visited (strong_uniform) 32 / 8 x
+// 131072 7739 -> 7686, 4 x 28 / 4 x 40000 8158 -> 7983; near-uniform 4 x 32 / 8 x 32768 and 2 x 28 / 4 x 80000 the same within 0.1 %.
 // In calls of fewer blocks its workgroups, a quarter as many and up to four times as long, end in a last wave that weighs: from 16384 blocks on
-// near-uniform 4 x 32 / 8 x 16384 6508 against 6558, strong_uniform 4 x 28 / 4 x 20000 2269 against 2284 and 28 / 4 x 100000 6212 against 6234, for concentrated 4 x 32 / 8 x
-// 16384 1925 -> 1879 and 2 x 32 / 8 x 32768 1615 -> 1605.
+// near-uniform 4 x 32 / 8 x 16384 6493 against 6545, strong_uniform 4 x 28 / 4 x 20000 2096 against 2103 and 28 / 4 x 100000 5976 against 5990, for concentrated 4 x 32 / 8 x
+// 16384 1875 -> 1854 and strong_uniform 2 x 32 / 8 x 32768 1771 -> 1761.
 // (The more blocks a row has, the less the gather weighs beside the attention: rows of more than 1024 lose nothing from 16384 blocks on.  strong_uniform 8 / 2 x
-// 262144 6769 -> 6747, 28 / 4 x 140000 8171 -> 8134, 14 / 2 x 160000 5675 -> 5647; near-uniform 8 / 2 x 262144 83.62 -> 83.68 ms, 16 / 16 x 131200 43.60 -> 43.64, inside the spread.)
+// 262144 6801 -> 6771, 28 / 4 x 140000 8147 -> 8106, 14 / 2 x 160000 5628 -> 5608; near-uniform 8 / 2 x 262144 83.62 -> 83.68 ms, 16 / 16 x 131200 43.60 -> 43.64, inside the spread.)
 constexpr int FEW = 4, LONG_ROW = 1024;
 bool few_each(int64_t blocks, int nb) { return blocks >= (nb > LONG_ROW ? 16384 : 32768); }
 __global__ __launch_bounds__(256) void gather_needed_kernel(GatherArgs a, TaskGroups t) {
