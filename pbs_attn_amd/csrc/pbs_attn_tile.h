@@ -306,8 +306,11 @@ constexpr int COPY_FIRST_GAP = 2;
 // A piece of the next tile's copy every so many matrix instructions: all of them are on their way before the middle of a tile, which leaves its second
 // half to the memory's latency.  In a tile of two column groups pieces 8 apart end with the tile, and its wait was a round trip to L2: passes of single
 // blocks, 8 apart -> 4, 4 / 1 heads x 8192 96.3 -> 92.0 us, 129.1 -> 124.3 in segments of 128, 8 / 2 x 2048 60.5 -> 59.2, 28 / 4 x 1000 53.5 -> 52.7;
-// 3 apart 93.7, 127.7, 59.7 and 52.8, 2 apart no better than 8.
-constexpr int copy_gap_step(int nq) { return 2 * nq; }
+// 3 apart 93.7, 127.7, 59.7 and 52.8, 2 apart no better than 8; rows of few selected blocks, 8 / 2 x 142981 in segments of 2048 2193 -> 2112.
+// The second block's diagonal tile, a pair's last, keeps 8: its copies, the next item's first tile, follow that item's sixteen query loads and hold up
+// what is behind them.  4 apart there -> 8: inside one segment 4 x 16 / 16 x 1152 41.0 -> 40.0 us, 2 x 32 / 8 x 1152 40.4 -> 39.5; 28 / 4 x 1000 in segments of 256 52.3 -> 51.8,
+// 32 / 8 x 32768 concentrated 826.5 -> 822.5, x 131072 2668 -> 2643.
+constexpr int copy_gap_step(int nq, bool ends_pair) { return nq == 2 && !ends_pair ? 4 : 8; }
 // NQ: the column groups the tile is worked on for, four or (a tile that only one of the pair's blocks sees) two
 template <int NQ>
 struct TileSchedule {
@@ -418,7 +421,7 @@ constexpr int check_schedule() {
     if (s.read_after[f] >= 0 && s.first_use[f] < s.read_after[f] + 6) return 5;
     if (f >= FRAG_BUFS && s.read_after[f] < s.last_use[f - FRAG_BUFS]) return 6;
   }
-  if (s.unit_gap(8 * NQ - 1, 6) >= s.N_MFMA || COPY_FIRST_GAP + 15 * copy_gap_step(NQ) >= s.N_MFMA) return 7;
+  if (s.unit_gap(8 * NQ - 1, 6) >= s.N_MFMA || COPY_FIRST_GAP + 15 * copy_gap_step(NQ, true) >= s.N_MFMA) return 7;
   return 0;
 }
 static_assert(check_schedule<4>() == 0 && check_schedule<2>() == 0, "tile schedule");
@@ -535,7 +538,7 @@ __device__ __forceinline__ void fast_tile(const uint32_t (&ka)[4], const uint32_
       __builtin_amdgcn_sched_barrier(0);
     }
     read_frag(std::integral_constant<int, frag_read_after<NQ>(i)>{});
-    constexpr int past = i - COPY_FIRST_GAP, step = copy_gap_step(NQ);
+    constexpr int past = i - COPY_FIRST_GAP, step = copy_gap_step(NQ, MASKED == 12);
     if constexpr (COPIES && past >= 0 && past % step == 0 && past / step < 16) {
       copy_piece<past / step>(copy);
       __builtin_amdgcn_sched_barrier(0);
